@@ -1,4 +1,4 @@
-"""Build recipe for libnmg_hip.so (hipcc, gfx950 only).  Run as ``python -m sten_amd.build``."""
+"""Build recipe for libnmg_hip.so (hipcc, gfx950 only) and the host path.  Run as ``python -m sten_amd.build``."""
 import os
 import subprocess
 import sys
@@ -11,11 +11,30 @@ SOURCES = ["nmg_runtime.hip", "nmg_sparsify.hip", "nmg_spmm.hip", "nmg_smfmac.hi
 # bench.py's measurement aid: a library of its own, outside the product ABI
 PROBE_LIB = os.path.join(HERE, "libnmg_probe.so")
 PROBE_SOURCES = ["nmg_probe.hip"]
+# the native host path: an extension module against torch's libraries, linked to LIB
+HOST_LIB = os.path.join(HERE, "_host.so")
+HOST_SOURCE = "nmg_host.cpp"
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option",
 ]
+
+
+def build_host(verbose=False):
+    """Compile the host path (no device code) and link it against torch and the library beside it."""
+    import sysconfig
+
+    from torch.utils.cpp_extension import include_paths, library_paths
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
+           "-I" + sysconfig.get_paths()["include"]]
+    cmd += ["-isystem" + p for p in include_paths() + ["/opt/rocm/include"]]
+    cmd += [os.path.join(CSRC, HOST_SOURCE), "-o", HOST_LIB, "-L" + HERE, "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN"]
+    cmd += ["-L" + p for p in library_paths()] + ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), file=sys.stderr)
+    subprocess.run(cmd, check=True)
+    return HOST_LIB
 
 
 def build(verbose=False, jobs=8, check=True):
@@ -42,6 +61,7 @@ def build(verbose=False, jobs=8, check=True):
     subprocess.run(cmd, check=True)
     probe_objs = [os.path.join(objdir, src.replace(".hip", ".o")) for src in PROBE_SOURCES]
     subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + probe_objs + ["-o", PROBE_LIB], check=True)
+    build_host(verbose)
     if check:
         from . import isa_check
         if isa_check.main([]) != 0:

@@ -1,0 +1,1258 @@
+// Host path of the grouped n:m products: operand caches, choice of the route, allocation of results
+// and workspaces, launch.  A product of a few tokens keeps the GPU busy for 7 to 15 us; the same
+// steps in Python (attribute look-ups, ctypes conversions, the generic dispatcher) took 24 to 37 us
+// per call, so they bounded every small product whatever its kernel did.  Built as the extension
+// module sten_amd._host and linked against libnmg_hip.so, whose C ABI stays the only way to a kernel.
+//
+// Everything here runs with the GIL held (nothing blocks); that is what makes the operand caches safe
+// with several threads.
+#include <Python.h>
+#include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/LegacyTypeDispatch.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <map>
+#include <sstream>
+#include <stdexcept>
+#include <string>
+#include <vector>
+
+#include "../../include/nmg_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+PyObject *g_nmg_error = nullptr;      // sten_amd.native.NmgError
+
+struct NmgError : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
+template <typename... A>
+[[noreturn]] void fail(const A &...parts)
+{
+    std::ostringstream s;
+    (s << ... << parts);
+    throw NmgError(s.str());
+}
+
+void check(int rc)
+{
+    if (rc != NMG_OK) fail("nmg call failed with status ", rc, ": ", nmg_last_error());
+}
+
+#define HOST_TRY try {
+#define HOST_CATCH(ret)                                                       \
+    }                                                                         \
+    catch (const NmgError &e) { PyErr_SetString(g_nmg_error, e.what()); return ret; } \
+    catch (python_error &e) { e.restore(); return ret; }                      \
+    catch (const c10::Error &e) { PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace()); return ret; } \
+    catch (const std::exception &e) { PyErr_SetString(PyExc_RuntimeError, e.what()); return ret; }
+
+// ---------------------------------------------------------------------------------- small helpers
+
+struct Text {
+    PyObject *kernel, *variant, *dense_variant, *slices, *expand, *cache_dense, *container, *dense_shape, *B, *s, *meta;
+} S_;
+
+int dtype_code(at::ScalarType t)
+{
+    switch (t) {
+    case at::kFloat: return NMG_F32;
+    case at::kHalf: return NMG_F16;
+    case at::kBFloat16: return NMG_BF16;
+    case at::kDouble: return NMG_F64;
+    default: fail("unsupported dtype ", t);
+    }
+}
+
+bool is16(const Tensor &t) { return t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16; }
+
+void require_gpu(const Tensor &t)
+{
+    if (!t.is_cuda())
+        fail("nmg kernels run on the GPU only; got a tensor on ", t.device(), " (move the tensor to an MI355X device)");
+}
+
+void *stream_of(const Tensor &t) { return (void *)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+Tensor new_empty(at::IntArrayRef size, const Tensor &like) { return at::empty(size, like.options()); }
+Tensor new_empty(at::IntArrayRef size, const Tensor &like, at::ScalarType dt) { return at::empty(size, like.options().dtype(dt)); }
+
+bool aligned16(const Tensor &t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+constexpr int64_t k2G = int64_t(1) << 31;
+constexpr int64_t kOstreamMaxTokens = 4;    // nmg_spmm_ostream: the token rows its lanes hold
+constexpr int64_t kOstreamAutoTokens = 2;   // ... and up to where it is ahead of the sliced kernel (4096 x 11008: 12.4 / 13.3 / 16.2 against 15.9 / 16.0 / 16.3 us at 1 / 2 / 3 tokens)
+constexpr int64_t kGstreamMaxTokens = 16;   // nmg_spmm_gstream: tokens up to which the stream of the weight bounds the product
+constexpr int64_t kF32GemmMaxTokens = 65535 * 32;   // one launch of the fp32 GEMM: token tiles of 32 in grid.y
+
+// ------------------------------------------------------------------------------- the tensor's core
+
+struct Geometry {
+    int nd = 0, n = 0, m = 0, g = 0, sdim = 0, gdim = 0;
+    std::vector<int64_t> dims;
+    int64_t G = 0, S = 0, nb = 0, cols = 0, chunks = 0;
+};
+
+// What is derived from val and idx for the products; dropped when either changes.
+struct Operands {
+    bool valid = false;
+    uint32_t val_version = 0, idx_version = 0;
+    Tensor pk_val, pk_pat, fp_val, fp_idx;      // rowpack, and fragpack where the pattern has one
+    Tensor frag[2];                             // densefrag per reduction direction
+    std::map<int64_t, Tensor> dense[2];         // dense copies per reduction direction, by row pitch
+    Tensor lp_val, lp_pat, gp, op;              // operands of the streamed few-token products
+};
+
+struct State {
+    Tensor val, idx;
+    PyObject *layout = nullptr, *opt = nullptr;
+    Geometry geo;
+    Operands ops;
+    bool slot_valid = false;
+    uint32_t slot_version = 0;
+    Tensor slot;
+};
+
+struct Core {
+    PyObject_HEAD
+    State *st;
+};
+
+PyTypeObject CoreType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+State &state_of(PyObject *o)
+{
+    if (!PyObject_TypeCheck(o, &CoreType)) fail("expected a GroupedNMTensor, got ", Py_TYPE(o)->tp_name);
+    return *reinterpret_cast<Core *>(o)->st;
+}
+
+State &matmul_state(PyObject *o)
+{
+    State &w = state_of(o);
+    if (w.geo.nd != 2) fail("matmul needs a 2-D grouped n:m tensor");
+    return w;
+}
+
+// The operands of the present val / idx: an in-place change of either shows in its version.
+Operands &operands(State &w)
+{
+    const uint32_t vv = w.val._version(), iv = w.idx._version();
+    if (!w.ops.valid || w.ops.val_version != vv || w.ops.idx_version != iv) {
+        w.ops = Operands();
+        w.ops.valid = true;
+        w.ops.val_version = vv;
+        w.ops.idx_version = iv;
+    }
+    return w.ops;
+}
+
+long opt_long(PyObject *d, PyObject *key, long dflt)
+{
+    PyObject *v = PyDict_GetItemWithError(d, key);
+    if (v == nullptr) {
+        if (PyErr_Occurred()) throw python_error();
+        return dflt;
+    }
+    const long r = PyLong_AsLong(v);
+    if (r == -1 && PyErr_Occurred()) throw python_error();
+    return r;
+}
+
+bool opt_bool(PyObject *d, PyObject *key, bool dflt)
+{
+    PyObject *v = PyDict_GetItemWithError(d, key);
+    if (v == nullptr) {
+        if (PyErr_Occurred()) throw python_error();
+        return dflt;
+    }
+    const int r = PyObject_IsTrue(v);
+    if (r < 0) throw python_error();
+    return r != 0;
+}
+
+struct Options {
+    std::string kernel = "auto";
+    long variant = -1, dense_variant = -1, slices = -1;
+    bool expand = true, cache_dense = true;
+};
+
+Options options_of(const State &w)
+{
+    Options o;
+    PyObject *k = PyDict_GetItemWithError(w.opt, S_.kernel);
+    if (k != nullptr) {
+        const char *c = PyUnicode_AsUTF8(k);
+        if (c == nullptr) throw python_error();
+        o.kernel = c;
+    }
+    if (PyDict_Size(w.opt) > (k != nullptr ? 1 : 0)) {
+        o.variant = opt_long(w.opt, S_.variant, -1);
+        o.dense_variant = opt_long(w.opt, S_.dense_variant, -1);
+        o.slices = opt_long(w.opt, S_.slices, -1);
+        o.expand = opt_bool(w.opt, S_.expand, true);
+        o.cache_dense = opt_bool(w.opt, S_.cache_dense, true);
+    }
+    return o;
+}
+
+// ------------------------------------------------------------------------------- derived operands
+
+void pack(State &w)
+{
+    Operands &o = operands(w);
+    if (o.pk_val.defined()) return;
+    const Geometry &q = w.geo;
+    require_gpu(w.val);
+    const bool narrow = nmg_rowpack_pat_bytes(q.n, q.m) == 1;
+    Tensor pk_val = new_empty({q.G, q.nb, q.n}, w.val);
+    Tensor pk_pat = new_empty({q.G, q.nb}, w.val, narrow ? at::kByte : at::kShort);
+    Tensor fp_val, fp_idx;
+    if (is16(w.val) && nmg_fragpack_supported(q.n, q.m)) {
+        int64_t ve = 0, iw = 0;
+        check(nmg_fragpack_sizes(q.G, q.S, &ve, &iw));
+        fp_val = new_empty({ve}, w.val);
+        fp_idx = new_empty({iw}, w.val, at::kInt);
+    }
+    check(nmg_pack_operands(w.val.data_ptr(), (const int16_t *)w.idx.data_ptr(), q.G, q.S, pk_val.data_ptr(), pk_pat.data_ptr(),
+                            fp_val.defined() ? fp_val.data_ptr() : nullptr, fp_idx.defined() ? fp_idx.data_ptr() : nullptr,
+                            q.n, q.m, q.g, dtype_code(w.val.scalar_type()), stream_of(w.val)));
+    o.pk_val = pk_val;
+    o.pk_pat = pk_pat;
+    o.fp_val = fp_val;
+    o.fp_idx = fp_idx;
+}
+
+// The weight as the A operand of the dense matrix cores, [outputs, reduction] in fragment order.
+Tensor densefrag(State &w, int rd, bool keep)
+{
+    Operands &o = operands(w);
+    if (keep && o.frag[rd].defined()) return o.frag[rd];
+    if (!keep) o.frag[0] = o.frag[1] = Tensor();
+    pack(w);
+    const Geometry &q = w.geo;
+    int64_t elems = 0;
+    check(nmg_densefrag_elems(q.dims[1 - rd], q.dims[rd], &elems));
+    Tensor df = new_empty({elems}, w.val);
+    // rowpack lines run along the group dim
+    check(nmg_densefrag(o.pk_val.data_ptr(), o.pk_pat.data_ptr(), q.G, q.S, q.gdim == rd ? 1 : 0, df.data_ptr(), q.n, q.m,
+                        dtype_code(w.val.scalar_type()), stream_of(w.val)));
+    if (keep) o.frag[rd] = df;
+    return df;
+}
+
+// Dense copy [outputs, reduction] of the weight, rows zero-padded to a multiple of pad_k.
+Tensor dense_operand(State &w, int rd, bool keep, int64_t pad_k)
+{
+    Operands &o = operands(w);
+    const Geometry &q = w.geo;
+    const int64_t O = q.dims[1 - rd], K = q.dims[rd], Kp = up(K, pad_k) * pad_k;
+    if (keep) {
+        auto it = o.dense[rd].find(Kp);
+        if (it != o.dense[rd].end()) return it->second;
+    }
+    pack(w);
+    Tensor out = Kp == K ? new_empty({O, Kp}, w.val) : at::zeros({O, Kp}, w.val.options());
+    check(nmg_rowpack_expand(o.pk_val.data_ptr(), o.pk_pat.data_ptr(), q.G, q.S, out.data_ptr(), Kp, q.gdim == rd ? 1 : 0, q.n,
+                             q.m, dtype_code(w.val.scalar_type()), stream_of(w.val)));
+    if (keep) o.dense[rd][Kp] = out;      // only an operand that was written is kept
+    return out;
+}
+
+void lanepack8(State &w)
+{
+    Operands &o = operands(w);
+    if (o.lp_val.defined()) return;
+    pack(w);
+    const Geometry &q = w.geo;
+    int64_t ve = 0, pb = 0;
+    check(nmg_lanepack8_sizes(q.G, q.S, q.n, &ve, &pb));
+    Tensor lp_val = new_empty({ve}, w.val), lp_pat = new_empty({pb}, w.val, at::kByte);
+    check(nmg_lanepack8(o.pk_val.data_ptr(), o.pk_pat.data_ptr(), q.G, q.S, q.n, lp_val.data_ptr(), lp_pat.data_ptr(),
+                        dtype_code(w.val.scalar_type()), stream_of(w.val)));
+    o.lp_val = lp_val;
+    o.lp_pat = lp_pat;
+}
+
+template <typename Bytes, typename Pack>
+void stream_operand(State &w, Tensor Operands::*slot, Bytes bytes_of, Pack pack_to)
+{
+    Operands &o = operands(w);
+    if ((o.*slot).defined()) return;
+    pack(w);
+    const Geometry &q = w.geo;
+    int64_t bytes = 0;
+    check(bytes_of(q.G, q.S, q.n, q.m, &bytes));
+    Tensor t = new_empty({std::max<int64_t>(bytes, 16)}, w.val, at::kByte);
+    check(pack_to(o.pk_val.data_ptr(), o.pk_pat.data_ptr(), q.G, q.S, q.n, q.m, t.data_ptr(), dtype_code(w.val.scalar_type()),
+                  stream_of(w.val)));
+    o.*slot = t;
+}
+
+void gpack(State &w) { stream_operand(w, &Operands::gp, nmg_gpack_bytes, nmg_gpack); }
+void opack(State &w) { stream_operand(w, &Operands::op, nmg_opack_bytes, nmg_opack); }
+
+Tensor slotmap(State &w)
+{
+    const Geometry &q = w.geo;
+    if (q.nd != 2) fail("the slot map needs a 2-D grouped n:m tensor");
+    const uint32_t iv = w.idx._version();
+    if (w.slot_valid && w.slot_version == iv) return w.slot;
+    require_gpu(w.idx);
+    Tensor slot = new_empty({q.nb, q.chunks * q.cols}, w.idx, at::kShort);
+    check(nmg_slotmap((const int16_t *)w.idx.data_ptr(), q.G, q.S, (int16_t *)slot.data_ptr(), q.n, q.m, q.g, stream_of(w.idx)));
+    w.slot = slot;
+    w.slot_version = iv;
+    w.slot_valid = true;
+    return slot;
+}
+
+// ------------------------------------------------------------------------------- views of dense data
+
+std::string shape_text(const Tensor &t)
+{
+    std::ostringstream s;
+    s << "(";
+    for (int64_t d = 0; d < t.dim(); d++) s << (d ? ", " : "") << t.size(d);
+    s << (t.dim() == 1 ? ",)" : ")");
+    return s.str();
+}
+
+// t as [batch, G, S] with element strides; `t` is replaced by a re-ordered copy where the other dims
+// do not collapse into one stride.
+nmg_view view_of(Tensor &t, const Geometry &q)
+{
+    if (t.sizes() != at::IntArrayRef(q.dims)) fail("the dense tensor must have the shape of the layout, got ", shape_text(t));
+    if (q.nd == 2) return nmg_view{1, q.G, q.S, 0, t.stride(q.gdim), t.stride(q.sdim)};
+    std::vector<int64_t> perm;
+    for (int d = 0; d < q.nd; d++)
+        if (d != q.sdim && d != q.gdim) perm.push_back(d);
+    perm.push_back(q.gdim);
+    perm.push_back(q.sdim);
+    t = t.permute(perm).reshape({-1, q.G, q.S});     // a view wherever there is one
+    return nmg_view{t.size(0), q.G, q.S, t.size(0) > 1 ? t.stride(0) : 0, t.stride(1), t.stride(2)};
+}
+
+Tensor gather(State &w, const Tensor &dense)
+{
+    require_gpu(dense);
+    require_gpu(w.val);
+    Tensor t = dense.scalar_type() == w.val.scalar_type() ? dense : dense.to(w.val.scalar_type());
+    nmg_view v = view_of(t, w.geo);
+    Tensor val = at::empty_like(w.val);
+    check(nmg_gather(t.data_ptr(), &v, (const int16_t *)w.idx.data_ptr(), val.data_ptr(), w.geo.n, w.geo.m, w.geo.g,
+                     dtype_code(val.scalar_type()), stream_of(t)));
+    return val;
+}
+
+// ---------------------------------------------------------------------------------------- products
+
+const char *dtype_name(const Tensor &t)
+{
+    switch (t.scalar_type()) {
+    case at::kFloat: return "torch.float32";
+    case at::kHalf: return "torch.float16";
+    case at::kBFloat16: return "torch.bfloat16";
+    case at::kDouble: return "torch.float64";
+    default: return "another dtype";
+    }
+}
+
+Tensor workspace(int64_t floats, const Tensor &like) { return new_empty({std::max<int64_t>(floats, 1)}, like, at::kFloat); }
+
+int64_t split_ws(int slices, int64_t T, int64_t O) { return slices * T * up(O, 256) * 256; }
+
+// Y = X @ op(W): rd = 1 is X [T, C] @ W^T (F.linear forward), rd = 0 is X [T, R] @ W (the input's gradient).
+Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
+{
+    const Geometry &q = w.geo;
+    require_gpu(x);
+    require_gpu(w.val);
+    if (bias.defined()) require_gpu(bias);
+    if (x.scalar_type() != w.val.scalar_type())
+        fail("dtype mismatch: activations ", dtype_name(x), ", weight ", dtype_name(w.val));
+    const bool reduce_sparse = rd == q.sdim;
+    const int64_t K = q.dims[rd], O = q.dims[1 - rd];
+    if (x.dim() != 2 || x.size(1) != K) fail("activations must be [tokens, ", K, "], got ", shape_text(x));
+    c10::DeviceGuard device(x.device());
+    at::AutoDispatchBelowADInplaceOrView raw;
+    if (x.stride(1) != 1) x = x.contiguous();
+    const int64_t T = x.size(0);
+    const int64_t ldx = T > 1 ? x.stride(0) : K;      // the stride of a dim of extent 1 means nothing
+    Tensor y = new_empty({T, O}, x);
+    if (bias.defined()) bias = bias.to(x.scalar_type()).contiguous();
+    const Options opt = options_of(w);
+    const std::string kname = kernel != nullptr ? kernel : opt.kernel;
+    const bool automatic = kname == "auto";
+    const int dt = dtype_code(x.scalar_type());
+    const bool half = is16(x), al = aligned16(x);
+    void *const stream = stream_of(x);
+    void *const xp = x.data_ptr(), *const yp = y.data_ptr(), *const bp = bias.defined() ? bias.data_ptr() : nullptr;
+
+    if (kname == "skinny" && T > 16) fail("the skinny kernel serves at most 16 tokens");
+    // Few tokens on blocks of 8 along the reduction (1:8, 2:8, 4:8): the rowpack operand holds 0.375 /
+    // 0.625 / 1.125 bytes per dense weight where the operand of the sparse matrix cores holds 1.125
+    // (and 4:8 has none): streamed once, expanded in registers, one kernel.
+    if ((automatic || kname == "sstream") && reduce_sparse && T <= 16 && half && nmg_spmm_sstream_supported(q.n, q.m) && K % 256 == 0
+        // weights of fewer than 3072 lines with more than 8 tokens: the operand of the sparse matrix
+        // cores streams as fast or faster although it is larger (4:8 has none)
+        && (!automatic || q.n == 4 || O >= 96 * 32 || T <= 8) && ldx % 8 == 0 && al
+        && T * std::max(ldx, K) * 2 < k2G && 32 * (K / 8) * q.n * 2 < k2G) {
+        lanepack8(w);
+        check(nmg_spmm_sstream(w.ops.lp_val.data_ptr(), w.ops.lp_pat.data_ptr(), O, K, xp, ldx, yp, O, bp, T, q.n, q.m, dt, stream));
+        return y;
+    }
+    if (kname == "sstream")
+        fail("the streaming product along the sparse dim needs 16-bit data, at most 16 tokens, "
+             "1:8, 2:8 or 4:8 and a reduction extent that is a multiple of 256");
+    const bool smf_ok = reduce_sparse && K % 8 == 0 && ldx % 8 == 0 && al && half;
+    bool packed = false;
+    if (smf_ok && (automatic || kname == "skinny" || kname == "smfmac")) {
+        pack(w);
+        packed = w.ops.fp_val.defined();
+    }
+    if (kname == "smfmac" && !packed)
+        fail("the sparse-matrix-core kernel needs 16-bit data, a 2-of-4 compatible n:m "
+             "pattern along the reduction dim and 16-byte aligned activations");
+    if (packed) {
+        const void *fv = w.ops.fp_val.data_ptr(), *fi = w.ops.fp_idx.data_ptr();
+        long variant = opt.variant;
+        const bool flat = T * ldx * 2 < k2G;
+        if (T <= 16 && kname != "smfmac")
+            variant = 5;      // decode shapes: streaming kernel on the same operand
+        else if (T <= 24 && automatic && variant == -1 && K % 128 == 0 && flat && opt.slices < 0)
+            // 17 .. 24 tokens: the streaming kernel with the second half of its 32 token columns in
+            // use is still ahead of the sliced reduction (4096 x 11008: 15.8 / 17.9 against 18.2 /
+            // 18.7 us at 17 / 24 tokens; at 32 tokens 20.1 against 19.3)
+            variant = 5;
+        if (T > 16 && variant == -1 && K % 64 == 0 && flat) {
+            // few tiles for the chip: the reduction is cut into slices, summed by a second kernel
+            int slices = 1;
+            int64_t bytes = 0;
+            check(nmg_splitk_plan(O, K, T, &slices, &bytes));
+            if (opt.slices >= 0) slices = (int)opt.slices;
+            if (slices > 1) {
+                Tensor ws = workspace(split_ws(slices, T, O), x);
+                check(nmg_spmm_smfmac_splitk(fv, fi, O, K, xp, ldx, yp, O, bp, T, dt, slices, ws.data_ptr(), ws.numel() * 4, stream));
+                return y;
+            }
+        }
+        check(nmg_spmm_smfmac(fv, fi, O, K, xp, ldx, yp, O, bp, T, dt, (int)variant, stream));
+        return y;
+    }
+    // Few tokens as well when the choice is automatic: without a sparse-core operand (another
+    // pattern, the reduction along the group dim, fp32) the alternative for <= 16 tokens is the untuned
+    // streaming kernel.  4096 x 11008 at 1 / 4 / 16 tokens: 4:8 25 / 25 / 26 us on the dense-core
+    // operand with the reduction cut into slices against 63 / 119 / 342; 2:4 reduced along the
+    // group dim (the reference's default orientation) 24 / 25 / 26 against 1190 / 1203 / 1286; fp32
+    // 65 / 65 / 65 against 70 / 134 / 361.
+    const int64_t min_t = automatic ? 1 : 17;
+    const bool flat = T * ldx * 2 < k2G;
+    // Few tokens with the reduction along the group dim (what F.linear does with a weight in the
+    // reference's default orientation): the compressed lines are streamed once and expanded in
+    // registers -- 51 MB instead of the 90 MB of the dense-core operand for 4096 x 11008 at 2:4.
+    // ... and with a handful of tokens at 2:4 every workgroup owns 16 outputs over the whole
+    // reduction: one kernel, no sums through memory (the token rows are then read by every
+    // workgroup, which is why this is for few of them)
+    const bool few_ok = !reduce_sparse && half && K % 8 == 0 && ldx % 8 == 0 && al && flat;
+    if ((automatic || kname == "ostream") && few_ok && T <= (automatic ? kOstreamAutoTokens : kOstreamMaxTokens)
+        && nmg_spmm_ostream_supported(q.n, q.m)) {
+        opack(w);
+        check(nmg_spmm_ostream(w.ops.op.data_ptr(), K, O, xp, ldx, yp, O, bp, T, q.n, q.m, dt, stream));
+        return y;
+    }
+    if (kname == "ostream")
+        fail("the product with 16 outputs per workgroup needs 16-bit data, 2:4, the reduction along "
+             "the group dim, at most ", kOstreamMaxTokens, " tokens and a reduction extent that is a multiple of 8");
+    if ((automatic || kname == "gstream") && few_ok && T <= kGstreamMaxTokens && nmg_spmm_gstream_supported(q.n, q.m)) {
+        gpack(w);
+        int slices = 1;
+        int64_t bytes = 0;
+        check(nmg_spmm_gstream_plan(K, O, T, q.n, q.m, &slices, &bytes));
+        Tensor ws = workspace(bytes / 4, x);
+        check(nmg_spmm_gstream(w.ops.gp.data_ptr(), K, O, xp, ldx, yp, O, bp, T, q.n, q.m, dt, ws.data_ptr(), ws.numel() * 4, stream));
+        return y;
+    }
+    if (kname == "gstream")
+        fail("the streaming product along the group dim needs 16-bit data, at most ", kGstreamMaxTokens,
+             " tokens, m = 4 or 8 with n = 1 or 2 and a reduction extent that is a multiple of 8");
+    const bool dense16 = T >= min_t && half && K % 64 == 0 && ldx % 8 == 0 && al && flat;
+    if ((automatic || kname == "mfma" || kname == "densefrag") && dense16 && nmg_densefrag_supported(q.n, q.m)
+        && (kname == "densefrag" || opt.expand)) {
+        // "expand, then multiply": one HBM-bound pass writes the weight in the register order of
+        // the dense matrix cores into scratch, the pipelined kernel multiplies from there
+        Tensor df = densefrag(w, rd, opt.cache_dense);
+        int slices = 1;
+        int64_t bytes = 0;
+        if (opt.dense_variant == -1)
+            // (the plan leaves 16 tokens and fewer to the streaming kernel of the sparse-core operand;
+            // here they are cut like 17)
+            check(nmg_splitk_plan(O, K, std::max<int64_t>(T, 17), &slices, &bytes));
+        if (opt.slices >= 0) slices = (int)opt.slices;
+        if (slices > 1) {
+            // few tiles for the chip: the reduction is cut into slices, summed by a second kernel
+            Tensor ws = workspace(split_ws(slices, T, O), x);
+            check(nmg_spmm_densefrag_splitk(df.data_ptr(), O, K, xp, ldx, yp, O, bp, T, dt, slices, ws.data_ptr(), ws.numel() * 4, stream));
+            return y;
+        }
+        check(nmg_spmm_densefrag(df.data_ptr(), O, K, xp, ldx, yp, O, bp, T, dt, (int)opt.dense_variant, stream));
+        return y;
+    }
+    if (kname == "densefrag")
+        fail("the densefrag route needs 16-bit data, more than 16 tokens, an m that is a power of two or three times one "
+             "and a reduction extent that is a multiple of 64");
+    if (kname == "expand") {
+        if (!(dense16 && O * K * 2 < k2G))
+            fail("the expand-then-multiply route needs 16-bit data, more than 16 tokens "
+                 "and a reduction extent that is a multiple of 64");
+        // the same idea with a plain row-major dense copy of the weight
+        Tensor a = dense_operand(w, rd, false, 1);
+        check(nmg_gemm_nt(a.data_ptr(), K, xp, ldx, yp, O, bp, O, K, T, dt, stream));
+        return y;
+    }
+    if (x.scalar_type() == at::kFloat && T >= min_t && automatic && opt.expand && T <= kF32GemmMaxTokens) {
+        // single precision: "expand, then multiply" as well -- a dense copy of the weight (kept per
+        // weight version) and the pipelined fp32 matrix-core kernel; the kernel below, which expands
+        // inside its reduction loop, runs at a tenth of that rate
+        // One dense copy [R, C] serves both directions: row-major operand of the product that
+        // reduces along dim 1, reduction-major operand of the one that reduces along dim 0.
+        Tensor a = dense_operand(w, 1, opt.cache_dense, 1);
+        auto entry = rd == 1 ? nmg_gemm_nt : nmg_gemm_nn;
+        check(entry(a.data_ptr(), a.stride(0), xp, ldx, yp, O, bp, O, K, T, dt, stream));
+        return y;
+    }
+    const int64_t Kp = up(K, 64) * 64;
+    if (half && T >= (reduce_sparse ? 4 : 1) && automatic && opt.expand && O * Kp * 2 < k2G && T * Kp * 2 < k2G) {
+        // 16-bit shapes that none of the matrix-core routes above takes as they are (a reduction
+        // extent that is not a multiple of 64 or 8, an m such as 5 or 7, unaligned activations):
+        // a dense copy of the weight with zero-padded rows (kept per weight version) and, where
+        // needed, a zero-padded copy of the activations, through the dense 16-bit GEMM -- the
+        // kernel below runs at a hundredth of its rate (from 4 tokens on where the reduction runs
+        // along the sparse dim: this GEMM does not cut its reduction, and at 1 token the streaming kernel
+        // below is ahead, 81 us against 132; along the group dim that kernel takes 470 us at 4096^2)
+        Tensor a = dense_operand(w, rd, opt.cache_dense, 64);
+        Tensor xq = x;
+        if (Kp != K || ldx % 8 != 0 || !al || !flat) {
+            xq = at::zeros({T, Kp}, x.options());
+            xq.narrow(1, 0, K).copy_(x);
+        }
+        check(nmg_gemm_nt(a.data_ptr(), Kp, xq.data_ptr(), T > 1 ? xq.stride(0) : Kp, yp, O, bp, O, Kp, T, dt, stream));
+        return y;
+    }
+    pack(w);
+    int code = NMG_KERNEL_AUTO;
+    if (kname == "mfma" || kname == "expand" || kname == "densefrag") code = NMG_KERNEL_MFMA;
+    else if (kname == "smfmac") code = NMG_KERNEL_SMFMAC;
+    else if (kname != "auto") code = NMG_KERNEL_SKINNY;
+    check(nmg_spmm(w.ops.pk_val.data_ptr(), w.ops.pk_pat.data_ptr(), q.G, q.S, xp, ldx, yp, O, bp, T, reduce_sparse ? 1 : 0, q.n, q.m,
+                   dt, code, stream));
+    return y;
+}
+
+// op(W) @ B in single precision with B and the result as they lie in memory: the dense copy of the
+// weight (kept per weight version; the same one for both directions) as the row operand of the fp32
+// matrix-core GEMM, B as its reduction-major operand.  Undefined when the route does not apply.
+Tensor mm_f32(State &w, Tensor b, int rd, const Options &opt)
+{
+    if (b.scalar_type() != at::kFloat || b.size(1) <= 16 || opt.kernel != "auto" || !opt.expand || b.size(1) > kF32GemmMaxTokens)
+        return Tensor();
+    const Geometry &q = w.geo;
+    const int64_t K = q.dims[rd], O = q.dims[1 - rd];
+    if (b.stride(1) != 1) b = b.contiguous();
+    const int64_t N = b.size(1);
+    // the one dense copy [R, C]: row-major row operand of W @ B, reduction-major row operand of W^T @ B
+    Tensor wd = dense_operand(w, 1, opt.cache_dense, 1);
+    auto entry = rd == 1 ? nmg_gemm_nn : nmg_gemm_tn;
+    Tensor c = new_empty({O, N}, b);
+    check(entry(b.data_ptr(), K > 1 ? b.stride(0) : N, wd.data_ptr(), wd.stride(0), c.data_ptr(), N, nullptr, N, K, O,
+                dtype_code(b.scalar_type()), stream_of(b)));
+    return c;
+}
+
+void check_mm(const State &w, const Tensor &b, int64_t K)
+{
+    require_gpu(b);
+    require_gpu(w.val);
+    if (b.dim() != 2 || b.size(0) != K) fail("B must be [", K, ", N], got ", shape_text(b));
+    if (b.scalar_type() != w.val.scalar_type()) fail("dtype mismatch: B ", dtype_name(b), ", weight ", dtype_name(w.val));
+}
+
+// C = W @ B (torch.mm): the sparse matrix cores with both dense operands as they lie in memory where
+// they can take it, else the transposed operands through spmm.
+Tensor spmm_tt(State &w, Tensor b)
+{
+    const Geometry &q = w.geo;
+    const int64_t R = q.dims[0], C = q.dims[1];
+    check_mm(w, b, C);
+    c10::DeviceGuard device(b.device());
+    at::AutoDispatchBelowADInplaceOrView raw;
+    const int64_t N = b.size(1);
+    const Options opt = options_of(w);
+    bool direct = q.sdim == 1 && is16(b) && C % 64 == 0 && N > 16 && (opt.kernel == "auto" || opt.kernel == "smfmac");
+    if (direct && b.stride(1) != 1) b = b.contiguous();
+    if (direct && (b.stride(0) % 8 != 0 || !aligned16(b))) direct = false;
+    if (direct) {
+        pack(w);
+        direct = w.ops.fp_val.defined();
+    }
+    if (!direct) {
+        Tensor c = mm_f32(w, b, 1, opt);
+        if (c.defined()) return c;
+        return spmm(w, b.t().contiguous(), Tensor(), 1, nullptr).t();
+    }
+    Tensor c = new_empty({R, N}, b);
+    check(nmg_spmm_smfmac_tt(w.ops.fp_val.data_ptr(), w.ops.fp_idx.data_ptr(), R, C, b.data_ptr(), b.stride(0), c.data_ptr(), N, nullptr,
+                             N, dtype_code(b.scalar_type()), stream_of(b)));
+    return c;
+}
+
+// op(W) @ B on the dense matrix cores with both dense operands as they lie in memory.
+Tensor spmm_tt_dense(State &w, Tensor b, int rd)
+{
+    const Geometry &q = w.geo;
+    const int64_t K = q.dims[rd], O = q.dims[1 - rd];
+    check_mm(w, b, K);
+    c10::DeviceGuard device(b.device());
+    at::AutoDispatchBelowADInplaceOrView raw;
+    const int64_t N = b.size(1);
+    const Options opt = options_of(w);
+    bool direct = is16(b) && K % 64 == 0 && N > 16 && nmg_densefrag_supported(q.n, q.m)
+                  && (opt.kernel == "auto" || opt.kernel == "densefrag") && opt.expand;
+    if (direct && b.stride(1) != 1) b = b.contiguous();
+    if (direct && (b.stride(0) % 8 != 0 || !aligned16(b) || b.stride(0) >= (int64_t(1) << 24))) direct = false;
+    if (!direct) {
+        Tensor c = mm_f32(w, b, rd, opt);
+        if (c.defined()) return c;
+        return spmm(w, b.t().contiguous(), Tensor(), rd, nullptr).t();
+    }
+    Tensor df = densefrag(w, rd, opt.cache_dense);
+    Tensor c = new_empty({O, N}, b);
+    check(nmg_spmm_densefrag_tt(df.data_ptr(), O, K, b.data_ptr(), b.stride(0), c.data_ptr(), N, nullptr, N, dtype_code(b.scalar_type()),
+                                stream_of(b)));
+    return c;
+}
+
+bool masked_product_supported(const State &w, const Tensor &rows, const Tensor &cols, bool last)
+{
+    const Geometry &q = w.geo;
+    if (q.nd != 2 || !is16(w.val) || rows.scalar_type() != w.val.scalar_type() || cols.scalar_type() != w.val.scalar_type()) return false;
+    for (const Tensor *t : {&rows, &cols})
+        if (t->stride(1) == 1 && (t->stride(0) % 8 != 0 || !aligned16(*t))) return false;
+    const int64_t pitch = std::max(rows.stride(0), cols.stride(0));
+    if (last) return rows.size(1) % 8 == 0 && pitch < (int64_t(1) << 22);
+    return q.dims[0] % 8 == 0 && q.dims[1] % 8 == 0 && pitch < (int64_t(1) << 25);
+}
+
+// val of the kept positions of rows^T @ cols (rows [T, R], cols [T, C]; with `last` rows [R, T], cols [C, T]).
+Tensor masked_product(State &w, Tensor rows, Tensor cols, bool last)
+{
+    const Geometry &q = w.geo;
+    if (q.nd != 2) fail("the masked product needs a 2-D grouped n:m tensor");
+    const int64_t R = q.dims[0], C = q.dims[1];
+    require_gpu(rows);
+    require_gpu(cols);
+    require_gpu(w.val);
+    const int td = last ? 1 : 0, fd = 1 - td;      // token dim / feature dim of the operands
+    if (rows.dim() != 2 || cols.dim() != 2 || rows.size(td) != cols.size(td) || rows.size(fd) != R || cols.size(fd) != C) {
+        if (last) fail("operands must be [", R, ", T] and [", C, ", T], got ", shape_text(rows), " and ", shape_text(cols));
+        fail("operands must be [T, ", R, "] and [T, ", C, "], got ", shape_text(rows), " and ", shape_text(cols));
+    }
+    if (rows.scalar_type() != w.val.scalar_type() || cols.scalar_type() != w.val.scalar_type())
+        fail("dtype mismatch: operands ", dtype_name(rows), " / ", dtype_name(cols), ", weight ", dtype_name(w.val));
+    c10::DeviceGuard device(w.val.device());
+    at::AutoDispatchBelowADInplaceOrView raw;
+    if (rows.stride(1) != 1) rows = rows.contiguous();
+    if (cols.stride(1) != 1) cols = cols.contiguous();
+    const Tensor &lines = q.gdim == 0 ? rows : cols, &pos = q.gdim == 0 ? cols : rows;
+    const int64_t T = rows.size(td);
+    if (T == 0) return at::zeros_like(w.val);
+    Tensor slot = slotmap(w);
+    Tensor val = at::empty_like(w.val);
+    auto entry = last ? nmg_sddmm_nt : nmg_sddmm;
+    check(entry(lines.data_ptr(), lines.stride(0), pos.data_ptr(), pos.stride(0), T, (const int16_t *)slot.data_ptr(), q.G, q.S,
+                val.data_ptr(), q.n, q.m, q.g, dtype_code(val.scalar_type()), stream_of(val)));
+    return val;
+}
+
+// Dense product on this library's matrix-core kernels, operands as they lie in memory: tn: x [K, T],
+// a [K, O] -> x^T @ a;  nt: x [T, K], a [O, K] -> x @ a^T.  fp32 always; 16-bit types where the kernels take
+// the shape (extents and pitches that are multiples of 8, 16-byte aligned bases; nt: K a multiple of 64) --
+// other 16-bit shapes go through the fp32 kernel (operands widened, result rounded once).  Undefined where
+// that does not take them either (double, more than 2 097 120 tokens).
+Tensor dense_product(bool tn, Tensor x, Tensor a)
+{
+    const at::ScalarType dt = x.scalar_type();
+    const int64_t T = x.size(tn ? 1 : 0), K = x.size(tn ? 0 : 1), O = a.size(tn ? 1 : 0);
+    const bool f32 = dt == at::kFloat, half = is16(x);
+    const bool sound = x.is_cuda() && a.scalar_type() == dt && (f32 || half) && T > 0 && O > 0 && K > 0;
+    if (!sound) return Tensor();
+    c10::DeviceGuard device(x.device());
+    at::AutoDispatchBelowADInplaceOrView raw;
+    if (x.stride(1) != 1) x = x.contiguous();
+    if (a.stride(1) != 1) a = a.contiguous();
+    bool ok;
+    if (half) {
+        ok = x.stride(0) % 8 == 0 && a.stride(0) % 8 == 0 && aligned16(x) && aligned16(a) && O % 8 == 0
+             && std::max(x.stride(0), a.stride(0)) < (int64_t(1) << 24);
+        ok = ok && (tn ? T % 8 == 0 : K % 64 == 0 && O * a.stride(0) * 2 < k2G && T * x.stride(0) * 2 < k2G);
+    } else {
+        ok = up(T, 32) <= 65535;
+    }
+    if (!ok) {
+        if (half && up(T, 32) <= 65535) return dense_product(tn, x.to(at::kFloat), a.to(at::kFloat)).to(dt);
+        return Tensor();
+    }
+    Tensor y = new_empty({T, O}, x);
+    auto entry = tn ? nmg_gemm_tn : nmg_gemm_nt;
+    check(entry(a.data_ptr(), a.stride(0), x.data_ptr(), x.stride(0), y.data_ptr(), O, nullptr, O, K, T, dtype_code(dt), stream_of(x)));
+    return y;
+}
+
+// x [T, K] @ dequantised(B, meta, s)^T for at most 16 token rows.
+Tensor w4_linear(const Tensor &B, const Tensor &meta, const Tensor &s, int64_t M, int64_t K, Tensor x, Tensor bias)
+{
+    c10::DeviceGuard device(x.device());
+    at::AutoDispatchBelowADInplaceOrView raw;
+    const int64_t T = x.size(0);
+    if (x.stride(1) != 1 || x.stride(0) % 8 != 0 || !aligned16(x)) x = x.contiguous();
+    if (bias.defined()) bias = bias.to(at::kHalf).contiguous();
+    Tensor y = new_empty({T, M}, x);
+    check(nmg_w4_linear(B.data_ptr(), meta.data_ptr(), s.data_ptr(), M, K, x.data_ptr(), T > 1 ? x.stride(0) : K, y.data_ptr(), M,
+                        bias.defined() ? bias.data_ptr() : nullptr, T, stream_of(x)));
+    return y;
+}
+
+// ------------------------------------------------------------------------------- Python: the core type
+
+PyObject *wrap(const Tensor &t) { return THPVariable_Wrap(t); }
+
+Tensor tensor_arg(PyObject *o, const char *what)
+{
+    if (!THPVariable_Check(o)) fail(what, " must be a tensor, got ", Py_TYPE(o)->tp_name);
+    return THPVariable_Unpack(o);
+}
+
+Tensor optional_arg(PyObject *o, const char *what) { return o == nullptr || o == Py_None ? Tensor() : tensor_arg(o, what); }
+
+int dim_arg(PyObject *o)
+{
+    const long d = PyLong_AsLong(o);
+    if (d == -1 && PyErr_Occurred()) throw python_error();
+    if (d != 0 && d != 1) fail("reduce_dim must be 0 or 1, got ", d);
+    return (int)d;
+}
+
+PyObject *core_new(PyTypeObject *type, PyObject *, PyObject *)
+{
+    PyObject *o = type->tp_alloc(type, 0);
+    if (o == nullptr) return nullptr;
+    State *st = new State();
+    st->layout = Py_None;
+    Py_INCREF(Py_None);
+    st->opt = PyDict_New();
+    reinterpret_cast<Core *>(o)->st = st;
+    return o;
+}
+
+void core_dealloc(PyObject *o)
+{
+    State *st = reinterpret_cast<Core *>(o)->st;
+    if (st != nullptr) {
+        Py_XDECREF(st->layout);
+        Py_XDECREF(st->opt);
+        delete st;
+    }
+    Py_TYPE(o)->tp_free(o);
+}
+
+int64_t int_attr(PyObject *o, const char *name)
+{
+    PyObject *v = PyObject_GetAttrString(o, name);
+    if (v == nullptr) throw python_error();
+    const long long r = PyLong_AsLongLong(v);
+    Py_DECREF(v);
+    if (r == -1 && PyErr_Occurred()) throw python_error();
+    return r;
+}
+
+void set_layout(State &w, PyObject *layout)
+{
+    Geometry q;
+    PyObject *shape = PyObject_GetAttr(layout, S_.dense_shape);
+    if (shape == nullptr) throw python_error();
+    PyObject *seq = PySequence_Fast(shape, "dense_shape must be a sequence");
+    Py_DECREF(shape);
+    if (seq == nullptr) throw python_error();
+    q.nd = (int)PySequence_Fast_GET_SIZE(seq);
+    for (int d = 0; d < q.nd; d++) q.dims.push_back(PyLong_AsLongLong(PySequence_Fast_GET_ITEM(seq, d)));
+    Py_DECREF(seq);
+    if (PyErr_Occurred()) throw python_error();
+    q.n = (int)int_attr(layout, "n");
+    q.m = (int)int_attr(layout, "m");
+    q.g = (int)int_attr(layout, "group_size");
+    q.sdim = (int)int_attr(layout, "sparse_dim");
+    q.gdim = (int)int_attr(layout, "group_dim");
+    q.G = q.dims.at(q.gdim);
+    q.S = q.dims.at(q.sdim);
+    q.nb = up(q.S, q.m);
+    q.cols = nmg_chunk(q.n, q.m) * q.g;
+    q.chunks = up(q.G, q.cols);
+    w.geo = std::move(q);
+    Py_INCREF(layout);
+    Py_XDECREF(w.layout);
+    w.layout = layout;
+}
+
+int set_tensor(PyObject *self, PyObject *v, void *slot)
+{
+    HOST_TRY
+    State &w = state_of(self);
+    if (v == nullptr) fail("the tensor cannot be deleted");
+    (w.*(slot == nullptr ? &State::val : &State::idx)) = tensor_arg(v, slot == nullptr ? "val" : "idx");
+    w.ops = Operands();
+    if (slot != nullptr) {
+        w.slot = Tensor();
+        w.slot_valid = false;
+    }
+    return 0;
+    HOST_CATCH(-1)
+}
+
+PyObject *get_tensor(PyObject *self, void *slot)
+{
+    HOST_TRY
+    State &w = state_of(self);
+    return wrap(slot == nullptr ? w.val : w.idx);
+    HOST_CATCH(nullptr)
+}
+
+PyObject *get_layout(PyObject *self, void *)
+{
+    PyObject *l = reinterpret_cast<Core *>(self)->st->layout;
+    Py_INCREF(l);
+    return l;
+}
+
+int put_layout(PyObject *self, PyObject *v, void *)
+{
+    HOST_TRY
+    State &w = state_of(self);
+    if (v == nullptr) fail("the layout cannot be deleted");
+    set_layout(w, v);
+    w.ops = Operands();
+    w.slot_valid = false;
+    return 0;
+    HOST_CATCH(-1)
+}
+
+PyObject *get_opt(PyObject *self, void *)
+{
+    PyObject *d = reinterpret_cast<Core *>(self)->st->opt;
+    Py_INCREF(d);
+    return d;
+}
+
+int put_opt(PyObject *self, PyObject *v, void *)
+{
+    if (v == nullptr || !PyDict_Check(v)) {
+        PyErr_SetString(PyExc_TypeError, "spmm_opt must be a dict");
+        return -1;
+    }
+    State &w = *reinterpret_cast<Core *>(self)->st;
+    Py_INCREF(v);
+    Py_XDECREF(w.opt);
+    w.opt = v;
+    return 0;
+}
+
+// {reduction direction: operand} of the operands kept for the present val and idx
+PyObject *get_frag_cache(PyObject *self, void *)
+{
+    HOST_TRY
+    Operands &o = operands(state_of(self));
+    PyObject *d = PyDict_New();
+    for (long rd = 0; rd < 2; rd++)
+        if (o.frag[rd].defined()) {
+            PyObject *k = PyLong_FromLong(rd), *t = wrap(o.frag[rd]);
+            PyDict_SetItem(d, k, t);
+            Py_DECREF(k);
+            Py_DECREF(t);
+        }
+    return d;
+    HOST_CATCH(nullptr)
+}
+
+// {reduction direction, or (direction, pitch) where the rows are padded: dense copy}
+PyObject *get_dense_cache(PyObject *self, void *)
+{
+    HOST_TRY
+    State &w = state_of(self);
+    Operands &o = operands(w);
+    PyObject *d = PyDict_New();
+    for (int rd = 0; rd < 2; rd++)
+        for (auto &e : o.dense[rd]) {
+            PyObject *k = e.first == w.geo.dims[rd] ? PyLong_FromLong(rd) : Py_BuildValue("(iL)", rd, (long long)e.first);
+            PyObject *t = wrap(e.second);
+            PyDict_SetItem(d, k, t);
+            Py_DECREF(k);
+            Py_DECREF(t);
+        }
+    return d;
+    HOST_CATCH(nullptr)
+}
+
+PyObject *pair_or_none(const Tensor &a, const Tensor &b)
+{
+    if (!a.defined()) Py_RETURN_NONE;
+    return Py_BuildValue("(NN)", wrap(a), wrap(b));
+}
+
+// a C++ scope for the operand methods: device of the weight, no autograd, a 2-D weight
+struct OperandScope {
+    State &w;
+    c10::DeviceGuard device;
+    at::AutoDispatchBelowADInplaceOrView raw;
+    explicit OperandScope(PyObject *self) : w(matmul_state(self)), device((require_gpu(w.val), w.val.device())) {}
+};
+
+PyObject *py_rowpack(PyObject *self, PyObject *)
+{
+    HOST_TRY
+    OperandScope s(self);
+    pack(s.w);
+    return pair_or_none(s.w.ops.pk_val, s.w.ops.pk_pat);
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_fragpack(PyObject *self, PyObject *)
+{
+    HOST_TRY
+    OperandScope s(self);
+    pack(s.w);
+    return pair_or_none(s.w.ops.fp_val, s.w.ops.fp_idx);
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_densefrag(PyObject *self, PyObject *arg)
+{
+    HOST_TRY
+    OperandScope s(self);
+    return wrap(densefrag(s.w, dim_arg(arg), options_of(s.w).cache_dense));
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_dense_operand(PyObject *self, PyObject *args, PyObject *kwargs)
+{
+    HOST_TRY
+    static const char *names[] = {"reduce_dim", "cached", "pad_k", nullptr};
+    PyObject *rd = nullptr;
+    int cached = 0;
+    long long pad_k = 1;
+    if (!PyArg_ParseTupleAndKeywords(args, kwargs, "O|pL", const_cast<char **>(names), &rd, &cached, &pad_k)) return nullptr;
+    OperandScope s(self);
+    return wrap(dense_operand(s.w, dim_arg(rd), cached && options_of(s.w).cache_dense, pad_k));
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_lanepack8(PyObject *self, PyObject *)
+{
+    HOST_TRY
+    OperandScope s(self);
+    lanepack8(s.w);
+    return pair_or_none(s.w.ops.lp_val, s.w.ops.lp_pat);
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_gpack(PyObject *self, PyObject *)
+{
+    HOST_TRY
+    OperandScope s(self);
+    gpack(s.w);
+    return wrap(s.w.ops.gp);
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_opack(PyObject *self, PyObject *)
+{
+    HOST_TRY
+    OperandScope s(self);
+    opack(s.w);
+    return wrap(s.w.ops.op);
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_slotmap(PyObject *self, PyObject *)
+{
+    HOST_TRY
+    State &w = state_of(self);
+    c10::DeviceGuard device(w.idx.device());
+    at::AutoDispatchBelowADInplaceOrView raw;
+    return wrap(slotmap(w));
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_drop(PyObject *self, PyObject *)
+{
+    reinterpret_cast<Core *>(self)->st->ops = Operands();
+    Py_RETURN_NONE;
+}
+
+// A tensor of the same class, pattern and options with other values.
+PyObject *with_val(PyObject *self, const Tensor &val)
+{
+    State &w = state_of(self);
+    PyObject *o = core_new(Py_TYPE(self), nullptr, nullptr);
+    if (o == nullptr) throw python_error();
+    State &n = *reinterpret_cast<Core *>(o)->st;
+    n.val = val;
+    n.idx = w.idx;
+    n.geo = w.geo;
+    Py_INCREF(w.layout);
+    Py_DECREF(n.layout);
+    n.layout = w.layout;
+    Py_DECREF(n.opt);
+    n.opt = PyDict_Copy(w.opt);
+    return o;
+}
+
+PyObject *py_gather(PyObject *self, PyObject *arg)
+{
+    HOST_TRY
+    State &w = state_of(self);
+    Tensor t = tensor_arg(arg, "the dense tensor");
+    require_gpu(t);
+    c10::DeviceGuard device(t.device());
+    at::AutoDispatchBelowADInplaceOrView raw;
+    return with_val(self, gather(w, t));
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_to_dense(PyObject *self, PyObject *)
+{
+    HOST_TRY
+    State &w = state_of(self);
+    const Geometry &q = w.geo;
+    require_gpu(w.val);
+    c10::DeviceGuard device(w.val.device());
+    at::AutoDispatchBelowADInplaceOrView raw;
+    Tensor out = new_empty(q.dims, w.val), t = out;
+    nmg_view v = view_of(t, q);
+    check(nmg_to_dense(w.val.data_ptr(), (const int16_t *)w.idx.data_ptr(), t.data_ptr(), &v, q.n, q.m, q.g,
+                       dtype_code(w.val.scalar_type()), stream_of(w.val)));
+    if (t.storage().data_ptr().get() != out.storage().data_ptr().get()) {
+        std::vector<int64_t> perm, sizes;
+        for (int d = 0; d < q.nd; d++)
+            if (d != q.sdim && d != q.gdim) perm.push_back(d);
+        perm.push_back(q.gdim);
+        perm.push_back(q.sdim);
+        for (int64_t d : perm) sizes.push_back(q.dims[d]);
+        std::vector<int64_t> inv(q.nd);
+        for (int i = 0; i < q.nd; i++) inv[perm[i]] = i;
+        out = t.view(sizes).permute(inv).contiguous();
+    }
+    return wrap(out);
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_masked_product(PyObject *self, PyObject *args)
+{
+    HOST_TRY
+    PyObject *r, *c;
+    int last = 0;
+    if (!PyArg_ParseTuple(args, "OOp", &r, &c, &last)) return nullptr;
+    State &w = state_of(self);
+    return with_val(self, masked_product(w, tensor_arg(r, "rows_op"), tensor_arg(c, "cols_op"), last != 0));
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_masked_product_supported(PyObject *self, PyObject *args)
+{
+    HOST_TRY
+    PyObject *r, *c;
+    int last = 0;
+    if (!PyArg_ParseTuple(args, "OOp", &r, &c, &last)) return nullptr;
+    return PyBool_FromLong(masked_product_supported(state_of(self), tensor_arg(r, "rows_op"), tensor_arg(c, "cols_op"), last != 0));
+    HOST_CATCH(nullptr)
+}
+
+PyGetSetDef core_getset[] = {
+    {"val", get_tensor, set_tensor, "kept values [outer, c, g, n]", nullptr},
+    {"idx", get_tensor, set_tensor, "int16 column positions [outer, c, g, 1]", (void *)1},
+    {"layout", get_layout, put_layout, "NMGLayout", nullptr},
+    {"spmm_opt", get_opt, put_opt, "options of the products", nullptr},
+    {"_densefrag", get_frag_cache, nullptr, "dense-core operands kept for the present values", nullptr},
+    {"_dense_operand", get_dense_cache, nullptr, "dense copies kept for the present values", nullptr},
+    {nullptr, nullptr, nullptr, nullptr, nullptr}};
+
+PyMethodDef core_methods[] = {
+    {"rowpack", py_rowpack, METH_NOARGS,
+     "(pk_val [G, nb, n], pk_pat [G, nb]) -- per line of the group dim and block of the sparse dim, the kept\n"
+     "values and the pattern number; cached until ``val`` changes."},
+    {"fragpack", py_fragpack, METH_NOARGS,
+     "Operand of the sparse-matrix-core kernel (values + 2-bit positions in instruction register order);\n"
+     "``None`` when the n:m pattern does not fit 2-of-4 groups or the dtype is not 16-bit.  Cached until ``val`` changes."},
+    {"densefrag", py_densefrag, METH_O,
+     "densefrag(reduce_dim): the weight as the A operand of the dense matrix cores, [outputs, reduction] in\n"
+     "fragment order, expanded from the rowpack operand.  It is as large as the dense weight.  It is kept until\n"
+     "``val`` changes (one copy per reduction direction), so a frozen weight, or the forward and backward of one\n"
+     "training step, pay the expansion once; ``spmm_opt[\"cache_dense\"] = False`` rebuilds it per call instead and\n"
+     "keeps the memory of the compressed format."},
+    {"dense_operand", (PyCFunction)(void (*)(void))py_dense_operand, METH_VARARGS | METH_KEYWORDS,
+     "dense_operand(reduce_dim, cached=False, pad_k=1): dense copy [outputs, reduction] of the weight (transposed\n"
+     "when the reduction runs along dim 0), expanded from the rowpack operand into fresh scratch.  ``cached``: kept\n"
+     "until ``val`` changes, like the densefrag operand (``spmm_opt[\"cache_dense\"] = False`` turns that off).\n"
+     "``pad_k``: the rows are padded with zeros to a multiple of it."},
+    {"lanepack8", py_lanepack8, METH_NOARGS,
+     "Operand of the streaming product on blocks of 8 along the reduction (1:8, 2:8, 4:8 with at most 16 tokens):\n"
+     "the rowpack values and pattern bytes in the order in which the lanes of ``nmg_spmm_sstream`` take them; as\n"
+     "large as the rowpack operand (0.625 bytes per dense weight at 2:8), kept until ``val`` changes."},
+    {"gpack", py_gpack, METH_NOARGS,
+     "Operand of the streaming product along the group dim (at most 16 tokens, m = 4 or 8 with n = 1 or 2): the\n"
+     "rowpack operand in tiles of 32 lines x 256 outputs, each one contiguous run in the order in which the lanes\n"
+     "of ``nmg_spmm_gstream`` take it, pattern numbers in 4 bits where there are at most 16; kept until ``val`` changes."},
+    {"opack", py_opack, METH_NOARGS,
+     "Operand of ``nmg_spmm_ostream`` (a handful of tokens, 2:4, reduction along the group dim): the rowpack operand\n"
+     "per span of 16 outputs and set of 256 lines in the order in which the lanes fetch it, pattern numbers in 4\n"
+     "bits; kept until ``val`` changes."},
+    {"slotmap", py_slotmap, METH_NOARGS,
+     "int16 [num_blocks, Gpad]: for every line of the (padded) group dim and block of the sparse dim, the slot that\n"
+     "holds it -- the inverse of ``idx``.  Operand of the masked weight-gradient kernel; depends on the pattern\n"
+     "only, cached until ``idx`` changes."},
+    {"to_dense", py_to_dense, METH_NOARGS, "The dense tensor, zeros at the positions that are not kept."},
+    {"_gather", py_gather, METH_O, nullptr},
+    {"_masked_product", py_masked_product, METH_VARARGS, nullptr},
+    {"_masked_product_supported", py_masked_product_supported, METH_VARARGS, nullptr},
+    {"_drop_operands", py_drop, METH_NOARGS, "Forget every operand derived from ``val`` (in-place updates call this)."},
+    {nullptr, nullptr, 0, nullptr}};
+
+// ---------------------------------------------------------------------------------- Python: functions
+
+PyObject *py_sparsify(PyObject *, PyObject *args)
+{
+    HOST_TRY
+    PyObject *self, *dense;
+    if (!PyArg_ParseTuple(args, "OO", &self, &dense)) return nullptr;
+    State &w = state_of(self);      // layout set, val and idx not yet
+    const Geometry &q = w.geo;
+    Tensor t = tensor_arg(dense, "the dense tensor");
+    require_gpu(t);
+    c10::DeviceGuard device(t.device());
+    at::AutoDispatchBelowADInplaceOrView raw;
+    nmg_view v = view_of(t, q);
+    const int64_t outer = v.batch * q.chunks * q.nb, c = nmg_chunk(q.n, q.m);
+    Tensor val = new_empty({outer, c, q.g, q.n}, t), idx = new_empty({outer, c, q.g, 1}, t, at::kShort);
+    check(nmg_sparsify(t.data_ptr(), &v, val.data_ptr(), (int16_t *)idx.data_ptr(), q.n, q.m, q.g, dtype_code(t.scalar_type()),
+                       stream_of(t)));
+    w.val = val;
+    w.idx = idx;
+    Py_RETURN_NONE;
+    HOST_CATCH(nullptr)
+}
+
+const char *kernel_arg(PyObject *o)
+{
+    if (o == nullptr || o == Py_None) return nullptr;
+    const char *c = PyUnicode_AsUTF8(o);
+    if (c == nullptr) throw python_error();
+    return c;
+}
+
+PyObject *py_spmm(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    HOST_TRY
+    if (n != 5) fail("spmm takes 5 arguments");
+    return wrap(spmm(matmul_state(a[0]), tensor_arg(a[1], "the activations"), optional_arg(a[2], "the bias"), dim_arg(a[3]), kernel_arg(a[4])));
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_spmm_tt(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    HOST_TRY
+    if (n != 2) fail("spmm_tt takes 2 arguments");
+    return wrap(spmm_tt(matmul_state(a[0]), tensor_arg(a[1], "B")));
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_spmm_tt_dense(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    HOST_TRY
+    if (n != 3) fail("spmm_tt_dense takes 3 arguments");
+    return wrap(spmm_tt_dense(matmul_state(a[0]), tensor_arg(a[1], "B"), dim_arg(a[2])));
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_dense_product(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    HOST_TRY
+    if (n != 3) fail("dense_product takes 3 arguments");
+    Tensor y = dense_product(PyObject_IsTrue(a[0]) == 1, tensor_arg(a[1], "x"), tensor_arg(a[2], "a"));
+    if (!y.defined()) Py_RETURN_NONE;
+    return wrap(y);
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_w4_linear(PyObject *, PyObject *args)
+{
+    HOST_TRY
+    PyObject *B, *meta, *s, *x, *bias;
+    long long M, K;
+    if (!PyArg_ParseTuple(args, "OOOLLOO", &B, &meta, &s, &M, &K, &x, &bias)) return nullptr;
+    return wrap(w4_linear(tensor_arg(B, "B"), tensor_arg(meta, "meta"), tensor_arg(s, "s"), M, K, tensor_arg(x, "the activations"),
+                          optional_arg(bias, "the bias")));
+    HOST_CATCH(nullptr)
+}
+
+PyObject *py_init(PyObject *, PyObject *arg)
+{
+    Py_INCREF(arg);
+    Py_XDECREF(g_nmg_error);
+    g_nmg_error = arg;
+    Py_RETURN_NONE;
+}
+
+PyMethodDef functions[] = {
+    {"init", py_init, METH_O, "init(error class)"},
+    {"sparsify", py_sparsify, METH_VARARGS, "sparsify(core, dense): fills val and idx of a core whose layout is set"},
+    {"spmm", (PyCFunction)(void (*)(void))py_spmm, METH_FASTCALL, "spmm(weight, x, bias, reduce_dim, kernel)"},
+    {"spmm_tt", (PyCFunction)(void (*)(void))py_spmm_tt, METH_FASTCALL, "spmm_tt(weight, b)"},
+    {"spmm_tt_dense", (PyCFunction)(void (*)(void))py_spmm_tt_dense, METH_FASTCALL, "spmm_tt_dense(weight, b, reduce_dim)"},
+    {"dense_product", (PyCFunction)(void (*)(void))py_dense_product, METH_FASTCALL, "dense_product(tn, x, a), None where no kernel takes it"},
+    {"w4_linear", py_w4_linear, METH_VARARGS, "w4_linear(B, meta, s, M, K, x, bias)"},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", "Native host path of the grouped n:m products.", -1, functions};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host()
+{
+    CoreType.tp_name = "sten_amd._host.Core";
+    CoreType.tp_doc = "Values, indices, geometry and cached operands of a grouped n:m tensor.";
+    CoreType.tp_basicsize = sizeof(Core);
+    CoreType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE;
+    CoreType.tp_new = core_new;
+    CoreType.tp_dealloc = core_dealloc;
+    CoreType.tp_getset = core_getset;
+    CoreType.tp_methods = core_methods;
+    if (PyType_Ready(&CoreType) < 0) return nullptr;
+    PyObject *m = PyModule_Create(&module_def);
+    if (m == nullptr) return nullptr;
+    g_nmg_error = PyExc_RuntimeError;
+    Py_INCREF(g_nmg_error);
+    S_ = {PyUnicode_InternFromString("kernel"), PyUnicode_InternFromString("variant"), PyUnicode_InternFromString("dense_variant"),
+          PyUnicode_InternFromString("slices"), PyUnicode_InternFromString("expand"), PyUnicode_InternFromString("cache_dense"),
+          PyUnicode_InternFromString("_wrapped_tensor_container"), PyUnicode_InternFromString("dense_shape"),
+          PyUnicode_InternFromString("B"), PyUnicode_InternFromString("s"), PyUnicode_InternFromString("meta")};
+    Py_INCREF(&CoreType);
+    if (PyModule_AddObject(m, "Core", (PyObject *)&CoreType) < 0) return nullptr;
+    return m;
+}

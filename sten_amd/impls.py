@@ -8,7 +8,7 @@ functions: this package's own ``dispatch`` module, or a real ``sten``.
 """
 import torch
 
-from . import native
+from ._host_loader import host as _host
 from .tensor import GroupedNMTensor, spmm, spmm_tt, spmm_tt_dense
 
 
@@ -58,34 +58,9 @@ def _dense_product(form, x, a):
     pitches that are multiples of 8, 16-byte aligned bases; ``"nt"``: K a multiple of 64) -- other
     16-bit shapes go through the fp32 kernel (operands widened, result rounded once); only what
     that does not take either (double, more than 2 097 120 tokens) goes to ``torch.mm``."""
-    dt = x.dtype
-    if form == "tn":
-        (K, T), O = x.shape, a.shape[1]
-    else:
-        (T, K), O = x.shape, a.shape[0]
-    ok = x.is_cuda and a.dtype == dt and dt in native.DTYPE_CODE and dt != torch.float64 and T > 0 and O > 0 and K > 0
-    if ok:
-        x = x if x.stride(1) == 1 else x.contiguous()
-        a = a if a.stride(1) == 1 else a.contiguous()
-    if ok and dt != torch.float32:
-        ok = (x.stride(0) % 8 == 0 and a.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and a.data_ptr() % 16 == 0
-              and O % 8 == 0 and max(x.stride(0), a.stride(0)) < 2 ** 24)
-        if form == "tn":
-            ok = ok and T % 8 == 0
-        else:
-            ok = ok and K % 64 == 0 and O * a.stride(0) * 2 < 2 ** 31 and T * x.stride(0) * 2 < 2 ** 31
-    if ok and dt == torch.float32:
-        ok = (T + 31) // 32 <= 65535
-    if not ok:
-        if (x.is_cuda and a.dtype == dt and dt in (torch.float16, torch.bfloat16) and T > 0 and O > 0 and K > 0
-                and (T + 31) // 32 <= 65535):
-            return _dense_product(form, x.float(), a.float()).to(dt)
-        return torch.mm(x.t(), a) if form == "tn" else torch.mm(x, a.t())
-    entry = native.load().nmg_gemm_tn if form == "tn" else native.load().nmg_gemm_nt
-    y = torch.empty((T, O), dtype=dt, device=x.device)
-    with torch.cuda.device(x.device):
-        native.check(entry(native.ptr(a), a.stride(0), native.ptr(x), x.stride(0), native.ptr(y), O,
-                           None, O, K, T, native.dtype_code(dt), native.stream_ptr(x.device)))
+    y = _host.dense_product(form == "tn", x, a)
+    if y is None:
+        y = torch.mm(x.t(), a) if form == "tn" else torch.mm(x, a.t())
     return y
 
 

@@ -125,21 +125,3 @@ class NMGLayout:
             "padded_sparse_dim": self.num_blocks * self.m,
             "padded_group_dim": self.num_chunks * self.cols,
         }
-
-
-def bgs_view(t, lay):
-    """Return (tensor, NmgView) presenting ``t`` as [batch, G, S] with element strides.
-
-    The returned tensor aliases ``t`` whenever the non-sparse, non-group dims collapse into one
-    stride (always for 2-D); otherwise it is a contiguous re-ordered copy."""
-    p = t.permute(lay.other_dims + [lay.group_dim, lay.sparse_dim])
-    G, S = p.shape[-2], p.shape[-1]
-    if p.dim() == 2:
-        q = p.unsqueeze(0)
-    else:
-        try:
-            q = p.view(-1, G, S)
-        except RuntimeError:
-            q = p.reshape(-1, G, S)
-    v = native.NmgView(q.shape[0], G, S, q.stride(0) if q.shape[0] > 1 else 0, q.stride(1), q.stride(2))
-    return q, v

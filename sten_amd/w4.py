@@ -10,6 +10,7 @@ import ctypes
 import torch
 
 from . import native
+from ._host_loader import host as _host
 
 
 class SparseMarlinSparsifier:
@@ -85,16 +86,7 @@ class SparseMarlinTensor:
         T = x2.shape[0]
         if T > 16:
             return torch.nn.functional.linear(x, self.to_dense(), bias)
-        if x2.stride(1) != 1 or x2.stride(0) % 8 != 0 or x2.data_ptr() % 16 != 0:
-            x2 = x2.contiguous()
-        if bias is not None:
-            bias = bias.to(torch.float16).contiguous()
-        y = torch.empty((T, M), dtype=torch.float16, device=x.device)
-        with torch.cuda.device(x.device):
-            native.check(native.load().nmg_w4_linear(
-                native.ptr(self.B), native.ptr(self.meta), native.ptr(self.s), M, K, native.ptr(x2),
-                x2.stride(0) if T > 1 else K, native.ptr(y), M, native.ptr(bias), T,
-                native.stream_ptr(x.device)))
+        y = _host.w4_linear(self.B, self.meta, self.s, M, K, x2, bias)
         return y.reshape(*x.shape[:-1], M)
 
 
