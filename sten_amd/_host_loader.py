@@ -5,11 +5,19 @@ import torch  # noqa: F401  (the extension is linked against torch's libraries, 
 
 from .native import NmgError
 
+INTERFACE = 2      # kInterface in csrc/nmg_host.cpp: what the Python side expects of the module
+
 
 class _Missing:
     class Core:
         def __new__(cls, *args, **kwargs):
             raise NmgError(_missing)
+
+    def make_torch_function(self, *args):
+        def missing(*args):
+            raise NmgError(_missing)
+
+        return staticmethod(missing)
 
     def __getattr__(self, name):
         raise NmgError(_missing)
@@ -17,6 +25,8 @@ class _Missing:
 
 try:
     from . import _host as host
+    if getattr(host, "INTERFACE", None) != INTERFACE:
+        raise ImportError("it was built from other sources")
     host.init(NmgError)
 except ImportError as e:
     host = _Missing()

@@ -13,8 +13,12 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
 #include <c10/hip/HIPStream.h>
+#include <pybind11/pybind11.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
 
 #include <map>
 #include <sstream>
@@ -28,6 +32,7 @@ namespace {
 
 using at::Tensor;
 
+constexpr long kInterface = 2;        // INTERFACE in sten_amd/_host_loader.py
 PyObject *g_nmg_error = nullptr;      // sten_amd.native.NmgError
 
 struct NmgError : std::runtime_error {
@@ -58,7 +63,7 @@ void check(int rc)
 // ---------------------------------------------------------------------------------- small helpers
 
 struct Text {
-    PyObject *kernel, *variant, *dense_variant, *slices, *expand, *cache_dense, *container, *dense_shape, *B, *s, *meta;
+    PyObject *kernel, *variant, *dense_variant, *slices, *expand, *cache_dense, *container, *dense_shape, *B, *s, *meta, *grad_fmt, *data, *alpha;
 } S_;
 
 int dtype_code(at::ScalarType t)
@@ -1211,6 +1216,384 @@ PyObject *py_w4_linear(PyObject *, PyObject *args)
     HOST_CATCH(nullptr)
 }
 
+// --------------------------------------------------------------------- the dispatch of wrapped tensors
+
+// `__torch_function__` of a dispatch module.  The operators that have a native route and the accessors that an
+// optimizer or a module touches on every step are served here; everything else, and whatever the native
+// route does not know (another format, a registered replacement, sparse outputs, other gradient formats),
+// goes to the module's own Python dispatcher.
+struct Dispatch {
+    PyObject *slow;        // (func, types, args, kwargs)
+    PyObject *failed;      // (func, exception): the dispatcher's warning before an exception leaves it
+    PyObject *plain;       // set: functions that run on the wrapper's own placeholder
+    PyObject *native;      // operator -> {format: [forward, dense gradient, pattern gradient: bit per arity, place of the weight]}
+    PyObject *grad_of;     // (wrapped, dtype and device of this tensor) -> wrapper of a weight gradient
+    PyObject *add_;        // torch.Tensor.add_
+    PyObject *keep_all, *dense_tensor, *tensor;      // the module's KeepAll and DenseTensor, torch.Tensor
+};
+
+Dispatch *dispatch_of(PyObject *capsule) { return (Dispatch *)PyCapsule_GetPointer(capsule, nullptr); }
+
+// The list that holds what a wrapper wraps; nullptr where `o` is no wrapper.
+PyObject *container_of(PyObject *o)
+{
+    PyObject **d = _PyObject_GetDictPtr(o);
+    if (d == nullptr || *d == nullptr) return nullptr;
+    PyObject *c = PyDict_GetItem(*d, S_.container);
+    return c != nullptr && PyList_CheckExact(c) && PyList_GET_SIZE(c) == 1 ? c : nullptr;
+}
+
+bool plain_tensor(PyObject *o) { return THPVariable_CheckExact(o); }
+
+bool has_bit(PyObject *masks, Py_ssize_t slot, int arity)
+{
+    const long m = PyLong_AsLong(PyList_GET_ITEM(masks, slot));
+    return (m >> arity & 1) != 0;
+}
+
+// The format of the weight gradient where the native backward knows it: 1 dense, 2 the weight's pattern, else 0.
+int grad_kind(const Dispatch &d, PyObject *weight, PyObject *wrapped)
+{
+    PyObject **dict = _PyObject_GetDictPtr(weight);
+    PyObject *f = dict != nullptr && *dict != nullptr ? PyDict_GetItem(*dict, S_.grad_fmt) : nullptr;
+    if (f == nullptr || !PyTuple_Check(f) || PyTuple_GET_SIZE(f) != 4) return 0;
+    if ((PyObject *)Py_TYPE(PyTuple_GET_ITEM(f, 0)) != d.keep_all || (PyObject *)Py_TYPE(PyTuple_GET_ITEM(f, 2)) != d.keep_all) return 0;
+    PyObject *tmp = PyTuple_GET_ITEM(f, 1), *out = PyTuple_GET_ITEM(f, 3);
+    if (tmp == d.tensor && out == d.dense_tensor) return 1;
+    if (tmp == (PyObject *)Py_TYPE(wrapped) && out == tmp) return 2;
+    return 0;
+}
+
+// val-layout gradient: the kept positions of lhs^T @ rhs (lhs [T, rows of W], rhs [T, columns of W]).  16-bit weights
+// take the fused kernel, which never stores the dense product; fp32 and extents that are not multiples of 8 go
+// through the dense product and the same-pattern gather.
+Tensor masked_weight_grad(State &w, const Tensor &lhs, Tensor rhs)
+{
+    if (rhs.scalar_type() != w.val.scalar_type()) rhs = rhs.to(w.val.scalar_type());
+    if (masked_product_supported(w, lhs, rhs, false)) return masked_product(w, lhs, rhs, false);
+    Tensor g = dense_product(true, lhs, rhs);
+    if (!g.defined()) g = at::mm(lhs.t(), rhs);
+    return gather(w, g);
+}
+
+// Backward of F.linear(x, W[, b]) (weight at place 1) and of torch.mm(W, B) (weight at place 0).
+struct ProductNode : public torch::autograd::Node {
+    torch::autograd::SavedVariable dense;      // x or B
+    PyObject *container = nullptr, *owner = nullptr;
+    int place = 1, kind = 1;
+    bool released = false;
+
+    ~ProductNode() override
+    {
+        if (!Py_IsInitialized()) return;
+        pybind11::gil_scoped_acquire gil;
+        Py_XDECREF(container);
+        Py_XDECREF(owner);
+    }
+    std::string name() const override { return place == 1 ? "SparseLinearBackward" : "SparseMmBackward"; }
+    void release_variables() override
+    {
+        dense.reset_data();
+        released = true;
+    }
+
+    Tensor weight_grad(PyObject *wrapped, const Tensor &g)
+    {
+        PyObject *payload = kind == 2 ? with_val(wrapped, g) : wrap(g);
+        PyObject *like = wrap(state_of(wrapped).val);
+        PyObject *r = PyObject_CallFunctionObjArgs(dispatch_of(owner)->grad_of, payload, like, kind == 2 ? Py_True : Py_False, nullptr);
+        Py_DECREF(payload);
+        Py_DECREF(like);
+        if (r == nullptr) throw python_error();
+        Tensor t = THPVariable_Unpack(r);
+        Py_DECREF(r);
+        return t;
+    }
+
+    void linear(PyObject *wrapped, const Tensor &gy, torch::autograd::variable_list &out)
+    {
+        State &w = matmul_state(wrapped);
+        Tensor x = dense.unpack();
+        Tensor g = gy.dim() == 2 ? gy : gy.reshape({-1, gy.size(-1)});
+        Tensor x2 = x.dim() == 2 ? x : x.reshape({-1, x.size(-1)});
+        if (g.scalar_type() != w.val.scalar_type()) g = g.to(w.val.scalar_type());
+        if (task_should_compute_output(0)) {
+            Tensor gx = spmm(w, g.contiguous(), Tensor(), 0, nullptr);
+            out[0] = x.dim() == 2 ? gx : gx.reshape(x.sizes());
+        }
+        if (task_should_compute_output(1)) {
+            Tensor gw;
+            if (kind == 2) {
+                gw = masked_weight_grad(w, g, x2);
+            } else {
+                // the dense weight gradient dY^T X from the operands as they lie (both token-major)
+                const Tensor r = x2.scalar_type() == g.scalar_type() ? x2 : x2.to(g.scalar_type());
+                gw = dense_product(true, g, r);
+                if (!gw.defined()) gw = at::mm(g.t(), r);
+            }
+            out[1] = weight_grad(wrapped, gw);
+        }
+        if (out.size() > 2 && task_should_compute_output(2)) out[2] = g.sum(0);
+    }
+
+    void mm(PyObject *wrapped, Tensor gc, torch::autograd::variable_list &out)
+    {
+        State &w = matmul_state(wrapped);
+        Tensor b = dense.unpack();
+        if (gc.scalar_type() != w.val.scalar_type()) gc = gc.to(w.val.scalar_type());
+        if (task_should_compute_output(1)) out[1] = spmm_tt_dense(w, gc, 0);      // W^T @ grad_out, both as they lie in memory
+        if (!task_should_compute_output(0)) return;
+        Tensor gw;
+        const Tensor r = b.scalar_type() == gc.scalar_type() ? b : b.to(gc.scalar_type());
+        if (kind == 2 && masked_product_supported(w, gc, b, true)) {
+            // grad_out [R, N] and B [C, N] are reduction-contiguous as they lie: no transposing copies
+            gw = masked_product(w, gc, b, true);
+        } else if (kind == 2 && !(gc.scalar_type() == at::kFloat && b.scalar_type() == at::kFloat)) {
+            gw = masked_weight_grad(w, gc.t(), b.t());
+        } else {
+            gw = dense_product(false, gc, r);      // grad_out @ B^T
+            if (!gw.defined()) gw = at::mm(gc, r.t());
+            if (kind == 2) gw = gather(w, gw);
+        }
+        out[0] = weight_grad(wrapped, gw);
+    }
+
+    torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override
+    {
+        torch::autograd::variable_list out(next_edges().size());
+        TORCH_CHECK(!released, torch::autograd::ERR_BACKWARD_TWICE);
+        if (!grads[0].defined()) return out;
+        c10::AutoGradMode no_grad(false);
+        pybind11::gil_scoped_acquire gil;
+        try {
+            c10::DeviceGuard device(grads[0].device());
+            PyObject *wrapped = PyList_GetItem(container, 0);
+            if (wrapped == nullptr) throw python_error();
+            Py_INCREF(wrapped);
+            std::unique_ptr<PyObject, void (*)(PyObject *)> hold(wrapped, [](PyObject *o) { Py_DECREF(o); });
+            if (place == 1) linear(wrapped, grads[0], out);
+            else mm(wrapped, grads[0], out);
+        } catch (const NmgError &e) {
+            PyErr_SetString(g_nmg_error, e.what());
+            python_error err;
+            err.persist();
+            throw std::move(err);
+        } catch (python_error &e) {
+            e.persist();
+            throw;
+        }
+        return out;
+    }
+};
+
+std::shared_ptr<ProductNode> new_node(PyObject *capsule, PyObject *container, int place, int kind, const Tensor &dense,
+                                      torch::autograd::edge_list edges)
+{
+    std::shared_ptr<ProductNode> node(new ProductNode(), torch::autograd::deleteNode);
+    Py_INCREF(container);
+    Py_INCREF(capsule);
+    node->container = container;
+    node->owner = capsule;
+    node->place = place;
+    node->kind = kind;
+    node->dense = torch::autograd::SavedVariable(dense, false);
+    node->set_next_edges(std::move(edges));
+    return node;
+}
+
+// A new reference to the result, or nullptr without an error where the native route does not apply.
+PyObject *native_product(PyObject *capsule, PyObject *formats, PyObject *args)
+{
+    Dispatch &d = *dispatch_of(capsule);
+    const Py_ssize_t n = PyTuple_GET_SIZE(args);
+    if (n < 2 || n > 3) return nullptr;
+    PyObject *a0 = PyTuple_GET_ITEM(args, 0), *a1 = PyTuple_GET_ITEM(args, 1);
+    const int guess = plain_tensor(a0) ? 1 : 0;      // where the weight would be
+    PyObject *pw = guess == 1 ? a1 : a0, *px = guess == 1 ? a0 : a1;
+    if (plain_tensor(pw) || !plain_tensor(px)) return nullptr;
+    PyObject *container = container_of(pw);
+    if (container == nullptr) return nullptr;
+    PyObject *wrapped = PyList_GET_ITEM(container, 0);
+    PyObject *masks = PyDict_GetItem(formats, (PyObject *)Py_TYPE(wrapped));
+    if (masks == nullptr || PyLong_AsLong(PyList_GET_ITEM(masks, 3)) != guess) return nullptr;
+    PyObject *pb = n == 3 ? PyTuple_GET_ITEM(args, 2) : Py_None;
+    if (pb != Py_None && !plain_tensor(pb)) return nullptr;
+    const int arity = pb == Py_None ? 2 : 3;
+    if (!has_bit(masks, 0, arity) || (guess == 0 && n != 2)) return nullptr;
+    const Tensor &x = THPVariable_Unpack(px), &wt = THPVariable_Unpack(pw);
+    Tensor bias = pb == Py_None ? Tensor() : THPVariable_Unpack(pb);
+    const bool grad = c10::GradMode::is_enabled() && (x.requires_grad() || wt.requires_grad() || (bias.defined() && bias.requires_grad()));
+    if (x.dim() < 2 && !(guess == 1 && x.dim() == 1)) return nullptr;
+    if (!PyObject_TypeCheck(wrapped, &CoreType)) {      // the int4 format: generation without gradients
+        if (grad || guess != 1 || !x.is_cuda() || x.scalar_type() != at::kHalf) return nullptr;
+        Tensor t[3];
+        PyObject *names[3] = {S_.B, S_.meta, S_.s};
+        for (int i = 0; i < 3; i++) {
+            PyObject *o = PyObject_GetAttr(wrapped, names[i]);
+            if (o == nullptr) throw python_error();
+            t[i] = tensor_arg(o, "a part of the int4 weight");
+            Py_DECREF(o);
+        }
+        PyObject *shape = PyObject_GetAttr(wrapped, S_.dense_shape);
+        if (shape == nullptr) throw python_error();
+        long long M = 0, K = 0;
+        const int ok = PyArg_ParseTuple(shape, "LL", &M, &K);
+        Py_DECREF(shape);
+        if (!ok) throw python_error();
+        if (x.size(-1) != K || x.numel() > 16 * K) return nullptr;
+        Tensor y = w4_linear(t[0], t[1], t[2], M, K, x.dim() == 2 ? x : x.reshape({-1, K}), bias);
+        if (x.dim() != 2) {
+            std::vector<int64_t> size(x.sizes().begin(), x.sizes().end());
+            size.back() = M;
+            y = y.reshape(size);
+        }
+        return wrap(y);
+    }
+    int kind = 0;
+    if (grad) {
+        kind = grad_kind(d, pw, wrapped);
+        if (kind == 0 || !has_bit(masks, kind, arity)) return nullptr;
+    }
+    State &w = matmul_state(wrapped);
+    Tensor y;
+    if (guess == 1) {
+        Tensor x2 = x;
+        {
+            at::AutoDispatchBelowADInplaceOrView raw;
+            if (x.dim() != 2) x2 = x.reshape({-1, x.size(-1)});
+            y = spmm(w, x2, bias, 1, nullptr);
+            if (x.dim() != 2) {
+                std::vector<int64_t> size(x.sizes().begin(), x.sizes().end());
+                size.back() = y.size(-1);
+                y = y.reshape(size);
+            }
+        }
+    } else {
+        y = spmm_tt(w, x);
+    }
+    if (grad) {
+        torch::autograd::edge_list edges = guess == 0 ? torch::autograd::collect_next_edges(wt, x)
+                                           : arity == 3 ? torch::autograd::collect_next_edges(x, wt, bias)
+                                                        : torch::autograd::collect_next_edges(x, wt);
+        torch::autograd::set_history(y, new_node(capsule, container, guess, kind, x, std::move(edges)));
+    }
+    return wrap(y);
+}
+
+bool same_tensor(const Tensor &a, const Tensor &b)
+{
+    return a.unsafeGetTensorImpl() == b.unsafeGetTensorImpl() || (a.data_ptr() == b.data_ptr() && a.sizes() == b.sizes());
+}
+
+// weight.add_(gradient, alpha=...): the step of an optimizer.  nullptr without an error where it is another call.
+PyObject *native_add_(const Dispatch &d, PyObject *args, PyObject *kwargs)
+{
+    if (PyTuple_GET_SIZE(args) != 2) return nullptr;
+    PyObject *alpha = nullptr;
+    if (kwargs != nullptr && PyDict_Size(kwargs) > 0) {
+        alpha = PyDict_GetItem(kwargs, S_.alpha);
+        if (alpha == nullptr || PyDict_Size(kwargs) != 1 || !(PyFloat_CheckExact(alpha) || PyLong_CheckExact(alpha))) return nullptr;
+    }
+    PyObject *cw = container_of(PyTuple_GET_ITEM(args, 0)), *cg = container_of(PyTuple_GET_ITEM(args, 1));
+    if (cw == nullptr || cg == nullptr) return nullptr;
+    PyObject *pw = PyList_GET_ITEM(cw, 0), *pg = PyList_GET_ITEM(cg, 0);
+    if (!PyObject_TypeCheck(pw, &CoreType)) return nullptr;
+    State &w = state_of(pw);
+    at::Scalar a = 1;
+    if (alpha != nullptr) {
+        if (PyFloat_CheckExact(alpha)) a = PyFloat_AS_DOUBLE(alpha);
+        else a = (int64_t)PyLong_AsLongLong(alpha);
+    }
+    if (PyObject_TypeCheck(pg, &CoreType)) {
+        State &g = state_of(pg);
+        if (g.layout != w.layout || !same_tensor(g.idx, w.idx)) return nullptr;
+        w.val.add_(g.val, a);
+    } else if ((PyObject *)Py_TYPE(pg) == d.dense_tensor) {
+        PyObject *o = PyObject_GetAttr(pg, S_.data);
+        if (o == nullptr) throw python_error();
+        const bool plain = plain_tensor(o);
+        Tensor t = plain ? THPVariable_Unpack(o) : Tensor();
+        Py_DECREF(o);
+        if (!plain || !t.is_cuda() || t.device() != w.val.device() || t.sizes() != at::IntArrayRef(w.geo.dims)) return nullptr;
+        c10::DeviceGuard device(t.device());
+        Tensor kept;
+        {
+            at::AutoDispatchBelowADInplaceOrView raw;
+            kept = gather(w, t);
+        }
+        w.val.add_(kept, a);
+    } else {
+        return nullptr;
+    }
+    w.ops = Operands();
+    PyObject *self = PyTuple_GET_ITEM(args, 0);
+    Py_INCREF(self);
+    return self;
+}
+
+PyObject *torch_function(PyObject *capsule, PyObject *const *a, Py_ssize_t n)
+{
+    if (n < 3 || n > 4 || !PyTuple_Check(a[2])) {
+        PyErr_SetString(PyExc_TypeError, "__torch_function__(func, types, args, kwargs=None)");
+        return nullptr;
+    }
+    Dispatch &d = *dispatch_of(capsule);
+    PyObject *func = a[0], *args = a[2], *kwargs = n == 4 && a[3] != Py_None ? a[3] : nullptr;
+    const int plain = PySet_Contains(d.plain, func);
+    if (plain < 0) return nullptr;
+    if (plain) {
+        const auto before = at::impl::PythonTorchFunctionTLS::get_disabled_state();
+        at::impl::PythonTorchFunctionTLS::set_disabled_state(at::impl::TorchFunctionDisabledState::SUBCLASSES_DISABLED);
+        PyObject *r = PyObject_Call(func, args, kwargs);
+        at::impl::PythonTorchFunctionTLS::set_disabled_state(before);
+        return r;
+    }
+    PyObject *r = nullptr;
+    bool bad = false;
+    try {
+        PyObject *formats = PyDict_GetItem(d.native, func);
+        if (formats != nullptr && (kwargs == nullptr || PyDict_Size(kwargs) == 0)) r = native_product(capsule, formats, args);
+        else if (func == d.add_) r = native_add_(d, args, kwargs);
+    }
+    catch (const NmgError &e) { PyErr_SetString(g_nmg_error, e.what()); bad = true; }
+    catch (python_error &e) { e.restore(); bad = true; }
+    catch (const c10::Error &e) { PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace()); bad = true; }
+    catch (const std::exception &e) { PyErr_SetString(PyExc_RuntimeError, e.what()); bad = true; }
+    if (bad) {
+        PyObject *type, *value, *trace;
+        PyErr_Fetch(&type, &value, &trace);
+        PyErr_NormalizeException(&type, &value, &trace);
+        PyObject *done = PyObject_CallFunctionObjArgs(d.failed, func, value, nullptr);
+        if (done == nullptr) {      // the warning was turned into an error
+            Py_XDECREF(type);
+            Py_XDECREF(value);
+            Py_XDECREF(trace);
+            return nullptr;
+        }
+        Py_DECREF(done);
+        PyErr_Restore(type, value, trace);
+        return nullptr;
+    }
+    if (r != nullptr) return r;
+    return PyObject_CallFunctionObjArgs(d.slow, func, a[1], args, kwargs != nullptr ? kwargs : Py_None, nullptr);
+}
+
+PyMethodDef torch_function_def = {"__torch_function__", (PyCFunction)(void (*)(void))torch_function, METH_FASTCALL, nullptr};
+
+PyObject *py_make_torch_function(PyObject *, PyObject *args)
+{
+    Dispatch d;
+    if (!PyArg_ParseTuple(args, "OOO!O!OOOOO", &d.slow, &d.failed, &PySet_Type, &d.plain, &PyDict_Type, &d.native, &d.grad_of, &d.add_,
+                          &d.keep_all, &d.dense_tensor, &d.tensor))
+        return nullptr;
+    Py_INCREF(args);      // a dispatch module lives as long as the process; so does what its callable refers to
+    PyObject *capsule = PyCapsule_New(new Dispatch(d), nullptr, nullptr);
+    if (capsule == nullptr) return nullptr;
+    PyObject *f = PyCFunction_New(&torch_function_def, capsule);
+    Py_DECREF(capsule);
+    return f;
+}
+
 PyObject *py_init(PyObject *, PyObject *arg)
 {
     Py_INCREF(arg);
@@ -1221,6 +1604,8 @@ PyObject *py_init(PyObject *, PyObject *arg)
 
 PyMethodDef functions[] = {
     {"init", py_init, METH_O, "init(error class)"},
+    {"make_torch_function", py_make_torch_function, METH_VARARGS,
+     "make_torch_function(slow, failed, plain, native, grad_of, add_, KeepAll, DenseTensor, Tensor)"},
     {"sparsify", py_sparsify, METH_VARARGS, "sparsify(core, dense): fills val and idx of a core whose layout is set"},
     {"spmm", (PyCFunction)(void (*)(void))py_spmm, METH_FASTCALL, "spmm(weight, x, bias, reduce_dim, kernel)"},
     {"spmm_tt", (PyCFunction)(void (*)(void))py_spmm_tt, METH_FASTCALL, "spmm_tt(weight, b)"},
@@ -1251,7 +1636,9 @@ PyMODINIT_FUNC PyInit__host()
     S_ = {PyUnicode_InternFromString("kernel"), PyUnicode_InternFromString("variant"), PyUnicode_InternFromString("dense_variant"),
           PyUnicode_InternFromString("slices"), PyUnicode_InternFromString("expand"), PyUnicode_InternFromString("cache_dense"),
           PyUnicode_InternFromString("_wrapped_tensor_container"), PyUnicode_InternFromString("dense_shape"),
-          PyUnicode_InternFromString("B"), PyUnicode_InternFromString("s"), PyUnicode_InternFromString("meta")};
+          PyUnicode_InternFromString("B"), PyUnicode_InternFromString("s"), PyUnicode_InternFromString("meta"),
+          PyUnicode_InternFromString("grad_fmt"), PyUnicode_InternFromString("data"), PyUnicode_InternFromString("alpha")};
+    if (PyModule_AddIntConstant(m, "INTERFACE", kInterface) < 0) return nullptr;
     Py_INCREF(&CoreType);
     if (PyModule_AddObject(m, "Core", (PyObject *)&CoreType) < 0) return nullptr;
     return m;

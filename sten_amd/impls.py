@@ -125,20 +125,28 @@ def install(api):
             grads.append(gy2.sum(dim=0))
         return tuple(grads)
 
+    # The dispatch module of this package serves these operators natively, by the rules written here
+    # (``ProductNode`` in csrc/nmg_host.cpp); any other STen-style dispatcher calls the functions.
+    def native(fn):
+        fn.native = True
+        return fn
+
+    native(linear_fwd)
     for arity in (2, 3):
         fmts = (torch.Tensor, GroupedNMTensor) + (torch.Tensor,) * (arity - 2)
         api.register_fwd_op_impl(operator=torch.nn.functional.linear, inp=fmts, out=[dense_fmt])(linear_fwd)
         api.register_bwd_op_impl(
             operator=torch.nn.functional.linear, grad_out=(torch.Tensor,),
             grad_inp=(dense_fmt,) * arity, inp=fmts,
-        )(lambda ctx, g, s: linear_bwd_common(ctx, g, compressed=False))
+        )(native(lambda ctx, g, s: linear_bwd_common(ctx, g, compressed=False)))
         api.register_bwd_op_impl(
             operator=torch.nn.functional.linear, grad_out=(torch.Tensor,),
             grad_inp=(dense_fmt, nmg_fmt) + (dense_fmt,) * (arity - 2), inp=fmts,
-        )(lambda ctx, g, s: linear_bwd_common(ctx, g, compressed=True))
+        )(native(lambda ctx, g, s: linear_bwd_common(ctx, g, compressed=True)))
 
     # ---- torch.mm(W_nmg, B) -----------------------------------------------------------------
     @api.register_fwd_op_impl(operator=torch.mm, inp=(GroupedNMTensor, torch.Tensor), out=[dense_fmt])
+    @native
     def mm_fwd(ctx, inputs, output_sparsifiers):
         weight, b = inputs
         ctx.save_for_backward(weight, b)
@@ -165,11 +173,11 @@ def install(api):
     api.register_bwd_op_impl(
         operator=torch.mm, grad_out=(torch.Tensor,), grad_inp=(dense_fmt, dense_fmt),
         inp=(GroupedNMTensor, torch.Tensor),
-    )(lambda ctx, g, s: mm_bwd_common(ctx, g, compressed=False))
+    )(native(lambda ctx, g, s: mm_bwd_common(ctx, g, compressed=False)))
     api.register_bwd_op_impl(
         operator=torch.mm, grad_out=(torch.Tensor,), grad_inp=(nmg_fmt, dense_fmt),
         inp=(GroupedNMTensor, torch.Tensor),
-    )(lambda ctx, g, s: mm_bwd_common(ctx, g, compressed=True))
+    )(native(lambda ctx, g, s: mm_bwd_common(ctx, g, compressed=True)))
 
     return {"dense_to_grouped_nm": dense_to_grouped_nm,
             "dense_to_same_grouped_nm": dense_to_same_grouped_nm}

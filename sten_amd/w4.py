@@ -106,6 +106,7 @@ def install(api):
         bias = inputs[2] if len(inputs) > 2 else None
         return weight.wrapped_tensor.linear(x, bias)
 
+    linear_fwd.native = True      # few tokens without gradients are served natively by this package's dispatch module
     api.register_fwd_op_impl(operator=torch.nn.functional.linear,
                              inp=(torch.Tensor, SparseMarlinTensor), out=[dense_fmt])(linear_fwd)
     api.register_fwd_op_impl(operator=torch.nn.functional.linear,

@@ -1,0 +1,59 @@
+"""The native dispatch of wrapped weights (csrc/nmg_host.cpp) against the Python dispatcher, which stays the
+route of every other call: same kernels, so the same bits."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+import sten_amd as sten
+from sten_amd import dispatch
+from helpers import seeded
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def weight(dtype, grad):
+    layer = torch.nn.Linear(128, 96, bias=True, device=DEV, dtype=dtype)
+    with torch.no_grad():
+        layer.weight.copy_(seeded((96, 128), dtype, seed=1, std=0.1).to(DEV))
+    builder = sten.SparsityBuilder()
+    builder.set_weight("weight", initial_sparsifier=sten.GroupedNMSparsifier(2, 4, 4), out_format=sten.GroupedNMTensor)
+    if grad == "pattern":
+        builder.set_weight_grad("weight", tmp_format=sten.GroupedNMTensor, out_format=sten.GroupedNMTensor)
+    return builder.sparsify_model_inplace(layer)
+
+
+def results(call, layer, x, shape):
+    x.grad = layer.weight.grad = layer.bias.grad = None
+    y = call()
+    y.backward(seeded(shape, x.dtype, seed=3).to(DEV))
+    g = layer.weight.grad.wrapped_tensor
+    out = [y.detach(), x.grad, g.val if isinstance(g, sten.GroupedNMTensor) else g.to_dense()]
+    return out + ([] if layer.bias.grad is None else [layer.bias.grad])
+
+
+@pytest.mark.parametrize("grad", ["dense", "pattern"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("op,lead", [("linear", (1,)), ("linear", (33,)), ("linear", (3, 5)), ("nobias", (17,)), ("mm", (40,))])
+def test_native_dispatch_gives_what_the_python_dispatcher_gives(op, lead, dtype, grad):
+    print(f"case {op} {lead} {dtype} {grad}", flush=True)
+    layer = weight(dtype, grad)
+    if op == "mm":
+        x = seeded((128, 40), dtype, seed=2).to(DEV).requires_grad_(True)
+        func, args, shape = torch.mm, (layer.weight, x), (96, 40)
+    else:
+        x = seeded(lead + (128,), dtype, seed=2).to(DEV).requires_grad_(True)
+        func, args, shape = F.linear, (x, layer.weight) + ((layer.bias,) if op == "linear" else ()), lead + (96,)
+    native = results(lambda: func(*args), layer, x, shape)
+    python = results(lambda: dispatch._torch_function(func, (), args, None), layer, x, shape)
+    assert len(native) == len(python)
+    for a, b in zip(native, python):
+        assert a.shape == b.shape and torch.equal(a, b)
+
+
+def test_a_graph_is_walked_once():
+    layer = weight(torch.float32, "dense")
+    y = layer(seeded((4, 128), torch.float32, seed=2).to(DEV))
+    y.sum().backward()
+    with pytest.raises(RuntimeError):
+        y.sum().backward()
