@@ -90,6 +90,16 @@ template <> struct Zero<__hip_bfloat16> {
     __device__ static __hip_bfloat16 v() { return __float2bfloat16(0.f); }
 };
 
+// Compressor for 32-bit scores, m <= 8 and at most 128 patterns (nmg_match.h); *done tells whether it took the shape.
+struct ViewDev;
+#define NMG_MATCH(name)                                                                                                    \
+    int name(const void *dense, void *val, int16_t *idx, const ViewDev &view, int64_t outer, int n, int m, int g, int c, \
+             int cols, hipStream_t stream, bool *done)
+NMG_MATCH(match_f32);
+NMG_MATCH(match_f16);
+NMG_MATCH(match_bf16);
+#undef NMG_MATCH
+
 // Address of element (group index gi, sparse index si) of batch b in a strided view.
 struct ViewDev {
     int64_t G, S, stride_b, stride_g, stride_s;

@@ -1,0 +1,998 @@
+// Dense -> grouped n:m for scores of 32 bits and m <= 8, at most 128 patterns: the tile as a matching problem.
+// Included by nmg_match_{f32,f16,bf16}.hip, one instantiation each.
+//
+// The sorted walk of the reference (nmg_sparsify.hip) accepts edges (column o, pattern p) in descending
+// order of one key that both ends share.  That is the stable matching of columns (one pattern each) with
+// patterns (g columns each) under preferences given by the key, and it is unique: whatever order the
+// columns propose in, deferred acceptance ends in it.  So all columns propose at once to their best pattern,
+// a pattern keeps its g best and sends the others away, those propose to the best pattern whose last kept
+// key is below theirs, and so on.  Inside a pattern the walk hands out slots in descending key order, so the
+// patterns' lists are kept sorted and are the result.
+//
+// The walk batched by "until the next pattern fills", which this replaced, took up to one round per pattern
+// over all free columns (6 / 28 / 70 rounds for 2:4, 2:8, 4:8).  Random weights need 4 / 7 / 8 rounds here,
+// and all but the first concern a few columns: 13 of 96 are sent away in total (2:4:16), 113 of 896
+// (2:8:32), 299 of 2240 (4:8:32).
+//
+// Later rounds insert proposals into the lists lane by lane (the code says how).  4096 x 4096 2:4:16 fp16: 99 -> 60 us,
+// 8192 x 8192 2:8:32: 727 -> 230 us, 4096 x 4096 4:8:32: 390 -> 160 us; of the 230 us, tile data and results take 55,
+// the first proposals 15, the first round 43; the later rounds are chains of LDS round trips.
+//
+// A round over all columns:
+//   1. every pending column computes its proposal (one thread per column; threshold of a pattern = key of its
+//      last slot, 0 while it has room);
+//   2. counting sort of the proposals by pattern;
+//   3. every proposal finds its rank: proposals of its pattern that are larger (all pairs) plus kept keys
+//      that are larger (binary search); every kept key of a pattern with proposals moves down by the
+//      proposals above it;
+//   4. what ranks below the pattern's capacity is written to its slot, the rest is pending.
+// Columns that have no pattern with room and a positive score wait.  In the walk they come last, together
+// with the zero columns beyond the end of the group dim, in descending column order, and each takes the
+// largest pattern with room: that is written in closed form.
+//
+// A block that reaches beyond the end of the sparse dim has positions that are zero for every column, so patterns
+// that agree in the real positions tie for every column: all columns propose to the largest of such a class, and
+// one pattern's worth of them is kept in a round.  `match_partial` does the first rounds of such a tile.
+#pragma once
+#include "nmg_common.h"
+
+#include <algorithm>
+
+namespace nmg {
+
+constexpr int match_binom(int m, int n)
+{
+    long r = 1;
+    for (int i = 1; i <= n; i++) r = r * (m - n + i) / i;
+    return (int)r;
+}
+
+// The patterns of n:m as position masks in the library's order (nmg_runtime.hip), at compile time.
+template <int N, int M> struct MatchMasks {
+    uint8_t mask[match_binom(M, N)] = {};
+    constexpr int fill(int at, int n, int m, bool flip, int high)
+    {
+        if (n == m || n == 0) {
+            mask[at] = (uint8_t)(((1 << n) - 1) | high);
+            return at + 1;
+        }
+        const int mid = fill(at, n, m - 1, true, high);
+        if (flip)
+            for (int i = at, j = mid - 1; i < j; i++, j--) {
+                const uint8_t t = mask[i];
+                mask[i] = mask[j];
+                mask[j] = t;
+            }
+        return fill(mid, n - 1, m - 1, !flip, high | (1 << (m - 1)));
+    }
+    constexpr MatchMasks() { fill(0, N, M, false, 0); }
+};
+
+struct MatchParams {
+    const void *dense;
+    void *val;
+    int16_t *idx;
+    ViewDev view;
+    int64_t outer;
+    int n, m, g, c, cols;
+    int region_bytes, r_mem, r_arr, r_int;     // LDS bytes of one tile, offsets inside
+    int unit;                                  // bytes of one load of the tile data (16, 8, 4, or one element)
+    int out4;                                  // four slots per thread on the way out
+    uint32_t masks[32];                        // position mask of every pattern, four per word
+    uint64_t magic_cols, magic_g;
+};
+
+template <int NT> __device__ __forceinline__ void match_sync()
+{
+    if (NT <= 64) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
+// Inclusive prefix sum over 64, 32 or 16 consecutive lanes: DPP shifts inside the rows of 16 lanes, then lane
+// 15 of rows 0 and 2 into rows 1 and 3, then lane 31 into rows 2 and 3.
+template <int CTRL, int ROWS> __device__ __forceinline__ int match_dpp(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, CTRL < 0x140);
+}
+template <int LANES> __device__ __forceinline__ int match_prefix(int v)
+{
+    v += match_dpp<0x111, 0xF>(v);
+    v += match_dpp<0x112, 0xF>(v);
+    v += match_dpp<0x114, 0xF>(v);
+    v += match_dpp<0x118, 0xF>(v);
+    if (LANES >= 32) v += match_dpp<0x142, 0xA>(v);
+    if (LANES == 64) v += match_dpp<0x143, 0xC>(v);
+    return v;
+}
+
+template <int CTRL> __device__ __forceinline__ uint64_t match_swap(uint64_t v)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, 0xF, 0xF, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, 0xF, 0xF, true);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+__device__ __forceinline__ float match_abs(float x) { return fabsf(x); }
+__device__ __forceinline__ float match_abs(__half x) { return fabsf(__half2float(x)); }
+__device__ __forceinline__ float match_abs(__hip_bfloat16 x) { return fabsf(__bfloat162float(x)); }
+
+// Key of the edge (column o, pattern p): patterns below each other in descending order of the number that they
+// put on top, so that a group of proposals is followed by smaller keys.  0: none.
+__device__ __forceinline__ uint64_t match_key(uint32_t score, int o, int p)
+{
+    return ((uint64_t)(((uint32_t)(127 - p) << 16) | (score >> 16)) << 32) | ((score << 16) | (uint32_t)o);
+}
+__device__ __forceinline__ int match_pattern(uint64_t key) { return 127 - (int)(key >> 48); }
+__device__ __forceinline__ int match_column(uint64_t key) { return (int)(key & 0xFFFFu); }
+
+constexpr int kMatchTables = 6;      // c ints each, and four counts (three of them for partial blocks only)
+constexpr int kMatchPad = 64;        // bytes behind the proposals: a batch of eight keys past the end of the last group
+
+// First rounds of a tile with `real_rows` < m real positions.  All columns' keys are sorted by pattern and key in
+// every round (compare-exchange network), since most of them are refused and sit in few, long groups.  A refused
+// column skips the patterns of its class that those ahead of it are certain to fill: all of them that have no other
+// class with the same score to turn to, which bit 0 of a key says here.  Stops when at most `few` columns are pending;
+// leaves s_mem, s_occ, the waiting columns in s_np[1] and the pending ones in s_arr and s_np[0].
+// A function of its own: its registers are not those of the other tiles.
+template <typename T, int NT>
+__device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, int r_int, int c, int m, int g, int so, int sr,
+                                           int real_cols, int real_rows, int few)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    for (int *x : {&region_at, &r_mem, &r_arr, &r_int, &c, &m, &g, &so, &sr, &real_cols, &real_rows, &few})
+        *x = __builtin_amdgcn_readfirstlane(*x);      // (arguments come in vector registers)
+    const uint32_t *s_mask = (const uint32_t *)smem + c;
+    const T *s_d = (const T *)(smem + region_at);
+    uint64_t *s_mem = (uint64_t *)(smem + region_at + r_mem), *s_arr = (uint64_t *)(smem + region_at + r_arr);
+    int *s_dem = (int *)(smem + region_at + r_int), *s_start = s_dem + c, *s_occ = s_start + c;
+    int *s_list = s_occ + c, *s_at = s_list + c, *s_last = s_at + c, *s_np = s_last + c;      // the classes, largest patterns first
+    const int tt = threadIdx.x % NT, real_mask = (1 << real_rows) - 1;
+    auto column = [](uint64_t key) { return (int)((key >> 1) & 0x7FFFu); };
+    auto propose = [&](int o, uint32_t at_score, int below) -> uint64_t {      // at that score only patterns up to `below`
+        float a[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++) a[r] = match_abs(s_d[o * so + min(r, m - 1) * sr]);
+        uint32_t best = 0, bmask = 0;
+        int bp = 0;
+        bool tied = false;
+        for (int p = 0; p < c; p++) {
+            const uint32_t mk = __builtin_amdgcn_readfirstlane(s_mask[p]);
+            const uint64_t last = s_mem[p * g + g - 1];
+            float acc = 0;
+#pragma unroll
+            for (int r = 0; r < 7; r++) {
+                if (r >= real_rows) break;
+                acc += (mk >> r) & 1 ? a[r] : 0.f;      // (adding 0 changes nothing)
+            }
+            const uint32_t sb = __float_as_uint(acc);
+            if (sb >= best && !(sb == at_score && p > below) && match_key(sb, o << 1, p) > last) {
+                tied = sb == best && (tied || ((mk ^ bmask) & real_mask) != 0);
+                best = sb;
+                bp = p;
+                bmask = mk;
+            }
+        }
+        return best == 0 ? 0 : match_key(best, o << 1, bp) | (tied ? 1 : 0);
+    };
+    for (int p = tt; p < c; p += NT) {
+        int before = 0, above = 0, size = 0;      // patterns of classes with a smaller mask, of the same one
+        for (int q = 0; q < c; q++) {
+            const int x = (int)(s_mask[q] & real_mask), y = (int)(s_mask[p] & real_mask);
+            before += x < y ? 1 : 0;
+            size += x == y ? 1 : 0;
+            above += x == y && q > p ? 1 : 0;
+        }
+        s_list[before + above] = p;
+        s_at[p] = before + above;
+        s_last[p] = before + size - 1;
+    }
+    for (int e = tt; e < real_cols; e += NT) s_arr[e] = propose(e, 0, 0);
+    int span = 1;      // log2
+    while ((1 << span) < real_cols) span++;
+    int left = 0;
+    for (int round = 0; round < real_cols * c + 2; round++) {
+        match_sync<NT>();
+        if (real_cols <= NT && NT >= 64) {
+            if (tt < 8) s_arr[real_cols + tt] = 0;
+            match_sync<NT>();
+            // one key per thread: its place is the number of larger ones (waiting columns, 0, go behind)
+            const uint64_t key = tt < real_cols ? s_arr[tt] : 0;
+            int at = 0;
+            for (int e = 0; e < real_cols; e += 8) {
+                uint64_t k8[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) k8[u] = s_arr[e + u];
+#pragma unroll
+                for (int u = 0; u < 8; u++) at += k8[u] > key ? 1 : 0;
+            }
+            match_sync<NT>();
+            if (tt < real_cols) s_arr[tt] = 0;
+            match_sync<NT>();
+            if (key != 0) s_arr[at] = key;
+            match_sync<NT>();
+        } else
+        // every exchange puts the larger key first, so what lies beyond the end takes no part
+        for (int size = 0; size < span; size++)
+            for (int dist = size; dist >= 0; dist--) {
+                for (int e = tt; e < 1 << (span - 1); e += NT) {
+                    const int lo = e & ((1 << dist) - 1), base = (e >> dist) << (dist + 1);
+                    const int i = base + lo, j = dist == size ? base + (2 << dist) - 1 - lo : i + (1 << dist);
+                    if (j < real_cols) {
+                        const uint64_t x = s_arr[i], y = s_arr[j];
+                        if (y > x) {
+                            s_arr[i] = y;
+                            s_arr[j] = x;
+                        }
+                    }
+                }
+                match_sync<NT>();
+            }
+        // groups; first refused column of every pattern that has another class to turn to
+        for (int p = tt; p < c; p += NT) {
+            s_start[p] = 0;
+            s_dem[p] = 0;
+            s_occ[p] = real_cols;
+        }
+        if (tt == 0) s_np[0] = 0;
+        match_sync<NT>();
+        for (int e = tt; e < real_cols; e += NT) {
+            const uint64_t key = s_arr[e], prev = e > 0 ? s_arr[e - 1] : ~0ull;
+            if (key != 0 && (e == 0 || match_pattern(prev) != match_pattern(key))) s_start[match_pattern(key)] = e;
+        }
+        match_sync<NT>();
+        for (int e = tt; e < real_cols; e += NT) {
+            const uint64_t key = s_arr[e], next = e + 1 < real_cols ? s_arr[e + 1] : 0;
+            if (key == 0) continue;
+            const int p = match_pattern(key), r = e - s_start[p];
+            if (next == 0 || match_pattern(next) != p) s_dem[p] = r + 1;
+            if (r == g - 1) s_mem[p * g + g - 1] = key;
+            if (r >= g) {
+                atomicAdd(s_np, 1);
+                if (key & 1) atomicMin(&s_occ[p], e);
+            }
+        }
+        match_sync<NT>();
+        left = s_np[0];
+        match_sync<NT>();
+        if (left <= few) break;
+        for (int e = tt; e < real_cols; e += NT) {
+            const uint64_t key = s_arr[e];
+            if (key == 0) continue;
+            const int p = match_pattern(key), r = e - s_start[p];
+            if (r < g) continue;
+            uint32_t score = 0;
+            int q = p;
+            if ((key & 1) == 0) {
+                score = (uint32_t)(key >> 16);
+                const int to = s_at[p] + (min(e, s_occ[p]) - s_start[p] - g) / g + 1;
+                q = to <= s_last[p] ? s_list[to] : -1;
+            }
+            s_arr[e] = propose(column(key), score, q);
+        }
+    }
+    // the lists, the pending columns in front of s_arr
+    constexpr int MOST = 10;      // keys that a thread holds while it re-orders s_arr
+    uint64_t mine[MOST];
+    int waiting = 0;
+    if (tt == 0) s_np[0] = 0;
+#pragma unroll
+    for (int i = 0; i < MOST; i++) {
+        const int e = tt + NT * i;
+        mine[i] = e < real_cols ? s_arr[e] : 0;
+        if (e < real_cols && mine[i] == 0) waiting++;
+    }
+    if (waiting != 0) atomicAdd(s_np + 1, waiting);
+    match_sync<NT>();
+#pragma unroll
+    for (int i = 0; i < MOST; i++)
+        if (mine[i] != 0) {
+            const int e = tt + NT * i, p = match_pattern(mine[i]), r = e - s_start[p];
+            if (r < g) s_mem[p * g + r] = (mine[i] & ~0xFFFFull) | (uint64_t)column(mine[i]);
+            else s_arr[atomicAdd(s_np, 1)] = (uint64_t)column(mine[i]);
+        }
+    for (int p = tt; p < c; p += NT) {
+        s_occ[p] = min(g, s_dem[p]);
+        s_dem[p] = 0;
+    }
+    match_sync<NT>();
+}
+
+// NT threads per tile, at most CPT columns each.  SN, SM, SG != 0: compiled for that n:m:g.  RC: the columns are
+// the contiguous dim of the dense tensor, and the tile data lies in LDS as [position][column]; otherwise
+// as [column][position].
+template <typename T, int NT, int CPT, int SN, int SM, int SG, bool RC>
+__global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT == 256 ? 5 : NT == 64 ? 6 : 7) void match_kernel(MatchParams Q)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int SC = SM ? match_binom(SM, SN) : 0;
+    constexpr int THREADS = NT <= 64 ? 256 : NT;
+    constexpr int TILES = THREADS / NT;
+    const int n = SN ? SN : Q.n, m = SM ? SM : Q.m, g = SG ? SG : Q.g, c = SC ? SC : Q.c;
+    const int cols = SC && SG ? SC * SG : Q.cols;
+    constexpr int V = 16 / (int)sizeof(T);
+    const int ldc = (cols + V - 1) / V * V;      // RC: columns per line of the tile data
+    const int tid = threadIdx.x;
+    const int tile = tid / NT, tt = tid % NT;
+
+    uint32_t *s_pos = (uint32_t *)smem;      // positions of a pattern, four bits each; behind them their masks
+    const int head_bytes = (c * 8 + 15) & ~15;
+    unsigned char *region = smem + head_bytes + (size_t)tile * Q.region_bytes;
+    T *s_d = (T *)region;
+    uint64_t *s_mem = (uint64_t *)(region + Q.r_mem);     // kept keys, every pattern's in descending order; 0: free slot
+    uint64_t *s_arr = (uint64_t *)(region + Q.r_arr);     // pending columns, then the proposals grouped by pattern
+    int *s_dem = (int *)(region + Q.r_int);               // proposals of the round per pattern
+    int *s_start = s_dem + c;                             // first of them in s_arr
+    int *s_occ = s_start + c;                             // slots taken
+    int *s_np = s_occ + 4 * c;                            // pending columns, waiting columns, pending columns of the later rounds
+
+    // ---- where the tiles lie ----
+    // Workgroups go to the 8 XCDs in turn, each with an L2 of its own, and neighbours along the sparse dim share
+    // 128-byte lines where that dim is contiguous: among every 64 workgroups XCD x takes 8x .. 8x+7.  Last tiles
+    // first: those of the last chunk hold fewer real columns and should not be the tail.
+    int64_t grp = blockIdx.x;
+    if (grp < (int64_t)(gridDim.x & ~63u)) grp = (grp & ~63LL) | ((grp & 7) << 3) | ((grp >> 3) & 7);
+    const T *dense = (const T *)Q.dense;
+    const int64_t nbl = Q.view.num_blocks, per_batch = Q.view.num_chunks * nbl;
+    int64_t wg = (int64_t)gridDim.x - 1 - grp;
+    if (Q.view.S % m != 0 && nbl >= TILES) {
+        // partial blocks take several times as long: their workgroups come first.  Number q of them is holder(q).
+        const int64_t lines = Q.outer / nbl;
+        auto holder = [&](int64_t q) { return ((q + 1) * nbl - 1) / TILES; };
+        if (grp < lines) {
+            wg = holder(grp);
+        } else {      // number `wg` of the others
+            int64_t q = wg * TILES / nbl;
+            while (q < lines && holder(q) - q <= wg) q++;
+            while (q > 0 && holder(q - 1) - (q - 1) > wg) q--;
+            wg += q;
+        }
+    }
+    const int64_t tile0 = wg * TILES;
+    const int64_t b_first = tile0 / per_batch;
+    const int64_t kc_first = (tile0 - b_first * per_batch) / nbl, mb_first = tile0 - b_first * per_batch - kc_first * nbl;
+    auto locate = [&](int tm, int64_t &b, int64_t &kc, int64_t &mb) {
+        b = b_first;
+        kc = kc_first;
+        mb = mb_first + tm;
+        while (mb >= nbl) {
+            mb -= nbl;
+            if (++kc == Q.view.num_chunks) {
+                kc = 0;
+                b++;
+            }
+        }
+    };
+
+    // ---- tile data to LDS, zeros beyond the ends; UB: bytes of one load ----
+    auto load = [&](auto ub) {
+        constexpr int UB = decltype(ub)::value, E = UB / (int)sizeof(T);
+        if constexpr (!RC && SM != 0 && (E > SM || SM % E != 0)) return;      // (the host does not ask for it)
+        using Unit = typename std::conditional<UB == 16, uint4, typename std::conditional<UB == 8, uint2,
+                     typename std::conditional<UB == 4, uint32_t, uint16_t>::type>::type>::type;
+        auto copy_unit = [&](T *dst, const T *src, int valid) {      // `valid` elements of the unit exist
+            if (valid >= E) {
+                *(Unit *)dst = *(const Unit *)src;
+            } else {
+#pragma unroll
+                for (int e = 0; e < E; e++) dst[e] = e < valid ? src[e] : Zero<T>::v();
+            }
+        };
+        if (RC) {
+            // lines of columns: consecutive threads take consecutive units of a line
+            const int upl = ldc / E, total = TILES * m * upl;
+#pragma unroll 4
+            for (int e = tid; e < total; e += THREADS) {
+                const int line = e / upl, o = (e - line * upl) * E;
+                const int tm = TILES == 1 ? 0 : line / m, r = line - tm * m;
+                int valid = 0;
+                const T *src = dense;
+                if (tile0 + tm < Q.outer) {
+                    int64_t b, kc, mb;
+                    locate(tm, b, kc, mb);
+                    if (mb * m + r < Q.view.S) {
+                        src = dense + b * Q.view.stride_b + (kc * cols + o) + (mb * m + r) * Q.view.stride_s;
+                        const int64_t left = min(Q.view.G - kc * cols, (int64_t)cols) - o;
+                        valid = left < 0 ? 0 : left < E ? (int)left : E;
+                    }
+                }
+                copy_unit((T *)(smem + head_bytes + (size_t)tm * Q.region_bytes) + r * ldc + o, src, valid);
+            }
+        } else {
+            // columns of m positions: consecutive threads take the units of a column, then the same column of the
+            // next tile (its neighbour in memory where the sparse dim is contiguous), then the next columns
+            const int upc = max(m / E, 1), across = TILES * upc, walkers = THREADS / across;
+            if (tid < walkers * across) {
+                const int o0 = tid / across, w = tid - o0 * across;
+                const int tm = w / upc, r = (w - tm * upc) * E;
+                T *dst = (T *)(smem + head_bytes + (size_t)tm * Q.region_bytes) + r;
+                const T *src = dense;
+                int real = 0, valid = 0;
+                if (tile0 + tm < Q.outer) {
+                    int64_t b, kc, mb;
+                    locate(tm, b, kc, mb);
+                    const int64_t left = Q.view.S - (mb * m + r);
+                    valid = left < 0 ? 0 : left < E ? (int)left : E;
+                    src = dense + b * Q.view.stride_b + kc * cols * Q.view.stride_g + (mb * m + r) * Q.view.stride_s;
+                    real = (int)min(Q.view.G - kc * cols, (int64_t)cols);
+                }
+                const int64_t sg = Q.view.stride_g;
+                if (valid == E && real == cols) {
+#pragma unroll 4
+                    for (int o = o0; o < cols; o += walkers) copy_unit(dst + o * m, src + o * sg, E);
+                } else {
+                    for (int o = o0; o < cols; o += walkers) copy_unit(dst + o * m, src + o * sg, o < real ? valid : 0);
+                }
+            }
+        }
+    };
+    if (Q.unit == 16) load(std::integral_constant<int, 16>{});
+    else if (Q.unit == 8) load(std::integral_constant<int, 8>{});
+    else if (Q.unit == 4 && (sizeof(T) == 4 || !RC)) load(std::integral_constant<int, 4>{});
+    else load(std::integral_constant<int, (int)sizeof(T)>{});
+    for (int p = tid; p < c; p += THREADS) {
+        uint32_t mk = (Q.masks[p >> 2] >> (8 * (p & 3))) & 0xFFu, pos = 0;
+        s_pos[c + p] = mk;
+        for (int j = 0; mk != 0; j++) {
+            pos |= (uint32_t)(__ffs(mk) - 1) << (4 * j);
+            mk &= mk - 1;
+        }
+        s_pos[p] = pos;
+    }
+    for (int s = tt; s < cols; s += NT) s_mem[s] = 0;
+    for (int p = tt; p < kMatchTables * c + 4; p += NT) s_dem[p] = 0;
+    __syncthreads();
+
+    const bool live = tile0 + tile < Q.outer;
+    int real_cols = cols, real_rows = m;
+    if (live) {
+        int64_t b, kc, mb;
+        locate(tile, b, kc, mb);
+        real_cols = (int)min(Q.view.G - kc * cols, (int64_t)cols);
+        real_rows = (int)min(Q.view.S - mb * m, (int64_t)m);
+    }
+    // the partial blocks among the workgroup's tiles, all threads on one after the other
+    if (Q.view.S % m != 0)
+        for (int tm = 0; tm < TILES && tile0 + tm < Q.outer; tm++) {
+            int64_t b, kc, mb;
+            locate(tm, b, kc, mb);
+            if (mb == nbl - 1)
+                match_partial<T, THREADS>(head_bytes + tm * Q.region_bytes, Q.r_mem, Q.r_arr, Q.r_int, c, m, g, RC ? 1 : m,
+                                          RC ? ldc : 1, (int)min(Q.view.G - kc * cols, (int64_t)cols), (int)(Q.view.S - mb * m), cols / 8);
+        }
+    auto mask_of = [&](int p) { return (int)((Q.masks[p >> 2] >> (8 * (p & 3))) & 0xFFu); };
+    auto group_of = [&](int s) { return SG ? s / SG : (int)(((uint64_t)s * Q.magic_g) >> 32); };
+    auto at = [&](int o, int r) { return RC ? r * ldc + o : o * m + r; };
+
+    // Proposal of column o: its best pattern among those with room or a last key below the column's (the
+    // larger pattern on equal scores); 0 where no such pattern has a positive score.  THR = false: all have room.
+    auto propose = [&](int o, auto thr_tag) -> uint64_t {
+        constexpr bool THR = decltype(thr_tag)::value;
+        float a[8];
+        if (!RC && sizeof(T) == 2 && SM == 8) {
+            const uint4 raw = *(const uint4 *)(s_d + o * 8);
+            T v[8];
+            __builtin_memcpy(v, &raw, 16);
+#pragma unroll
+            for (int r = 0; r < 8; r++) a[r] = match_abs(v[r]);
+        } else if (!RC && sizeof(T) == 2 && SM == 4) {
+            const uint2 raw = *(const uint2 *)(s_d + o * 4);
+            T v[4];
+            __builtin_memcpy(v, &raw, 8);
+#pragma unroll
+            for (int r = 0; r < 8; r++) a[r] = r < 4 ? match_abs(v[r & 3]) : 0.f;
+        } else {
+#pragma unroll
+            for (int r = 0; r < 8; r++) a[r] = r < m ? match_abs(s_d[at(o, r)]) : 0.f;
+        }
+        uint32_t best = 0;
+        int bp = 0, later = 0;
+        auto consider = [&](float acc, int p) {
+            const uint32_t sb = __float_as_uint(acc);
+            bool ok = sb >= best;
+            if (THR) {
+                const uint64_t last = s_mem[p * g + g - 1 + later];
+                ok = ok && match_key(sb, o, p) > last;
+            }
+            if (ok) {
+                best = sb;
+                bp = p;
+            }
+        };
+        if constexpr (SM != 0) {
+            constexpr MatchMasks<SN ? SN : 1, SM ? SM : 1> tab;
+#pragma unroll
+            for (int p = 0; p < SC; p++) {
+                float acc = 0;
+                bool any = false;
+#pragma unroll
+                for (int r = 0; r < SM; r++)
+                    if ((tab.mask[p] >> r) & 1) {
+                        acc = any ? acc + a[r] : a[r];      // left to right, in ascending positions
+                        any = true;
+                    }
+                consider(acc, p);
+                // all sums and thresholds in flight at once would not fit the registers
+                if (SC > 8 && p % 8 == 7) {
+                    if (THR) asm volatile("" : "+v"(later), "+v"(best));
+#pragma unroll
+                    for (int r = 0; r < SM; r++) asm volatile("" : "+v"(a[r]), "+v"(best));
+                }
+            }
+        } else {
+            for (int p = 0; p < c; p++) {
+                const int mk = mask_of(p);
+                float acc = 0;
+#pragma unroll
+                for (int r = 0; r < 8; r++)
+                    if ((mk >> r) & 1) acc += a[r];
+                consider(acc, p);
+            }
+        }
+        return best == 0 ? 0 : match_key(best, o, bp);
+    };
+
+    if (live) {
+        int pend = real_cols;
+        // a quarter of the tile and fewer go on in the registers below
+        const int few = SG != 0 ? cols / 4 : 0;
+        // every proposal that is not the last word of its column is refused once per (column, pattern) at most
+        const int limit = cols * c + 2;
+        if (real_rows < m) {
+            pend = s_np[0];
+            match_sync<NT>();
+        }
+        for (int round = real_rows < m ? 1 : 0; round < limit && pend > (round == 0 ? 0 : few); round++) {
+            const int ns = (pend + NT - 1) / NT;
+            // 1. proposals
+            if (round == 0) {
+                for (int e = tt; e < pend; e += NT) s_arr[e] = propose(e, std::false_type{});
+            } else {
+                for (int e = tt; e < pend; e += NT) s_arr[e] = propose((int)s_arr[e], std::true_type{});
+            }
+            // 2. counting sort by pattern
+            uint64_t key[CPT];
+            int pos[CPT];
+#pragma unroll
+            for (int i = 0; i < CPT; i++) {
+                const int e = tt + NT * i;
+                key[i] = 0;
+                pos[i] = 0;
+                if (i < ns && e < pend) {
+                    key[i] = s_arr[e];      // this thread's own entries
+                    if (key[i] != 0) pos[i] = atomicAdd(&s_dem[match_pattern(key[i])], 1);
+                    else atomicAdd(s_np + 1, 1);      // waits
+                }
+            }
+            match_sync<NT>();
+            if (tt < 64) {
+                constexpr int LANES = NT < 64 ? NT : 64;
+                const int p0 = 2 * tt, p1 = p0 + 1;
+                const int d0 = p0 < c ? s_dem[p0] : 0, d1 = p1 < c ? s_dem[p1] : 0;
+                const int excl = match_prefix<LANES>(d0 + d1) - (d0 + d1);
+                if (p0 < c) s_start[p0] = excl;
+                if (p1 < c) s_start[p1] = excl + d0;
+                if (tt == LANES - 1) s_np[0] = excl + d0 + d1;      // proposals of this round
+            }
+            match_sync<NT>();
+            const int props = s_np[0];
+#pragma unroll
+            for (int i = 0; i < CPT; i++)
+                if (i < ns && key[i] != 0) s_arr[s_start[match_pattern(key[i])] + pos[i]] = key[i];
+            if (tt < 8) s_arr[props + tt] = 0;      // what the last batch of the last group reads
+            match_sync<NT>();
+            // 3. ranks.  Thread e takes the proposal that the sort put at e: the lanes of a wavefront then read the
+            //    same few groups.  A proposal that has seen as many larger keys as its pattern has slots stops.
+            const int nr = (props + NT - 1) / NT;
+#pragma unroll
+            for (int i = 0; i < CPT; i++) {
+                const int e = tt + NT * i;
+                key[i] = 0;
+                if (i < nr && e < props) {
+                    const uint64_t mine = s_arr[e];
+                    const int p = match_pattern(mine), d = s_dem[p];
+                    int r = 0;
+                    if (round > 0) {
+                        const uint64_t *kept = s_mem + p * g;
+                        for (int step = 1 << (31 - __clz(g)); step > 0; step >>= 1)
+                            if (r + step <= g && kept[r + step - 1] > mine) r += step;
+                    }
+                    const uint64_t *grp_k = s_arr + s_start[p];
+                    // whole batches: behind the group lie smaller keys
+                    for (int j0 = 0; j0 < d && r < g; j0 += 8) {
+                        uint64_t k8[8];
+#pragma unroll
+                        for (int u = 0; u < 8; u++) k8[u] = grp_k[j0 + u];
+#pragma unroll
+                        for (int u = 0; u < 8; u++) r += k8[u] > mine ? 1 : 0;
+                    }
+                    key[i] = mine;
+                    pos[i] = r;
+                }
+            }
+            uint64_t mkey[CPT];      // kept keys that move, and by how much
+            int mshift[CPT];
+            if (round > 0) {
+#pragma unroll
+                for (int i = 0; i < CPT; i++) {
+                    const int s = tt + NT * i;
+                    mshift[i] = 0;
+                    if (s < cols) {
+                        const int p = group_of(s), d = s_dem[p];
+                        if (d > 0) {
+                            mkey[i] = s_mem[s];
+                            const uint64_t *grp_k = s_arr + s_start[p];
+                            if (mkey[i] != 0)
+                                for (int j = 0; j < d; j++) mshift[i] += grp_k[j] > mkey[i] ? 1 : 0;
+                        }
+                    }
+                }
+            }
+            if (tt == 0) s_np[0] = 0;
+            match_sync<NT>();
+            // 4. the new lists; what a pattern has no slot for is pending
+            if (round > 0) {
+#pragma unroll
+                for (int i = 0; i < CPT; i++)
+                    if (mshift[i] > 0) {
+                        const int p = match_pattern(mkey[i]);
+                        const int s = tt + NT * i + mshift[i];
+                        if (s - p * g < g) s_mem[s] = mkey[i];
+                        else s_arr[atomicAdd(s_np, 1)] = (uint64_t)match_column(mkey[i]);
+                    }
+            }
+#pragma unroll
+            for (int i = 0; i < CPT; i++)
+                if (i < nr && key[i] != 0) {
+                    const int p = match_pattern(key[i]);
+                    if (pos[i] < g) s_mem[p * g + pos[i]] = key[i];
+                    else s_arr[atomicAdd(s_np, 1)] = (uint64_t)match_column(key[i]);
+                }
+            for (int p = tt; p < c; p += NT) {
+                s_occ[p] = min(g, s_occ[p] + s_dem[p]);
+                s_dem[p] = 0;
+            }
+            match_sync<NT>();
+            pend = s_np[0];
+        }
+
+        if constexpr (SG != 0) {
+            // Later rounds: a few columns.  L lanes hold a pattern's list, one key each in descending order, and insert a
+            // proposal by one shift along the lanes.  A pattern takes at most BUCKET proposals in a round; the rest stay
+            // pending.  In a tile of several wavefronts the first one ends the matching alone, without barriers.
+            constexpr int L = SG <= 16 ? 16 : 32, BUCKET = SG / 2 < 8 ? SG / 2 : 8, EIGHT = 8;
+            static_assert(SG <= 32 && SC * SG % 4 == 0, "a list fits its lanes; lists and buckets fit the proposals' place");
+            uint16_t *pending = (uint16_t *)s_arr, *next = pending + cols;
+            uint64_t *s_bkt = (uint64_t *)(next + cols);
+            {
+                constexpr int I = (CPT + 3) / 4;      // the columns left over come as entries of eight bytes
+                uint16_t o[I];
+#pragma unroll
+                for (int i = 0; i < I; i++) o[i] = tt + NT * i < pend ? (uint16_t)s_arr[tt + NT * i] : 0;
+                match_sync<NT>();
+#pragma unroll
+                for (int i = 0; i < I; i++)
+                    if (tt + NT * i < pend) pending[tt + NT * i] = o[i];
+            }
+            int round = 0;
+            auto late = [&](auto active_tag, int until) {      // threads of the tile that take part
+                constexpr int A = decltype(active_tag)::value, W = A < 64 ? A : 64, WAVES = A / W, ROWS = W / L;
+                const int wave = tt / W, lane = tt % W, row = lane / L, r = lane % L;
+                for (const int limit = cols * c + 2; round < limit && pend > until; round++) {
+                    match_sync<A>();
+                    int *count = s_np + 2 + (round & 1);      // zero; the other one is cleared on the way
+                    auto put = [&](int o, uint64_t key) {
+                        if (key == 0) {
+                            atomicAdd(s_np + 1, 1);
+                            return;
+                        }
+                        const int p = match_pattern(key), place = atomicAdd(&s_dem[p], 1);
+                        if (place < BUCKET) s_bkt[p * BUCKET + place] = key;
+                        else next[atomicAdd(count, 1)] = (uint16_t)o;
+                    };
+                    if (SC > 8 && pend * EIGHT <= A) {
+                        // eight lanes per column, each a part of the patterns
+                        const int e = tt / EIGHT, sub = tt % EIGHT;
+                        if (e < pend) {
+                            const int o = (int)pending[e];
+                            uint32_t best = 0;
+                            int bp = 0;
+#pragma unroll 3
+                            for (int i = 0; i < (SC + EIGHT - 1) / EIGHT; i++) {
+                                const int p = min(sub + EIGHT * i, SC - 1);
+                                const uint32_t ps = s_pos[p];
+                                float acc = match_abs(s_d[at(o, (int)(ps & 15u))]);
+#pragma unroll
+                                for (int j = 1; j < SN; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
+                                const uint32_t sb = __float_as_uint(acc);
+                                if (sb >= best && match_key(sb, o, p) > s_mem[p * SG + SG - 1]) {
+                                    best = sb;
+                                    bp = p;
+                                }
+                            }
+                            uint64_t top = ((uint64_t)best << 32) | (uint32_t)bp;
+                            top = max(top, match_swap<0xB1>(top));       // lanes 1 apart, 2 apart, the two quads
+                            top = max(top, match_swap<0x4E>(top));
+                            top = max(top, match_swap<0x141>(top));
+                            if (sub == 0) put(o, (top >> 32) == 0 ? 0 : match_key((uint32_t)(top >> 32), o, (int)(top & 0xFFu)));
+                        }
+                    } else {
+                        for (int e = tt; e < pend; e += A) {
+                            const int o = (int)pending[e];
+                            put(o, propose(o, std::true_type{}));
+                        }
+                    }
+                    match_sync<A>();
+                    // The patterns with proposals, ROWS at a time; wavefront w has those with p / ROWS = w (mod WAVES).
+                    for (int p0 = 0; p0 < SC; p0 += W) {
+                        const int dl = p0 + lane < SC && (p0 + lane) / ROWS % WAVES == wave ? s_dem[p0 + lane] : 0;
+                        uint64_t open = __ballot(dl > 0);
+                        if (W < 64) open = (open >> (threadIdx.x & 63 & ~(W - 1))) & ((1ull << (W & 63)) - 1);
+                        while (open != 0) {
+                            uint64_t mine_bits = open;
+#pragma unroll
+                            for (int i = 0; i < ROWS; i++) {
+                                if (i < row) mine_bits &= mine_bits - 1;
+                                open &= open - 1;
+                            }
+                            if (mine_bits != 0) {
+                                const int p = p0 + __ffsll((unsigned long long)mine_bits) - 1;
+                                const int d = min(s_dem[p], BUCKET);
+                                uint64_t key = r < SG ? s_mem[p * SG + r] : 0;
+                                const uint64_t was = key;
+                                for (int j = 0; j < d; j++) {
+                                    const uint64_t in = s_bkt[p * BUCKET + j];
+                                    const uint64_t before = match_swap<(L == 16 ? 0x111 : 0x138)>(key);      // row_shr:1, wave_shr:1
+                                    const bool stays = key > in, behind = r == 0 || before > in;
+                                    if (r == SG - 1) {
+                                        const uint64_t out = stays ? in : key;      // what the list has no place for
+                                        if (out != 0) next[atomicAdd(count, 1)] = (uint16_t)match_column(out);
+                                    }
+                                    key = stays ? key : behind ? in : before;
+                                }
+                                if (key != was && r < SG) s_mem[p * SG + r] = key;
+                                if (r == 0) s_dem[p] = 0;
+                            }
+                        }
+                    }
+                    if (tt == 0) s_np[2 + ((round & 1) ^ 1)] = 0;
+                    match_sync<A>();
+                    pend = *count;
+                    uint16_t *t = pending;
+                    pending = next;
+                    next = t;
+                }
+            };
+            if constexpr (NT > 64) {
+                late(std::integral_constant<int, NT>{}, 16);
+                __syncthreads();
+                if (tt < 64) late(std::integral_constant<int, 64>{}, 0);
+                __syncthreads();
+            } else {
+                late(std::integral_constant<int, NT>{}, 0);
+                match_sync<NT>();
+            }
+            if (real_cols - s_np[1] < cols) {      // slots taken per pattern, for the columns that come last
+                for (int p = tt; p < c; p += NT) s_occ[p] = 0;
+                match_sync<NT>();
+                for (int s = tt; s < cols; s += NT)
+                    if (s_mem[s] != 0) atomicAdd(&s_occ[group_of(s)], 1);
+                match_sync<NT>();
+            }
+        }
+
+        // ---- closed form: zero columns beyond the end, then the columns that wait ----
+        // Number k in descending column order takes free slot number k, the slots in descending pattern order.
+        const int placed = real_cols - s_np[1];
+        if (placed < cols) {
+            const int npad = cols - real_cols;
+            int16_t *s_wait = (int16_t *)s_arr;                  // waiting columns in descending order
+            if (placed < real_cols) {
+                int16_t *s_flag = s_wait + cols;
+                for (int o = tt; o < cols; o += NT) s_flag[o] = 0;
+                match_sync<NT>();
+                for (int s = tt; s < cols; s += NT)
+                    if (s_mem[s] != 0) s_flag[match_column(s_mem[s])] = 1;
+                match_sync<NT>();
+                // a column's number: those of the higher runs of LANES columns, then of the higher lanes of its own
+                constexpr int LANES = NT < 64 ? NT : 64;
+                int *s_runs = (int *)(s_flag + cols);
+                const int lane = tt % LANES, nruns = (real_cols + LANES - 1) / LANES;
+                auto waits = [&](int run) {
+                    const int o = run * LANES + lane;
+                    const uint64_t b = __ballot(o < real_cols && s_flag[o] == 0);
+                    return LANES == 64 ? b : (b >> (threadIdx.x & 63 & ~(LANES - 1))) & ((1ull << (LANES & 63)) - 1);
+                };
+                for (int run = tt / LANES; run < nruns; run += NT / LANES) {
+                    const uint64_t b = waits(run);
+                    if (lane == 0) s_runs[run] = __popcll(b);
+                }
+                match_sync<NT>();
+                for (int run = tt / LANES; run < nruns; run += NT / LANES) {
+                    const uint64_t b = waits(run);
+                    int k = 0;
+                    for (int u = run + 1; u < nruns; u++) k += s_runs[u];
+                    if ((b >> lane) & 1) s_wait[k + __popcll(b >> lane) - 1] = (int16_t)(run * LANES + lane);
+                }
+            }
+            if (tt < 64) {
+                constexpr int LANES = NT < 64 ? NT : 64;
+                const int p0 = c - 1 - 2 * tt, p1 = p0 - 1;
+                const int r0 = p0 >= 0 ? g - s_occ[p0] : 0, r1 = p1 >= 0 ? g - s_occ[p1] : 0;
+                const int excl = match_prefix<LANES>(r0 + r1) - (r0 + r1);
+                if (p0 >= 0) s_start[p0] = excl;
+                if (p1 >= 0) s_start[p1] = excl + r0;
+            }
+            match_sync<NT>();
+            for (int e = tt; e < cols; e += NT) {
+                if (s_mem[e] != 0) continue;
+                const int p = group_of(e), k = s_start[p] + (e - p * g) - s_occ[p];
+                const int o = k < npad ? cols - 1 - k : (int)s_wait[k - npad];
+                s_mem[e] = (1ull << 48) | (uint32_t)o;
+            }
+        }
+    }
+
+    // ---- the workgroup's slots, contiguous in val and idx ----
+    __syncthreads();
+    T *val = (T *)Q.val;
+    auto elem = [&](const unsigned char *reg, uint64_t key, uint32_t ps, int j) {
+        const int o = match_column(key), r = (int)((ps >> (4 * j)) & 15u);
+        return ((const T *)reg)[at(o, r)];
+    };
+    if constexpr (SN != 0 && SG % 4 == 0 && SG != 0) {
+        if (Q.out4) {
+            constexpr int BYTES = 4 * SN * (int)sizeof(T);
+            constexpr int W = BYTES % 16 == 0 ? 4 : 2;          // words per store
+            for (int e = 4 * tid; e < TILES * cols; e += 4 * THREADS) {
+                const int tm = TILES == 1 ? 0 : e / cols, slot = e - tm * cols;
+                const int64_t t = tile0 + tm;
+                if (t >= Q.outer) break;
+                const unsigned char *reg = smem + head_bytes + (size_t)tm * Q.region_bytes;
+                T v[4 * SN];
+                int16_t o4[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const uint64_t k = ((const uint64_t *)(reg + Q.r_mem))[slot + u];
+                    const uint32_t ps = s_pos[(slot + u) / SG];
+                    o4[u] = (int16_t)match_column(k);
+#pragma unroll
+                    for (int j = 0; j < SN; j++) v[u * SN + j] = elem(reg, k, ps, j);
+                }
+                const int64_t to = t * (int64_t)cols + slot;
+                uint2 raw;
+                __builtin_memcpy(&raw, o4, 8);
+                *(uint2 *)(Q.idx + to) = raw;
+#pragma unroll
+                for (int w = 0; w < BYTES / (4 * W); w++) {
+                    if constexpr (W == 4) {
+                        uint4 x;
+                        __builtin_memcpy(&x, (const char *)v + 16 * w, 16);
+                        ((uint4 *)(val + to * SN))[w] = x;
+                    } else {
+                        uint2 x;
+                        __builtin_memcpy(&x, (const char *)v + 8 * w, 8);
+                        ((uint2 *)(val + to * SN))[w] = x;
+                    }
+                }
+            }
+            return;
+        }
+    }
+    for (int e = tid; e < TILES * cols; e += THREADS) {
+        const int tm = (int)(((uint64_t)e * Q.magic_cols) >> 32), slot = e - tm * cols;
+        const int64_t t = tile0 + tm;
+        if (t >= Q.outer) break;
+        const unsigned char *reg = smem + head_bytes + (size_t)tm * Q.region_bytes;
+        const uint64_t k = ((const uint64_t *)(reg + Q.r_mem))[slot];
+        const uint32_t ps = s_pos[group_of(slot)];
+        const int64_t to = t * (int64_t)cols + slot;
+        Q.idx[to] = (int16_t)match_column(k);
+        for (int j = 0; j < n; j++) val[to * n + j] = elem(reg, k, ps, j);
+    }
+}
+
+template <typename T, int NT, int CPT, int SN, int SM, int SG, bool RC>
+static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
+{
+    *done = false;
+    constexpr int TILES = NT <= 64 ? 256 / NT : 1, THREADS = NT <= 64 ? 256 : NT;
+    const int cols = Q.cols, m = Q.m, c = Q.c, V = 16 / (int)sizeof(T);
+    if (cols > NT * CPT || c > 128 || (NT < 64 && c > 2 * NT)) return NMG_OK;      // prefix sums: two patterns per lane
+    if ((int64_t)TILES * cols >= 65536) return NMG_OK;                              // the magic divisions hold below 2^16
+    auto up = [](int x, int a) { return (x + a - 1) / a * a; };
+    int off = RC ? m * up(cols, V) * (int)sizeof(T) : up(cols * m * (int)sizeof(T), 16);
+    Q.r_mem = off;
+    off += cols * 8;
+    Q.r_arr = off;
+    off += cols * 8 + kMatchPad;
+    Q.r_int = off;
+    off = up(off + (kMatchTables * c + 4) * 4, 16);
+    // the tiles of a wavefront run the same offsets of their regions: spread them over the banks
+    if (NT < 64)
+        while (off % 256 != (NT == 16 ? 64 : 128)) off += 16;
+    Q.region_bytes = off;
+    const size_t lds = (size_t)up(c * 8, 16) + (size_t)TILES * off;
+    if (lds > 160 * 1024) return NMG_OK;
+    Q.out4 = cols % 4 == 0 && (uintptr_t)Q.val % 16 == 0 && (uintptr_t)Q.idx % 8 == 0;
+    auto kern = match_kernel<T, NT, CPT, SN, SM, SG, RC>;
+    if (lds > 64 * 1024)
+        NMG_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const int64_t grid = (Q.outer + TILES - 1) / TILES;
+    NMG_REQUIRE(grid <= 0x7fffffffLL, NMG_ERR_UNSUPPORTED, "too many tiles (%lld)", (long long)grid);
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(THREADS), lds, stream, Q);
+    NMG_HIP_TRY(hipGetLastError());
+    *done = true;
+    return NMG_OK;
+}
+
+template <typename T, bool RC> static int match_dispatch(MatchParams &Q, hipStream_t stream, bool *done)
+{
+    const int n = Q.n, m = Q.m, g = Q.g;
+    auto is = [&](int a, int b, int d) { return n == a && m == b && g == d; };
+#ifndef MATCH_24
+#define MATCH_24 32, 3
+#define MATCH_18 64, 4
+#define MATCH_36 64, 4
+#define MATCH_28 256, 4
+#define MATCH_48 512, 5
+#endif
+    if (is(2, 4, 16)) return match_launch<T, MATCH_24, 2, 4, 16, RC>(Q, stream, done);
+    if (is(1, 8, 32)) return match_launch<T, MATCH_18, 1, 8, 32, RC>(Q, stream, done);
+    if (is(3, 6, 12)) return match_launch<T, MATCH_36, 3, 6, 12, RC>(Q, stream, done);
+    if (is(2, 8, 32)) return match_launch<T, MATCH_28, 2, 8, 32, RC>(Q, stream, done);
+    if (is(4, 8, 32)) {
+        // (fp32 tiles with the data in LDS leave one workgroup per CU)
+        const int rc = match_launch<T, MATCH_48, 4, 8, 32, RC>(Q, stream, done);
+        if (rc != NMG_OK || *done) return rc;
+    }
+    if (Q.cols <= 64 && Q.c <= 32) return match_launch<T, 16, 4, 0, 0, 0, RC>(Q, stream, done);
+    if (Q.cols <= 128 && Q.c <= 20) return match_launch<T, 32, 4, 0, 0, 0, RC>(Q, stream, done);
+    if (Q.cols <= 256) return match_launch<T, 64, 4, 0, 0, 0, RC>(Q, stream, done);
+    if (Q.cols <= 1024) return match_launch<T, 256, 4, 0, 0, 0, RC>(Q, stream, done);
+    if (Q.cols <= 2560) return match_launch<T, 512, 5, 0, 0, 0, RC>(Q, stream, done);
+    return match_launch<T, 1024, 4, 0, 0, 0, RC>(Q, stream, done);
+}
+
+template <typename T>
+static int match_run(const void *dense, void *val, int16_t *idx, const ViewDev &view, int64_t outer, int n, int m, int g, int c, int cols,
+               hipStream_t stream, bool *done)
+{
+    *done = false;
+    if (m > 8 || n < 1 || c > 128 || cols < 16) return NMG_OK;
+    MatchParams Q{};
+    Q.dense = dense;
+    Q.val = val;
+    Q.idx = idx;
+    Q.view = view;
+    Q.outer = outer;
+    Q.n = n;
+    Q.m = m;
+    Q.g = g;
+    Q.c = c;
+    Q.cols = cols;
+    const int8_t *order = host_order(n, m);
+    NMG_REQUIRE(order != nullptr, NMG_ERR_ARG, "invalid n:m = %d:%d", n, m);
+    for (int p = 0; p < c; p++)
+        for (int j = 0; j < n; j++) Q.masks[p / 4] |= 1u << (8 * (p % 4) + order[p * n + j]);
+    Q.magic_cols = (((uint64_t)1 << 32) + cols - 1) / cols;
+    Q.magic_g = (((uint64_t)1 << 32) + g - 1) / g;
+    const bool rc = view.stride_g == 1 && view.stride_s != 1;
+    // the widest load that every unit of the tile data is aligned to
+    Q.unit = (int)sizeof(T);
+    auto fits = [&](int64_t elements, int ub) { return elements * (int64_t)sizeof(T) % ub == 0; };
+    for (int ub = 16; ub > (int)sizeof(T); ub /= 2) {
+        const bool lines = rc ? fits(cols, ub) && fits(view.stride_s, ub)
+                              : view.stride_s == 1 && fits(m, ub) && fits(view.stride_g, ub);
+        if (lines && fits(view.stride_b, ub) && (uintptr_t)dense % ub == 0) {
+            Q.unit = ub;
+            break;
+        }
+    }
+    return rc ? match_dispatch<T, true>(Q, stream, done) : match_dispatch<T, false>(Q, stream, done);
+}
+
+}  // namespace nmg

@@ -1,0 +1,38 @@
+"""The matching form of the compressor (csrc/nmg_match.h) at the edges of its tiles, against the CPU oracle: values and
+indices must be identical."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import sten_amd as sten
+from helpers import oracle_sparsify, same_bits, to_np
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,m,g", [(2, 4, 16), (1, 8, 32), (2, 8, 32), (3, 6, 12), (4, 8, 32), (2, 6, 5), (3, 8, 24)])
+@pytest.mark.parametrize("along", [0, 1])
+def test_tiles_at_their_edges(n, m, g, dtype, along):
+    # two chunks of the group dim, the second of one column, half of the columns or all but one; blocks that reach
+    # beyond the end by every number of positions; continuous values, few magnitudes, zeros
+    cols = math.comb(m, n) * g
+    gen = torch.Generator().manual_seed(n * 100 + m * 10 + along)
+    extras = (1,) if cols > 1000 else (1, cols // 2, cols - 1)
+    for k, extra in enumerate(extras):
+        for rest in range(m) if cols <= 1000 else (0, 2, m - 1):
+            w = torch.randn(cols + extra, 2 * m + rest, generator=gen) * 0.02
+            if (rest + k) % 3 == 1:
+                w = torch.randint(-3, 4, w.shape, generator=gen).float() * 0.25
+            if (rest + k) % 3 == 2:
+                w[torch.rand(w.shape, generator=gen) < 0.5] = 0
+            w = w.to(dtype)
+            w = w if along == 1 else w.t().contiguous()
+            print(f"case {n}:{m}:{g} {dtype} shape={tuple(w.shape)} along={along}", flush=True)
+            val, idx, _ = oracle_sparsify(w, n, m, along, g, 1 - along)
+            t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
+            assert np.array_equal(to_np(t.idx), idx)
+            assert same_bits(t.val, val)
