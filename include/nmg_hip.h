@@ -225,12 +225,18 @@ int nmg_gemm_nn(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void
 int nmg_gemm_tn(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy,
                 const void *d_bias, int64_t O, int64_t K, int64_t T, int dtype, void *stream);
 
+/* dst [dst_rows, dst_cols] = src [rows, cols] in a 16-bit type, zeros beyond the source; any pitches and
+ * alignments.  Brings operands into the shape of the matrix-core products (row starts, K steps), or a padded
+ * result back.  No counterpart in the reference. */
+int nmg_copy_rows16(const void *d_src, int64_t rows, int64_t cols, int64_t ld_src, void *d_dst, int64_t dst_rows,
+                    int64_t dst_cols, int64_t ld_dst, void *stream);
+
 /* ---- "densefrag": the weight expanded into the register order of V_MFMA_F32_32X32X16, for the
  * products the sparse matrix cores cannot do: patterns that do not fit 2-of-4 groups, and the
  * reduction along the group dim (gradient with respect to the activations).
  * densefrag [OB][K/16][64][8] (dtype F16/BF16): outputs O = G lines (transpose = 0) or S positions
- * (transpose = 1), padded to OB*32 = a multiple of 256; reduction K = the other extent, which
- * must be a multiple of 64; m must be a power of two or three times one (3, 6, 12, 24, 48).  Built from the rowpack operand per call or
+ * (transpose = 1), padded to OB*32 = a multiple of 256; reduction K = the other extent, padded
+ * with zeros to a multiple of 64; m must be a power of two or three times one (3, 6, 12, 24, 48).  Built from the rowpack operand per call or
  * cached by the caller.  No counterpart in the reference. */
 int nmg_densefrag_supported(int n, int m);
 int nmg_densefrag_elems(int64_t O, int64_t K, int64_t *elems);
@@ -280,6 +286,11 @@ int nmg_slotmap(const int16_t *d_idx, int64_t G, int64_t S, int16_t *d_slot, int
 int nmg_sddmm(const void *d_lines, int64_t ld_lines, const void *d_pos, int64_t ld_pos, int64_t T,
               const int16_t *d_slot, int64_t G, int64_t S, void *d_val, int n, int m, int g, int dtype,
               void *stream);
+/* The same for any G and S: the rows of both operands are readable, with zeros behind G and S, up to the next
+ * multiple of 8. */
+int nmg_sddmm_padded(const void *d_lines, int64_t ld_lines, const void *d_pos, int64_t ld_pos, int64_t T,
+                     const int16_t *d_slot, int64_t G, int64_t S, void *d_val, int n, int m, int g, int dtype,
+                     void *stream);
 /* The same with the operands given reduction-contiguous: L^T [G, T] and P^T [S, T] (leading
  * dimensions >= T), as the operands of the weight gradient of torch.mm(W, B) lie in memory
  * (grad_out [R, N] and B [C, N]); T % 8 == 0, any G and S.  Replaces the transposing copies the

@@ -8,7 +8,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libnmg_hip.so")
 SOURCES = ["nmg_runtime.hip", "nmg_sparsify.hip", "nmg_match_f32.hip", "nmg_match_f16.hip", "nmg_match_bf16.hip",
            "nmg_spmm.hip", "nmg_smfmac.hip", "nmg_dense.hip",
-           "nmg_densefrag.hip", "nmg_w4.hip", "nmg_pack.hip", "nmg_sddmm.hip", "nmg_perfect.hip", "nmg_gstream.hip", "nmg_sstream.hip", "nmg_ostream.hip"]
+           "nmg_densefrag.hip", "nmg_w4.hip", "nmg_pack.hip", "nmg_sddmm.hip", "nmg_perfect.hip", "nmg_gstream.hip", "nmg_sstream.hip", "nmg_ostream.hip", "nmg_align.hip"]
 # bench.py's measurement aid: a library of its own, outside the product ABI
 PROBE_LIB = os.path.join(HERE, "libnmg_probe.so")
 PROBE_SOURCES = ["nmg_probe.hip"]

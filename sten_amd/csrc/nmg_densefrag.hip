@@ -19,7 +19,7 @@
 // positions), lane l holds the 8 weights of output ob*32 + l%32 at reduction positions
 // k16*16 + 8*(l/32) + 0..7 -- the A operand of V_MFMA_F32_32X32X16, which the first form of the
 // multiplication used; the 16 x 16 x 32 instruction finds its fragments in it with another lane
-// offset (below).  OB is padded to a multiple of 8 (256 outputs), the reduction extent must be a
+// offset (below).  OB is padded to a multiple of 8 (256 outputs), the reduction extent to a
 // multiple of 64; padding is zero.
 #include "nmg_common.h"
 #include "nmg_tile.h"
@@ -561,8 +561,7 @@ extern "C" int nmg_densefrag_supported(int n, int m)
 extern "C" int nmg_densefrag_elems(int64_t O, int64_t K, int64_t *elems)
 {
     NMG_REQUIRE(O >= 0 && K >= 0 && elems, NMG_ERR_ARG, "invalid extents");
-    NMG_REQUIRE(K % 64 == 0, NMG_ERR_UNSUPPORTED, "the reduction extent must be a multiple of 64");
-    *elems = ((O + 255) / 256) * 256 * K;
+    *elems = ((O + 255) / 256) * 256 * ((K + 63) / 64 * 64);
     return NMG_OK;
 }
 
@@ -573,9 +572,7 @@ extern "C" int nmg_densefrag(const void *d_pk_val, const void *d_pk_pat, int64_t
                 "densefrag needs m to be a power of two or three times one (at most 64), got %d:%d", n, m);
     NMG_REQUIRE(dtype == NMG_F16 || dtype == NMG_BF16, NMG_ERR_UNSUPPORTED, "densefrag takes f16/bf16");
     NMG_REQUIRE(G >= 0 && S >= 0, NMG_ERR_ARG, "negative extent");
-    const int64_t O = transpose ? S : G, K = transpose ? G : S;
-    NMG_REQUIRE(K % 64 == 0, NMG_ERR_UNSUPPORTED, "the reduction extent (%lld) must be a multiple of 64",
-                (long long)K);
+    const int64_t O = transpose ? S : G, K = transpose ? G : S, Kp = (K + 63) / 64 * 64;
     if (O == 0 || K == 0) return NMG_OK;
     NMG_REQUIRE(d_pk_val && d_pk_pat && d_df, NMG_ERR_ARG, "null device pointer");
     DfExpandParams P{};
@@ -587,15 +584,15 @@ extern "C" int nmg_densefrag(const void *d_pk_val, const void *d_pk_pat, int64_t
     P.S = S;
     P.nb = (S + m - 1) / m;
     P.OB = (O + 255) / 256 * 8;
-    P.K16 = K / 16;
+    P.K16 = Kp / 16;
     P.n = n;
     P.m = m;
     P.pat_bytes = binom(m, n) <= 256 ? 1 : 2;
     P.pt = densefrag_tile_positions(m);
     P.bpt = P.pt / m;
     P.transpose = transpose ? 1 : 0;
-    // the grid covers the padded operand: outputs up to a multiple of 256
-    const int64_t Gp = transpose ? G : P.OB * 32, Sp = transpose ? P.OB * 32 : S;
+    // the grid covers the padded operand: outputs up to a multiple of 256, the reduction to one of 64
+    const int64_t Gp = transpose ? Kp : P.OB * 32, Sp = transpose ? P.OB * 32 : Kp;
     const int64_t gx = (Sp + P.pt - 1) / P.pt, gy = (Gp + DFX_L - 1) / DFX_L;
     NMG_REQUIRE(gx <= 0x7fffffffLL && gy <= 65535, NMG_ERR_UNSUPPORTED, "weight too large for one launch");
     dim3 grid((unsigned)gx, (unsigned)gy);

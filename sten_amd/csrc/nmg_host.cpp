@@ -93,6 +93,21 @@ Tensor new_empty(at::IntArrayRef size, const Tensor &like, at::ScalarType dt) { 
 bool aligned16(const Tensor &t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
 
 int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+int64_t round_up(int64_t a, int64_t b) { return up(a, b) * b; }
+
+// t (16-bit, 2-D) as rows of at least `cols` elements that start on 16 bytes, zeros from t's extent on, and at
+// least `rows` of them: t itself where it is that already, else a copy.
+Tensor padded(const Tensor &t, int64_t rows, int64_t cols)
+{
+    const int64_t R = t.size(0), C = t.size(1);
+    const Tensor s = C <= 1 || t.stride(1) == 1 ? t : t.contiguous();
+    if (R == rows && C == cols && (R <= 1 || s.stride(0) % 8 == 0) && aligned16(s)) return s;
+    Tensor out = new_empty({rows, cols}, t);
+    check(nmg_copy_rows16(s.data_ptr(), R, C, R > 1 ? s.stride(0) : C, out.data_ptr(), rows, cols, cols, stream_of(t)));
+    return out;
+}
+
+int64_t pitch_of(const Tensor &t) { return t.size(0) > 1 ? t.stride(0) : t.size(1); }
 
 constexpr int64_t k2G = int64_t(1) << 31;
 constexpr int64_t kOstreamMaxTokens = 4;    // nmg_spmm_ostream: the token rows its lanes hold
@@ -419,8 +434,35 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
     if (kname == "sstream")
         fail("the streaming product along the sparse dim needs 16-bit data, at most 16 tokens, "
              "1:8, 2:8 or 4:8 and a reduction extent that is a multiple of 256");
-    const bool smf_ok = reduce_sparse && K % 8 == 0 && ldx % 8 == 0 && al && half;
+    const bool flat = T * ldx * 2 < k2G;
+    // An extent, a pitch or a start that the matrix-core kernels do not read gets a copy of the activations with
+    // whole K steps of 64 (nmg_align.hip).  The sparse cores' operand holds whole steps anyway, the dense cores'
+    // operand is padded; in both, what lies behind the reduction is zero.  Reductions that are a multiple of 8 but
+    // not of 64 are copied as well from 17 tokens on: the kernel with guarded loads that takes them as they are has
+    // no split reduction (1768 x 2216, 298 tokens: 39 us against 14).
+    const bool plain8 = K % 8 == 0 && ldx % 8 == 0 && al, plain64 = K % 64 == 0 && plain8;
+    const bool pad_ok = half && (automatic || kname == "densefrag") && opt.expand && T * round_up(K, 64) * 2 < k2G && T > 0 && K > 0;
+    const bool smf_pad = pad_ok && automatic && opt.variant == -1 && reduce_sparse && (T > 16 ? plain8 && !plain64 : !plain8)
+                         && nmg_fragpack_supported(q.n, q.m);
+    const bool smf_ok = reduce_sparse && plain8 && half;
     bool packed = false;
+    if (smf_pad) {
+        pack(w);
+        packed = w.ops.fp_val.defined();
+        const int64_t Kp = round_up(K, 64);
+        const Tensor xq = padded(x, T, Kp);
+        const void *fv = w.ops.fp_val.data_ptr(), *fi = w.ops.fp_idx.data_ptr();
+        int slices = 1;
+        int64_t bytes = 0;
+        if (T > 16) check(nmg_splitk_plan(O, Kp, T, &slices, &bytes));
+        if (slices > 1) {
+            Tensor ws = workspace(split_ws(slices, T, O), x);
+            check(nmg_spmm_smfmac_splitk(fv, fi, O, Kp, xq.data_ptr(), pitch_of(xq), yp, O, bp, T, dt, slices, ws.data_ptr(), ws.numel() * 4, stream));
+        } else {
+            check(nmg_spmm_smfmac(fv, fi, O, Kp, xq.data_ptr(), pitch_of(xq), yp, O, bp, T, dt, T <= 16 ? 5 : -1, stream));
+        }
+        return y;
+    }
     if (smf_ok && (automatic || kname == "skinny" || kname == "smfmac")) {
         pack(w);
         packed = w.ops.fp_val.defined();
@@ -431,7 +473,6 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
     if (packed) {
         const void *fv = w.ops.fp_val.data_ptr(), *fi = w.ops.fp_idx.data_ptr();
         long variant = opt.variant;
-        const bool flat = T * ldx * 2 < k2G;
         if (T <= 16 && kname != "smfmac")
             variant = 5;      // decode shapes: streaming kernel on the same operand
         else if (T <= 24 && automatic && variant == -1 && K % 128 == 0 && flat && opt.slices < 0)
@@ -461,14 +502,30 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
     // group dim (the reference's default orientation) 24 / 25 / 26 against 1190 / 1203 / 1286; fp32
     // 65 / 65 / 65 against 70 / 134 / 361.
     const int64_t min_t = automatic ? 1 : 17;
-    const bool flat = T * ldx * 2 < k2G;
     // Few tokens with the reduction along the group dim (what F.linear does with a weight in the
     // reference's default orientation): the compressed lines are streamed once and expanded in
     // registers -- 51 MB instead of the 90 MB of the dense-core operand for 4096 x 11008 at 2:4.
     // ... and with a handful of tokens at 2:4 every workgroup owns 16 outputs over the whole
     // reduction: one kernel, no sums through memory (the token rows are then read by every
     // workgroup, which is why this is for few of them)
-    const bool few_ok = !reduce_sparse && half && K % 8 == 0 && ldx % 8 == 0 && al && flat;
+    if (pad_ok && automatic && !reduce_sparse && T <= kGstreamMaxTokens && !plain8 && nmg_spmm_gstream_supported(q.n, q.m)) {
+        // the streams take lines in groups of 8; those behind the last are zero in the operand and in the copy
+        const int64_t Kp = round_up(K, 8);
+        const Tensor xq = padded(x, T, Kp);
+        if (T <= kOstreamAutoTokens && nmg_spmm_ostream_supported(q.n, q.m)) {
+            opack(w);
+            check(nmg_spmm_ostream(w.ops.op.data_ptr(), Kp, O, xq.data_ptr(), pitch_of(xq), yp, O, bp, T, q.n, q.m, dt, stream));
+            return y;
+        }
+        gpack(w);
+        int slices = 1;
+        int64_t bytes = 0;
+        check(nmg_spmm_gstream_plan(Kp, O, T, q.n, q.m, &slices, &bytes));
+        Tensor ws = workspace(bytes / 4, x);
+        check(nmg_spmm_gstream(w.ops.gp.data_ptr(), Kp, O, xq.data_ptr(), pitch_of(xq), yp, O, bp, T, q.n, q.m, dt, ws.data_ptr(), ws.numel() * 4, stream));
+        return y;
+    }
+    const bool few_ok = !reduce_sparse && half && plain8 && flat;
     if ((automatic || kname == "ostream") && few_ok && T <= (automatic ? kOstreamAutoTokens : kOstreamMaxTokens)
         && nmg_spmm_ostream_supported(q.n, q.m)) {
         opack(w);
@@ -490,12 +547,16 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
     if (kname == "gstream")
         fail("the streaming product along the group dim needs 16-bit data, at most ", kGstreamMaxTokens,
              " tokens, m = 4 or 8 with n = 1 or 2 and a reduction extent that is a multiple of 8");
-    const bool dense16 = T >= min_t && half && K % 64 == 0 && ldx % 8 == 0 && al && flat;
-    if ((automatic || kname == "mfma" || kname == "densefrag") && dense16 && nmg_densefrag_supported(q.n, q.m)
+    const bool dense16 = T >= min_t && half && plain64 && flat;
+    if ((automatic || kname == "mfma" || kname == "densefrag") && (dense16 || (pad_ok && T >= min_t)) && nmg_densefrag_supported(q.n, q.m)
         && (kname == "densefrag" || opt.expand)) {
         // "expand, then multiply": one HBM-bound pass writes the weight in the register order of
         // the dense matrix cores into scratch, the pipelined kernel multiplies from there
         Tensor df = densefrag(w, rd, opt.cache_dense);
+        const int64_t Kp = round_up(K, 64);
+        const Tensor xq = dense16 ? x : padded(x, T, Kp);
+        const void *const xp = xq.data_ptr();
+        const int64_t ldx = dense16 ? (T > 1 ? x.stride(0) : K) : pitch_of(xq), K = Kp;
         int slices = 1;
         int64_t bytes = 0;
         if (opt.dense_variant == -1)
@@ -535,22 +596,17 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
         check(entry(a.data_ptr(), a.stride(0), xp, ldx, yp, O, bp, O, K, T, dt, stream));
         return y;
     }
-    const int64_t Kp = up(K, 64) * 64;
+    const int64_t Kp = round_up(K, 64);
     if (half && T >= (reduce_sparse ? 4 : 1) && automatic && opt.expand && O * Kp * 2 < k2G && T * Kp * 2 < k2G) {
-        // 16-bit shapes that none of the matrix-core routes above takes as they are (a reduction
-        // extent that is not a multiple of 64 or 8, an m such as 5 or 7, unaligned activations):
+        // 16-bit shapes that none of the matrix-core routes above takes (an m such as 5 or 7):
         // a dense copy of the weight with zero-padded rows (kept per weight version) and, where
         // needed, a zero-padded copy of the activations, through the dense 16-bit GEMM -- the
         // kernel below runs at a hundredth of its rate (from 4 tokens on where the reduction runs
         // along the sparse dim: this GEMM does not cut its reduction, and at 1 token the streaming kernel
         // below is ahead, 81 us against 132; along the group dim that kernel takes 470 us at 4096^2)
         Tensor a = dense_operand(w, rd, opt.cache_dense, 64);
-        Tensor xq = x;
-        if (Kp != K || ldx % 8 != 0 || !al || !flat) {
-            xq = at::zeros({T, Kp}, x.options());
-            xq.narrow(1, 0, K).copy_(x);
-        }
-        check(nmg_gemm_nt(a.data_ptr(), Kp, xq.data_ptr(), T > 1 ? xq.stride(0) : Kp, yp, O, bp, O, Kp, T, dt, stream));
+        const Tensor xq = plain64 && flat ? x : padded(x.contiguous(), T, Kp);
+        check(nmg_gemm_nt(a.data_ptr(), Kp, xq.data_ptr(), pitch_of(xq), yp, O, bp, O, Kp, T, dt, stream));
         return y;
     }
     pack(w);
@@ -591,6 +647,15 @@ void check_mm(const State &w, const Tensor &b, int64_t K)
     if (b.scalar_type() != w.val.scalar_type()) fail("dtype mismatch: B ", dtype_name(b), ", weight ", dtype_name(w.val));
 }
 
+Tensor spmm_tt_dense(State &w, Tensor b, int rd);
+
+// The dense matrix cores take B as it lies (padded where needed).
+bool tt_dense_ok(const State &w, const Tensor &b, const Options &opt)
+{
+    return is16(b) && b.size(0) > 0 && b.size(1) > 16 && nmg_densefrag_supported(w.geo.n, w.geo.m) && (opt.kernel == "auto" || opt.kernel == "densefrag")
+           && opt.expand && round_up(b.size(1), 8) < (int64_t(1) << 24);
+}
+
 // C = W @ B (torch.mm): the sparse matrix cores with both dense operands as they lie in memory where
 // they can take it, else the transposed operands through spmm.
 Tensor spmm_tt(State &w, Tensor b)
@@ -602,20 +667,28 @@ Tensor spmm_tt(State &w, Tensor b)
     at::AutoDispatchBelowADInplaceOrView raw;
     const int64_t N = b.size(1);
     const Options opt = options_of(w);
-    bool direct = q.sdim == 1 && is16(b) && C % 64 == 0 && N > 16 && (opt.kernel == "auto" || opt.kernel == "smfmac");
-    if (direct && b.stride(1) != 1) b = b.contiguous();
-    if (direct && (b.stride(0) % 8 != 0 || !aligned16(b))) direct = false;
-    if (direct) {
+    bool direct = q.sdim == 1 && is16(b) && N > 16 && C > 0 && round_up(N, 8) < (int64_t(1) << 24) && (opt.kernel == "auto" || opt.kernel == "smfmac");
+    if (direct && nmg_fragpack_supported(q.n, q.m)) {
         pack(w);
         direct = w.ops.fp_val.defined();
+    } else {
+        direct = false;
     }
     if (!direct) {
         Tensor c = mm_f32(w, b, 1, opt);
         if (c.defined()) return c;
+        // the dense cores take B as it lies too: fewer launches, and the padding of odd extents happens once
+        // (large products are faster on a transposed copy, see launch_dense16)
+        if (opt.kernel == "auto" && tt_dense_ok(w, b, opt) && (C % 64 != 0 || N % 8 != 0 || R * C * N < (int64_t(1) << 33)))
+            return spmm_tt_dense(w, b, 1);
         return spmm(w, b.t().contiguous(), Tensor(), 1, nullptr).t();
     }
+    // (whole K steps and pieces of 8 columns: see `padded`)
+    const int64_t Cp = round_up(C, 64);
+    const Tensor bq = b.stride(1) == 1 && b.stride(0) % 8 == 0 && aligned16(b) && b.stride(0) < (int64_t(1) << 24) && C == Cp ? b
+                      : padded(b, Cp, round_up(N, 8));
     Tensor c = new_empty({R, N}, b);
-    check(nmg_spmm_smfmac_tt(w.ops.fp_val.data_ptr(), w.ops.fp_idx.data_ptr(), R, C, b.data_ptr(), b.stride(0), c.data_ptr(), N, nullptr,
+    check(nmg_spmm_smfmac_tt(w.ops.fp_val.data_ptr(), w.ops.fp_idx.data_ptr(), R, Cp, bq.data_ptr(), bq.stride(0), c.data_ptr(), N, nullptr,
                              N, dtype_code(b.scalar_type()), stream_of(b)));
     return c;
 }
@@ -630,18 +703,17 @@ Tensor spmm_tt_dense(State &w, Tensor b, int rd)
     at::AutoDispatchBelowADInplaceOrView raw;
     const int64_t N = b.size(1);
     const Options opt = options_of(w);
-    bool direct = is16(b) && K % 64 == 0 && N > 16 && nmg_densefrag_supported(q.n, q.m)
-                  && (opt.kernel == "auto" || opt.kernel == "densefrag") && opt.expand;
-    if (direct && b.stride(1) != 1) b = b.contiguous();
-    if (direct && (b.stride(0) % 8 != 0 || !aligned16(b) || b.stride(0) >= (int64_t(1) << 24))) direct = false;
-    if (!direct) {
+    if (!tt_dense_ok(w, b, opt)) {
         Tensor c = mm_f32(w, b, rd, opt);
         if (c.defined()) return c;
         return spmm(w, b.t().contiguous(), Tensor(), rd, nullptr).t();
     }
     Tensor df = densefrag(w, rd, opt.cache_dense);
+    const int64_t Kp = round_up(K, 64);
+    const Tensor bq = b.stride(1) == 1 && b.stride(0) % 8 == 0 && aligned16(b) && b.stride(0) < (int64_t(1) << 24) && K == Kp ? b
+                      : padded(b, Kp, round_up(N, 8));
     Tensor c = new_empty({O, N}, b);
-    check(nmg_spmm_densefrag_tt(df.data_ptr(), O, K, b.data_ptr(), b.stride(0), c.data_ptr(), N, nullptr, N, dtype_code(b.scalar_type()),
+    check(nmg_spmm_densefrag_tt(df.data_ptr(), O, Kp, bq.data_ptr(), bq.stride(0), c.data_ptr(), N, nullptr, N, dtype_code(b.scalar_type()),
                                 stream_of(b)));
     return c;
 }
@@ -650,11 +722,8 @@ bool masked_product_supported(const State &w, const Tensor &rows, const Tensor &
 {
     const Geometry &q = w.geo;
     if (q.nd != 2 || !is16(w.val) || rows.scalar_type() != w.val.scalar_type() || cols.scalar_type() != w.val.scalar_type()) return false;
-    for (const Tensor *t : {&rows, &cols})
-        if (t->stride(1) == 1 && (t->stride(0) % 8 != 0 || !aligned16(*t))) return false;
-    const int64_t pitch = std::max(rows.stride(0), cols.stride(0));
-    if (last) return rows.size(1) % 8 == 0 && pitch < (int64_t(1) << 22);
-    return q.dims[0] % 8 == 0 && q.dims[1] % 8 == 0 && pitch < (int64_t(1) << 25);
+    const int64_t longest = std::max({rows.size(1), cols.size(1), rows.stride(0), cols.stride(0)});
+    return longest < (int64_t(1) << (last ? 21 : 24));
 }
 
 // val of the kept positions of rows^T @ cols (rows [T, R], cols [T, C]; with `last` rows [R, T], cols [C, T]).
@@ -675,24 +744,24 @@ Tensor masked_product(State &w, Tensor rows, Tensor cols, bool last)
         fail("dtype mismatch: operands ", dtype_name(rows), " / ", dtype_name(cols), ", weight ", dtype_name(w.val));
     c10::DeviceGuard device(w.val.device());
     at::AutoDispatchBelowADInplaceOrView raw;
-    if (rows.stride(1) != 1) rows = rows.contiguous();
-    if (cols.stride(1) != 1) cols = cols.contiguous();
+    rows = padded(rows, rows.size(0), round_up(rows.size(1), 8));
+    cols = padded(cols, cols.size(0), round_up(cols.size(1), 8));
     const Tensor &lines = q.gdim == 0 ? rows : cols, &pos = q.gdim == 0 ? cols : rows;
-    const int64_t T = rows.size(td);
+    const int64_t T = rows.size(td);      // (padded with zeros where the tokens are the fast dim)
     if (T == 0) return at::zeros_like(w.val);
     Tensor slot = slotmap(w);
     Tensor val = at::empty_like(w.val);
-    auto entry = last ? nmg_sddmm_nt : nmg_sddmm;
-    check(entry(lines.data_ptr(), lines.stride(0), pos.data_ptr(), pos.stride(0), T, (const int16_t *)slot.data_ptr(), q.G, q.S,
+    auto entry = last ? nmg_sddmm_nt : nmg_sddmm_padded;
+    check(entry(lines.data_ptr(), pitch_of(lines), pos.data_ptr(), pitch_of(pos), T, (const int16_t *)slot.data_ptr(), q.G, q.S,
                 val.data_ptr(), q.n, q.m, q.g, dtype_code(val.scalar_type()), stream_of(val)));
     return val;
 }
 
 // Dense product on this library's matrix-core kernels, operands as they lie in memory: tn: x [K, T],
 // a [K, O] -> x^T @ a;  nt: x [T, K], a [O, K] -> x @ a^T.  fp32 always; 16-bit types where the kernels take
-// the shape (extents and pitches that are multiples of 8, 16-byte aligned bases; nt: K a multiple of 64) --
-// other 16-bit shapes go through the fp32 kernel (operands widened, result rounded once).  Undefined where
-// that does not take them either (double, more than 2 097 120 tokens).
+// the shape (extents and pitches that are multiples of 8, 16-byte aligned bases; nt: K a multiple of 64),
+// else padded copies of the operands and, tn, a padded result.  Undefined where neither applies (double, extents
+// beyond the kernels').
 Tensor dense_product(bool tn, Tensor x, Tensor a)
 {
     const at::ScalarType dt = x.scalar_type();
@@ -704,21 +773,32 @@ Tensor dense_product(bool tn, Tensor x, Tensor a)
     at::AutoDispatchBelowADInplaceOrView raw;
     if (x.stride(1) != 1) x = x.contiguous();
     if (a.stride(1) != 1) a = a.contiguous();
-    bool ok;
-    if (half) {
-        ok = x.stride(0) % 8 == 0 && a.stride(0) % 8 == 0 && aligned16(x) && aligned16(a) && O % 8 == 0
-             && std::max(x.stride(0), a.stride(0)) < (int64_t(1) << 24);
-        ok = ok && (tn ? T % 8 == 0 : K % 64 == 0 && O * a.stride(0) * 2 < k2G && T * x.stride(0) * 2 < k2G);
-    } else {
-        ok = up(T, 32) <= 65535;
+    void *const stream = stream_of(x);
+    if (!half) {
+        if (up(T, 32) > 65535) return Tensor();
+        Tensor y = new_empty({T, O}, x);
+        auto entry = tn ? nmg_gemm_tn : nmg_gemm_nt;
+        check(entry(a.data_ptr(), a.stride(0), x.data_ptr(), x.stride(0), y.data_ptr(), O, nullptr, O, K, T, dtype_code(dt), stream));
+        return y;
     }
-    if (!ok) {
-        if (half && up(T, 32) <= 65535) return dense_product(tn, x.to(at::kFloat), a.to(at::kFloat)).to(dt);
-        return Tensor();
+    if (tn) {
+        const int64_t T8 = round_up(T, 8), O8 = round_up(O, 8);
+        if (std::max({T8, O8, x.stride(0), a.stride(0)}) >= (int64_t(1) << 24)) return Tensor();
+        x = padded(x, K, T8);
+        a = padded(a, K, O8);
+        Tensor y = new_empty({T8, O8}, x);
+        check(nmg_gemm_tn(a.data_ptr(), pitch_of(a), x.data_ptr(), pitch_of(x), y.data_ptr(), O8, nullptr, O8, K, T8, dtype_code(dt), stream));
+        if (O8 == O) return T8 == T ? y : y.narrow(0, 0, T);
+        Tensor out = new_empty({T, O}, x);
+        check(nmg_copy_rows16(y.data_ptr(), T, O, O8, out.data_ptr(), T, O, O, stream));
+        return out;
     }
+    const int64_t K64 = round_up(K, 64);
+    if (O * std::max(K64, a.stride(0)) * 2 >= k2G || T * std::max(K64, x.stride(0)) * 2 >= k2G) return Tensor();
+    x = padded(x, T, K64);
+    a = padded(a, O, K64);
     Tensor y = new_empty({T, O}, x);
-    auto entry = tn ? nmg_gemm_tn : nmg_gemm_nt;
-    check(entry(a.data_ptr(), a.stride(0), x.data_ptr(), x.stride(0), y.data_ptr(), O, nullptr, O, K, T, dtype_code(dt), stream_of(x)));
+    check(nmg_gemm_nt(a.data_ptr(), pitch_of(a), x.data_ptr(), pitch_of(x), y.data_ptr(), O, nullptr, O, K64, T, dtype_code(dt), stream));
     return y;
 }
 
@@ -896,7 +976,7 @@ PyObject *get_frag_cache(PyObject *self, void *)
     HOST_CATCH(nullptr)
 }
 
-// {reduction direction, or (direction, pitch) where the rows are padded: dense copy}
+// {reduction direction, or (direction, extent) where the reduction is padded: dense copy, as rows or in fragment order}
 PyObject *get_dense_cache(PyObject *self, void *)
 {
     HOST_TRY
@@ -907,6 +987,13 @@ PyObject *get_dense_cache(PyObject *self, void *)
         for (auto &e : o.dense[rd]) {
             PyObject *k = e.first == w.geo.dims[rd] ? PyLong_FromLong(rd) : Py_BuildValue("(iL)", rd, (long long)e.first);
             PyObject *t = wrap(e.second);
+            PyDict_SetItem(d, k, t);
+            Py_DECREF(k);
+            Py_DECREF(t);
+        }
+    for (int rd = 0; rd < 2; rd++)
+        if (o.frag[rd].defined() && w.geo.dims[rd] % 64 != 0) {
+            PyObject *k = Py_BuildValue("(iL)", rd, (long long)round_up(w.geo.dims[rd], 64)), *t = wrap(o.frag[rd]);
             PyDict_SetItem(d, k, t);
             Py_DECREF(k);
             Py_DECREF(t);
@@ -1075,7 +1162,10 @@ PyObject *py_masked_product(PyObject *self, PyObject *args)
     int last = 0;
     if (!PyArg_ParseTuple(args, "OOp", &r, &c, &last)) return nullptr;
     State &w = state_of(self);
-    return with_val(self, masked_product(w, tensor_arg(r, "rows_op"), tensor_arg(c, "cols_op"), last != 0));
+    const Tensor rows = tensor_arg(r, "rows_op"), cols = tensor_arg(c, "cols_op");
+    if (last && rows.dim() == 2 && rows.size(1) % 8 != 0)      // (the backward of torch.mm pads its operands)
+        fail("reduction-contiguous operands need a token count that is a multiple of 8, got ", rows.size(1));
+    return with_val(self, masked_product(w, rows, cols, last != 0));
     HOST_CATCH(nullptr)
 }
 
@@ -1085,7 +1175,8 @@ PyObject *py_masked_product_supported(PyObject *self, PyObject *args)
     PyObject *r, *c;
     int last = 0;
     if (!PyArg_ParseTuple(args, "OOp", &r, &c, &last)) return nullptr;
-    return PyBool_FromLong(masked_product_supported(state_of(self), tensor_arg(r, "rows_op"), tensor_arg(c, "cols_op"), last != 0));
+    const Tensor rows = tensor_arg(r, "rows_op"), cols = tensor_arg(c, "cols_op");
+    return PyBool_FromLong(masked_product_supported(state_of(self), rows, cols, last != 0) && !(last && rows.size(1) % 8 != 0));
     HOST_CATCH(nullptr)
 }
 
@@ -1265,8 +1356,8 @@ int grad_kind(const Dispatch &d, PyObject *weight, PyObject *wrapped)
 }
 
 // val-layout gradient: the kept positions of lhs^T @ rhs (lhs [T, rows of W], rhs [T, columns of W]).  16-bit weights
-// take the fused kernel, which never stores the dense product; fp32 and extents that are not multiples of 8 go
-// through the dense product and the same-pattern gather.
+// take the fused kernel, which never stores the dense product; fp32 goes through the dense product and the
+// same-pattern gather.
 Tensor masked_weight_grad(State &w, const Tensor &lhs, Tensor rhs)
 {
     if (rhs.scalar_type() != w.val.scalar_type()) rhs = rhs.to(w.val.scalar_type());

@@ -293,7 +293,8 @@ __global__ __launch_bounds__(256, 1) void sddmm16_kernel(SddmmParams P)
     // beyond the extent repeat the last one (never stored).
     const bool is_l = wave >= 2;
     const unsigned char *gsrc = (const unsigned char *)(is_l ? P.lop : P.pop);
-    const int64_t ld = is_l ? P.ldl : P.ldp, ext = is_l ? P.G : P.S, f0 = is_l ? l0 : p0;
+    const int64_t ld = is_l ? P.ldl : P.ldp, f0 = is_l ? l0 : p0;
+    const int64_t ext = NT ? (is_l ? P.G : P.S) : ((is_l ? P.G : P.S) + 7) & ~(int64_t)7;      // (rows end on whole pieces)
     uint32_t g_off[SD_LPW];
 #pragma unroll
     for (int i = 0; i < SD_LPW; i++) {
@@ -725,7 +726,7 @@ extern "C" int nmg_slotmap(const int16_t *d_idx, int64_t G, int64_t S, int16_t *
     return NMG_OK;
 }
 
-static int sddmm_impl(bool nt, const void *d_lines, int64_t ld_lines, const void *d_pos, int64_t ld_pos, int64_t T,
+static int sddmm_impl(bool nt, bool padded, const void *d_lines, int64_t ld_lines, const void *d_pos, int64_t ld_pos, int64_t T,
                       const int16_t *d_slot, int64_t G, int64_t S, void *d_val, int n, int m, int g, int dtype,
                       void *stream)
 {
@@ -734,11 +735,11 @@ static int sddmm_impl(bool nt, const void *d_lines, int64_t ld_lines, const void
     NMG_REQUIRE(G >= 0 && S >= 0 && T >= 0, NMG_ERR_ARG, "negative extent");
     const int64_t cg = binom(m, n) * g;
     NMG_REQUIRE(cg < 32768, NMG_ERR_ARG, "c*g must be below 2^15");
-    NMG_REQUIRE(nt ? (ld_lines >= T && ld_pos >= T) : (ld_lines >= G && ld_pos >= S), NMG_ERR_ARG,
+    NMG_REQUIRE(nt ? (ld_lines >= T && ld_pos >= T) : (ld_lines >= G && ld_pos >= S), NMG_ERR_ARG,      // (and multiples of 8)
                 "leading dimension smaller than row length");
     if (G == 0 || S == 0 || n == 0) return NMG_OK;
     NMG_REQUIRE(T > 0, NMG_ERR_UNSUPPORTED, "no tokens: clear val instead");
-    NMG_REQUIRE((nt || (G % 8 == 0 && S % 8 == 0)) && ld_lines % 8 == 0 && ld_pos % 8 == 0 &&
+    NMG_REQUIRE((nt || padded || (G % 8 == 0 && S % 8 == 0)) && ld_lines % 8 == 0 && ld_pos % 8 == 0 &&
                     ((uintptr_t)d_lines % 16) == 0 && ((uintptr_t)d_pos % 16) == 0,
                 NMG_ERR_UNSUPPORTED, "needs extents and leading dimensions that are multiples of 8 and 16-byte aligned operands");
     NMG_REQUIRE(ld_lines < ((int64_t)1 << (nt ? 22 : 25)) && ld_pos < ((int64_t)1 << (nt ? 22 : 25)), NMG_ERR_UNSUPPORTED,
@@ -878,12 +879,19 @@ extern "C" int nmg_sddmm(const void *d_lines, int64_t ld_lines, const void *d_po
                          const int16_t *d_slot, int64_t G, int64_t S, void *d_val, int n, int m, int g,
                          int dtype, void *stream)
 {
-    return sddmm_impl(false, d_lines, ld_lines, d_pos, ld_pos, T, d_slot, G, S, d_val, n, m, g, dtype, stream);
+    return sddmm_impl(false, false, d_lines, ld_lines, d_pos, ld_pos, T, d_slot, G, S, d_val, n, m, g, dtype, stream);
+}
+
+extern "C" int nmg_sddmm_padded(const void *d_lines, int64_t ld_lines, const void *d_pos, int64_t ld_pos, int64_t T,
+                                const int16_t *d_slot, int64_t G, int64_t S, void *d_val, int n, int m, int g,
+                                int dtype, void *stream)
+{
+    return sddmm_impl(false, true, d_lines, ld_lines, d_pos, ld_pos, T, d_slot, G, S, d_val, n, m, g, dtype, stream);
 }
 
 extern "C" int nmg_sddmm_nt(const void *d_lines_t, int64_t ld_lines, const void *d_pos_t, int64_t ld_pos, int64_t T,
                             const int16_t *d_slot, int64_t G, int64_t S, void *d_val, int n, int m, int g,
                             int dtype, void *stream)
 {
-    return sddmm_impl(true, d_lines_t, ld_lines, d_pos_t, ld_pos, T, d_slot, G, S, d_val, n, m, g, dtype, stream);
+    return sddmm_impl(true, false, d_lines_t, ld_lines, d_pos_t, ld_pos, T, d_slot, G, S, d_val, n, m, g, dtype, stream);
 }

@@ -32,8 +32,7 @@ class GroupedNMSparsifier:
 def _masked_weight_grad(weight, lhs_t, rhs):
     """val-layout gradient: the kept positions of ``lhs_t^T @ rhs`` (``lhs_t`` [T, rows of W],
     ``rhs`` [T, columns of W]).  16-bit weights take the fused kernel, which never stores the dense
-    product; fp32 (``nmg_gemm_tn``) and extents that are not multiples of 8 go through the dense
-    product and the same-pattern gather."""
+    product; fp32 (``nmg_gemm_tn``) goes through the dense product and the same-pattern gather."""
     if rhs.dtype != weight.dtype:
         rhs = rhs.to(weight.dtype)
     if weight.masked_product_supported(lhs_t, rhs):
@@ -55,9 +54,8 @@ def _dense_product(form, x, a):
     """Dense product on this library's matrix-core kernels, operands as they lie in memory:
     ``"tn"``: x [K, T], a [K, O] -> x^T @ a (``nmg_gemm_tn``);  ``"nt"``: x [T, K], a [O, K] -> x @ a^T
     (``nmg_gemm_nt``).  fp32 always; 16-bit types where the kernels take the shape (extents and
-    pitches that are multiples of 8, 16-byte aligned bases; ``"nt"``: K a multiple of 64) -- other
-    16-bit shapes go through the fp32 kernel (operands widened, result rounded once); only what
-    that does not take either (double, more than 2 097 120 tokens) goes to ``torch.mm``."""
+    pitches that are multiples of 8, 16-byte aligned bases; ``"nt"``: K a multiple of 64), else padded
+    copies of the operands; only what neither takes (double, extents beyond 2^24) goes to ``torch.mm``."""
     y = _host.dense_product(form == "tn", x, a)
     if y is None:
         y = torch.mm(x.t(), a) if form == "tn" else torch.mm(x, a.t())
