@@ -101,7 +101,7 @@ Tensor padded(const Tensor &t, int64_t rows, int64_t cols)
 {
     const int64_t R = t.size(0), C = t.size(1);
     const Tensor s = C <= 1 || t.stride(1) == 1 ? t : t.contiguous();
-    if (R == rows && C == cols && (R <= 1 || s.stride(0) % 8 == 0) && aligned16(s)) return s;
+    if (R == rows && C == cols && (R <= 1 || (s.stride(0) % 8 == 0 && s.stride(0) >= C)) && aligned16(s)) return s;
     Tensor out = new_empty({rows, cols}, t);
     check(nmg_copy_rows16(s.data_ptr(), R, C, R > 1 ? s.stride(0) : C, out.data_ptr(), rows, cols, cols, stream_of(t)));
     return out;
