@@ -1049,6 +1049,7 @@ extern "C" int nmg_gemm_nt(const void *d_a, int64_t lda, const void *d_x, int64_
     if (O == 0 || T == 0) return NMG_OK;
     NMG_REQUIRE(K > 0, NMG_ERR_UNSUPPORTED, "gemm_nt needs K > 0");
     NMG_REQUIRE(d_a && d_x && d_y, NMG_ERR_ARG, "null device pointer");
+    if (dense_rows16_pays(O, T)) return dense_rows16(d_a, lda, d_x, ldx, d_y, ldy, d_bias, O, K, T, dtype, stream);
     DenseParams P{};
     P.pk_val = d_a;
     P.x = d_x;

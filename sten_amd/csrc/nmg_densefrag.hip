@@ -158,6 +158,7 @@ struct DfParams {
     void *y;
     const void *bias;
     int64_t O, K, T, ldx, ldy;
+    int64_t lda;         // ROWA: row pitch of the weight, in elements
     int KP;              // K steps of 64
     int tiles_m, tiles_n;
     // reduction cut into slices (0 / 1: whole): slice s of a tile stores its sums in single
@@ -201,7 +202,11 @@ template <> struct DfMma16<__hip_bfloat16> {
     __device__ static f32x4 run(F a, F b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 };
 
-template <typename T, int TB, int NH, bool XT = false>
+// ROWA = true takes the weight as rows in memory, A [O, K] with pitch lda, in place of the fragment order: a
+// lane's 16 bytes are those of its output row at the lane's reduction positions, a load touches 64 bytes of 16 rows
+// (the two loads of a K step the two halves of a 128-byte line).  Both operands of Y = X A^T as they lie.
+// CT = true stores the result transposed, C [O, T].
+template <typename T, int TB, int NH, bool XT = false, bool CT = XT, bool ROWA = false>
 __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
 {
     using Mm = DfMma16<T>;
@@ -246,9 +251,19 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     const unsigned char *av_base[2];
 #pragma unroll
     for (int o = 0; o < 2; o++)
-        av_base[o] = (const unsigned char *)P.df + (((int64_t)(ob0 + o) * KPT + kp_lo) * 4) * 1024;
+        av_base[o] = (const unsigned char *)P.df +
+                     (ROWA ? (int64_t)kp_lo * 128 : (((int64_t)(ob0 + o) * KPT + kp_lo) * 4) * 1024);
     const int r16 = lane & 15, kq = lane >> 4;
     const uint32_t lane_a = (uint32_t)((kq >> 1) * 1024 + ((kq & 1) * 32 + r16) * 16);
+    uint32_t row_a[ROWA ? AB : 1];
+    if constexpr (ROWA) {
+#pragma unroll
+        for (int ab = 0; ab < AB; ab++) {
+            int64_t row = f0 + wave * 64 + ab * 16 + r16;
+            if (row >= P.O) row = P.O - 1;            // clamped rows are computed, never stored
+            row_a[ab] = (uint32_t)(row * P.lda * 2 + kq * 16);
+        }
+    }
     // K step kp of the activations starts kp * XSTEP bytes into the operand
     const int64_t XSTEP = XT ? 64 * P.ldx * 2 : 128;
     const unsigned char *x_base = (const unsigned char *)P.x + (int64_t)kp_lo * XSTEP;
@@ -301,10 +316,11 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
 #pragma unroll
                 for (int k32 = 0; k32 < 2; k32++)
                     if (XL + ab * 2 + k32 == i) {
-                        const unsigned char *av = av_base[ab >> 1] + (int64_t)kp * 4096;
+                        const unsigned char *av = av_base[ab >> 1] + (int64_t)kp * (ROWA ? 128 : 4096);
                         asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3"
                                      : "=v"(w.a[ab][k32])
-                                     : "v"(lane_a), "s"(av), "n"(k32 * 2048 + (ab & 1) * 256)
+                                     : "v"(ROWA ? row_a[ROWA ? ab : 0] : lane_a), "s"(av),
+                                       "n"(ROWA ? k32 * 64 : k32 * 2048 + (ab & 1) * 256)
                                      : "memory");
                     }
         }
@@ -492,13 +508,13 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
         return;
     }
     const TileOut out{P.y, P.bias, P.O, P.T, P.ldy};
-    if constexpr (XT)
+    if constexpr (CT)
         store_tile16_t<T, AB, TB>(acc, smem + wave * (AB * 16 * (TT * 2 + 16)), lane, f0 + wave * 64, t0, out);
     else
         store_tile16<T, AB, TB>(acc, smem + wave * (TT * (AB * 32 + 16)), lane, f0 + wave * 64, t0, out);
 }
 
-template <typename T, int TB, int NH, bool XT = false> static int launch_dense16(DfParams &P, hipStream_t s)
+template <typename T, int TB, int NH, bool XT = false, bool CT = XT, bool ROWA = false> static int launch_dense16(DfParams &P, hipStream_t s)
 {
     constexpr int TT = TB * 16;
     P.tiles_m = (int)((P.O + 255) / 256);
@@ -506,10 +522,10 @@ template <typename T, int TB, int NH, bool XT = false> static int launch_dense16
     const int slices = P.ksplit > 1 ? P.ksplit : 1;
     dim3 grid((unsigned)(P.tiles_m * P.tiles_n * slices));
     constexpr size_t ring = (size_t)DD_NS * TT * 128;
-    constexpr size_t stg = XT ? (size_t)4 * 64 * (TT * 2 + 16) : (size_t)4 * TT * (4 * 32 + 16);
+    constexpr size_t stg = CT ? (size_t)4 * 64 * (TT * 2 + 16) : (size_t)4 * TT * (4 * 32 + 16);
     constexpr size_t lds = ring > stg ? ring : stg;
     static_assert(lds <= 160 * 1024, "LDS");
-    auto k = dense16_direct_kernel<T, TB, NH, XT>;
+    auto k = dense16_direct_kernel<T, TB, NH, XT, CT, ROWA>;
     NMG_HIP_TRY(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k, grid, dim3(256), lds, s, P);
     NMG_HIP_TRY(hipGetLastError());
@@ -520,7 +536,15 @@ template <typename T, int TB, int NH, bool XT = false> static int launch_dense16
     return NMG_OK;
 }
 
-template <typename T> static int launch_dense(DfParams &P, int variant, hipStream_t s)
+static bool dense16_square(int64_t O, int64_t T)
+{
+    const int64_t tm = (O + 255) / 256, t256 = tm * ((T + 255) / 256), t128 = tm * ((T + 127) / 128);
+    const double fill256 = (double)t256 / (double)((t256 + 255) / 256 * 256);
+    const double fill128 = (double)t128 / (double)((t128 + 255) / 256 * 256);
+    return t256 >= 256 && fill256 * 1.055 >= fill128;
+}
+
+template <typename T, bool CT = false> static int launch_dense(DfParams &P, int variant, hipStream_t s)
 {
     // Variant 0: 256 outputs x 128 tokens per workgroup, 1: 256 x 256.  The larger tile moves fewer
     // bytes per flop through the vector caches and is 5-6 % faster per flop in steady state; one
@@ -528,14 +552,36 @@ template <typename T> static int launch_dense(DfParams &P, int variant, hipStrea
     // (A sixteen-phase form of the 256 x 256 tile on the 32 x 32 x 16 instruction once gave wrong
     // values now and then; the forms here pass the static check of their hand-tracked loads and
     // the repeated full-chip test.)
-    if (variant < 0) {
-        const int64_t tm = (P.O + 255) / 256, t256 = tm * ((P.T + 255) / 256), t128 = tm * ((P.T + 127) / 128);
-        const double fill256 = (double)t256 / (double)((t256 + 255) / 256 * 256);
-        const double fill128 = (double)t128 / (double)((t128 + 255) / 256 * 256);
-        variant = (P.ksplit <= 1 && t256 >= 256 && fill256 * 1.055 >= fill128) ? 1 : 0;
-    }
-    if (variant == 1) return launch_dense16<T, 16, 4>(P, s);
-    return launch_dense16<T, 8, 2>(P, s);
+    if (variant < 0) variant = P.ksplit <= 1 && dense16_square(P.O, P.T) ? 1 : 0;
+    if (variant == 1) return launch_dense16<T, 16, 4, false, CT>(P, s);
+    return launch_dense16<T, 8, 2, false, CT>(P, s);
+}
+
+// Y[T, O] = X[T, K] A[O, K]^T (+ bias), both operands rows in memory, on 256 x 256 tiles.  The caller has checked
+// extents, pitches and alignment (nmg_gemm_nt).  Bound by the vector memory path: a weight load touches 16 rows.  us,
+// 256 x 128 kernel of nmg_gemm_nt -> this one: 4096 x 4096, K = 2048 (the weight gradient of torch.mm) 77 -> 68;
+// 16384 x 4096, K = 512 112 -> 94.  On 256 x 128 tiles this form is behind (8192 x 512, K = 4096: 60 -> 83), so it
+// takes the results that fill the chip with 256 x 256 tiles.
+bool dense_rows16_pays(int64_t O, int64_t T) { return dense16_square(O, T); }
+
+int dense_rows16(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy, const void *d_bias,
+                 int64_t O, int64_t K, int64_t T, int dtype, void *stream)
+{
+    DfParams P{};
+    P.df = d_a;
+    P.lda = lda;
+    P.x = d_x;
+    P.y = d_y;
+    P.bias = d_bias;
+    P.O = O;
+    P.K = K;
+    P.T = T;
+    P.ldx = ldx;
+    P.ldy = ldy;
+    P.KP = (int)(K / 64);
+    hipStream_t s = (hipStream_t)stream;
+    return dtype == NMG_F16 ? launch_dense16<__half, 16, 4, false, false, true>(P, s)
+                            : launch_dense16<__hip_bfloat16, 16, 4, false, false, true>(P, s);
 }
 
 }  // namespace nmg
@@ -673,6 +719,33 @@ extern "C" int nmg_spmm_densefrag_tt(const void *d_df, int64_t O, int64_t K, con
     // the 256 x 256 tile, which doubles them per wavefront, measured slower (16384x4096 x 4096
     // columns: 724 against 582 us; the plain product on a transposed copy: 360 + 60 for the copy).
     return dtype == NMG_F16 ? launch_dense16<__half, 8, 2, true>(P, s) : launch_dense16<__hip_bfloat16, 8, 2, true>(P, s);
+}
+
+// C[O, T] = A X^T for X [T, K]: the product above with a transposed result.
+extern "C" int nmg_spmm_densefrag_ct(const void *d_df, int64_t O, int64_t K, const void *d_x, int64_t ldx, void *d_c,
+                                     int64_t ldc, const void *d_bias, int64_t T, int dtype, void *stream)
+{
+    NMG_REQUIRE(dtype == NMG_F16 || dtype == NMG_BF16, NMG_ERR_UNSUPPORTED, "densefrag takes f16/bf16");
+    NMG_REQUIRE(O >= 0 && K >= 0 && T >= 0, NMG_ERR_ARG, "negative extent");
+    NMG_REQUIRE(ldx >= K && ldc >= T, NMG_ERR_ARG, "leading dimension smaller than row length");
+    NMG_REQUIRE(K % 64 == 0 && K > 0 && ldx % 8 == 0 && ((uintptr_t)d_x % 16) == 0, NMG_ERR_UNSUPPORTED,
+                "needs K %% 64 == 0 and 16-byte aligned activation rows");
+    NMG_REQUIRE(T * ldx * 2 < ((int64_t)1 << 31), NMG_ERR_UNSUPPORTED, "activations must be smaller than 2 GiB");
+    if (O == 0 || T == 0) return NMG_OK;
+    NMG_REQUIRE(d_df && d_x && d_c, NMG_ERR_ARG, "null device pointer");
+    DfParams P{};
+    P.df = d_df;
+    P.x = d_x;
+    P.y = d_c;
+    P.bias = d_bias;
+    P.O = O;
+    P.K = K;
+    P.T = T;
+    P.ldx = ldx;
+    P.ldy = ldc;
+    P.KP = (int)(K / 64);
+    hipStream_t s = (hipStream_t)stream;
+    return dtype == NMG_F16 ? launch_dense<__half, true>(P, -1, s) : launch_dense<__hip_bfloat16, true>(P, -1, s);
 }
 
 extern "C" int nmg_spmm_densefrag_splitk(const void *d_df, int64_t O, int64_t K, const void *d_x, int64_t ldx,

@@ -1,0 +1,24 @@
+"""Dense product of two operands as rows in memory, on 256 x 256 tiles and beside their limit."""
+import pytest
+import torch
+
+from sten_amd import native
+from helpers import rel_l2, seeded
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# two roundings of the result (the bias is added to the rounded product), each half an ulp of 2^-10 / 2^-7 relative
+TOL = {torch.float16: 1e-3, torch.bfloat16: 8e-3}
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("O,K,T,pad", [(4096, 64, 4096, 0), (4000, 192, 4090, 8), (8192, 128, 1801, 0), (1, 64, 65537, 0)])
+def test_gemm_nt_square_tiles(O, K, T, pad, dtype):
+    A, X = seeded((O, K + pad), dtype, seed=1).to(DEV), seeded((T, K + pad), dtype, seed=2).to(DEV)
+    bias = seeded((O,), dtype, seed=3).to(DEV)
+    Y = torch.full((T, O + 8), 7.0, dtype=dtype, device=DEV)
+    native.check(native.load().nmg_gemm_nt(native.ptr(A), K + pad, native.ptr(X), K + pad, native.ptr(Y), O + 8, native.ptr(bias), O, K, T,
+                                           native.dtype_code(dtype), None))
+    want = X[:, :K].float() @ A[:, :K].float().t() + bias.float()
+    assert bool((Y[:, O:] == 7.0).all())
+    assert rel_l2(Y[:, :O].float().cpu().numpy(), want.cpu().numpy()) <= TOL[dtype]
