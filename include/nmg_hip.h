@@ -156,6 +156,9 @@ int nmg_spmm_smfmac(const void *d_fp_val, const void *d_fp_idx, int64_t M, int64
 int nmg_spmm_smfmac_tt(const void *d_fp_val, const void *d_fp_idx, int64_t M, int64_t K, const void *d_b,
                        int64_t ldb, void *d_c, int64_t ldc, const void *d_bias, int64_t T, int dtype,
                        void *stream);
+/* The same result from activations X [T, K] (B transposed beforehand, nmg_transpose16): C [M, T] = W * X^T. */
+int nmg_spmm_smfmac_ct(const void *d_fp_val, const void *d_fp_idx, int64_t M, int64_t K, const void *d_x, int64_t ldx,
+                       void *d_c, int64_t ldc, const void *d_bias, int64_t T, int dtype, void *stream);
 
 /* The same product with the reduction cut into slices, for token counts between the decode shapes
  * and a batch that fills the chip (a 4096 x 11008 weight x 17..512 tokens is 16..64 tiles of
@@ -230,6 +233,9 @@ int nmg_gemm_tn(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void
  * result back.  No counterpart in the reference. */
 int nmg_copy_rows16(const void *d_src, int64_t rows, int64_t cols, int64_t ld_src, void *d_dst, int64_t dst_rows,
                     int64_t dst_cols, int64_t ld_dst, void *stream);
+/* dst [cols, dst_cols] = src [rows, cols] transposed in a 16-bit type, zeros from `rows` on; dst_cols a multiple of 8. */
+int nmg_transpose16(const void *d_src, int64_t rows, int64_t cols, int64_t ld_src, void *d_dst, int64_t dst_cols,
+                    int64_t ld_dst, void *stream);
 
 /* ---- "densefrag": the weight expanded into the register order of V_MFMA_F32_32X32X16, for the
  * products the sparse matrix cores cannot do: patterns that do not fit 2-of-4 groups, and the
@@ -258,6 +264,9 @@ int nmg_spmm_densefrag(const void *d_df, int64_t O, int64_t K, const void *d_x, 
  * transpose_b / transpose_c meaning as dace_gnm_mult.py:572-627. */
 int nmg_spmm_densefrag_tt(const void *d_df, int64_t O, int64_t K, const void *d_b, int64_t ldb, void *d_c,
                           int64_t ldc, const void *d_bias, int64_t T, int dtype, void *stream);
+/* The same result from activations X [T, K]: C [O, T] = A * X^T. */
+int nmg_spmm_densefrag_ct(const void *d_df, int64_t O, int64_t K, const void *d_x, int64_t ldx, void *d_c, int64_t ldc,
+                          const void *d_bias, int64_t T, int dtype, void *stream);
 /* nmg_spmm_densefrag with the reduction cut into slices (see nmg_splitk_plan). */
 int nmg_spmm_densefrag_splitk(const void *d_df, int64_t O, int64_t K, const void *d_x, int64_t ldx,
                               void *d_y, int64_t ldy, const void *d_bias, int64_t T, int dtype, int slices,

@@ -95,15 +95,33 @@ bool aligned16(const Tensor &t) { return reinterpret_cast<uintptr_t>(t.data_ptr(
 int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 int64_t round_up(int64_t a, int64_t b) { return up(a, b) * b; }
 
+// t (2-D) with contiguous rows that do not overlap: t itself where they lie so, else a copy.
+Tensor rows_of(const Tensor &t)
+{
+    const int64_t R = t.size(0), C = t.size(1);
+    return (C <= 1 || t.stride(1) == 1) && (R <= 1 || t.stride(0) >= C) ? t : t.contiguous();
+}
+
 // t (16-bit, 2-D) as rows of at least `cols` elements that start on 16 bytes, zeros from t's extent on, and at
 // least `rows` of them: t itself where it is that already, else a copy.
 Tensor padded(const Tensor &t, int64_t rows, int64_t cols)
 {
     const int64_t R = t.size(0), C = t.size(1);
-    const Tensor s = C <= 1 || t.stride(1) == 1 ? t : t.contiguous();
-    if (R == rows && C == cols && (R <= 1 || (s.stride(0) % 8 == 0 && s.stride(0) >= C)) && aligned16(s)) return s;
+    const Tensor s = rows_of(t);
+    if (R == rows && C == cols && (R <= 1 || s.stride(0) % 8 == 0) && aligned16(s)) return s;
     Tensor out = new_empty({rows, cols}, t);
     check(nmg_copy_rows16(s.data_ptr(), R, C, R > 1 ? s.stride(0) : C, out.data_ptr(), rows, cols, cols, stream_of(t)));
+    return out;
+}
+
+// b^T (b [K, N], 16-bit) as rows of Kp >= K elements that start on 16 bytes, zeros from K on.
+Tensor transposed(const Tensor &b, int64_t Kp)
+{
+    const int64_t K = b.size(0), N = b.size(1);
+    if (b.stride(0) == 1 && b.stride(1) != 1) return padded(b.t(), N, Kp);
+    const Tensor s = rows_of(b);
+    Tensor out = new_empty({N, Kp}, b);
+    check(nmg_transpose16(s.data_ptr(), K, N, K > 1 ? s.stride(0) : N, out.data_ptr(), Kp, Kp, stream_of(b)));
     return out;
 }
 
@@ -649,15 +667,57 @@ void check_mm(const State &w, const Tensor &b, int64_t K)
 
 Tensor spmm_tt_dense(State &w, Tensor b, int rd);
 
-// The dense matrix cores take B as it lies (padded where needed).
+// C = op(W) B from a transposed copy of B rather than from B as it lies: the copy (4 us, K N / 0.55 * 10^6 us beyond
+// a few MB) and the kernel on it, whose activation fragments are 16-byte LDS reads, against a kernel whose fragments
+// are transposing reads at half that rate.  us, as it lies -> copy and kernel, sparse / dense cores: 4096 x 4096 x 2048
+// columns 85 -> 52 / 83 -> 66; 512 x 4096 x 4096 75 -> 50 / 70 -> 62; 1024^3 20 -> 15 / 20 -> 18; 768 x 768 x 512
+// 14.3 -> 13.3 / 16.3 -> 15.8; 4096 x 512 x 4096 29 -> 24 / 31 -> 28; 512 x 512 x 64 9.2 -> 11.4 / 10.9 -> 12.8.  What is
+// saved grows with the reduction steps that a CU walks, rounds of 256 tiles times the reduction.  Operands that need
+// a padded copy anyway take the transposed one.
+bool transposed_pays(int64_t O, int64_t K, int64_t N, bool as_it_lies)
+{
+    const int64_t rounds = up(up(O, 256) * up(N, 128), 256);
+    return N * round_up(K, 64) * 2 < k2G && (!as_it_lies || rounds * K >= 768);
+}
+
+// Whether op(W) B with few columns is better cut along the reduction (as spmm does it, its result transposed
+// back) than run whole on the CUs that its tiles occupy.  A reduction step of 64 takes about 0.45 us on the sparse and
+// 0.6 us on the dense cores; the cut saves the steps of all slices but one and costs about 11 us of launches beside
+// the partial sums, written and read once.  us, whole -> cut: sparse cores 4096 x 11008 x 32 columns 81 -> 27, x 512
+// 102 -> 58, 4096 x 4096 x 128 31 -> 25 (8 slices), x 512 32 -> 41 (4 slices); dense cores 1024 x 16384 x 128 141 -> 31,
+// 4096 x 4096 x 512 46 -> 41, x 1024 50 -> 57.
+bool tt_split_pays(const Options &opt, int64_t O, int64_t K, int64_t N, bool sparse)
+{
+    if (opt.kernel != "auto" || opt.variant != -1 || opt.dense_variant != -1 || opt.slices >= 0 || !opt.expand || N * round_up(K, 64) * 2 >= k2G)
+        return false;
+    int slices = 1;
+    int64_t bytes = 0;
+    check(nmg_splitk_plan(O, K, N, &slices, &bytes));
+    const double saved = (double)up(K, 64) * (1.0 - 1.0 / slices) * (sparse ? 0.45 : 0.6);
+    return slices > 1 && saved > 11.0 + (double)slices * (double)(N * O) * 8 / 4e6;
+}
+
+Tensor tt_split(State &w, const Tensor &b, int rd)
+{
+    const int64_t K = b.size(0), N = b.size(1);
+    const Tensor y = spmm(w, transposed(b, round_up(K, 64)).narrow(1, 0, K), Tensor(), rd, nullptr);
+    return N % 8 == 0 ? transposed(y, N) : y.t().contiguous();
+}
+
+bool tt_as_it_lies(const Tensor &b)
+{
+    return b.stride(1) == 1 && b.stride(0) % 8 == 0 && b.stride(0) >= b.size(1) && aligned16(b) && b.stride(0) < (int64_t(1) << 24);
+}
+
+// The dense matrix cores take B as it lies, or a copy of it.
 bool tt_dense_ok(const State &w, const Tensor &b, const Options &opt)
 {
     return is16(b) && b.size(0) > 0 && b.size(1) > 16 && nmg_densefrag_supported(w.geo.n, w.geo.m) && (opt.kernel == "auto" || opt.kernel == "densefrag")
            && opt.expand && round_up(b.size(1), 8) < (int64_t(1) << 24);
 }
 
-// C = W @ B (torch.mm): the sparse matrix cores with both dense operands as they lie in memory where
-// they can take it, else the transposed operands through spmm.
+// C = W @ B (torch.mm): the sparse matrix cores where they can take it, else the dense ones, else the transposed
+// operands through spmm.
 Tensor spmm_tt(State &w, Tensor b)
 {
     const Geometry &q = w.geo;
@@ -677,23 +737,28 @@ Tensor spmm_tt(State &w, Tensor b)
     if (!direct) {
         Tensor c = mm_f32(w, b, 1, opt);
         if (c.defined()) return c;
-        // the dense cores take B as it lies too: fewer launches, and the padding of odd extents happens once
-        // (large products are faster on a transposed copy, see launch_dense16)
-        if (opt.kernel == "auto" && tt_dense_ok(w, b, opt) && (C % 64 != 0 || N % 8 != 0 || R * C * N < (int64_t(1) << 33)))
+        if (opt.kernel == "auto" && tt_dense_ok(w, b, opt))
             return spmm_tt_dense(w, b, 1);
         return spmm(w, b.t().contiguous(), Tensor(), 1, nullptr).t();
     }
     // (whole K steps and pieces of 8 columns: see `padded`)
+    if (tt_split_pays(opt, R, C, N, true)) return tt_split(w, b, 1);
     const int64_t Cp = round_up(C, 64);
-    const Tensor bq = b.stride(1) == 1 && b.stride(0) % 8 == 0 && aligned16(b) && b.stride(0) < (int64_t(1) << 24) && C == Cp ? b
-                      : padded(b, Cp, round_up(N, 8));
+    const bool as_it_lies = tt_as_it_lies(b) && C == Cp;
     Tensor c = new_empty({R, N}, b);
+    if (transposed_pays(R, C, N, as_it_lies)) {
+        const Tensor bt = transposed(b, Cp);
+        check(nmg_spmm_smfmac_ct(w.ops.fp_val.data_ptr(), w.ops.fp_idx.data_ptr(), R, Cp, bt.data_ptr(), pitch_of(bt), c.data_ptr(), N,
+                                 nullptr, N, dtype_code(b.scalar_type()), stream_of(b)));
+        return c;
+    }
+    const Tensor bq = as_it_lies ? b : padded(b, Cp, round_up(N, 8));
     check(nmg_spmm_smfmac_tt(w.ops.fp_val.data_ptr(), w.ops.fp_idx.data_ptr(), R, Cp, bq.data_ptr(), bq.stride(0), c.data_ptr(), N, nullptr,
                              N, dtype_code(b.scalar_type()), stream_of(b)));
     return c;
 }
 
-// op(W) @ B on the dense matrix cores with both dense operands as they lie in memory.
+// op(W) @ B on the dense matrix cores.
 Tensor spmm_tt_dense(State &w, Tensor b, int rd)
 {
     const Geometry &q = w.geo;
@@ -708,11 +773,18 @@ Tensor spmm_tt_dense(State &w, Tensor b, int rd)
         if (c.defined()) return c;
         return spmm(w, b.t().contiguous(), Tensor(), rd, nullptr).t();
     }
+    if (tt_split_pays(opt, O, K, N, false)) return tt_split(w, b, rd);
     Tensor df = densefrag(w, rd, opt.cache_dense);
     const int64_t Kp = round_up(K, 64);
-    const Tensor bq = b.stride(1) == 1 && b.stride(0) % 8 == 0 && aligned16(b) && b.stride(0) < (int64_t(1) << 24) && K == Kp ? b
-                      : padded(b, Kp, round_up(N, 8));
+    const bool as_it_lies = tt_as_it_lies(b) && K == Kp;
     Tensor c = new_empty({O, N}, b);
+    if (transposed_pays(O, K, N, as_it_lies)) {
+        const Tensor bt = transposed(b, Kp);
+        check(nmg_spmm_densefrag_ct(df.data_ptr(), O, Kp, bt.data_ptr(), pitch_of(bt), c.data_ptr(), N, nullptr, N, dtype_code(b.scalar_type()),
+                                    stream_of(b)));
+        return c;
+    }
+    const Tensor bq = as_it_lies ? b : padded(b, Kp, round_up(N, 8));
     check(nmg_spmm_densefrag_tt(df.data_ptr(), O, Kp, bq.data_ptr(), bq.stride(0), c.data_ptr(), N, nullptr, N, dtype_code(b.scalar_type()),
                                 stream_of(b)));
     return c;
@@ -1432,7 +1504,7 @@ struct ProductNode : public torch::autograd::Node {
         State &w = matmul_state(wrapped);
         Tensor b = dense.unpack();
         if (gc.scalar_type() != w.val.scalar_type()) gc = gc.to(w.val.scalar_type());
-        if (task_should_compute_output(1)) out[1] = spmm_tt_dense(w, gc, 0);      // W^T @ grad_out, both as they lie in memory
+        if (task_should_compute_output(1)) out[1] = spmm_tt_dense(w, gc, 0);      // W^T @ grad_out
         if (!task_should_compute_output(0)) return;
         Tensor gw;
         const Tensor r = b.scalar_type() == gc.scalar_type() ? b : b.to(gc.scalar_type());

@@ -296,7 +296,8 @@ constexpr int DR_NS = 4;                // activation stages in LDS (>= DR_D + 1
 // reduction positions of its token -- is four LDS transpose reads (DS_READ_B64_TR_B16: in every
 // group of 16 lanes, lane i receives as element j the 16-bit element i%4 of the 8 bytes addressed
 // by lane 4j + i/4); the epilogue stages [feature][token] and stores token-contiguous rows.
-template <typename T, int FB, int TB, int WM, int WN, int NH, bool XT = false>
+// CT = true alone is that epilogue on activations [T, K]: C = W B with B transposed beforehand.
+template <typename T, int FB, int TB, int WM, int WN, int NH, bool XT = false, bool CT = XT>
 __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
 {
     using S = Smf<T>;
@@ -644,7 +645,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
         return;
     }
     const TileOut out{P.y, P.bias, P.M, P.T, P.ldy};
-    if constexpr (XT)
+    if constexpr (CT)
         smf_store_tile_t<T, FB, TB>(acc, smem + wave * (FB * 32 * (TB * 64 + 16)), lane, f0 + wm * FB * 32,
                                     t0 + wn * TB * 32, out);
     else
@@ -652,7 +653,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
                                   t0 + wn * TB * 32, out);
 }
 
-template <typename T, int FB, int TB, int WM, int WN, int NH, bool XT = false>
+template <typename T, int FB, int TB, int WM, int WN, int NH, bool XT = false, bool CT = XT>
 static int launch_smfmac_direct(SmfParams &P, hipStream_t s)
 {
     constexpr int TF = WM * FB * 32, TT = WN * TB * 32;
@@ -666,11 +667,11 @@ static int launch_smfmac_direct(SmfParams &P, hipStream_t s)
     const int slices = P.ksplit > 1 ? P.ksplit : 1;
     dim3 grid((unsigned)(P.tiles_m * P.tiles_n * slices));
     constexpr size_t ring = (size_t)DR_NS * TT * 128;
-    constexpr size_t stg = XT ? (size_t)4 * FB * 32 * (TB * 64 + 16) : (size_t)4 * TB * 32 * (FB * 64 + 16);
+    constexpr size_t stg = CT ? (size_t)4 * FB * 32 * (TB * 64 + 16) : (size_t)4 * TB * 32 * (FB * 64 + 16);
     constexpr size_t lds = ring > stg ? ring : stg;
     static_assert(lds <= 160 * 1024, "LDS");
     static_assert(!XT || (TT == 128 && WN == 1), "the transposed tile is 64 rows of 128 tokens");
-    auto k = spmm_smfmac_direct_kernel<T, FB, TB, WM, WN, NH, XT>;
+    auto k = spmm_smfmac_direct_kernel<T, FB, TB, WM, WN, NH, XT, CT>;
     NMG_HIP_TRY(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k, grid, dim3(256), lds, s, P);
     NMG_HIP_TRY(hipGetLastError());
@@ -1160,18 +1161,22 @@ static int launch_smfmac_cfg(SmfParams &P, hipStream_t s)
     return NMG_OK;
 }
 
+// The tile of the direct kernel: 6 = 256 x 128, 8 = 256 x 256.
+static int smfmac_tile(const SmfParams &P)
+{
+    // Large-batch default.  The 256 x 256 tile moves a quarter fewer bytes per flop through the
+    // vector caches and is 2-4 % faster per flop in steady state (16384 x 4096 x 4096 tokens:
+    // 267 against 273 us; 8192^2 x 4096, 2:8: 250 against 260); what decides is how the tiles
+    // fill the chip: rounds of 256 tiles, a 256 x 256 tile taking twice the time of a 256 x 128
+    // one (both are one workgroup per CU: 260 and 448 registers per lane).
+    const int64_t tm = (P.M + 255) / 256, t256 = tm * ((P.T + 255) / 256), t128 = tm * ((P.T + 127) / 128);
+    const double cost128 = (double)((t128 + 255) / 256), cost256 = (double)((t256 + 255) / 256) * 2.0 / 1.025;
+    return (P.ksplit <= 1 && cost256 < cost128) ? 8 : 6;
+}
+
 template <typename T> static int launch_smfmac(SmfParams &P, int variant, hipStream_t s)
 {
-    if (variant < 0) {
-        // Large-batch default.  The 256 x 256 tile moves a quarter fewer bytes per flop through the
-        // vector caches and is 2-4 % faster per flop in steady state (16384 x 4096 x 4096 tokens:
-        // 267 against 273 us; 8192^2 x 4096, 2:8: 250 against 260); what decides is how the tiles
-        // fill the chip: rounds of 256 tiles, a 256 x 256 tile taking twice the time of a 256 x 128
-        // one (both are one workgroup per CU: 260 and 448 registers per lane).
-        const int64_t tm = (P.M + 255) / 256, t256 = tm * ((P.T + 255) / 256), t128 = tm * ((P.T + 127) / 128);
-        const double cost128 = (double)((t128 + 255) / 256), cost256 = (double)((t256 + 255) / 256) * 2.0 / 1.025;
-        variant = (P.ksplit <= 1 && cost256 < cost128) ? 8 : 6;
-    }
+    if (variant < 0) variant = smfmac_tile(P);
     switch (variant) {
     case 0: return launch_smfmac_cfg<T, 2, 2, 4, 2, 1>(P, s);  // register-prefetch kernel, 256 lines x 128 tokens: any K
     case 5:                                                     // decode shapes, T <= 16 (staged form: <= 32)
@@ -1331,6 +1336,42 @@ extern "C" int nmg_spmm_smfmac_tt(const void *d_fp_val, const void *d_fp_idx, in
     hipStream_t s = (hipStream_t)stream;
     return dtype == NMG_F16 ? launch_smfmac_direct<__half, 2, 4, 4, 1, 2, true>(P, s)
                             : launch_smfmac_direct<__hip_bfloat16, 2, 4, 4, 1, 2, true>(P, s);
+}
+
+// ---- C[M, T] = W * X^T (+ bias per row) for X [T, K]: the untransposed product with a transposed result ----
+extern "C" int nmg_spmm_smfmac_ct(const void *d_fp_val, const void *d_fp_idx, int64_t M, int64_t K,
+                                  const void *d_x, int64_t ldx, void *d_c, int64_t ldc, const void *d_bias,
+                                  int64_t T, int dtype, void *stream)
+{
+    NMG_REQUIRE(dtype == NMG_F16 || dtype == NMG_BF16, NMG_ERR_UNSUPPORTED,
+                "the sparse matrix cores take f16/bf16 only");
+    NMG_REQUIRE(M >= 0 && K >= 0 && T >= 0, NMG_ERR_ARG, "negative extent");
+    NMG_REQUIRE(ldx >= K && ldc >= T, NMG_ERR_ARG, "leading dimension smaller than row length");
+    NMG_REQUIRE((K % 64) == 0 && K > 0 && (ldx % 8) == 0 && ((uintptr_t)d_x % 16) == 0, NMG_ERR_UNSUPPORTED,
+                "needs K %% 64 == 0 and 16-byte aligned activation rows");
+    NMG_REQUIRE(T * ldx * 2 < ((int64_t)1 << 31), NMG_ERR_UNSUPPORTED, "activations must be smaller than 2 GiB");
+    if (M == 0 || T == 0) return NMG_OK;
+    NMG_REQUIRE(d_fp_val && d_fp_idx && d_x && d_c, NMG_ERR_ARG, "null device pointer");
+    SmfParams P{};
+    P.fp_val = d_fp_val;
+    P.fp_idx = (const uint32_t *)d_fp_idx;
+    P.x = d_x;
+    P.y = d_c;
+    P.bias = d_bias;
+    P.M = M;
+    P.K = K;
+    P.T = T;
+    P.ldx = ldx;
+    P.ldy = ldc;
+    P.MB = (int)((M + 255) / 256 * 8);
+    P.KP = (int)(K / 64);
+    hipStream_t s = (hipStream_t)stream;
+    auto launch = [&](auto tag) -> int {
+        using T16 = decltype(tag);
+        if (smfmac_tile(P) == 8) return launch_smfmac_direct<T16, 2, 8, 4, 1, 4, false, true>(P, s);
+        return launch_smfmac_direct<T16, 2, 4, 4, 1, 2, false, true>(P, s);
+    };
+    return dtype == NMG_F16 ? launch(__half{}) : launch(__hip_bfloat16{});
 }
 
 // ---- the split reduction for callers that cannot allocate -----------------------------------

@@ -54,6 +54,7 @@ SIGNATURES = {
     "nmg_densefrag": (_I, [_P, _P, _I64, _I64, _I, _P, _I, _I, _I, _P]),
     "nmg_spmm_densefrag": (_I, [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _I, _P]),
     "nmg_spmm_densefrag_splitk": (_I, [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _I, _P, _I64, _P]),
+    "nmg_spmm_densefrag_ct": (_I, [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _P]),
     "nmg_spmm_densefrag_tt": (_I, [_P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _P]),
     "nmg_w4_sizes": (_I, [_I64, _I64] + [ctypes.POINTER(ctypes.c_int64)] * 3),
     "nmg_w4_pack": (_I, [_P, _I64, _I64, _I64, _P, _P, _P, _P]),
@@ -70,6 +71,7 @@ SIGNATURES = {
     "nmg_slotmap": (_I, [_P, _I64, _I64, _P, _I, _I, _I, _P]),
     "nmg_sddmm": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I, _I, _I, _I, _P]),
     "nmg_sddmm_padded": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I, _I, _I, _I, _P]),
+    "nmg_transpose16": (_I, [_P, _I64, _I64, _I64, _P, _I64, _I64, _P]),
     "nmg_copy_rows16": (_I, [_P, _I64, _I64, _I64, _P, _I64, _I64, _I64, _P]),
     "nmg_sddmm_nt": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I, _I, _I, _I, _P]),
     "nmg_perfect_nm": (_I, [_P, _I64, _I64, _I64, _P, _P, _I, _I, _I, _P]),
@@ -77,6 +79,7 @@ SIGNATURES = {
     "nmg_noalloc_scratch_bytes": (_I64, []),
     "nmg_noalloc_prepare": (_I, []),
     "nmg_spmm_smfmac_splitk_noalloc": (_I, [_P, _P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _I, _P]),
+    "nmg_spmm_smfmac_ct": (_I, [_P, _P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _P]),
     "nmg_spmm_smfmac_tt": (_I, [_P, _P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _P]),
     "nmg_spmm_gstream_supported": (_I, [_I, _I]),
     "nmg_spmm_gstream_plan": (_I, [_I64, _I64, _I64, _I, _I, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int64)]),

@@ -187,19 +187,18 @@ class GroupedNMTensor(_host.Core):
 
 
 def spmm_tt(weight, b):
-    """C = W @ B for a 2-D ``GroupedNMTensor`` W [R, C] and a dense B [C, N] (``torch.mm``), without
-    transposing copies when the sparse matrix cores can take it (16-bit, 2-of-4 compatible pattern
-    along dim 1, C % 64 == 0, more than 16 columns, B row-contiguous with a row pitch that is a
-    multiple of 8); otherwise through ``spmm`` on the transposed operands."""
+    """C = W @ B for a 2-D ``GroupedNMTensor`` W [R, C] and a dense B [C, N] (``torch.mm``), contiguous where N > 16 and
+    the data is 16-bit.  On the sparse matrix cores where the pattern fits 2 of 4 along dim 1, else on the dense ones:
+    from a transposed copy of B, from B as it lies where that is faster (short reductions), or cut along the reduction
+    (few columns).  What these do not take goes through ``spmm`` on the transposed operands."""
     return _host.spmm_tt(weight, b)
 
 
 def spmm_tt_dense(weight, b, *, reduce_dim):
-    """C = op(W) @ B with both dense operands as they lie in memory, on the dense matrix cores:
+    """C = op(W) @ B on the dense matrix cores:
     ``reduce_dim=0``: B is [R, N], C = W^T @ B is [C, N] (the gradient with respect to B of
-    ``torch.mm(W, B)``); ``reduce_dim=1``: B is [C, N], C = W @ B is [R, N].  Needs 16-bit data, a
-    m that is a power of two or three times one, a reduction extent that is a multiple of 64, more than 16 columns and a B that is
-    row-contiguous with a row pitch that is a multiple of 8; otherwise through ``spmm`` on the
+    ``torch.mm(W, B)``); ``reduce_dim=1``: B is [C, N], C = W @ B is [R, N].  Takes 16-bit data, an
+    m that is a power of two or three times one and more than 16 columns; the rest goes through ``spmm`` on the
     transposed operands."""
     return _host.spmm_tt_dense(weight, b, reduce_dim)
 
