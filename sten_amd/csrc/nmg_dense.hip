@@ -687,8 +687,8 @@ struct GemmF32Params {
     int vec;   // rows are 16-byte aligned: load four reduction positions at a time
 };
 
-// FAST: rows 16-byte aligned and K a multiple of BKT -- the loads of a step are one 128-bit load
-// per element through pointers computed once (rows past the end are clamped to the last one; their
+// FAST: rows 16-byte aligned, K a multiple of BKT, rows of reduction-major operands in whole groups of four -- the
+// loads of a step are one 128-bit load per element through pointers computed once (rows past the end are clamped to the last one; their
 // results are never stored), nothing else stands between the MFMAs.
 // AKM: the weight-side operand is given as A[K, O] (reduction-major: Y = X * A, the dense operand of
 // torch.mm as it lies in memory).  Its loads then run along the outputs and the tile is transposed
@@ -727,14 +727,10 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
         f32x4 r = {0.f, 0.f, 0.f, 0.f};
         if (row < nrows) {
             const float *src = base + row * ld + k;
-            if (P.vec && k + 3 < P.K) {
-                r = *(const f32x4 *)src;
-            } else {
-                if (k < P.K) r[0] = src[0];
-                if (k + 1 < P.K) r[1] = src[1];
-                if (k + 2 < P.K) r[2] = src[2];
-                if (k + 3 < P.K) r[3] = src[3];
-            }
+            if (k < P.K) r[0] = src[0];
+            if (k + 1 < P.K) r[1] = src[1];
+            if (k + 2 < P.K) r[2] = src[2];
+            if (k + 3 < P.K) r[3] = src[3];
         }
         return r;
     };
@@ -758,7 +754,42 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
         const int64_t row = r0 + e / KV < nrows ? r0 + e / KV : nrows - 1;
         return base + row * ld + (e % KV) * 4;
     };
+    // General form (any K, pitch and alignment): the same 16-byte loads -- a global load needs no more than the
+    // alignment of its elements -- with guards in the step that holds the end of the reduction only.  A group of four
+    // rows of a reduction-major operand that reaches past the last row is loaded from the last four and shifted
+    // on its way into LDS.  us, element by element -> this: 2139 x 504, K 2333 174 -> 72; 1676 x 3410, K 3456 with both
+    // operands reduction-major 596 -> 385; 1273 x 3204, K 291 51 -> 31.
+    typedef f32x4 f32x4_any __attribute__((aligned(4)));
+    auto shift_of = [&](int64_t r0, int64_t nrows, int e) {
+        const int64_t over = r0 + (e / BKT) * 4 + 4 - nrows;
+        return nrows >= 4 && over > 0 && over < 4 ? (int)over : 0;
+    };
+    auto shifted = [&](const f32x4 &g, int c, int s) {
+        float t = g[c];
+        if (c < 3) t = s == 1 ? g[(c + 1) & 3] : t;
+        if (c < 2) t = s == 2 ? g[(c + 2) & 3] : t;
+        if (c < 1) t = s == 3 ? g[3] : t;
+        return t;
+    };
     struct Stage { f32x4 x[XV], a[AV]; };
+    int xs[XV] = {}, as[AV] = {};
+    if constexpr (!FAST && XKM)
+#pragma unroll
+        for (int v = 0; v < XV; v++) xs[v] = shift_of(tok0, P.T, tid + v * 256);
+    if constexpr (!FAST && AKM)
+#pragma unroll
+        for (int v = 0; v < AV; v++) as[v] = shift_of(o0, P.O, tid + v * 256);
+    auto load_any = [&](const float *base, const float *p, int64_t ld, int64_t r0, int64_t nrows, int e, int64_t k0, bool km) {
+        const bool whole = k0 + BKT <= P.K;
+        if (km) {
+            if (nrows < 4) return fetch_km(base, ld, r0 + (e / BKT) * 4, nrows, k0 + e % BKT);
+            f32x4 r = {0.f, 0.f, 0.f, 0.f};
+            if (whole || k0 + e % BKT < P.K) r = *(const f32x4_any *)(p + k0 * ld);
+            return r;
+        }
+        if (whole) return (f32x4)*(const f32x4_any *)(p + k0);
+        return fetch_rm(base, ld, r0 + e / KV, nrows, k0 + (e % KV) * 4);
+    };
     const float *xp[XV], *ap[AV];
 #pragma unroll
     for (int v = 0; v < XV; v++)
@@ -773,27 +804,25 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
             const int e = tid + o * 256;
             if constexpr (FAST) G.x[o] = *(const f32x4 *)(xp[o] + (XKM ? k0 * P.ldx : k0));
             else if (XE % 256 == 0 || e < XE)
-                G.x[o] = XKM ? fetch_km(P.x, P.ldx, tok0 + (e / BKT) * 4, P.T, k0 + e % BKT)
-                             : fetch_rm(P.x, P.ldx, tok0 + e / KV, P.T, k0 + (e % KV) * 4);
+                G.x[o] = load_any(P.x, xp[o], P.ldx, tok0, P.T, e, k0, XKM);
         } else {
             const int v = o - XV, e = tid + v * 256;
             if constexpr (FAST) G.a[v] = *(const f32x4 *)(ap[v] + (AKM ? k0 * P.lda : k0));
             else if (AE % 256 == 0 || e < AE)
-                G.a[v] = AKM ? fetch_km(P.a, P.lda, o0 + (e / BKT) * 4, P.O, k0 + e % BKT)
-                             : fetch_rm(P.a, P.lda, o0 + e / KV, P.O, k0 + (e % KV) * 4);
+                G.a[v] = load_any(P.a, ap[v], P.lda, o0, P.O, e, k0, AKM);
         }
     };
     auto store_op = [&](const Stage &G, int buf, int o) {
         if (o < CSX * XV) {
             const int v = o / CSX, c = o % CSX, e = tid + v * 256;
             if (XE % 256 == 0 || e < XE) {
-                if constexpr (XKM) Xs[(buf * BM + (e / BKT) * 4 + c) * PITCH + e % BKT] = G.x[v][c];
+                if constexpr (XKM) Xs[(buf * BM + (e / BKT) * 4 + c) * PITCH + e % BKT] = FAST ? G.x[v][c] : shifted(G.x[v], c, xs[v]);
                 else *(f32x4 *)(Xs + (buf * BM + e / KV) * PITCH + (e % KV) * 4) = G.x[v];
             }
         } else {
             const int v = (o - CSX * XV) / CSA, c = (o - CSX * XV) % CSA, e = tid + v * 256;
             if (AE % 256 == 0 || e < AE) {
-                if constexpr (AKM) As[(buf * BN + (e / BKT) * 4 + c) * PITCH + e % BKT] = G.a[v][c];
+                if constexpr (AKM) As[(buf * BN + (e / BKT) * 4 + c) * PITCH + e % BKT] = FAST ? G.a[v][c] : shifted(G.a[v], c, as[v]);
                 else *(f32x4 *)(As + (buf * BN + e / KV) * PITCH + (e % KV) * 4) = G.a[v];
             }
         }
@@ -962,9 +991,12 @@ static void launch_gemm_f32(const GemmF32Params &Q, int form, hipStream_t st)
 // A CU works its tiles off one after the other as far as the matrix pipe is concerned, so a launch
 // costs ceil(tiles / 256) x the cost of one tile; the shape with the smallest product wins (768
 // outputs x 4096 tokens: 192 tiles of 128 x 128 leave a quarter of the CUs idle, 256 of 128 x 96 none).
+// 64 x 96 (two wavefronts per sub-tile, each half of the reduction) sits between: 3072 outputs x 512 tokens, K 768
+// 33.0 -> 30.6 us, 1408 x 985, K 2304 75 -> 62; with both operands reduction-major it gains nothing over
+// 128 x 64 (3840 x 328, K 512: 23.4 against 21.2).  32 x 64 was no faster than twice 32 x 32 and is not there.
 struct GemmF32Shape { int bm, bn; double eff; };
 static const GemmF32Shape kGemmF32Shapes[] = {
-    {128, 128, 1.00}, {128, 96, 0.97}, {128, 64, 0.92}, {64, 64, 0.80}, {32, 32, 0.55},
+    {128, 128, 1.00}, {128, 96, 0.97}, {128, 64, 0.92}, {64, 96, 0.88}, {64, 64, 0.80}, {32, 32, 0.55},
 };
 
 }  // namespace nmg
@@ -997,14 +1029,16 @@ static int gemm_f32_host(const void *d_a, int64_t lda, const void *d_x, int64_t 
     for (int c = 0; c < (int)(sizeof(kGemmF32Shapes) / sizeof(kGemmF32Shapes[0])); c++) {
         const GemmF32Shape &S = kGemmF32Shapes[c];
         const int64_t tiles = ((T + S.bm - 1) / S.bm) * ((O + S.bn - 1) / S.bn);
-        const double cost = (double)((tiles + 255) / 256) * S.bm * S.bn / S.eff;
+        const double eff = form == 2 && S.bm == 64 && S.bn == 96 ? 0.68 : S.eff;
+        const double cost = (double)((tiles + 255) / 256) * S.bm * S.bn / eff;
         if (c == 0 || cost < best_cost) { best = c; best_cost = cost; }
     }
     switch (best) {
     case 0: launch_gemm_f32<2, 2, 1, 2, 2>(Q, form, st); break;
     case 1: launch_gemm_f32<4, 1, 1, 1, 3>(Q, form, st); break;
     case 2: launch_gemm_f32<2, 2, 1, 2, 1>(Q, form, st); break;
-    case 3: launch_gemm_f32<2, 2, 1, 1, 1>(Q, form, st); break;
+    case 3: launch_gemm_f32<2, 1, 2, 1, 3>(Q, form, st); break;
+    case 4: launch_gemm_f32<2, 2, 1, 1, 1>(Q, form, st); break;
     default: launch_gemm_f32<1, 1, 4, 1, 1>(Q, form, st); break;
     }
     NMG_HIP_TRY(hipGetLastError());
