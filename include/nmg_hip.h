@@ -236,6 +236,8 @@ int nmg_copy_rows16(const void *d_src, int64_t rows, int64_t cols, int64_t ld_sr
 /* dst [cols, dst_cols] = src [rows, cols] transposed in a 16-bit type, zeros from `rows` on; dst_cols a multiple of 8. */
 int nmg_transpose16(const void *d_src, int64_t rows, int64_t cols, int64_t ld_src, void *d_dst, int64_t dst_cols,
                     int64_t ld_dst, void *stream);
+/* y [cols] = sum of the rows of x [rows, cols] (row pitch ld), single-precision sums (f32, f16, bf16). */
+int nmg_colsum(const void *d_x, int64_t rows, int64_t cols, int64_t ld, void *d_y, int dtype, void *stream);
 
 /* ---- "densefrag": the weight expanded into the register order of V_MFMA_F32_32X32X16, for the
  * products the sparse matrix cores cannot do: patterns that do not fit 2-of-4 groups, and the

@@ -7,6 +7,7 @@
 // alignment, they only touch one more line).  1857 x 10385 and its like: 3 us for 512 rows against 14 us for a fill
 // and a strided copy.
 #include "nmg_common.h"
+#include "nmg_tile.h"
 
 namespace nmg {
 
@@ -82,6 +83,51 @@ __global__ __launch_bounds__(256) void transpose16_kernel(Transpose16 P)
     }
 }
 
+// y[c] = sum over the rows of x[r, c], single-precision sums, rounded once: the bias gradient of a linear layer.  A
+// workgroup owns 32 columns (32 lanes x 4 bytes, 64 columns in pairs of the 16-bit types) over all rows, 32 rows at a time with
+// 16 loads per lane in flight, and adds its 32 partial rows through LDS in order: one launch, no semaphores to clear.
+// Bound by latency at the sizes it takes (512 x 768 in single precision: 4.0 us; the library's sum and the fill in front of it 11.5).
+struct ColSum {
+    const void *x;
+    void *y;
+    int64_t rows, cols, ld;
+};
+constexpr int CS_ROWS = 32, CS_DEEP = 16;
+
+template <typename T> __global__ __launch_bounds__(1024) void colsum_kernel(ColSum P)
+{
+    constexpr int E = 4 / (int)sizeof(T);
+    __shared__ float part[CS_ROWS][32 * E + 1];
+    const int tid = threadIdx.x, cl = tid & 31, rl = tid >> 5;
+    const int64_t c = ((int64_t)blockIdx.x * 32 + cl) * E;
+    float acc[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) acc[e] = 0.f;
+    for (int64_t r0 = rl; r0 < P.rows; r0 += CS_ROWS * CS_DEEP) {
+        float v[CS_DEEP][E];
+#pragma unroll
+        for (int u = 0; u < CS_DEEP; u++) {
+            const int64_t r = r0 + u * CS_ROWS;
+#pragma unroll
+            for (int e = 0; e < E; e++) v[u][e] = r < P.rows && c + e < P.cols ? to_f32(((const T *)P.x)[r * P.ld + c + e]) : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < CS_DEEP; u++)
+#pragma unroll
+            for (int e = 0; e < E; e++) acc[e] += v[u][e];
+    }
+#pragma unroll
+    for (int e = 0; e < E; e++) part[rl][cl * E + e] = acc[e];
+    __syncthreads();
+    if (tid >= 32 * E) return;
+    const int64_t col = (int64_t)blockIdx.x * 32 * E + tid;
+    if (col >= P.cols) return;
+    float s = 0.f;
+    for (int r = 0; r < CS_ROWS; r++) s += part[r][tid];
+    if constexpr (sizeof(T) == 4) ((float *)P.y)[col] = s;
+    else ((uint16_t *)P.y)[col] = f32_to_bits16(s, (T *)nullptr);
+}
+
 }  // namespace nmg
 
 using namespace nmg;
@@ -115,6 +161,25 @@ extern "C" int nmg_transpose16(const void *d_src, int64_t rows, int64_t cols, in
     const int64_t tiles = P.tiles_c * ((dst_cols + TR_ROWS - 1) / TR_ROWS);
     NMG_REQUIRE(tiles <= 0x7fffffffLL, NMG_ERR_UNSUPPORTED, "matrix too large for one launch");
     hipLaunchKernelGGL(transpose16_kernel, dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream, P);
+    NMG_HIP_TRY(hipGetLastError());
+    return NMG_OK;
+}
+
+extern "C" int nmg_colsum(const void *d_x, int64_t rows, int64_t cols, int64_t ld, void *d_y, int dtype, void *stream)
+{
+    NMG_REQUIRE(dtype == NMG_F32 || dtype == NMG_F16 || dtype == NMG_BF16, NMG_ERR_UNSUPPORTED, "colsum takes f32/f16/bf16");
+    NMG_REQUIRE(rows >= 0 && cols >= 0 && (rows <= 1 || ld >= cols), NMG_ERR_ARG, "invalid extents");
+    if (cols == 0) return NMG_OK;
+    NMG_REQUIRE(d_y && (d_x || rows == 0), NMG_ERR_ARG, "null device pointer");
+    ColSum P{d_x, d_y, rows, cols, ld};
+    const int64_t per = dtype == NMG_F32 ? 32 : 64, blocks = (cols + per - 1) / per;
+    NMG_REQUIRE(blocks <= 0x7fffffffLL, NMG_ERR_UNSUPPORTED, "too many columns for one launch");
+    hipStream_t s = (hipStream_t)stream;
+    switch (dtype) {
+    case NMG_F32: hipLaunchKernelGGL(colsum_kernel<float>, dim3((unsigned)blocks), dim3(1024), 0, s, P); break;
+    case NMG_F16: hipLaunchKernelGGL(colsum_kernel<__half>, dim3((unsigned)blocks), dim3(1024), 0, s, P); break;
+    default: hipLaunchKernelGGL(colsum_kernel<__hip_bfloat16>, dim3((unsigned)blocks), dim3(1024), 0, s, P); break;
+    }
     NMG_HIP_TRY(hipGetLastError());
     return NMG_OK;
 }

@@ -71,6 +71,7 @@ SIGNATURES = {
     "nmg_slotmap": (_I, [_P, _I64, _I64, _P, _I, _I, _I, _P]),
     "nmg_sddmm": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I, _I, _I, _I, _P]),
     "nmg_sddmm_padded": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I, _I, _I, _I, _P]),
+    "nmg_colsum": (_I, [_P, _I64, _I64, _I64, _P, _I, _P]),
     "nmg_transpose16": (_I, [_P, _I64, _I64, _I64, _P, _I64, _I64, _P]),
     "nmg_copy_rows16": (_I, [_P, _I64, _I64, _I64, _P, _I64, _I64, _I64, _P]),
     "nmg_sddmm_nt": (_I, [_P, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I, _I, _I, _I, _P]),
