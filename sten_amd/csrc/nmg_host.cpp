@@ -804,7 +804,8 @@ Tensor spmm_tt_dense(State &w, Tensor b, int rd)
 Tensor column_sum(const Tensor &g)
 {
     const at::ScalarType dt = g.scalar_type();
-    if (!(dt == at::kFloat || is16(g)) || g.size(0) == 0 || g.size(0) > 4096 || g.size(1) == 0) return g.sum(0);
+    if (!g.is_cuda() || !(dt == at::kFloat || is16(g)) || g.size(0) == 0 || g.size(0) > 4096 || g.size(1) == 0) return g.sum(0);
+    c10::DeviceGuard device(g.device());
     at::AutoDispatchBelowADInplaceOrView raw;
     const Tensor s = rows_of(g);
     Tensor y = new_empty({g.size(1)}, g);
@@ -1364,6 +1365,16 @@ PyObject *py_spmm(PyObject *, PyObject *const *a, Py_ssize_t n)
     HOST_CATCH(nullptr)
 }
 
+PyObject *py_column_sum(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    HOST_TRY
+    if (n != 1) fail("column_sum takes 1 argument");
+    const Tensor x = tensor_arg(a[0], "x");
+    if (x.dim() != 2) fail("column_sum takes a matrix");
+    return wrap(column_sum(x));
+    HOST_CATCH(nullptr)
+}
+
 PyObject *py_spmm_tt(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
     HOST_TRY
@@ -1793,6 +1804,7 @@ PyMethodDef functions[] = {
      "make_torch_function(slow, failed, plain, native, grad_of, add_, KeepAll, DenseTensor, Tensor)"},
     {"sparsify", py_sparsify, METH_VARARGS, "sparsify(core, dense): fills val and idx of a core whose layout is set"},
     {"spmm", (PyCFunction)(void (*)(void))py_spmm, METH_FASTCALL, "spmm(weight, x, bias, reduce_dim, kernel)"},
+    {"column_sum", (PyCFunction)(void (*)(void))py_column_sum, METH_FASTCALL, "column_sum(x): sum over the rows"},
     {"spmm_tt", (PyCFunction)(void (*)(void))py_spmm_tt, METH_FASTCALL, "spmm_tt(weight, b)"},
     {"spmm_tt_dense", (PyCFunction)(void (*)(void))py_spmm_tt_dense, METH_FASTCALL, "spmm_tt_dense(weight, b, reduce_dim)"},
     {"dense_product", (PyCFunction)(void (*)(void))py_dense_product, METH_FASTCALL, "dense_product(tn, x, a), None where no kernel takes it"},
