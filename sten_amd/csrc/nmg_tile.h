@@ -279,24 +279,26 @@ __device__ __forceinline__ void store_partial_tile16(const f32x4 (&acc)[AB][TB],
     }
 }
 
-template <typename T> __global__ __launch_bounds__(256) void splitk_sum_kernel(SplitSum P)
+// Bound by memory.  A workgroup takes 1024 outputs of one token (no division per thread), a thread four outputs: the
+// slices' sums are all requested before the first is added (the kernel is a chain of round trips to memory
+// otherwise: the sums were written through other L2s), added in slice order, and stored as one 8-byte word.
+// 777 x 4096 in two slices, 32 MB: 10.7 -> 8.0 us against the form
+// with a division per thread, sixteen guarded loads whatever the number of slices and 2-byte stores.
+template <typename T, int U> __global__ __launch_bounds__(256) void splitk_sum_kernel(SplitSum P)
 {
-    const int64_t quads = (P.M + 3) / 4;
-    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= P.T * quads) return;
-    const int64_t tok = gid / quads, f = (gid - tok * quads) * 4;
+    const uint32_t groups = (uint32_t)((P.M + 1023) / 1024);
+    const int64_t tok = blockIdx.x / groups, f = ((int64_t)(blockIdx.x - (uint32_t)tok * groups) * 256 + threadIdx.x) * 4;
+    if (f >= P.M) return;
     const float *src = P.part + tok * P.part_ld + f;
-    // sixteen slices are fetched at a time (the kernel is a chain of round trips to memory otherwise:
-    // the sums were written through other L2s) and added in slice order
     const int64_t step = P.T * P.part_ld;
     float4 sum = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < P.slices; s0 += 16) {
-        float4 v[16];
+    for (int s0 = 0; s0 < P.slices; s0 += U) {
+        float4 v[U];
 #pragma unroll
-        for (int u = 0; u < 16; u++)
+        for (int u = 0; u < U; u++)
             v[u] = s0 + u < P.slices ? *(const float4 *)(src + (int64_t)(s0 + u) * step) : float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int u = 0; u < 16; u++) {
+        for (int u = 0; u < U; u++) {
             sum.x += v[u].x;
             sum.y += v[u].y;
             sum.z += v[u].z;
@@ -306,15 +308,27 @@ template <typename T> __global__ __launch_bounds__(256) void splitk_sum_kernel(S
     const float o[4] = {sum.x, sum.y, sum.z, sum.w};
     uint16_t *dst = (uint16_t *)P.y + tok * P.ldy + f;
     const T *bias = (const T *)P.bias;
+    uint16_t h[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-        if (f + i < P.M) dst[i] = f32_to_bits16(o[i] + (bias ? to_f32(bias[f + i]) : 0.f), (T *)nullptr);
+    for (int i = 0; i < 4; i++) h[i] = f32_to_bits16(o[i] + (bias && f + i < P.M ? to_f32(bias[f + i]) : 0.f), (T *)nullptr);
+    if (f + 4 <= P.M) {
+        __builtin_memcpy(dst, h, 8);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (f + i < P.M) dst[i] = h[i];
+    }
 }
 
 template <typename T> static inline int launch_splitk_sum(const SplitSum &P, hipStream_t s)
 {
-    const int64_t threads = P.T * ((P.M + 3) / 4);
-    hipLaunchKernelGGL(splitk_sum_kernel<T>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, P);
+    const int64_t blocks = P.T * ((P.M + 1023) / 1024);
+    NMG_REQUIRE(blocks <= 0x7fffffffLL, NMG_ERR_UNSUPPORTED, "product too large for one launch");
+    const dim3 grid((unsigned)blocks);
+    if (P.slices <= 2) hipLaunchKernelGGL((splitk_sum_kernel<T, 2>), grid, dim3(256), 0, s, P);
+    else if (P.slices <= 4) hipLaunchKernelGGL((splitk_sum_kernel<T, 4>), grid, dim3(256), 0, s, P);
+    else if (P.slices <= 8) hipLaunchKernelGGL((splitk_sum_kernel<T, 8>), grid, dim3(256), 0, s, P);
+    else hipLaunchKernelGGL((splitk_sum_kernel<T, 16>), grid, dim3(256), 0, s, P);
     NMG_HIP_TRY(hipGetLastError());
     return NMG_OK;
 }

@@ -61,3 +61,15 @@ def test_odd_extents(R, C, T, n, m, g, along, dtype):
     assert gd.shape == (R, C) and rel_l2(to_np(gd), G.T @ X) <= TOL[dtype]
     gn = _dense_product("nt", gy.t().contiguous().to(DEV), x.t().contiguous().to(DEV))
     assert gn.shape == (R, C) and rel_l2(to_np(gn), G.T @ X) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("R,T", [(3, 17), (1021, 20), (1028, 33), (2050, 130)])
+@pytest.mark.parametrize("slices", [2, 3, 8, 16])      # 16 steps: none leaves a slice empty
+def test_sum_of_slices(R, T, slices, dtype):
+    w = sten.GroupedNMTensor.from_dense(seeded((R, 1024), dtype, seed=1, std=0.5).to(DEV), 2, 4, sparse_dim=0, group_size=4, group_dim=1)
+    x, bias = seeded((T, 1024), dtype, seed=2), seeded((R,), dtype, seed=3)
+    w.spmm_opt["slices"] = slices
+    y = sten.spmm(w, x.to(DEV), bias.to(DEV), reduce_dim=1)
+    want = to_np(x).astype(np.float64) @ to_np(w.to_dense()).astype(np.float64).T + to_np(bias).astype(np.float64)
+    assert rel_l2(to_np(y), want) <= TOL[dtype]
