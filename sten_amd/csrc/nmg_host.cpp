@@ -1597,6 +1597,16 @@ std::shared_ptr<ProductNode> new_node(PyObject *capsule, PyObject *container, in
     return node;
 }
 
+// A tensor with a forward-mode tangent or inside a function transform (vmap, grad): what the Python dispatcher's
+// autograd.Function refuses must reach it, the kernels see neither.
+bool transformed(const Tensor &t)
+{
+    return t.defined()
+           && (t._fw_grad(0).defined()
+               || t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                                           c10::DispatchKey::Functionalize})));
+}
+
 // A new reference to the result, or nullptr without an error where the native route does not apply.
 PyObject *native_product(PyObject *capsule, PyObject *formats, PyObject *args)
 {
@@ -1618,6 +1628,7 @@ PyObject *native_product(PyObject *capsule, PyObject *formats, PyObject *args)
     if (!has_bit(masks, 0, arity) || (guess == 0 && n != 2)) return nullptr;
     const Tensor &x = THPVariable_Unpack(px), &wt = THPVariable_Unpack(pw);
     Tensor bias = pb == Py_None ? Tensor() : THPVariable_Unpack(pb);
+    if (transformed(x) || transformed(wt) || transformed(bias)) return nullptr;
     const bool grad = c10::GradMode::is_enabled() && (x.requires_grad() || wt.requires_grad() || (bias.defined() && bias.requires_grad()));
     if (x.dim() < 2 && !(guess == 1 && x.dim() == 1)) return nullptr;
     if (!PyObject_TypeCheck(wrapped, &CoreType)) {      // the int4 format: generation without gradients

@@ -57,3 +57,21 @@ def test_a_graph_is_walked_once():
     y.sum().backward()
     with pytest.raises(RuntimeError):
         y.sum().backward()
+
+
+def test_transforms_reach_the_python_dispatcher():
+    """Forward-mode tangents and function transforms: refused there, never dropped."""
+    import torch.autograd.forward_ad as forward_ad
+    layer = weight(torch.float32, "dense")
+    x = seeded((4, 128), torch.float32, seed=2).to(DEV)
+    with forward_ad.dual_level():
+        with pytest.raises(NotImplementedError):
+            layer(forward_ad.make_dual(x, torch.ones_like(x)))
+        bias = forward_ad.make_dual(layer.bias.detach(), torch.ones_like(layer.bias))
+        with pytest.raises(NotImplementedError):
+            F.linear(x, layer.weight, bias)
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.func.vmap(layer)(x.reshape(2, 2, 128))
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.func.grad(lambda v: layer(v).sum())(x)
+    assert layer(x).shape == (4, 96)
