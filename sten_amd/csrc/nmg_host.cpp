@@ -19,6 +19,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <map>
 #include <sstream>
@@ -1610,6 +1611,9 @@ bool transformed(const Tensor &t)
 // A new reference to the result, or nullptr without an error where the native route does not apply.
 PyObject *native_product(PyObject *capsule, PyObject *formats, PyObject *args)
 {
+    // torch.jit.trace records the allocation of the result but no launch: the graph would return memory that nothing
+    // has written.  The Python dispatcher's autograd.Function is recorded whole.
+    if (torch::jit::tracer::isTracing()) return nullptr;
     Dispatch &d = *dispatch_of(capsule);
     const Py_ssize_t n = PyTuple_GET_SIZE(args);
     if (n < 2 || n > 3) return nullptr;

@@ -75,3 +75,36 @@ def test_transforms_reach_the_python_dispatcher():
     with pytest.raises(RuntimeError, match="functorch"):
         torch.func.grad(lambda v: layer(v).sum())(x)
     assert layer(x).shape == (4, 96)
+
+
+class Product(torch.nn.Module):
+    """One operator on a sparse weight, with the weight (and bias) of ``layer``."""
+
+    def __init__(self, layer, op):
+        super().__init__()
+        self.weight, self.bias, self.op = layer.weight, layer.bias, op
+
+    def forward(self, x):
+        if self.op == "mm":
+            return torch.mm(self.weight, x)
+        return F.linear(x, self.weight, self.bias if self.op == "linear" else None)
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("op", ["linear", "nobias", "mm", "int4"])
+def test_a_traced_module_computes(op, grad):
+    """torch.jit.trace of a module: the graph holds the product, not the bare allocation of its result."""
+    print(f"case {op} grad={grad}", flush=True)
+    if op == "int4":
+        layer = torch.nn.Linear(128, 96, device=DEV, dtype=torch.float16)
+        builder = sten.SparsityBuilder()
+        builder.set_weight("weight", initial_sparsifier=sten.SparseMarlinSparsifier(), out_format=sten.SparseMarlinTensor)
+        module = Product(builder.sparsify_model_inplace(layer).requires_grad_(False), "linear")
+    else:
+        module = Product(weight(torch.float16, "dense").requires_grad_(grad), op)
+    shape = (128, 40) if op == "mm" else (8, 128)
+    first, second = (seeded(shape, torch.float16, seed=s).to(DEV) for s in (4, 5))
+    with torch.set_grad_enabled(grad):
+        traced = torch.jit.trace(module, (first,), check_trace=False)
+        for x in (second, first):
+            assert torch.equal(traced(x), module(x))
