@@ -65,6 +65,7 @@ void check(int rc)
 
 struct Text {
     PyObject *kernel, *variant, *dense_variant, *slices, *expand, *cache_dense, *container, *dense_shape, *B, *s, *meta, *grad_fmt, *data, *alpha;
+    PyObject *arguments[4], *nothing;      // names of __torch_function__'s, ()
 } S_;
 
 int dtype_code(at::ScalarType t)
@@ -1742,14 +1743,36 @@ PyObject *native_add_(const Dispatch &d, PyObject *args, PyObject *kwargs)
     return self;
 }
 
-PyObject *torch_function(PyObject *capsule, PyObject *const *a, Py_ssize_t n)
+// __torch_function__(func, types, args=(), kwargs=None), by position or by name
+PyObject *torch_function(PyObject *capsule, PyObject *const *a, Py_ssize_t n, PyObject *names)
 {
-    if (n < 3 || n > 4 || !PyTuple_Check(a[2])) {
-        PyErr_SetString(PyExc_TypeError, "__torch_function__(func, types, args, kwargs=None)");
+    PyObject *given[4] = {nullptr, nullptr, nullptr, nullptr};
+    bool known = n <= 4;
+    for (Py_ssize_t i = 0; i < n && known; i++) given[i] = a[i];
+    for (Py_ssize_t k = 0; names != nullptr && k < PyTuple_GET_SIZE(names) && known; k++) {
+        int i = 0;
+        while (i < 4 && PyUnicode_Compare(PyTuple_GET_ITEM(names, k), S_.arguments[i]) != 0) i++;
+        known = i < 4 && given[i] == nullptr;
+        if (known) given[i] = a[n + k];
+    }
+    if (!known || given[0] == nullptr || given[1] == nullptr) {
+        PyErr_SetString(PyExc_TypeError, "__torch_function__(func, types, args=(), kwargs=None)");
         return nullptr;
     }
     Dispatch &d = *dispatch_of(capsule);
-    PyObject *func = a[0], *args = a[2], *kwargs = n == 4 && a[3] != Py_None ? a[3] : nullptr;
+    PyObject *func = given[0], *args = given[2] != nullptr ? given[2] : S_.nothing;
+    PyObject *kwargs = given[3] != Py_None ? given[3] : nullptr;
+    pybind11::object own_args, own_kwargs;      // any sequence and any mapping will do
+    if (!PyTuple_Check(args)) {
+        own_args = pybind11::reinterpret_steal<pybind11::object>(PySequence_Tuple(args));
+        if (!own_args) return nullptr;
+        args = own_args.ptr();
+    }
+    if (kwargs != nullptr && !PyDict_Check(kwargs)) {
+        own_kwargs = pybind11::reinterpret_steal<pybind11::object>(PyDict_New());
+        if (!own_kwargs || PyDict_Update(own_kwargs.ptr(), kwargs) < 0) return nullptr;
+        kwargs = own_kwargs.ptr();
+    }
     const int plain = PySet_Contains(d.plain, func);
     if (plain < 0) return nullptr;
     if (plain) {
@@ -1786,10 +1809,10 @@ PyObject *torch_function(PyObject *capsule, PyObject *const *a, Py_ssize_t n)
         return nullptr;
     }
     if (r != nullptr) return r;
-    return PyObject_CallFunctionObjArgs(d.slow, func, a[1], args, kwargs != nullptr ? kwargs : Py_None, nullptr);
+    return PyObject_CallFunctionObjArgs(d.slow, func, given[1], args, kwargs != nullptr ? kwargs : Py_None, nullptr);
 }
 
-PyMethodDef torch_function_def = {"__torch_function__", (PyCFunction)(void (*)(void))torch_function, METH_FASTCALL, nullptr};
+PyMethodDef torch_function_def = {"__torch_function__", (PyCFunction)(void (*)(void))torch_function, METH_FASTCALL | METH_KEYWORDS, nullptr};
 
 PyObject *py_make_torch_function(PyObject *, PyObject *args)
 {
@@ -1849,7 +1872,10 @@ PyMODINIT_FUNC PyInit__host()
           PyUnicode_InternFromString("slices"), PyUnicode_InternFromString("expand"), PyUnicode_InternFromString("cache_dense"),
           PyUnicode_InternFromString("_wrapped_tensor_container"), PyUnicode_InternFromString("dense_shape"),
           PyUnicode_InternFromString("B"), PyUnicode_InternFromString("s"), PyUnicode_InternFromString("meta"),
-          PyUnicode_InternFromString("grad_fmt"), PyUnicode_InternFromString("data"), PyUnicode_InternFromString("alpha")};
+          PyUnicode_InternFromString("grad_fmt"), PyUnicode_InternFromString("data"), PyUnicode_InternFromString("alpha"),
+          {PyUnicode_InternFromString("func"), PyUnicode_InternFromString("types"), PyUnicode_InternFromString("args"),
+           PyUnicode_InternFromString("kwargs")},
+          PyTuple_New(0)};
     if (PyModule_AddIntConstant(m, "INTERFACE", kInterface) < 0) return nullptr;
     Py_INCREF(&CoreType);
     if (PyModule_AddObject(m, "Core", (PyObject *)&CoreType) < 0) return nullptr;

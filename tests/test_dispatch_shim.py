@@ -176,6 +176,33 @@ def test_unregistered_operator_falls_back_or_raises():
             torch.relu(w2)
 
 
+def test_torch_function_by_name_and_from_a_subclass():
+    """The protocol method takes its arguments by name, args and kwargs have defaults, a subclass may extend it."""
+    model, _, sb = sparse_linear(2)
+    model = sb.sparsify_model_inplace(model)
+    x = torch.randn(3, 6)
+    F, want = torch.nn.functional.linear, model(x)
+    hook = type(model.weight).__torch_function__
+    assert torch.equal(hook(F, (), args=(x, model.weight, model.bias), kwargs=None), want)
+    assert torch.equal(hook(func=F, types=(), args=[x, model.weight], kwargs={"bias": model.bias}), want)
+    assert torch.equal(hook(F, (), kwargs={"input": x, "weight": model.weight, "bias": model.bias}), want)
+    assert hook(torch.Tensor.is_leaf.__get__, (), args=(model.weight,)) is True
+    seen = []
+
+    class Watched(sten.SparseTensorWrapper):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return super().__torch_function__(func, types, args=args, kwargs=kwargs or {})
+
+    w = Watched(model.weight._wrapped_tensor_container, False, model.weight.grad_fmt)
+    assert torch.equal(torch.nn.functional.linear(x, w, model.bias), want)
+    assert F in seen
+    for bad in (lambda: hook(F), lambda: hook(F, (), func=F), lambda: hook(F, (), other=1), lambda: hook(F, (), (), None, 0)):
+        with pytest.raises(TypeError):
+            bad()
+
+
 def test_wrapper_copy_detach_pickle():
     w = _to_mask(EvenSparsifier(), torch.randn(4, 4).requires_grad_(True))
     d = w.detach()
