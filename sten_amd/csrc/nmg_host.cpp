@@ -1743,6 +1743,25 @@ PyObject *native_add_(const Dispatch &d, PyObject *args, PyObject *kwargs)
     return self;
 }
 
+// The dispatcher's warning in front of the error that is set; the error stays, or the one that the warning became.
+void warn_of_failure(const Dispatch &d, PyObject *func)
+{
+    if (!PyErr_ExceptionMatches(PyExc_Exception)) return;
+    PyObject *type, *value, *trace;
+    PyErr_Fetch(&type, &value, &trace);
+    PyErr_NormalizeException(&type, &value, &trace);
+    if (trace != nullptr) PyException_SetTraceback(value, trace);
+    PyObject *done = PyObject_CallFunctionObjArgs(d.failed, func, value, nullptr);
+    if (done != nullptr) {
+        Py_DECREF(done);
+        PyErr_Restore(type, value, trace);
+        return;
+    }
+    Py_XDECREF(type);
+    Py_XDECREF(value);
+    Py_XDECREF(trace);
+}
+
 // __torch_function__(func, types, args=(), kwargs=None), by position or by name
 PyObject *torch_function(PyObject *capsule, PyObject *const *a, Py_ssize_t n, PyObject *names)
 {
@@ -1780,6 +1799,7 @@ PyObject *torch_function(PyObject *capsule, PyObject *const *a, Py_ssize_t n, Py
         at::impl::PythonTorchFunctionTLS::set_disabled_state(at::impl::TorchFunctionDisabledState::SUBCLASSES_DISABLED);
         PyObject *r = PyObject_Call(func, args, kwargs);
         at::impl::PythonTorchFunctionTLS::set_disabled_state(before);
+        if (r == nullptr) warn_of_failure(d, func);
         return r;
     }
     PyObject *r = nullptr;
@@ -1794,18 +1814,7 @@ PyObject *torch_function(PyObject *capsule, PyObject *const *a, Py_ssize_t n, Py
     catch (const c10::Error &e) { PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace()); bad = true; }
     catch (const std::exception &e) { PyErr_SetString(PyExc_RuntimeError, e.what()); bad = true; }
     if (bad) {
-        PyObject *type, *value, *trace;
-        PyErr_Fetch(&type, &value, &trace);
-        PyErr_NormalizeException(&type, &value, &trace);
-        PyObject *done = PyObject_CallFunctionObjArgs(d.failed, func, value, nullptr);
-        if (done == nullptr) {      // the warning was turned into an error
-            Py_XDECREF(type);
-            Py_XDECREF(value);
-            Py_XDECREF(trace);
-            return nullptr;
-        }
-        Py_DECREF(done);
-        PyErr_Restore(type, value, trace);
+        warn_of_failure(d, func);
         return nullptr;
     }
     if (r != nullptr) return r;

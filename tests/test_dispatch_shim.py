@@ -203,6 +203,20 @@ def test_torch_function_by_name_and_from_a_subclass():
             bad()
 
 
+@pytest.mark.parametrize("call,error", [
+    (lambda w: w.retain_grad(), RuntimeError),                            # runs on the placeholder
+    (lambda w: setattr(w, "grad", 1), TypeError),
+    (lambda w: torch.nn.functional.linear(torch.ones(2, 5), w, torch.ones(4)), RuntimeError),
+])
+def test_every_failing_call_is_announced(call, error):
+    w = _to_mask(EvenSparsifier(), torch.randn(4, 6))
+    with pytest.warns(UserWarning, match="Exception raised during handling"), pytest.raises(error):
+        call(w)
+    with warnings.catch_warnings(), pytest.raises(UserWarning, match="Exception raised during handling"):
+        warnings.simplefilter("error")
+        call(w)
+
+
 def test_wrapper_copy_detach_pickle():
     w = _to_mask(EvenSparsifier(), torch.randn(4, 4).requires_grad_(True))
     d = w.detach()
