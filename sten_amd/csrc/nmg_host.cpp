@@ -421,6 +421,21 @@ Tensor workspace(int64_t floats, const Tensor &like) { return new_empty({std::ma
 
 int64_t split_ws(int slices, int64_t T, int64_t O) { return slices * T * up(O, 256) * 256; }
 
+// The code of the kernel that takes what no other route does; KeyError for a name that there is no kernel of.
+int kernel_code(const std::string &name)
+{
+    static const std::map<std::string, int> codes = {
+        {"mfma", NMG_KERNEL_MFMA}, {"expand", NMG_KERNEL_MFMA}, {"densefrag", NMG_KERNEL_MFMA},
+        {"smfmac", NMG_KERNEL_SMFMAC}, {"skinny", NMG_KERNEL_SKINNY}, {"gstream", NMG_KERNEL_SKINNY},
+        {"sstream", NMG_KERNEL_SKINNY}, {"ostream", NMG_KERNEL_SKINNY}};
+    const auto it = codes.find(name);
+    if (it != codes.end()) return it->second;
+    PyObject *key = PyUnicode_FromString(name.c_str());
+    if (key != nullptr) PyErr_SetObject(PyExc_KeyError, key);
+    Py_XDECREF(key);
+    throw python_error();
+}
+
 // Y = X @ op(W): rd = 1 is X [T, C] @ W^T (F.linear forward), rd = 0 is X [T, R] @ W (the input's gradient).
 Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
 {
@@ -443,6 +458,7 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
     const Options opt = options_of(w);
     const std::string kname = kernel != nullptr ? kernel : opt.kernel;
     const bool automatic = kname == "auto";
+    const int code = automatic ? NMG_KERNEL_AUTO : kernel_code(kname);
     const int dt = dtype_code(x.scalar_type());
     const bool half = is16(x), al = aligned16(x);
     void *const stream = stream_of(x);
@@ -640,10 +656,6 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
         return y;
     }
     pack(w);
-    int code = NMG_KERNEL_AUTO;
-    if (kname == "mfma" || kname == "expand" || kname == "densefrag") code = NMG_KERNEL_MFMA;
-    else if (kname == "smfmac") code = NMG_KERNEL_SMFMAC;
-    else if (kname != "auto") code = NMG_KERNEL_SKINNY;
     check(nmg_spmm(w.ops.pk_val.data_ptr(), w.ops.pk_pat.data_ptr(), q.G, q.S, xp, ldx, yp, O, bp, T, reduce_sparse ? 1 : 0, q.n, q.m,
                    dt, code, stream));
     return y;
@@ -1356,7 +1368,7 @@ const char *kernel_arg(PyObject *o)
     if (o == nullptr || o == Py_None) return nullptr;
     const char *c = PyUnicode_AsUTF8(o);
     if (c == nullptr) throw python_error();
-    return c;
+    return *c != 0 ? c : nullptr;
 }
 
 PyObject *py_spmm(PyObject *, PyObject *const *a, Py_ssize_t n)

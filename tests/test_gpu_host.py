@@ -5,7 +5,7 @@ import torch
 import torch.nn.functional as F
 
 import sten_amd as sten
-from sten_amd import dispatch
+from sten_amd import dispatch, native
 from helpers import seeded
 
 pytestmark = pytest.mark.gpu
@@ -108,3 +108,26 @@ def test_a_traced_module_computes(op, grad):
         traced = torch.jit.trace(module, (first,), check_trace=False)
         for x in (second, first):
             assert torch.equal(traced(x), module(x))
+
+
+def test_kernel_names():
+    """A name that there is no kernel of is refused on every route; "" leaves the choice to the weight's options."""
+    layer = weight(torch.float16, "dense")
+    w = layer.weight.wrapped_tensor
+    x = seeded((4, 128), torch.float16, seed=6).to(DEV)
+    want = sten.spmm(w, x, reduce_dim=1)
+    for name in ("x", "MFMA", "auto "):
+        for reduce_dim in (0, 1):
+            with pytest.raises(KeyError, match=name):
+                sten.spmm(w, x[:, :w.shape[reduce_dim]].contiguous(), reduce_dim=reduce_dim, kernel=name)
+        w.spmm_opt["kernel"] = name
+        for call in (lambda: layer(x), lambda: torch.mm(layer.weight, x.t().contiguous())):
+            with pytest.raises(KeyError, match=name), pytest.warns(UserWarning, match="Exception raised during handling"):
+                call()
+        w.spmm_opt["kernel"] = "auto"
+    assert torch.equal(sten.spmm(w, x, reduce_dim=1, kernel=""), want)
+    for name in native.KERNELS:
+        try:
+            sten.spmm(w, x, reduce_dim=1, kernel=name)
+        except native.NmgError:      # the kernel does not take the shape
+            pass
