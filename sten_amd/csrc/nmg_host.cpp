@@ -203,7 +203,10 @@ long opt_long(PyObject *d, PyObject *key, long dflt)
         if (PyErr_Occurred()) throw python_error();
         return dflt;
     }
-    const long r = PyLong_AsLong(v);
+    PyObject *whole = PyNumber_Long(v);      // what int() takes
+    if (whole == nullptr) throw python_error();
+    const long r = PyLong_AsLong(whole);
+    Py_DECREF(whole);
     if (r == -1 && PyErr_Occurred()) throw python_error();
     return r;
 }
@@ -222,7 +225,7 @@ bool opt_bool(PyObject *d, PyObject *key, bool dflt)
 
 struct Options {
     std::string kernel = "auto";
-    long variant = -1, dense_variant = -1, slices = -1;
+    long variant = -1, dense_variant = -1, slices = -1;      // slices: -1 where none are asked for
     bool expand = true, cache_dense = true;
 };
 
@@ -238,7 +241,7 @@ Options options_of(const State &w)
     if (PyDict_Size(w.opt) > (k != nullptr ? 1 : 0)) {
         o.variant = opt_long(w.opt, S_.variant, -1);
         o.dense_variant = opt_long(w.opt, S_.dense_variant, -1);
-        o.slices = opt_long(w.opt, S_.slices, -1);
+        if (PyDict_Contains(w.opt, S_.slices) == 1) o.slices = std::max(opt_long(w.opt, S_.slices, 0), 0L);
         o.expand = opt_bool(w.opt, S_.expand, true);
         o.cache_dense = opt_bool(w.opt, S_.cache_dense, true);
     }

@@ -6,7 +6,7 @@ import torch.nn.functional as F
 
 import sten_amd as sten
 from sten_amd import dispatch, native
-from helpers import seeded
+from helpers import rel_l2, seeded, to_np
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -131,3 +131,13 @@ def test_kernel_names():
             sten.spmm(w, x, reduce_dim=1, kernel=name)
         except native.NmgError:      # the kernel does not take the shape
             pass
+
+
+def test_options_are_converted_like_int_does():
+    w = weight(torch.float16, "dense").weight.wrapped_tensor
+    x = seeded((40, 96), torch.float16, seed=7).to(DEV)
+    want = to_np(sten.spmm(w, x, reduce_dim=0))
+    for name, value in (("variant", "-1"), ("dense_variant", -1.0), ("slices", "1"), ("slices", -1)):
+        w.spmm_opt[name] = value
+        assert rel_l2(to_np(sten.spmm(w, x, reduce_dim=0)), want) < 2e-3      # two roundings of the result to 11 bits
+        del w.spmm_opt[name]
