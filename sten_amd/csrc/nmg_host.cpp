@@ -98,11 +98,12 @@ int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 int64_t round_up(int64_t a, int64_t b) { return up(a, b) * b; }
 
 // t (2-D) with contiguous rows that do not overlap: t itself where they lie so, else a copy.
-Tensor rows_of(const Tensor &t)
+bool rows_lie(const Tensor &t)
 {
     const int64_t R = t.size(0), C = t.size(1);
-    return (C <= 1 || t.stride(1) == 1) && (R <= 1 || t.stride(0) >= C) ? t : t.contiguous();
+    return (C <= 1 || t.stride(1) == 1) && (R <= 1 || t.stride(0) >= C);
 }
+Tensor rows_of(const Tensor &t) { return rows_lie(t) ? t : t.contiguous(); }
 
 // t (16-bit, 2-D) as rows of at least `cols` elements that start on 16 bytes, zeros from t's extent on, and at
 // least `rows` of them: t itself where it is that already, else a copy.
@@ -128,6 +129,13 @@ Tensor transposed(const Tensor &b, int64_t Kp)
 }
 
 int64_t pitch_of(const Tensor &t) { return t.size(0) > 1 ? t.stride(0) : t.size(1); }
+
+// pitch_of(padded(t, t.size(0), round_up(t.size(1), 8)))
+int64_t pitch_of_whole_pieces(const Tensor &t)
+{
+    const bool kept = rows_lie(t) && t.size(0) > 1 && t.size(1) % 8 == 0 && t.stride(0) % 8 == 0 && aligned16(t);
+    return kept ? t.stride(0) : round_up(t.size(1), 8);
+}
 
 constexpr int64_t k2G = int64_t(1) << 31;
 constexpr int64_t kOstreamMaxTokens = 4;    // nmg_spmm_ostream: the token rows its lanes hold
@@ -834,8 +842,8 @@ bool masked_product_supported(const State &w, const Tensor &rows, const Tensor &
 {
     const Geometry &q = w.geo;
     if (q.nd != 2 || !is16(w.val) || rows.scalar_type() != w.val.scalar_type() || cols.scalar_type() != w.val.scalar_type()) return false;
-    const int64_t longest = std::max({rows.size(1), cols.size(1), rows.stride(0), cols.stride(0)});
-    return longest < (int64_t(1) << (last ? 21 : 24));
+    // the pitches that the kernel's 32-bit offsets reach
+    return std::max(pitch_of_whole_pieces(rows), pitch_of_whole_pieces(cols)) < (int64_t(1) << (last ? 22 : 25));
 }
 
 // val of the kept positions of rows^T @ cols (rows [T, R], cols [T, C]; with `last` rows [R, T], cols [C, T]).

@@ -229,6 +229,40 @@ def test_weight_gradient_of_torch_mm_from_its_operands_as_they_lie():
     assert float((got.val.float() - ref.val.float()).norm() / ref.val.float().norm()) <= 1e-3
 
 
+def test_rows_up_to_the_longest_that_the_kernel_takes():
+    """Operands with the reduction contiguous: rows below 2^22; with the features contiguous: pitches below 2^25.  What
+    counts is the pitch that the kernel is given: a row that gets a copy has the copy's."""
+    print("case sddmm longest rows", flush=True)
+    torch.manual_seed(5)
+    R, C, gen = 48, 64, torch.Generator(DEV).manual_seed(5)
+    W = (torch.randn(R, C) * 0.1).half().to(DEV)
+    w = sten.GroupedNMTensor.from_dense(W, 2, 4, sparse_dim=1, group_size=4, group_dim=0)
+
+    def check(got, gw):
+        ref = to_np(w._gather(gw).val).astype(np.float64)
+        # 2^17 K steps summed in fp32: at most sqrt(2^17) * 2^-24 = 2.2e-5 beside the rounding to fp16
+        assert rel_l2(to_np(got.val), ref) <= TOL[torch.float16]
+
+    T = 2 ** 22 - 8
+    gc, b = ((torch.randn(n, T + 8, device=DEV, generator=gen) * 0.1).half() for n in (R, C))
+    assert not w.masked_product_supported(gc, b, reduction_last=True)
+    gc, b = gc[:, :T].contiguous(), b[:, :T].contiguous()
+    assert w.masked_product_supported(gc, b, reduction_last=True)
+    check(w.masked_product(gc, b, reduction_last=True), sum((p.double() @ q.double().t()) for p, q in zip(gc.split(2 ** 20, 1), b.split(2 ** 20, 1))))
+    del gc, b
+
+    T, pitch = 33, 2 ** 25 - 8
+    buf = torch.zeros(T * pitch, dtype=torch.float16, device=DEV)
+    gy, x = buf.as_strided((T, R), (pitch, 1)), torch.randn(T, C, device=DEV, generator=gen).half()
+    gy.copy_(torch.randn(T, R, device=DEV, generator=gen))
+    assert w.masked_product_supported(gy, x)
+    check(w.masked_product(gy, x), gy.double().t() @ x.double())
+    assert not w.masked_product_supported(buf.as_strided((T - 1, R), (pitch + 8, 1)), x[1:])
+    moved = buf.as_strided((T - 1, R), (pitch + 9, 1), 3)      # starts on no 16 bytes: copied, so its own pitch is no limit
+    assert w.masked_product_supported(moved, x[1:])
+    check(w.masked_product(moved, x[1:]), moved.double().t() @ x[1:].double())
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("R,C,T,bias", [
     (256, 256, 64, False),       # one tile, whole K steps
