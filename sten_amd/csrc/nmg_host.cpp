@@ -880,8 +880,9 @@ Tensor masked_product(State &w, Tensor rows, Tensor cols, bool last)
 // Dense product on this library's matrix-core kernels, operands as they lie in memory: tn: x [K, T],
 // a [K, O] -> x^T @ a;  nt: x [T, K], a [O, K] -> x @ a^T.  fp32 always; 16-bit types where the kernels take
 // the shape (extents and pitches that are multiples of 8, 16-byte aligned bases; nt: K a multiple of 64),
-// else padded copies of the operands and, tn, a padded result.  Undefined where neither applies (double, extents
-// beyond the kernels').
+// else padded copies of the operands and, tn, a padded result; what lies beyond the 16-bit kernels' 32-bit offsets
+// (operands of 2 GiB, rows of 2^24) is widened for the fp32 kernel, the result rounded once.  Undefined where none
+// applies (double, more than 2 097 120 rows of the result in fp32).
 Tensor dense_product(bool tn, Tensor x, Tensor a)
 {
     const at::ScalarType dt = x.scalar_type();
@@ -894,16 +895,21 @@ Tensor dense_product(bool tn, Tensor x, Tensor a)
     if (x.stride(1) != 1) x = x.contiguous();
     if (a.stride(1) != 1) a = a.contiguous();
     void *const stream = stream_of(x);
-    if (!half) {
+    const int64_t T8 = round_up(T, 8), O8 = round_up(O, 8), K64 = round_up(K, 64);
+    const bool reached = tn ? std::max({T8, O8, x.stride(0), a.stride(0)}) < (int64_t(1) << 24)
+                            : std::max(O * std::max(K64, a.stride(0)), T * std::max(K64, x.stride(0))) * 2 < k2G;
+    if (!half || !reached) {
         if (up(T, 32) > 65535) return Tensor();
+        if (half) {
+            x = x.to(at::kFloat).contiguous();
+            a = a.to(at::kFloat).contiguous();
+        }
         Tensor y = new_empty({T, O}, x);
         auto entry = tn ? nmg_gemm_tn : nmg_gemm_nt;
-        check(entry(a.data_ptr(), a.stride(0), x.data_ptr(), x.stride(0), y.data_ptr(), O, nullptr, O, K, T, dtype_code(dt), stream));
-        return y;
+        check(entry(a.data_ptr(), a.stride(0), x.data_ptr(), x.stride(0), y.data_ptr(), O, nullptr, O, K, T, NMG_F32, stream));
+        return half ? y.to(dt) : y;
     }
     if (tn) {
-        const int64_t T8 = round_up(T, 8), O8 = round_up(O, 8);
-        if (std::max({T8, O8, x.stride(0), a.stride(0)}) >= (int64_t(1) << 24)) return Tensor();
         x = padded(x, K, T8);
         a = padded(a, K, O8);
         Tensor y = new_empty({T8, O8}, x);
@@ -913,8 +919,6 @@ Tensor dense_product(bool tn, Tensor x, Tensor a)
         check(nmg_copy_rows16(y.data_ptr(), T, O, O8, out.data_ptr(), T, O, O, stream));
         return out;
     }
-    const int64_t K64 = round_up(K, 64);
-    if (O * std::max(K64, a.stride(0)) * 2 >= k2G || T * std::max(K64, x.stride(0)) * 2 >= k2G) return Tensor();
     x = padded(x, T, K64);
     a = padded(a, O, K64);
     Tensor y = new_empty({T, O}, x);

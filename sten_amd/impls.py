@@ -55,7 +55,8 @@ def _dense_product(form, x, a):
     ``"tn"``: x [K, T], a [K, O] -> x^T @ a (``nmg_gemm_tn``);  ``"nt"``: x [T, K], a [O, K] -> x @ a^T
     (``nmg_gemm_nt``).  fp32 always; 16-bit types where the kernels take the shape (extents and
     pitches that are multiples of 8, 16-byte aligned bases; ``"nt"``: K a multiple of 64), else padded
-    copies of the operands; only what neither takes (double, extents beyond 2^24) goes to ``torch.mm``."""
+    copies of the operands, and the fp32 kernel beyond their offsets (2 GiB, rows of 2^24); only what none takes
+    (double, beyond those offsets also more than 2 097 120 rows of the result) goes to ``torch.mm``."""
     y = _host.dense_product(form == "tn", x, a)
     if y is None:
         y = torch.mm(x.t(), a) if form == "tn" else torch.mm(x, a.t())
