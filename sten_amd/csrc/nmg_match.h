@@ -78,6 +78,7 @@ struct MatchParams {
     int region_bytes, r_mem, r_arr, r_int;     // LDS bytes of one tile, offsets inside
     int unit;                                  // bytes of one load of the tile data (16, 8, 4, or one element)
     int out4;                                  // four slots per thread on the way out
+    int lanes_log2;                            // lanes that hold a pattern's list in the later rounds; 0: no such rounds
     uint32_t masks[32];                        // position mask of every pattern, four per word
     uint64_t magic_cols, magic_g;
 };
@@ -301,16 +302,25 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
     match_sync<NT>();
 }
 
+// Wavefronts per SIMD that the registers are cut for.  The kernels compiled for a pattern gain from the most, whatever
+// they spill (4096 x 4096 fp16 2:4:4 with 5 / 7: 134 / 116 us); so do those of up to a wavefront per tile that take any pattern
+// (2:4:12 with 4 / 6: 136 / 125), which spill more where the columns are contiguous (1:8:8 with 5 / 6: 77 / 87).
+constexpr int match_waves(int nt, bool compiled, bool rc)
+{
+    return nt > 256 ? 4 : compiled ? (nt == 256 ? 5 : nt == 64 ? 6 : 7) : nt > 64 ? 4 : rc ? 5 : 6;
+}
+
 // NT threads per tile, at most CPT columns each.  SN, SM, SG != 0: compiled for that n:m:g.  RC: the columns are
 // the contiguous dim of the dense tensor, and the tile data lies in LDS as [position][column]; otherwise
 // as [column][position].
 template <typename T, int NT, int CPT, int SN, int SM, int SG, bool RC>
-__global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT == 256 ? 5 : NT == 64 ? 6 : 7) void match_kernel(MatchParams Q)
+__global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) void match_kernel(MatchParams Q)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int SC = SM ? match_binom(SM, SN) : 0;
     constexpr int THREADS = NT <= 64 ? 256 : NT;
     constexpr int TILES = THREADS / NT;
+    constexpr bool LISTS = NT > 16 || SM != 0;
     const int n = SN ? SN : Q.n, m = SM ? SM : Q.m, g = SG ? SG : Q.g, c = SC ? SC : Q.c;
     const int cols = SC && SG ? SC * SG : Q.cols;
     constexpr int V = 16 / (int)sizeof(T);
@@ -463,7 +473,6 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT =
                 match_partial<T, THREADS>(head_bytes + tm * Q.region_bytes, Q.r_mem, Q.r_arr, Q.r_int, c, m, g, RC ? 1 : m,
                                           RC ? ldc : 1, (int)min(Q.view.G - kc * cols, (int64_t)cols), (int)(Q.view.S - mb * m), cols / 8);
         }
-    auto mask_of = [&](int p) { return (int)((Q.masks[p >> 2] >> (8 * (p & 3))) & 0xFFu); };
     auto group_of = [&](int s) { return SG ? s / SG : (int)(((uint64_t)s * Q.magic_g) >> 32); };
     auto at = [&](int o, int r) { return RC ? r * ldc + o : o * m + r; };
 
@@ -523,12 +532,14 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT =
                 }
             }
         } else {
+            uint32_t four = Q.masks[0];
             for (int p = 0; p < c; p++) {
-                const int mk = mask_of(p);
+                const uint32_t mk = four & 0xFFu;
+                four = (p & 3) == 3 ? Q.masks[((p + 1) >> 2) & 31] : four >> 8;
                 float acc = 0;
 #pragma unroll
                 for (int r = 0; r < 8; r++)
-                    if ((mk >> r) & 1) acc += a[r];
+                    acc += __uint_as_float(__float_as_uint(a[r]) & (0u - ((mk >> r) & 1u)));      // a[r] or 0, without a branch
                 consider(acc, p);
             }
         }
@@ -538,7 +549,8 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT =
     if (live) {
         int pend = real_cols;
         // a quarter of the tile and fewer go on in the registers below
-        const int few = SG != 0 ? cols / 4 : 0;
+        const bool lists = LISTS && (SG != 0 || Q.lanes_log2 != 0);
+        const int few = lists ? cols / 4 : 0;
         // every proposal that is not the last word of its column is refused once per (column, pattern) at most
         const int limit = cols * c + 2;
         if (real_rows < m) {
@@ -659,14 +671,15 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT =
             pend = s_np[0];
         }
 
-        if constexpr (SG != 0) {
-            // Later rounds: a few columns.  L lanes hold a pattern's list, one key each in descending order, and insert a
-            // proposal by one shift along the lanes.  A pattern takes at most BUCKET proposals in a round; the rest stay
+        if constexpr (LISTS) if (lists) {
+            // Later rounds: a few columns, whatever the pattern.  L lanes hold a pattern's list, one key each in descending order, and insert a
+            // proposal by one shift along the lanes.  A pattern takes at most `bucket` proposals in a round; the rest stay
             // pending.  In a tile of several wavefronts the first one ends the matching alone, without barriers.
-            constexpr int L = SG <= 16 ? 16 : 32, BUCKET = SG / 2 < 8 ? SG / 2 : 8, EIGHT = 8;
-            static_assert(SG <= 32 && SC * SG % 4 == 0, "a list fits its lanes; lists and buckets fit the proposals' place");
+            constexpr int EIGHT = 8;
+            const int ll = SG != 0 ? (SG <= 16 ? 4 : 5) : Q.lanes_log2, L = 1 << ll, bucket = min(g / 2, 8);
+            static_assert(SG <= 32 && SG != 1, "a list fits its lanes; lists and buckets fit the proposals' place");
             uint16_t *pending = (uint16_t *)s_arr, *next = pending + cols;
-            uint64_t *s_bkt = (uint64_t *)(next + cols);
+            uint64_t *s_bkt = s_arr + (cols + 1) / 2;
             {
                 constexpr int I = (CPT + 3) / 4;      // the columns left over come as entries of eight bytes
                 uint16_t o[I];
@@ -679,8 +692,9 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT =
             }
             int round = 0;
             auto late = [&](auto active_tag, int until) {      // threads of the tile that take part
-                constexpr int A = decltype(active_tag)::value, W = A < 64 ? A : 64, WAVES = A / W, ROWS = W / L;
-                const int wave = tt / W, lane = tt % W, row = lane / L, r = lane % L;
+                constexpr int A = decltype(active_tag)::value, W = A < 64 ? A : 64, WAVES = A / W;
+                const int rows_log2 = (W == 64 ? 6 : W == 32 ? 5 : 4) - ll, rows = 1 << rows_log2;
+                const int wave = tt / W, lane = tt % W, row = lane >> ll, r = lane & (L - 1);
                 for (const int limit = cols * c + 2; round < limit && pend > until; round++) {
                     match_sync<A>();
                     int *count = s_np + 2 + (round & 1);      // zero; the other one is cleared on the way
@@ -690,10 +704,10 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT =
                             return;
                         }
                         const int p = match_pattern(key), place = atomicAdd(&s_dem[p], 1);
-                        if (place < BUCKET) s_bkt[p * BUCKET + place] = key;
+                        if (place < bucket) s_bkt[p * bucket + place] = key;
                         else next[atomicAdd(count, 1)] = (uint16_t)o;
                     };
-                    if (SC > 8 && pend * EIGHT <= A) {
+                    if (c > 8 && pend * EIGHT <= A) {
                         // eight lanes per column, each a part of the patterns
                         const int e = tt / EIGHT, sub = tt % EIGHT;
                         if (e < pend) {
@@ -701,14 +715,14 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT =
                             uint32_t best = 0;
                             int bp = 0;
 #pragma unroll 3
-                            for (int i = 0; i < (SC + EIGHT - 1) / EIGHT; i++) {
-                                const int p = min(sub + EIGHT * i, SC - 1);
+                            for (int i = 0; i < (c + EIGHT - 1) / EIGHT; i++) {
+                                const int p = min(sub + EIGHT * i, c - 1);
                                 const uint32_t ps = s_pos[p];
                                 float acc = match_abs(s_d[at(o, (int)(ps & 15u))]);
 #pragma unroll
-                                for (int j = 1; j < SN; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
+                                for (int j = 1; j < n; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
                                 const uint32_t sb = __float_as_uint(acc);
-                                if (sb >= best && match_key(sb, o, p) > s_mem[p * SG + SG - 1]) {
+                                if (sb >= best && match_key(sb, o, p) > s_mem[p * g + g - 1]) {
                                     best = sb;
                                     bp = p;
                                 }
@@ -726,34 +740,34 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT =
                         }
                     }
                     match_sync<A>();
-                    // The patterns with proposals, ROWS at a time; wavefront w has those with p / ROWS = w (mod WAVES).
-                    for (int p0 = 0; p0 < SC; p0 += W) {
-                        const int dl = p0 + lane < SC && (p0 + lane) / ROWS % WAVES == wave ? s_dem[p0 + lane] : 0;
+                    // The patterns with proposals, `rows` at a time; wavefront w has those with p / rows = w (mod WAVES).
+                    for (int p0 = 0; p0 < c; p0 += W) {
+                        const int dl = p0 + lane < c && ((p0 + lane) >> rows_log2) % WAVES == wave ? s_dem[p0 + lane] : 0;
                         uint64_t open = __ballot(dl > 0);
                         if (W < 64) open = (open >> (threadIdx.x & 63 & ~(W - 1))) & ((1ull << (W & 63)) - 1);
                         while (open != 0) {
                             uint64_t mine_bits = open;
 #pragma unroll
-                            for (int i = 0; i < ROWS; i++) {
+                            for (int i = 0; i < rows; i++) {
                                 if (i < row) mine_bits &= mine_bits - 1;
                                 open &= open - 1;
                             }
                             if (mine_bits != 0) {
                                 const int p = p0 + __ffsll((unsigned long long)mine_bits) - 1;
-                                const int d = min(s_dem[p], BUCKET);
-                                uint64_t key = r < SG ? s_mem[p * SG + r] : 0;
+                                const int d = min(s_dem[p], bucket);
+                                uint64_t key = r < g ? s_mem[p * g + r] : 0;
                                 const uint64_t was = key;
                                 for (int j = 0; j < d; j++) {
-                                    const uint64_t in = s_bkt[p * BUCKET + j];
-                                    const uint64_t before = match_swap<(L == 16 ? 0x111 : 0x138)>(key);      // row_shr:1, wave_shr:1
+                                    const uint64_t in = s_bkt[p * bucket + j];
+                                    const uint64_t before = match_swap<(SG != 0 && SG <= 16 ? 0x111 : 0x138)>(key);      // row_shr:1, wave_shr:1
                                     const bool stays = key > in, behind = r == 0 || before > in;
-                                    if (r == SG - 1) {
+                                    if (r == g - 1) {
                                         const uint64_t out = stays ? in : key;      // what the list has no place for
                                         if (out != 0) next[atomicAdd(count, 1)] = (uint16_t)match_column(out);
                                     }
                                     key = stays ? key : behind ? in : before;
                                 }
-                                if (key != was && r < SG) s_mem[p * SG + r] = key;
+                                if (key != was && r < g) s_mem[p * g + r] = key;
                                 if (r == 0) s_dem[p] = 0;
                             }
                         }
@@ -843,12 +857,12 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT =
         const int o = match_column(key), r = (int)((ps >> (4 * j)) & 15u);
         return ((const T *)reg)[at(o, r)];
     };
-    if constexpr (SN != 0 && SG % 4 == 0 && SG != 0) {
+    if constexpr (SN != 0 && SG % 4 == 0) {
         if (Q.out4) {
             constexpr int BYTES = 4 * SN * (int)sizeof(T);
             constexpr int W = BYTES % 16 == 0 ? 4 : 2;          // words per store
             for (int e = 4 * tid; e < TILES * cols; e += 4 * THREADS) {
-                const int tm = TILES == 1 ? 0 : e / cols, slot = e - tm * cols;
+                const int tm = TILES == 1 ? 0 : SG != 0 ? e / cols : (int)(((uint64_t)e * Q.magic_cols) >> 32), slot = e - tm * cols;
                 const int64_t t = tile0 + tm;
                 if (t >= Q.outer) break;
                 const unsigned char *reg = smem + head_bytes + (size_t)tm * Q.region_bytes;
@@ -857,7 +871,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, SG == 0 || NT > 256 ? 4 : NT =
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const uint64_t k = ((const uint64_t *)(reg + Q.r_mem))[slot + u];
-                    const uint32_t ps = s_pos[(slot + u) / SG];
+                    const uint32_t ps = s_pos[group_of(slot + u)];
                     o4[u] = (int16_t)match_column(k);
 #pragma unroll
                     for (int j = 0; j < SN; j++) v[u * SN + j] = elem(reg, k, ps, j);
@@ -917,6 +931,14 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     Q.region_bytes = off;
     const size_t lds = (size_t)up(c * 8, 16) + (size_t)TILES * off;
     if (lds > 160 * 1024) return NMG_OK;
+    // Two wavefronts per tile while eight tiles or more share a CU, else four (4096 x 4096, fp32 2:8:16: 137 us against
+    // 162; 2:4:80: 148 against 143).
+    if (NT == 128 && lds > 20 * 1024) return NMG_OK;
+    // Lists of 2 to 64 keys that fit the lanes of a tile.  Below 32 columns a round over all of them is the shorter way
+    // (4096 x 4096 fp16, lists -> rounds: 2:4:4 204 -> 192 us, 1:2:8 238 -> 215; from there on 2:4:8 147 -> 140, 2:4:32
+    // 131 -> 117, 2:8:8 188 -> 140, 4:8:16 482 -> 365, rounds -> lists).
+    Q.lanes_log2 = Q.g < 2 || Q.g > 64 ? 0 : Q.g <= 16 ? 4 : Q.g <= 32 ? 5 : 6;
+    if ((1 << Q.lanes_log2) > NT || cols < 32) Q.lanes_log2 = 0;
     Q.out4 = cols % 4 == 0 && (uintptr_t)Q.val % 16 == 0 && (uintptr_t)Q.idx % 8 == 0;
     auto kern = match_kernel<T, NT, CPT, SN, SM, SG, RC>;
     if (lds > 64 * 1024)
@@ -949,9 +971,26 @@ template <typename T, bool RC> static int match_dispatch(MatchParams &Q, hipStre
         const int rc = match_launch<T, MATCH_48, 4, 8, 32, RC>(Q, stream, done);
         if (rc != NMG_OK || *done) return rc;
     }
+    // Small tiles, a quarter of a wavefront each: what counts is the instructions of a proposal.  The kernels compiled for
+    // a pattern, any g, need the fewest (4096 x 4096 fp16, any pattern -> compiled: 2:4:8 112 -> 75 us, 1:4:8 107 -> 69, 1:2:16
+    // 131 -> 94, 1:5:4 164 -> 122).
+    if (Q.cols <= 64 && m <= 5 && Q.c <= 6) {
+        if (m == 2 && n == 1) return match_launch<T, 16, 4, 1, 2, 0, RC>(Q, stream, done);
+        if (m == 3 && n == 1) return match_launch<T, 16, 4, 1, 3, 0, RC>(Q, stream, done);
+        if (m == 3 && n == 2) return match_launch<T, 16, 4, 2, 3, 0, RC>(Q, stream, done);
+        if (m == 4 && n == 1) return match_launch<T, 16, 4, 1, 4, 0, RC>(Q, stream, done);
+        if (m == 4 && n == 2) return match_launch<T, 16, 4, 2, 4, 0, RC>(Q, stream, done);
+        if (m == 4 && n == 3) return match_launch<T, 16, 4, 3, 4, 0, RC>(Q, stream, done);
+        if (m == 5 && n == 1) return match_launch<T, 16, 4, 1, 5, 0, RC>(Q, stream, done);
+        if (m == 5 && n == 4) return match_launch<T, 16, 4, 4, 5, 0, RC>(Q, stream, done);
+    }
     if (Q.cols <= 64 && Q.c <= 32) return match_launch<T, 16, 4, 0, 0, 0, RC>(Q, stream, done);
     if (Q.cols <= 128 && Q.c <= 20) return match_launch<T, 32, 4, 0, 0, 0, RC>(Q, stream, done);
     if (Q.cols <= 256) return match_launch<T, 64, 4, 0, 0, 0, RC>(Q, stream, done);
+    if (Q.cols <= 512) {
+        const int rc = match_launch<T, 128, 4, 0, 0, 0, RC>(Q, stream, done);
+        if (rc != NMG_OK || *done) return rc;
+    }
     if (Q.cols <= 1024) return match_launch<T, 256, 4, 0, 0, 0, RC>(Q, stream, done);
     if (Q.cols <= 2560) return match_launch<T, 512, 5, 0, 0, 0, RC>(Q, stream, done);
     return match_launch<T, 1024, 4, 0, 0, 0, RC>(Q, stream, done);

@@ -36,3 +36,33 @@ def test_tiles_at_their_edges(n, m, g, dtype, along):
             t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
             assert np.array_equal(to_np(t.idx), idx)
             assert same_bits(t.val, val)
+
+
+# every kind of tile: lists of 2 to 64 keys in 16, 32 and 64 lanes, lists that are too long or too short for them, odd
+# numbers of columns, a quarter of a wavefront up to sixteen wavefronts per tile, patterns compiled in and any
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n,m,g", [
+    (1, 2, 8), (1, 2, 16), (1, 2, 17), (1, 2, 33), (1, 2, 64), (1, 2, 65),
+    (1, 3, 7), (2, 3, 21), (1, 4, 4), (1, 4, 8), (3, 4, 16), (1, 5, 4), (4, 5, 12),
+    (2, 4, 3), (2, 4, 5), (2, 4, 6), (2, 4, 10), (2, 4, 11), (2, 4, 21), (2, 4, 22), (2, 4, 32), (2, 4, 33), (2, 4, 43), (2, 4, 64), (2, 4, 85),
+    (2, 5, 3), (2, 5, 6), (2, 5, 7), (3, 5, 33), (1, 6, 4), (5, 6, 10), (2, 6, 1), (2, 6, 2), (3, 6, 1), (3, 6, 3), (3, 6, 25),
+    (1, 7, 9), (3, 7, 2), (3, 7, 29), (1, 8, 2), (1, 8, 8), (7, 8, 5), (2, 8, 1), (2, 8, 2), (2, 8, 3), (2, 8, 4), (2, 8, 17),
+    (2, 8, 64), (3, 8, 1), (3, 8, 50), (4, 8, 1), (4, 8, 7), (4, 8, 15),
+])
+def test_any_group_size(n, m, g, dtype):
+    cols = math.comb(m, n) * g
+    gen = torch.Generator().manual_seed(n * 1000 + m * 100 + g)
+    for along in (0, 1):
+        for k, (extra, blocks, rest) in enumerate(((cols - 1, 17, 0), (cols // 2, 3, m - 1), (1, 2, 1))):
+            w = torch.randn(cols + extra, blocks * m + rest, generator=gen) * 0.02
+            if (k + along) % 3 == 1:
+                w = torch.randint(-3, 4, w.shape, generator=gen).float() * 0.25
+            if (k + along) % 3 == 2:
+                w[torch.rand(w.shape, generator=gen) < 0.5] = 0
+            w = w.to(dtype)
+            w = w if along == 1 else w.t().contiguous()
+            print(f"case {n}:{m}:{g} {dtype} shape={tuple(w.shape)} along={along}", flush=True)
+            val, idx, _ = oracle_sparsify(w, n, m, along, g, 1 - along)
+            t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
+            assert np.array_equal(to_np(t.idx), idx)
+            assert same_bits(t.val, val)
