@@ -16,7 +16,11 @@
 //
 // Later rounds insert proposals into the lists lane by lane (the code says how).  4096 x 4096 2:4:16 fp16: 99 -> 60 us,
 // 8192 x 8192 2:8:32: 727 -> 230 us, 4096 x 4096 4:8:32: 390 -> 160 us; of the 230 us, tile data and results take 55,
-// the first proposals 15, the first round 43; the later rounds are chains of LDS round trips.
+// the first proposals 15, the first round 43; the later rounds are chains of LDS round trips.  Other group sizes, 4096 x 4096
+// fp16 with the blocks along the contiguous / the slow dim, the batched walk -> this: 2:4:4 168 -> 116 / 231 -> 113 us, 2:4:8 115 -> 75 /
+// 146 -> 76, 2:4:32 118 -> 105 / 135 -> 116, 2:4:64 130 -> 118 / 146 -> 129, 1:4:8 99 -> 69 / 151 -> 70, 1:2:8 192 -> 147 /
+// 302 -> 145, 2:8:8 293 -> 130 / 326 -> 134, 4:8:16 870 -> 366 / 810 -> 388.  Slower than the walk is 1:4:17 (107 -> 110), and where the
+// sparse extent is odd and slow, 1:4:32 (4095 x 4093: 118 -> 126) and 1:2:64 (172 -> 182).
 //
 // A round over all columns:
 //   1. every pending column computes its proposal (one thread per column; threshold of a pattern = key of its
@@ -931,9 +935,10 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     Q.region_bytes = off;
     const size_t lds = (size_t)up(c * 8, 16) + (size_t)TILES * off;
     if (lds > 160 * 1024) return NMG_OK;
-    // Two wavefronts per tile while eight tiles or more share a CU, else four (4096 x 4096, fp32 2:8:16: 137 us against
-    // 162; 2:4:80: 148 against 143).
-    if (NT == 128 && lds > 20 * 1024) return NMG_OK;
+    // Two wavefronts per tile where every CU gets eight tiles and their data fits beside each other, else four: us with two /
+    // four, 4096 x 4096 fp16 2:4:64 118 / 157 and 2:8:16 130 / 135, the latter in fp32 (22 KB a tile) 162 / 137;
+    // 777 x 1001 fp16 2:4:64 (750 tiles) 52 / 39, 2:8:16 85 / 56.
+    if (NT == 128 && (lds > 20 * 1024 || Q.outer < 8 * 256)) return NMG_OK;
     // Lists of 2 to 64 keys that fit the lanes of a tile.  Below 32 columns a round over all of them is the shorter way
     // (4096 x 4096 fp16, lists -> rounds: 2:4:4 204 -> 192 us, 1:2:8 238 -> 215; from there on 2:4:8 147 -> 140, 2:4:32
     // 131 -> 117, 2:8:8 188 -> 140, 4:8:16 482 -> 365, rounds -> lists).
