@@ -40,11 +40,12 @@ int device_order(int n, int m, const int8_t **d_order);
 // 256 bytes of zeros on the current device (file-scope array, never written).
 int device_zero_page(const void **d_zero);
 
-
-// Y[G, S] = L[T, G]^T P[T, S] (+ bias[s]) in a 16-bit type on the matrix cores (nmg_sddmm.hip).
+// Y[T, O] = X[T, K] A[O, K]^T (+ bias[o]) in a 16-bit type, both operands as rows, on 256 x 256 tiles (nmg_densefrag.hip);
+// whether that is the faster form for the extents.
 bool dense_rows16_pays(int64_t O, int64_t T);
 int dense_rows16(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy, const void *d_bias,
                  int64_t O, int64_t K, int64_t T, int dtype, void *stream);
+// Y[G, S] = L[T, G]^T P[T, S] (+ bias[s]) in a 16-bit type on the matrix cores (nmg_sddmm.hip).
 int dense_tn16(const void *d_lines, int64_t ld_lines, const void *d_pos, int64_t ld_pos, int64_t T, int64_t G, int64_t S,
                void *d_y, int64_t ldy, const void *d_bias, int dtype, void *stream);
 

@@ -664,8 +664,9 @@ static int match_tiles(const SparsifyParams &, const double *, hipStream_t, bool
 
 template <typename T> static int dispatch_sparsify(SparsifyParams &P, hipStream_t stream)
 {
-    // Tiles of at least 16 columns with at most 128 patterns of at most 8 positions: nmg_match.h.  Smaller tiles are
-    // faster in the lane teams (2:4:2, 4096 x 4096 fp16: 200 us against 315).
+    // Tiles of at least 16 columns with at most 128 patterns of at most 8 positions: nmg_match.h.  Most smaller tiles are
+    // faster in the lane teams (4096 x 4096 fp16, teams / matching: 1:2:4 201 / 265 us, 1:8:1 163 / 203, 1:4:2 165 / 206, 2:3:5
+    // 164 / 186, 2:4:2 188 / 181, 4:5:3 281 / 146; from 16 columns on 1:2:8 179 / 148, 1:4:4 256 / 121, 2:4:4 312 / 116).
     bool matched = false;
     if (int rc = match_tiles(P, (const T *)P.dense, stream, &matched)) return rc;
     if (matched) return NMG_OK;
