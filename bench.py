@@ -107,7 +107,7 @@ PMC_SUMMARIES = {
     "c2": "spmm_c2_pmc.txt",
     "decode_1": "spmm_decode_1_pmc.txt",
     "c4_b1": "w4_linear_c4_b1_pmc.txt",
-    "sparsify_c2": "sparsify_rounds_sparsify_c2_pmc.txt",
+    "sparsify_c2": "match_sparsify_pmc.txt",
 }
 
 # measured beside the headline workload in the default run: (workload, steps, warm-up)
