@@ -66,3 +66,20 @@ def test_any_group_size(n, m, g, dtype):
             t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
             assert np.array_equal(to_np(t.idx), idx)
             assert same_bits(t.val, val)
+
+
+@pytest.mark.parametrize("n,m,g,dtype", [(2, 4, 43, torch.float16), (2, 4, 85, torch.float32), (1, 8, 33, torch.float32),
+                                         (2, 8, 18, torch.float16), (3, 6, 20, torch.bfloat16), (1, 4, 66, torch.float16)])
+def test_two_wavefronts_per_tile(n, m, g, dtype):
+    """Tiles of 257 to 512 columns, enough of them to fill the chip; the last chunk and the last block are partial."""
+    cols = math.comb(m, n) * g
+    gen = torch.Generator().manual_seed(g)
+    w = (torch.randn(cols + cols // 3, 1030 * m + 1, generator=gen) * 0.02).to(dtype)
+    w[torch.rand(w.shape, generator=gen) < 0.1] = 0
+    for along in (0, 1):
+        x = w if along == 1 else w.t().contiguous()
+        print(f"case {n}:{m}:{g} {dtype} shape={tuple(x.shape)} along={along}", flush=True)
+        val, idx, _ = oracle_sparsify(x, n, m, along, g, 1 - along)
+        t = sten.GroupedNMTensor.from_dense(x.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
+        assert np.array_equal(to_np(t.idx), idx)
+        assert same_bits(t.val, val)
