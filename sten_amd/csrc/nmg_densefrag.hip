@@ -161,6 +161,7 @@ struct DfParams {
     int64_t lda;         // ROWA: row pitch of the weight, in elements
     int KP;              // K steps of 64
     int tiles_m, tiles_n;
+    int turn;            // XCD x starts its walk of the reduction x / 8 of the way in
     // reduction cut into slices (0 / 1: whole): slice s of a tile stores its sums in single
     // precision at part[s][token][output], part_ld outputs per token
     int ksplit;
@@ -246,6 +247,7 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     const int kp_per = P.ksplit > 1 ? (KPT + P.ksplit - 1) / P.ksplit : KPT;
     const int kp_lo = slice * kp_per;
     const int KP = min(KPT, kp_lo + kp_per) - kp_lo;
+    const int first = P.turn ? (int)(blockIdx.x & 7) * KP / 8 : 0;
     const int ob0 = (int)(f0 / 32) + wave * 2;
 
     const unsigned char *av_base[2];
@@ -300,8 +302,11 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     // data is unused.
     auto issue_one = [&](int kp, WSet &w, int i) {
         if (kp >= KP) kp = KP - 1;
+        const int stage = kp & (DD_NS - 1);
+        kp += first;
+        if (kp >= KP) kp -= KP;
         if (i < XL) {
-            unsigned char *base = smem + (kp & (DD_NS - 1)) * STAGE;
+            unsigned char *base = smem + stage * STAGE;
             const unsigned char *xb = x_base + (int64_t)kp * XSTEP;
 #pragma unroll
             for (int q = 0; q < XL; q++)
@@ -521,6 +526,7 @@ template <typename T, int TB, int NH, bool XT = false, bool CT = XT, bool ROWA =
     P.tiles_n = (int)((P.T + TT - 1) / TT);
     const int slices = P.ksplit > 1 ? P.ksplit : 1;
     dim3 grid((unsigned)(P.tiles_m * P.tiles_n * slices));
+    P.turn = stagger_xcds(grid.x, P.KP / slices, P.KP * (P.O + P.T) * 128) ? 1 : 0;
     constexpr size_t ring = (size_t)DD_NS * TT * 128;
     constexpr size_t stg = CT ? (size_t)4 * 64 * (TT * 2 + 16) : (size_t)4 * TT * (4 * 32 + 16);
     constexpr size_t lds = ring > stg ? ring : stg;

@@ -62,6 +62,8 @@ struct SmfParams {
     int MB, KP;          // feature blocks of 32, k pairs of 64
     int tiles_m, tiles_n;
     int band;            // direct kernel: line tiles per band of the tile walk (4 or 8)
+    int turn;            // direct kernel: XCD x starts its walk of the reduction x / 8 of the way in
+    bool in_order;       // a tile asked for by number: sums in the order of the reduction, alike for every tile
     // direct kernel with the reduction cut into slices (0 / 1: whole): slice s of a tile writes
     // its sums in single precision to part[s][token][feature], part_ld features per token
     int ksplit;
@@ -334,6 +336,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
     const int kp_per = P.ksplit > 1 ? (KPT + P.ksplit - 1) / P.ksplit : KPT;
     const int kp_lo = slice * kp_per;
     const int KP = min(KPT, kp_lo + kp_per) - kp_lo;
+    const int first = P.turn ? (int)(blockIdx.x & 7) * KP / 8 : 0;
     const int wm = wave / WN, wn = wave % WN;
     const int mb0 = (int)(f0 / 32) + wm * FB;
 
@@ -383,8 +386,11 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
     // the operation count stays uniform, the data is unused.
     auto issue_one = [&](int kp, WSet &w, int i) {
         if (kp >= KP) kp = KP - 1;
+        const int stage = kp & (DR_NS - 1);
+        kp += first;
+        if (kp >= KP) kp -= KP;
         if (i < XL) {
-            unsigned char *base = smem + (kp & (DR_NS - 1)) * STAGE;
+            unsigned char *base = smem + stage * STAGE;
             const unsigned char *xb = x_base + (int64_t)kp * XSTEP;
 #pragma unroll
             for (int q = 0; q < XL; q++)
@@ -666,6 +672,7 @@ static int launch_smfmac_direct(SmfParams &P, hipStream_t s)
     P.band = (int64_t)TT * 2 * 8 > (int64_t)TF * 9 ? 8 : 4;   // bytes per reduction position: TT * 2 against TF * 9 / 8
     const int slices = P.ksplit > 1 ? P.ksplit : 1;
     dim3 grid((unsigned)(P.tiles_m * P.tiles_n * slices));
+    P.turn = !P.in_order && stagger_xcds(grid.x, P.KP / slices, P.KP * (int64_t)(P.MB * 32 * 72 + P.T * 128)) ? 1 : 0;
     constexpr size_t ring = (size_t)DR_NS * TT * 128;
     constexpr size_t stg = CT ? (size_t)4 * FB * 32 * (TB * 64 + 16) : (size_t)4 * TB * 32 * (FB * 64 + 16);
     constexpr size_t lds = ring > stg ? ring : stg;
@@ -1176,6 +1183,7 @@ static int smfmac_tile(const SmfParams &P)
 
 template <typename T> static int launch_smfmac(SmfParams &P, int variant, hipStream_t s)
 {
+    P.in_order = variant >= 0;
     if (variant < 0) variant = smfmac_tile(P);
     switch (variant) {
     case 0: return launch_smfmac_cfg<T, 2, 2, 4, 2, 1>(P, s);  // register-prefetch kernel, 256 lines x 128 tokens: any K

@@ -18,6 +18,19 @@ __device__ __forceinline__ uint16_t f32_to_bits16(float x, __hip_bfloat16 *)
     return *reinterpret_cast<uint16_t *>(&b);
 }
 
+// Grids of at most one workgroup per CU: all workgroups walk the reduction in step, so that the XCDs that share a weight
+// or an activation (2 and 4 of the 8 where the tiles are 16 x 16) ask memory for the same line at the same moment and all
+// wait for it.  Started x / 8 of the reduction apart, XCD by XCD, the first one to come by brings a line into the
+// memory-side cache and the others find it there.  Operands new in every pass, us: 4096 x 11008 2:4 fp16 x 2048 tokens
+// 114.5 -> 106, x 777 67 -> 60.5; its transpose on the dense cores x 512 58.5 -> 54; torch.mm 4096^2 x 2048 with both
+// gradients 183 -> 177.  Shorter walks put the XCDs a few steps apart only (21 steps of 64: 39.4 -> 42, 32 steps: 56.8 -> 59);
+// operands beyond that cache of 256 MB are gone before the others come by (268 MB, dense cores, 16384 x 4096 transposed x
+// 4096: 0.5 to 0.8 % of a training step lost); and with more than one round of workgroups the XCDs drift apart by themselves.
+inline bool stagger_xcds(unsigned workgroups, int steps, int64_t operand_bytes)
+{
+    return workgroups <= 256 && steps >= 64 && operand_bytes <= (int64_t)192 << 20;
+}
+
 // Where an output tile goes: Y[T, M] row-major with leading dimension ldy, optional bias[M].
 struct TileOut {
     void *y;
