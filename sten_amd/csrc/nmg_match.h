@@ -14,9 +14,12 @@
 // and all but the first concern a few columns: 13 of 96 are sent away in total (2:4:16), 113 of 896
 // (2:8:32), 299 of 2240 (4:8:32).
 //
-// Later rounds insert proposals into the lists lane by lane (the code says how).  4096 x 4096 2:4:16 fp16: 99 -> 60 us,
-// 8192 x 8192 2:8:32: 727 -> 230 us, 4096 x 4096 4:8:32: 390 -> 160 us; of the 230 us, tile data and results take 55,
-// the first proposals 15, the first round 43; the later rounds are chains of LDS round trips.  Other group sizes, 4096 x 4096
+// Later rounds insert proposals into the lists lane by lane (the code says how).  4096 x 4096 2:4:16 fp16: 99 -> 58 us,
+// 8192 x 8192 2:8:32: 727 -> 201 us, 4096 x 4096 4:8:32: 390 -> 140 us.  What bounds it is the issue of vector instructions (1200 for a
+// wavefront of two tiles 2:4:16, 0.74 of the time; 0.66 at 2:8:32) and, in the later rounds, chains of LDS round trips: of the 201 us,
+// tile data and results take 52, the first proposals 15, the first round 44, the later rounds 90.  A list in 16 lanes of one or two
+// keys, merged two proposals at a time, and eight lanes (2:4: two) on a column's patterns took these from 122 (whole kernel 233; 2:4:16
+// 59.3 -> 57.8, 1:8:32 43.5 -> 39.5, 4:8:32 172 -> 140, fp32 238 -> 191).  Other group sizes, 4096 x 4096
 // fp16 with the blocks along the contiguous / the slow dim, the batched walk -> this: 2:4:4 168 -> 116 / 231 -> 113 us, 2:4:8 115 -> 75 /
 // 146 -> 76, 2:4:32 118 -> 105 / 135 -> 116, 2:4:64 130 -> 118 / 146 -> 129, 1:4:8 99 -> 69 / 151 -> 70, 1:2:8 192 -> 147 /
 // 302 -> 145, 2:8:8 293 -> 130 / 326 -> 134, 4:8:16 870 -> 366 / 810 -> 388.  Slower than the walk is 1:4:17 (107 -> 110), and where the
@@ -129,9 +132,9 @@ __device__ __forceinline__ float match_abs(__hip_bfloat16 x) { return fabsf(__bf
 // put on top, so that a group of proposals is followed by smaller keys.  0: none.
 __device__ __forceinline__ uint64_t match_key(uint32_t score, int o, int p)
 {
-    return ((uint64_t)(((uint32_t)(127 - p) << 16) | (score >> 16)) << 32) | ((score << 16) | (uint32_t)o);
+    return ((uint64_t)(((uint32_t)(255 - p) << 16) | (score >> 16)) << 32) | ((score << 16) | (uint32_t)o);
 }
-__device__ __forceinline__ int match_pattern(uint64_t key) { return 127 - (int)(key >> 48); }
+__device__ __forceinline__ int match_pattern(uint64_t key) { return 255 - (int)(key >> 48); }
 __device__ __forceinline__ int match_column(uint64_t key) { return (int)(key & 0xFFFFu); }
 
 constexpr int kMatchTables = 6;      // c ints each, and four counts (three of them for partial blocks only)
@@ -676,14 +679,14 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
         }
 
         if constexpr (LISTS) if (lists) {
-            // Later rounds: a few columns, whatever the pattern.  L lanes hold a pattern's list, one key each in descending order, and insert a
-            // proposal by one shift along the lanes.  A pattern takes at most `bucket` proposals in a round; the rest stay
-            // pending.  In a tile of several wavefronts the first one ends the matching alone, without barriers.
-            constexpr int EIGHT = 8;
-            const int ll = SG != 0 ? (SG <= 16 ? 4 : 5) : Q.lanes_log2, L = 1 << ll, bucket = min(g / 2, 8);
+            // Later rounds: a few columns, whatever the pattern.  L lanes hold a pattern's list, KPL keys each in descending
+            // order, and insert a proposal by one shift along the lanes.  A pattern takes at most `bucket` proposals in a round;
+            // the rest stay pending.  In a tile of several wavefronts the first one ends the matching alone, without barriers.
+            constexpr int EIGHT = 8, KPL = SG > 16 ? 2 : 1;
+            const int ll = SG != 0 ? 4 : Q.lanes_log2, L = 1 << ll, bucket = min(g / 2, 8);
             static_assert(SG <= 32 && SG != 1, "a list fits its lanes; lists and buckets fit the proposals' place");
             uint16_t *pending = (uint16_t *)s_arr, *next = pending + cols;
-            uint64_t *s_bkt = s_arr + (cols + 1) / 2;
+            uint64_t *s_bkt = s_arr + (cols + 1) / 2;      // free places hold 0
             {
                 constexpr int I = (CPT + 3) / 4;      // the columns left over come as entries of eight bytes
                 uint16_t o[I];
@@ -693,6 +696,14 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 #pragma unroll
                 for (int i = 0; i < I; i++)
                     if (tt + NT * i < pend) pending[tt + NT * i] = o[i];
+                for (int i = tt; i < c * bucket; i += NT) s_bkt[i] = 0;
+            }
+            // a column's patterns go to EL lanes; the positions of a lane's patterns stay in registers
+            constexpr int EL = SC >= 16 ? 8 : SC >= 8 ? 4 : 2, PER = SG != 0 ? (SC + EL - 1) / EL : 1;
+            uint32_t mypos[PER];
+            if constexpr (SG != 0) {
+#pragma unroll
+                for (int i = 0; i < PER; i++) mypos[i] = s_pos[min(tt % EL + EL * i, SC - 1)];
             }
             int round = 0;
             auto late = [&](auto active_tag, int until) {      // threads of the tile that take part
@@ -711,8 +722,31 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                         if (place < bucket) s_bkt[p * bucket + place] = key;
                         else next[atomicAdd(count, 1)] = (uint16_t)o;
                     };
-                    if (c > 8 && pend * EIGHT <= A) {
-                        // eight lanes per column, each a part of the patterns
+                    auto best_of = [&](int o, int p, uint32_t ps, uint32_t &best, int &bp) {
+                        float acc = match_abs(s_d[at(o, (int)(ps & 15u))]);
+#pragma unroll
+                        for (int j = 1; j < n; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
+                        const uint32_t sb = __float_as_uint(acc);
+                        if (sb >= best && match_key(sb, o, p) > s_mem[p * g + g - 1]) {
+                            best = sb;
+                            bp = p;
+                        }
+                    };
+                    if constexpr (SG != 0) {
+                        const int sub = tt % EL;
+                        for (int e = tt / EL; e < pend; e += A / EL) {
+                            const int o = (int)pending[e];
+                            uint32_t best = 0;
+                            int bp = 0;
+#pragma unroll
+                            for (int i = 0; i < PER; i++) best_of(o, min(sub + EL * i, SC - 1), mypos[i], best, bp);
+                            uint64_t top = ((uint64_t)best << 32) | (uint32_t)bp;
+                            top = max(top, match_swap<0xB1>(top));                    // lanes 1 apart, 2 apart, the two quads
+                            if (EL >= 4) top = max(top, match_swap<0x4E>(top));
+                            if (EL >= 8) top = max(top, match_swap<0x141>(top));
+                            if (sub == 0) put(o, (top >> 32) == 0 ? 0 : match_key((uint32_t)(top >> 32), o, (int)(top & 0xFFu)));
+                        }
+                    } else if (c > 8 && pend * EIGHT <= A) {
                         const int e = tt / EIGHT, sub = tt % EIGHT;
                         if (e < pend) {
                             const int o = (int)pending[e];
@@ -721,18 +755,10 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 #pragma unroll 3
                             for (int i = 0; i < (c + EIGHT - 1) / EIGHT; i++) {
                                 const int p = min(sub + EIGHT * i, c - 1);
-                                const uint32_t ps = s_pos[p];
-                                float acc = match_abs(s_d[at(o, (int)(ps & 15u))]);
-#pragma unroll
-                                for (int j = 1; j < n; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
-                                const uint32_t sb = __float_as_uint(acc);
-                                if (sb >= best && match_key(sb, o, p) > s_mem[p * g + g - 1]) {
-                                    best = sb;
-                                    bp = p;
-                                }
+                                best_of(o, p, s_pos[p], best, bp);
                             }
                             uint64_t top = ((uint64_t)best << 32) | (uint32_t)bp;
-                            top = max(top, match_swap<0xB1>(top));       // lanes 1 apart, 2 apart, the two quads
+                            top = max(top, match_swap<0xB1>(top));
                             top = max(top, match_swap<0x4E>(top));
                             top = max(top, match_swap<0x141>(top));
                             if (sub == 0) put(o, (top >> 32) == 0 ? 0 : match_key((uint32_t)(top >> 32), o, (int)(top & 0xFFu)));
@@ -744,36 +770,72 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                         }
                     }
                     match_sync<A>();
+                    // a pattern's proposals into its list, AT at a time
+                    auto merge = [&](int p) {
+                        constexpr int AT = SG != 0 ? 2 : 1;
+                        static_assert(SG == 0 || (SG / 2 < 8 ? SG / 2 : 8) % AT == 0, "whole batches");
+                        uint64_t *list = s_mem + p * g + r * KPL, *bkt = s_bkt + p * bucket;
+                        uint64_t key[KPL], in[AT], ahead[AT];
+#pragma unroll
+                        for (int i = 0; i < KPL; i++) key[i] = r * KPL + i < g ? list[i] : 0;
+#pragma unroll
+                        for (int u = 0; u < AT; u++) in[u] = bkt[u];
+                        for (int j = AT; in[0] != 0; j += AT) {
+#pragma unroll
+                            for (int u = 0; u < AT; u++) ahead[u] = bkt[j + u];      // (the last batch reads past the bucket)
+                            uint64_t out[AT];
+#pragma unroll
+                            for (int u = 0; u < AT; u++) {
+                                // key(i) = max(key(i), min(key(i - 1), in)): the keys are positive doubles and no NaN
+                                auto lo = [](uint64_t x, uint64_t y) {
+                                    return __builtin_bit_cast(uint64_t, __builtin_fmin(__builtin_bit_cast(double, x), __builtin_bit_cast(double, y)));
+                                };
+                                auto hi = [](uint64_t x, uint64_t y) {
+                                    return __builtin_bit_cast(uint64_t, __builtin_fmax(__builtin_bit_cast(double, x), __builtin_bit_cast(double, y)));
+                                };
+                                uint64_t before = match_swap<(SG != 0 ? 0x111 : 0x138)>(key[KPL - 1]);      // row_shr:1, wave_shr:1
+                                if (r == 0) before = in[u];
+                                out[u] = lo(key[(g - 1) % KPL], in[u]);
+#pragma unroll
+                                for (int i = KPL - 1; i > 0; i--) key[i] = hi(key[i], lo(key[i - 1], in[u]));
+                                key[0] = hi(key[0], lo(before, in[u]));
+                            }
+                            if (r == (g - 1) / KPL) {      // what the list has no place for
+                                int has = 0;
+#pragma unroll
+                                for (int u = 0; u < AT; u++) has += out[u] != 0 ? 1 : 0;
+                                if (has != 0) {
+                                    int to = atomicAdd(count, has);
+#pragma unroll
+                                    for (int u = 0; u < AT; u++)
+                                        if (out[u] != 0) next[to++] = (uint16_t)match_column(out[u]);
+                                }
+                            }
+#pragma unroll
+                            for (int u = 0; u < AT; u++) in[u] = j < bucket ? ahead[u] : 0;
+                        }
+#pragma unroll
+                        for (int i = 0; i < KPL; i++)
+                            if (r * KPL + i < g) list[i] = key[i];
+                        if (r < bucket) bkt[r] = 0;
+                        if (r == 0) s_dem[p] = 0;
+                    };
                     // The patterns with proposals, `rows` at a time; wavefront w has those with p / rows = w (mod WAVES).
                     for (int p0 = 0; p0 < c; p0 += W) {
                         const int dl = p0 + lane < c && ((p0 + lane) >> rows_log2) % WAVES == wave ? s_dem[p0 + lane] : 0;
                         uint64_t open = __ballot(dl > 0);
                         if (W < 64) open = (open >> (threadIdx.x & 63 & ~(W - 1))) & ((1ull << (W & 63)) - 1);
-                        while (open != 0) {
-                            uint64_t mine_bits = open;
+                        using Bits = typename std::conditional<W == 64, uint64_t, uint32_t>::type;
+                        Bits left = (Bits)open;
+                        while (left != 0) {
+                            int p = -1;
 #pragma unroll
                             for (int i = 0; i < rows; i++) {
-                                if (i < row) mine_bits &= mine_bits - 1;
-                                open &= open - 1;
+                                const int q = W == 64 ? __ffsll((unsigned long long)left) : __ffs((unsigned)left);      // 0: none
+                                if (row == i) p = q - 1;
+                                left &= left - 1;
                             }
-                            if (mine_bits != 0) {
-                                const int p = p0 + __ffsll((unsigned long long)mine_bits) - 1;
-                                const int d = min(s_dem[p], bucket);
-                                uint64_t key = r < g ? s_mem[p * g + r] : 0;
-                                const uint64_t was = key;
-                                for (int j = 0; j < d; j++) {
-                                    const uint64_t in = s_bkt[p * bucket + j];
-                                    const uint64_t before = match_swap<(SG != 0 && SG <= 16 ? 0x111 : 0x138)>(key);      // row_shr:1, wave_shr:1
-                                    const bool stays = key > in, behind = r == 0 || before > in;
-                                    if (r == g - 1) {
-                                        const uint64_t out = stays ? in : key;      // what the list has no place for
-                                        if (out != 0) next[atomicAdd(count, 1)] = (uint16_t)match_column(out);
-                                    }
-                                    key = stays ? key : behind ? in : before;
-                                }
-                                if (key != was && r < g) s_mem[p * g + r] = key;
-                                if (r == 0) s_dem[p] = 0;
-                            }
+                            if (p >= 0) merge(p0 + p);
                         }
                     }
                     if (tt == 0) s_np[2 + ((round & 1) ^ 1)] = 0;
@@ -785,7 +847,9 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                 }
             };
             if constexpr (NT > 64) {
-                late(std::integral_constant<int, NT>{}, 16);
+                // (4096 x 4096 fp16, 16 -> 8 columns left to the first wavefront: 2:8:64 164 -> 145 us, 2:8:32 60.5 -> 58.5; with
+                // two wavefronts 3:8:8 244 -> 264 / 240 -> 222)
+                late(std::integral_constant<int, NT>{}, NT >= 256 ? 8 : 16);
                 __syncthreads();
                 if (tt < 64) late(std::integral_constant<int, 64>{}, 0);
                 __syncthreads();

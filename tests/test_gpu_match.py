@@ -83,3 +83,22 @@ def test_two_wavefronts_per_tile(n, m, g, dtype):
         t = sten.GroupedNMTensor.from_dense(x.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
         assert np.array_equal(to_np(t.idx), idx)
         assert same_bits(t.val, val)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n,m,g", [(2, 4, 16), (1, 8, 32), (2, 8, 32), (3, 6, 12), (4, 8, 32), (2, 4, 8), (2, 4, 32), (2, 8, 8), (3, 8, 8)])
+def test_columns_that_want_the_same_patterns(n, m, g, dtype):
+    # magnitudes that fall along the block: most columns propose to one pattern, lists and buckets run over, and the
+    # refusals come in long chains; mild, so that the later rounds see them, and steep
+    cols = math.comb(m, n) * g
+    gen = torch.Generator().manual_seed(n * 100 + m * 10 + g)
+    for along in (0, 1):
+        for fall in (0.9, 0.6):
+            w = (torch.randn(2 * cols - 3, 3 * m, generator=gen) * 0.1 + 1) * fall ** (torch.arange(3 * m) % m)
+            w = w.to(dtype)
+            w = w if along == 1 else w.t().contiguous()
+            print(f"case {n}:{m}:{g} {dtype} along={along} fall={fall}", flush=True)
+            val, idx, _ = oracle_sparsify(w, n, m, along, g, 1 - along)
+            t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
+            assert np.array_equal(to_np(t.idx), idx)
+            assert same_bits(t.val, val)
