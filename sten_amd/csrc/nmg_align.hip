@@ -84,48 +84,63 @@ __global__ __launch_bounds__(256) void transpose16_kernel(Transpose16 P)
 }
 
 // y[c] = sum over the rows of x[r, c], single-precision sums, rounded once: the bias gradient of a linear layer.  A
-// workgroup owns 32 columns (32 lanes x 4 bytes, 64 columns in pairs of the 16-bit types) over all rows, 32 rows at a time with
-// 16 loads per lane in flight, and adds its 32 partial rows through LDS in order: one launch, no semaphores to clear.
-// Bound by latency at the sizes it takes (512 x 768 in single precision: 4.0 us; the library's sum and the fill in front of it 11.5).
+// workgroup owns 64 or 128 bytes of every row (lanes of 16 bytes; narrow, so that a few hundred columns still are a few
+// dozen workgroups), 256 or 128 rows at a time with four loads per lane in flight, and adds its partial rows through LDS in
+// order: one launch, no semaphores to clear.  Bound by the loads that a few dozen workgroups keep in flight.  us, lanes of 4 bytes
+// and 32 rows at a time -> this: bf16 1667 x 3840 32.5 -> 5.7, 2184 x 1472 40.0 -> 5.4, 3881 x 1640 70.3 -> 9.6, fp16 4096 x 16384
+// 104 -> 28 (4.8 TB/s), fp32 512 x 768 3.3 -> 3.2 (the library's sum and the fill in front of it 11.5), 4096 x 4096 19.3 -> 19.1.
 struct ColSum {
     const void *x;
     void *y;
     int64_t rows, cols, ld;
 };
-constexpr int CS_ROWS = 32, CS_DEEP = 16;
+constexpr int CS_THREADS = 1024, CS_DEEP = 4;
 
-template <typename T> __global__ __launch_bounds__(1024) void colsum_kernel(ColSum P)
+template <typename T, int CS_LANES> __global__ __launch_bounds__(CS_THREADS) void colsum_kernel(ColSum P)
 {
-    constexpr int E = 4 / (int)sizeof(T);
-    __shared__ float part[CS_ROWS][32 * E + 1];
-    const int tid = threadIdx.x, cl = tid & 31, rl = tid >> 5;
-    const int64_t c = ((int64_t)blockIdx.x * 32 + cl) * E;
+    constexpr int CS_ROWS = CS_THREADS / CS_LANES;
+    constexpr int E = 16 / (int)sizeof(T), W = CS_LANES * E, GROUPS = CS_THREADS / W;
+    __shared__ float part[CS_ROWS][W + 4], sums[GROUPS][W];
+    const int tid = threadIdx.x, cl = tid % CS_LANES, rl = tid / CS_LANES;
+    const int64_t c = (int64_t)blockIdx.x * W + cl * E;
+    const int valid = (int)min((int64_t)E, P.cols - c);      // columns of the lane that exist
     float acc[E];
 #pragma unroll
     for (int e = 0; e < E; e++) acc[e] = 0.f;
-    for (int64_t r0 = rl; r0 < P.rows; r0 += CS_ROWS * CS_DEEP) {
-        float v[CS_DEEP][E];
+    const T *x = (const T *)P.x + c;
+    if (valid == E) {
+        for (int64_t r0 = rl; r0 < P.rows; r0 += CS_ROWS * CS_DEEP) {
+            T v[CS_DEEP][E];
 #pragma unroll
-        for (int u = 0; u < CS_DEEP; u++) {
-            const int64_t r = r0 + u * CS_ROWS;
+            for (int u = 0; u < CS_DEEP; u++)      // (a global load needs the alignment of its elements only)
+                __builtin_memcpy(v[u], x + min(r0 + u * CS_ROWS, P.rows - 1) * P.ld, 16);
 #pragma unroll
-            for (int e = 0; e < E; e++) v[u][e] = r < P.rows && c + e < P.cols ? to_f32(((const T *)P.x)[r * P.ld + c + e]) : 0.f;
+            for (int u = 0; u < CS_DEEP; u++)
+#pragma unroll
+                for (int e = 0; e < E; e++) acc[e] += r0 + u * CS_ROWS < P.rows ? to_f32(v[u][e]) : 0.f;
         }
+    } else {
+        for (int64_t r = rl; r < P.rows; r += CS_ROWS)
 #pragma unroll
-        for (int u = 0; u < CS_DEEP; u++)
-#pragma unroll
-            for (int e = 0; e < E; e++) acc[e] += v[u][e];
+            for (int e = 0; e < E; e++)
+                if (e < valid) acc[e] += to_f32(x[r * P.ld + e]);
     }
 #pragma unroll
     for (int e = 0; e < E; e++) part[rl][cl * E + e] = acc[e];
     __syncthreads();
-    if (tid >= 32 * E) return;
-    const int64_t col = (int64_t)blockIdx.x * 32 * E + tid;
-    if (col >= P.cols) return;
+    const int col = tid % W, grp = tid / W;
     float s = 0.f;
-    for (int r = 0; r < CS_ROWS; r++) s += part[r][tid];
-    if constexpr (sizeof(T) == 4) ((float *)P.y)[col] = s;
-    else ((uint16_t *)P.y)[col] = f32_to_bits16(s, (T *)nullptr);
+#pragma unroll
+    for (int r = 0; r < CS_ROWS / GROUPS; r++) s += part[grp * (CS_ROWS / GROUPS) + r][col];
+    sums[grp][col] = s;
+    __syncthreads();
+    const int64_t to = (int64_t)blockIdx.x * W + tid;
+    if (tid >= W || to >= P.cols) return;
+    s = 0.f;
+#pragma unroll
+    for (int r = 0; r < GROUPS; r++) s += sums[r][tid];
+    if constexpr (sizeof(T) == 4) ((float *)P.y)[to] = s;
+    else ((uint16_t *)P.y)[to] = f32_to_bits16(s, (T *)nullptr);
 }
 
 }  // namespace nmg
@@ -172,13 +187,18 @@ extern "C" int nmg_colsum(const void *d_x, int64_t rows, int64_t cols, int64_t l
     if (cols == 0) return NMG_OK;
     NMG_REQUIRE(d_y && (d_x || rows == 0), NMG_ERR_ARG, "null device pointer");
     ColSum P{d_x, d_y, rows, cols, ld};
-    const int64_t per = dtype == NMG_F32 ? 32 : 64, blocks = (cols + per - 1) / per;
+    const int64_t row_bytes = cols * (dtype == NMG_F32 ? 4 : 2);
+    // us, 4 / 8 / 16 lanes: 3881 x 1640 bf16 9.6 / 13.1 / 23.1, 1667 x 3840 bf16 6.1 / 5.7 / 8.1, 4096 x 4096 fp32 22.9 / 19.1 / 24.8,
+    // 4096 x 16384 fp16 42.6 / 28.1 / 29.1: whole 128-byte lines from the width on that still gives enough workgroups
+    const int lanes = row_bytes >= 56 * 128 ? 8 : 4;
+    const int64_t blocks = (row_bytes + 16 * lanes - 1) / (16 * lanes);
     NMG_REQUIRE(blocks <= 0x7fffffffLL, NMG_ERR_UNSUPPORTED, "too many columns for one launch");
     hipStream_t s = (hipStream_t)stream;
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(CS_THREADS), 0, s, P); };
     switch (dtype) {
-    case NMG_F32: hipLaunchKernelGGL(colsum_kernel<float>, dim3((unsigned)blocks), dim3(1024), 0, s, P); break;
-    case NMG_F16: hipLaunchKernelGGL(colsum_kernel<__half>, dim3((unsigned)blocks), dim3(1024), 0, s, P); break;
-    default: hipLaunchKernelGGL(colsum_kernel<__hip_bfloat16>, dim3((unsigned)blocks), dim3(1024), 0, s, P); break;
+    case NMG_F32: launch(lanes == 4 ? colsum_kernel<float, 4> : colsum_kernel<float, 8>); break;
+    case NMG_F16: launch(lanes == 4 ? colsum_kernel<__half, 4> : colsum_kernel<__half, 8>); break;
+    default: launch(lanes == 4 ? colsum_kernel<__hip_bfloat16, 4> : colsum_kernel<__hip_bfloat16, 8>); break;
     }
     NMG_HIP_TRY(hipGetLastError());
     return NMG_OK;

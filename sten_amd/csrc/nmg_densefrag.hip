@@ -297,17 +297,18 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
         u32x4 a[AB][2];   // [block of 16 outputs][k-step of 32]
     };
     WSet ws[DD_D + 1];
-    // load number i (0 .. OPS-1) of K step kp: first the XL activation DMA loads, then the 2 * AB
-    // weight fragments.  Steps beyond the last repeat it: the operation count stays uniform, the
+    // load number i (0 .. OPS-1) of the walk's K step kp, step `at` of the operands: first the XL activation DMA loads, then
+    // the 2 * AB weight fragments.  Steps beyond the last fetch the last one again: the operation count stays uniform, the
     // data is unused.
+    int at = first;
+    auto advance = [&](int kp) {      // after the loads of step kp
+        const int after = at + 1 == KP ? 0 : at + 1;      // (selects: no branch between the hand-tracked loads)
+        at = kp + 1 < KP ? after : at;
+    };
     auto issue_one = [&](int kp, WSet &w, int i) {
-        if (kp >= KP) kp = KP - 1;
-        const int stage = kp & (DD_NS - 1);
-        kp += first;
-        if (kp >= KP) kp -= KP;
         if (i < XL) {
-            unsigned char *base = smem + stage * STAGE;
-            const unsigned char *xb = x_base + (int64_t)kp * XSTEP;
+            unsigned char *base = smem + (kp & (DD_NS - 1)) * STAGE;
+            const unsigned char *xb = x_base + (int64_t)at * XSTEP;
 #pragma unroll
             for (int q = 0; q < XL; q++)
                 if (q == i)
@@ -321,7 +322,7 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
 #pragma unroll
                 for (int k32 = 0; k32 < 2; k32++)
                     if (XL + ab * 2 + k32 == i) {
-                        const unsigned char *av = av_base[ab >> 1] + (int64_t)kp * (ROWA ? 128 : 4096);
+                        const unsigned char *av = av_base[ab >> 1] + (int64_t)at * (ROWA ? 128 : 4096);
                         asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3"
                                      : "=v"(w.a[ab][k32])
                                      : "v"(ROWA ? row_a[ROWA ? ab : 0] : lane_a), "s"(av),
@@ -422,9 +423,11 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
 
     // prologue: steps 0 .. DD_D-1 in flight, then wait for step 0
 #pragma unroll
-    for (int st = 0; st < DD_D; st++)
+    for (int st = 0; st < DD_D; st++) {
 #pragma unroll
         for (int i = 0; i < OPS; i++) issue_one(st, ws[st], i);
+        advance(st);
+    }
     landed(ws[0]);
     asm volatile("s_barrier" ::: "memory");
 #pragma unroll
@@ -434,7 +437,7 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
 #pragma unroll
         for (int u = 0; u <= DD_D; u++) {
             const int kp = kp0 + u;
-            if (kp >= KP) break;
+            if (kp >= KP) goto walked;      // (past the loop: a break would be tested again there)
             const unsigned char *base = smem + (kp & (DD_NS - 1)) * STAGE;
             const unsigned char *next = smem + ((kp + 1) & (DD_NS - 1)) * STAGE;
             // A phase: its MFMAs, and behind one MFMA each the fragment reads of the next phase and
@@ -444,6 +447,7 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
             auto phase = [&](auto ph_tag) {
                 constexpr int PH = decltype(ph_tag)::value;
                 if constexpr (PH == NP - 1) {
+                    advance(kp + DD_D);
                     mma(ws[u], fr[PH % 2], ph_tag, 0);
                     mma(ws[u], fr[PH % 2], ph_tag, 1);
                     __builtin_amdgcn_sched_barrier(0);
@@ -493,6 +497,7 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
             static_assert(NP == 2 || NP == 4 || NP == 8, "one, two or four token parts");
         }
     }
+walked:
     pin_acc();
     // The loads of the steps beyond the last are still in flight and nothing reads what they bring:
     // every register of the ring passes through the final wait.

@@ -381,17 +381,18 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
         uint32_t ix[FB];
     };
     WSet ws[DR_D + 1];
-    // Load number i (0 .. OPS-1) of K step kp: first the XL activation DMA loads, then per
-    // feature block two weight fragments and the index word.  Steps beyond the last repeat it:
-    // the operation count stays uniform, the data is unused.
+    // Load number i (0 .. OPS-1) of the K step that is the walk's step kp, step `at` of the operands: first the XL activation
+    // DMA loads, then per feature block two weight fragments and the index word.  Steps beyond the last
+    // fetch the last one again: the operation count stays uniform, the data is unused.
+    int at = first;
+    auto advance = [&](int kp) {      // after the loads of step kp
+        const int after = at + 1 == KP ? 0 : at + 1;      // (selects: no branch between the hand-tracked loads)
+        at = kp + 1 < KP ? after : at;
+    };
     auto issue_one = [&](int kp, WSet &w, int i) {
-        if (kp >= KP) kp = KP - 1;
-        const int stage = kp & (DR_NS - 1);
-        kp += first;
-        if (kp >= KP) kp -= KP;
         if (i < XL) {
-            unsigned char *base = smem + stage * STAGE;
-            const unsigned char *xb = x_base + (int64_t)kp * XSTEP;
+            unsigned char *base = smem + (kp & (DR_NS - 1)) * STAGE;
+            const unsigned char *xb = x_base + (int64_t)at * XSTEP;
 #pragma unroll
             for (int q = 0; q < XL; q++)
                 if (q == i)
@@ -406,8 +407,8 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
             // still in flight would copy stale data.
 #pragma unroll
             for (int fb = 0; fb < FB; fb++) {
-                const unsigned char *av = av_base[fb] + (int64_t)kp * 2048;
-                const unsigned char *ai = ai_base[fb] + (int64_t)kp * 256;
+                const unsigned char *av = av_base[fb] + (int64_t)at * 2048;
+                const unsigned char *ai = ai_base[fb] + (int64_t)at * 256;
                 if (XL + fb * 3 == i)
                     asm volatile("global_load_dwordx4 %0, %1, %2" : "=a"(w.a[fb][0]) : "v"(lane16), "s"(av) : "memory");
                 if (XL + fb * 3 + 1 == i)
@@ -420,6 +421,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
     auto issue_step = [&](int kp, WSet &w) {
 #pragma unroll
         for (int i = 0; i < OPS; i++) issue_one(kp, w, i);
+        advance(kp);
     };
 
     f32x16 acc[FB][TB];
@@ -547,7 +549,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
 #pragma unroll
         for (int u = 0; u <= DR_D; u++) {
             const int kp = kp0 + u;
-            if (kp >= KP) break;
+            if (kp >= KP) goto walked;      // (past the loop: a break would be tested again there)
             const unsigned char *base = smem + (kp & (DR_NS - 1)) * STAGE;
             const unsigned char *next = smem + ((kp + 1) & (DR_NS - 1)) * STAGE;
             // One phase: two MFMAs; the LDS reads of the next phase into the other fragment set;
@@ -566,6 +568,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int i = L0; i < OPS; i++) issue_one(kp + DR_D, ws[(u + DR_D) % (DR_D + 1)], i);
+                    advance(kp + DR_D);
                     __builtin_amdgcn_sched_barrier(0);
                     // fragments of step kp are in registers, my share of step kp+1 has landed ...
                     landed(ws[(u + 1) % (DR_D + 1)]);
@@ -632,6 +635,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
             static_assert(NP == 2 || NP == 4 || NP == 8, "one, two or four token parts");
         }
     }
+walked:
     pin_acc();
     // The loads of the steps beyond the last are still in flight and nothing reads what they bring:
     // every register of the ring passes through the final wait, so that none of them is given to

@@ -23,6 +23,21 @@ def test_colsum(rows, cols, pitch, dtype):
     assert bool(((y.double() - want).abs() <= bound * x[:, :cols].double().abs().sum(0)).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,row_bytes,extra", [
+    (255, 64, 0), (257, 68, 0), (1025, 7164, 2), (1023, 7168, 0), (129, 7172, 6), (2, 8192, 10),      # lanes of 64 and of 128 bytes, either side
+])
+def test_colsum_at_the_edges_of_its_tiles(rows, row_bytes, extra, dtype):
+    # a pitch and a first element that are no multiple of 16 bytes; whole numbers: the sums are exact, one rounding at the end
+    cols = row_bytes // dtype.itemsize
+    pitch = cols + extra + 1
+    x = torch.full((rows * pitch + 1,), float("nan"), dtype=dtype, device=DEV)[1:].view(rows, pitch)
+    x[:, :cols] = torch.randint(-8, 9, (rows, cols), generator=torch.Generator().manual_seed(1)).to(dtype).to(DEV)
+    y = torch.empty(cols, dtype=dtype, device=DEV)
+    native.check(native.load().nmg_colsum(native.ptr(x), rows, cols, pitch, native.ptr(y), native.dtype_code(dtype), None))
+    assert torch.equal(y, x[:, :cols].double().sum(0).to(dtype))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("n,m,g", [(2, 4, 16), (3, 6, 12), (4, 8, 32)])
 @pytest.mark.parametrize("R,C", [(100, 203), (768, 520)])
