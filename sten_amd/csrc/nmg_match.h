@@ -19,7 +19,7 @@
 // wavefront of two tiles 2:4:16, 0.74 of the time; 0.66 at 2:8:32) and, in the later rounds, chains of LDS round trips: of the 201 us,
 // tile data and results take 52, the first proposals 15, the first round 44, the later rounds 90.  A list in 16 lanes of one or two
 // keys, merged two proposals at a time, and eight lanes (2:4: two) on a column's patterns took these from 122 (whole kernel 233; 2:4:16
-// 59.3 -> 57.8, 1:8:32 43.5 -> 39.5, 4:8:32 172 -> 140, fp32 238 -> 191).  Other group sizes, 4096 x 4096
+// 59.3 -> 57.8, 1:8:32 43.5 -> 39.5, 4:8:32 170 -> 136, fp32 238 -> 200).  Other group sizes, 4096 x 4096
 // fp16 with the blocks along the contiguous / the slow dim, the batched walk -> this: 2:4:4 168 -> 116 / 231 -> 113 us, 2:4:8 115 -> 75 /
 // 146 -> 76, 2:4:32 118 -> 105 / 135 -> 116, 2:4:64 130 -> 118 / 146 -> 129, 1:4:8 99 -> 69 / 151 -> 70, 1:2:8 192 -> 147 /
 // 302 -> 145, 2:8:8 293 -> 130 / 326 -> 134, 4:8:16 870 -> 366 / 810 -> 388.  Slower than the walk is 1:4:17 (107 -> 110), and where the
@@ -732,7 +732,9 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                             bp = p;
                         }
                     };
-                    if constexpr (SG != 0) {
+                    // (many patterns and more columns than one pass of the lanes takes: a column per lane, as a lone tile waits
+                    // less for it.  4:8:32 fp16, lanes of a column -> this: 1024 x 1024 22.2 -> 20.8 us, 4096 x 4096 141 -> 136, fp32 189 -> 200.)
+                    if (SG != 0 && (SC <= 32 || pend * EL <= A)) {
                         const int sub = tt % EL;
                         for (int e = tt / EL; e < pend; e += A / EL) {
                             const int o = (int)pending[e];
@@ -746,7 +748,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                             if (EL >= 8) top = max(top, match_swap<0x141>(top));
                             if (sub == 0) put(o, (top >> 32) == 0 ? 0 : match_key((uint32_t)(top >> 32), o, (int)(top & 0xFFu)));
                         }
-                    } else if (c > 8 && pend * EIGHT <= A) {
+                    } else if (SG == 0 && c > 8 && pend * EIGHT <= A) {
                         const int e = tt / EIGHT, sub = tt % EIGHT;
                         if (e < pend) {
                             const int o = (int)pending[e];
