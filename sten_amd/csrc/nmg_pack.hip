@@ -12,6 +12,8 @@
 // whole line, and gathered every fragment value by value from global memory.
 #include "nmg_common.h"
 
+#include <algorithm>
+
 namespace nmg {
 
 struct PackParams {
@@ -32,7 +34,7 @@ struct PackParams {
 };
 
 template <typename T, typename PT>
-__global__ __launch_bounds__(256) void pack_kernel(PackParams P)
+__global__ __launch_bounds__(1024) void pack_kernel(PackParams P)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr PT ABSENT = (PT)~(PT)0;
@@ -377,7 +379,9 @@ extern "C" int nmg_pack_operands(const void *d_val, const int16_t *d_idx, int64_
     const int elem = (int)dtype_size(dtype);
     const int pat_bytes = (int)nmg_rowpack_pat_bytes(n, m);
     const bool pow2 = (m & (m - 1)) == 0;
-    const int64_t R64 = (int64_t)tg.cols / gcd64(tg.cols, 32) * 32;   // lcm(cols, 32)
+    int64_t R64 = (int64_t)tg.cols / gcd64(tg.cols, 32) * 32;   // lcm(cols, 32)
+    // a single chunk that is mostly padding: the lines that exist (with the fragments' padding) are enough
+    if (tg.num_chunks == 1) R64 = std::min(R64, frag ? (G + 255) / 256 * 256 : (G + 31) / 32 * 32);
     const int nbw_unit = frag ? (64 / m > 0 ? 64 / m : 1) : 1;   // blocks per 64 positions
     const int64_t per_block = R64 * ((int64_t)n * elem + pat_bytes);
     // about 24 KiB of LDS per workgroup (many small workgroups hide each other's latencies: 55 us
@@ -385,9 +389,25 @@ extern "C" int nmg_pack_operands(const void *d_val, const int16_t *d_idx, int64_
     // where a line's run would otherwise be a few bytes
     int64_t NBW = per_block > 0 ? (24 * 1024) / per_block : 0;
     if (NBW < 3 && per_block > 0) NBW = (64 * 1024) / per_block < 3 ? (64 * 1024) / per_block : 3;
+    if (nbw_unit == 1) {      // runs of a line that are whole words, whatever n
+        if (NBW >= 6) NBW = (NBW + 2) / 8 * 8;
+        else if (NBW == 3 && per_block * 4 <= 90 * 1024) NBW = 4;
+    }
     NBW = NBW / nbw_unit * nbw_unit;
     if (NBW < nbw_unit) NBW = nbw_unit;
     if (NBW > 256) NBW = 256 / nbw_unit * nbw_unit;
+    // lines: the chunks' padded extent, and for the fragments the 256-line padding of the operand
+    int64_t lines = tg.num_chunks == 1 ? R64 : tg.num_chunks * tg.cols;
+    if (frag) lines = std::max(lines, (G + 255) / 256 * 256);
+    auto workgroups = [&](int64_t nbw) { return (lines + R64 - 1) / R64 * ((tg.num_blocks + nbw - 1) / nbw); };
+    // A workgroup's tile is a chain of passes through LDS, so a small weight wants many small tiles: halved down to 8 blocks
+    // until there are two workgroups for every CU.  And with less than that, or large tiles, more threads on a tile.
+    // us before -> now: 1:8:32 6656 x 1280 31 -> 16.6, 2584 x 1472 30 -> 10.1; 2:8:32 14152 x 1192 35 -> 31, 8192^2 80 -> 76; 3:6:12
+    // 14464 x 1920 38 -> 30, 1912 x 1640 17 -> 11.5; 2:4:16 1024^2 12 -> 6.9, 896 x 3840 13 -> 10.5 (4096^2: 21).
+    const int64_t least = std::max<int64_t>(nbw_unit, 8);
+    while (NBW > least && workgroups(NBW) < 512) NBW = std::max(least, NBW / 2 / least * least);
+    int threads = R64 * NBW > 6000 ? 512 : 256;
+    if (workgroups(NBW) <= 512) threads *= 2;
     // Pitch of a line in LDS: odd, so that the 32 lines a fragment reads side by side fall on
     // different banks (-10 % on 2:4:16: 6 workgroups of 23.7 KB per CU instead of 7 of 23.2), but
     // only where six padded workgroups still fit a CU: at 2:8:32 the padding takes the CU from
@@ -437,9 +457,6 @@ extern "C" int nmg_pack_operands(const void *d_val, const int16_t *d_idx, int64_
         for (int p = 0; p < tg.c; p++)
             for (int j = 0; j < n; j++) P.masks[p / 4] |= 1u << (8 * (p % 4) + order[p * n + j]);
     }
-    // lines: the chunks' padded extent, and for the fragments the 256-line padding of the operand
-    int64_t lines = tg.num_chunks * tg.cols;
-    if (frag && (int64_t)P.MBtot * 32 > lines) lines = (int64_t)P.MBtot * 32;
     const int64_t gy = (lines + R64 - 1) / R64, gx = (tg.num_blocks + NBW - 1) / NBW;
     NMG_REQUIRE(gy <= 65535 && gx <= 0x7fffffffLL, NMG_ERR_UNSUPPORTED, "weight too large for the pack kernel");
     dim3 grid((unsigned)gx, (unsigned)gy);
@@ -448,7 +465,7 @@ extern "C" int nmg_pack_operands(const void *d_val, const int16_t *d_idx, int64_
         auto kern = pack_kernel<T, PT>;                                                               \
         if (lds > 64 * 1024)                                                                          \
             NMG_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
-        hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, P);                                         \
+        hipLaunchKernelGGL(kern, grid, dim3(threads), lds, s, P);                                         \
     } while (0)
     if (dtype == NMG_F32) {
         if (pat_bytes == 1) NMG_PACK_LAUNCH(float, uint8_t); else NMG_PACK_LAUNCH(float, uint16_t);

@@ -53,6 +53,11 @@ def bits(x):
     (2300, 72, 4, 8, 32),       # no sparse-matrix-core operand: rowpack alone
     (200, 90, 3, 6, 4),         # m not a power of two
     (100, 48, 5, 12, 2),        # 792 patterns: 16-bit pattern numbers, scatter kernels
+    # one chunk that is mostly padding: tiles of the lines that exist
+    (1, 200, 2, 4, 16), (33, 264, 1, 8, 32), (257, 1040, 2, 8, 32), (895, 72, 2, 8, 32), (31, 100, 4, 8, 32), (2239, 40, 4, 8, 32), (65, 90, 3, 6, 12),
+    # tiles of 8 to 48 blocks, 256 to 1024 threads
+    (1024, 4096, 2, 4, 16), (5000, 4000, 2, 4, 16), (3000, 2056, 1, 8, 32), (8192, 1544, 1, 8, 32), (8000, 1000, 2, 8, 32),
+    (1000, 3000, 3, 6, 12), (6000, 2000, 3, 6, 12), (2500, 2100, 4, 8, 32),
 ])
 def test_one_pass_matches_the_scatter_kernels(dtype, G, S, n, m, g):
     print(f"case pack {dtype} G={G} S={S} {n}:{m}:{g}", flush=True)
