@@ -863,12 +863,12 @@ struct TiledParams {
 // weight).  The region of NT tiles that are neighbours along the sparse dim is then NT*m rows (one
 // per position) of c*g contiguous columns; LDS holds it as [position][column].
 template <typename T, bool GATHER, bool GC>
-__global__ __launch_bounds__(256) void scatter_tiled_kernel(TiledParams Q)
+__global__ __launch_bounds__(1024) void scatter_tiled_kernel(TiledParams Q)
 {
     const ScatterParams &P = Q.sp;
     extern __shared__ __align__(16) unsigned char smem[];
     T *tile = (T *)smem;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, nthr = blockDim.x;
     const int n = P.n, m = P.m, cols = P.cols, nt = Q.nt, pitch = Q.pitch;
     // workgroup -> (batch, group-dim chunk, first block)
     const int64_t wg = blockIdx.x;
@@ -894,7 +894,7 @@ __global__ __launch_bounds__(256) void scatter_tiled_kernel(TiledParams Q)
 
     if (GATHER) {
         // region -> LDS (zeros beyond G / S)
-        for (int i = tid; i < all_rows * wv; i += 256) {
+        for (int i = tid; i < all_rows * wv; i += nthr) {
             const int r = i / wv, cc = (i - r * wv) * V;
             T *dst = tile + r * pitch + cc;
             const T *src = dense + (int64_t)r * row_stride + cc;
@@ -907,14 +907,14 @@ __global__ __launch_bounds__(256) void scatter_tiled_kernel(TiledParams Q)
         }
     } else {
         const uint4 z = {0, 0, 0, 0};
-        for (int i = tid; i < all_rows * pitch * (int)sizeof(T) / 16; i += 256) ((uint4 *)tile)[i] = z;
+        for (int i = tid; i < all_rows * pitch * (int)sizeof(T) / 16; i += nthr) ((uint4 *)tile)[i] = z;
     }
     // the order table in LDS where it fits: a slot's positions are then one LDS read away instead
     // of a round trip to L2 behind the load of its index
     __shared__ int8_t s_ord[1024];
     const bool ord_lds = P.c * n <= 1024;
     if (ord_lds)
-        for (int i = tid; i < P.c * n; i += 256) s_ord[i] = P.order[i];
+        for (int i = tid; i < P.c * n; i += nthr) s_ord[i] = P.order[i];
     const int8_t *order = ord_lds ? s_ord : P.order;
     __syncthreads();
     // slots of the NT tiles: contiguous in val / idx (slot e of the workgroup is element
@@ -929,18 +929,18 @@ __global__ __launch_bounds__(256) void scatter_tiled_kernel(TiledParams Q)
         constexpr int NV = decltype(nv_tag)::value;
         constexpr int WB = NV * (int)sizeof(T);            // bytes of a slot's word
         using Word = typename std::conditional<WB == 8, uint2, uint32_t>::type;
-        for (int base = tid; base < total; base += 4 * 256) {
+        for (int base = tid; base < total; base += 4 * nthr) {
             int o[4];
             Word vw[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const int e = base + u * 256;
+                const int e = base + u * nthr;
                 o[u] = e < total ? (int)P.idx[at0 + e] : -1;
                 if (!GATHER && NV > 0) vw[u] = ((const Word *)P.val)[at0 + (e < total ? e : 0)];
             }
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const int e = base + u * 256;
+                const int e = base + u * nthr;
                 if (e >= total) continue;
                 const int tm = (int)(((uint64_t)e * Q.magic_cols) >> 32), slot = e - tm * cols;
                 const int p = (int)(((uint64_t)slot * Q.magic_g) >> 32);
@@ -982,7 +982,7 @@ __global__ __launch_bounds__(256) void scatter_tiled_kernel(TiledParams Q)
     if (GATHER) return;
     __syncthreads();
     // LDS -> region
-    for (int i = tid; i < rows * wv; i += 256) {
+    for (int i = tid; i < rows * wv; i += nthr) {
         const int r = i / wv, cc = (i - r * wv) * V;
         if (cc >= valid_w) continue;
         const T *src = tile + r * pitch + cc;
@@ -1010,6 +1010,11 @@ static int launch_scatter_tiled(bool gather, ScatterParams &P, hipStream_t s, bo
     const int64_t per_tile = (int64_t)P.cols * P.m * (int64_t)sizeof(T);
     int nt = (int)std::min<int64_t>(64, (8 * 1024) / per_tile);
     if (nt < 8) nt = 8;
+    // whole 128-byte lines of the dense rows where enough workgroups stay (4096^2 2:4:16 fp16 gather / scatter with 10 tiles 21.4 / 16.2
+    // us, with 16 15.2 / 14.5; 640 x 512 4.4 / 4.0 against 5.0 / 4.5)
+    const int64_t chunks = P.outer / P.view.num_blocks;   // batches x group-dim chunks
+    const int line = (int)(128 / (P.m * (int64_t)sizeof(T)));
+    if (!gc && 128 % (P.m * (int)sizeof(T)) == 0 && nt < line && nt * 2 > line && chunks * (P.view.num_blocks / line) >= 512) nt = line;
     nt = (int)std::min<int64_t>(nt, P.view.num_blocks);
     auto pitch_of = [&](int tiles, bool pad) { return (((gc ? P.cols : tiles * P.m) + V - 1) / V) * V + (pad ? V : 0); };
     bool pad = true;
@@ -1032,14 +1037,17 @@ static int launch_scatter_tiled(bool gather, ScatterParams &P, hipStream_t s, bo
     Q.magic_g = (((uint64_t)1 << 32) + P.g - 1) / P.g;
     const size_t lds = lds_of(nt, pad);
     if ((int64_t)nt * P.cols >= 65536) return NMG_OK;
-    const int64_t chunks = P.outer / P.view.num_blocks;   // batches x group-dim chunks
     const int64_t grid = chunks * Q.groups_per_chunk;
     if (grid > 0x7fffffffLL) return NMG_OK;
     auto kern = gc ? (gather ? scatter_tiled_kernel<T, true, true> : scatter_tiled_kernel<T, false, true>)
                    : (gather ? scatter_tiled_kernel<T, true, false> : scatter_tiled_kernel<T, false, false>);
     if (lds > 64 * 1024)
         NMG_HIP_TRY(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, s, Q);
+    // Large regions leave few workgroups on a CU: as many threads as it can use.  us, gather / scatter, 256 threads -> this, fp16:
+    // 2:8:32 8192^2 141 / 81 -> 57 / 44, 14152 x 1192 45 / 29 -> 21 / 18; 4:8:32 4096^2 37 / 24 -> 24 / 19; 3:6:12 4096^2 27 / 23 -> 22 / 20;
+    // 1:8:32 2584 x 1472 9.4 / 8.4 -> 6.3 / 6.4.  At 2:4:16 (8 to 12 KB) more threads lose: 4096^2 21 / 16 -> 21 / 22.
+    const int threads = lds >= 48 * 1024 ? 1024 : lds >= 16 * 1024 ? 512 : 256;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), lds, s, Q);
     NMG_HIP_TRY(hipGetLastError());
     *done = true;
     return NMG_OK;

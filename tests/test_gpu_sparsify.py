@@ -201,3 +201,25 @@ def test_preserved_magnitude_between_random_and_perfect():
             pd = p.to_dense()
             assert pd.shape == x.shape and sten.is_correct_nm(x, pd, sparse_dim, n, m)
             assert float(pd.abs().sum() / x.abs().sum()) >= kept - 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n,m,g,G,S", [
+    (2, 4, 16, 2112, 2050),     # lines of 128 bytes: enough workgroups; a partial tile and a partial block at the ends
+    (2, 4, 16, 500, 2048),      # too few
+    (1, 8, 32, 600, 1003), (3, 6, 12, 1000, 500), (2, 8, 32, 2000, 204), (4, 8, 32, 2300, 100), (2, 8, 32, 100, 36),
+])
+@pytest.mark.parametrize("along", [0, 1])
+def test_dense_copy_and_gather_of_every_tile_shape(n, m, g, G, S, along, dtype):
+    # regions of 8 to 115 KB, 256 to 1024 threads: a dense copy holds the kept values and nothing else, and gathering another
+    # dense tensor at the pattern gives what its copy holds there
+    print(f"case {n}:{m}:{g} {G}x{S} along={along} {dtype}", flush=True)
+    shape = (G, S) if along == 1 else (S, G)
+    w = seeded(shape, dtype, seed=G + S)
+    val, idx, lay = oracle_sparsify(w, n, m, along, g, 1 - along)
+    t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
+    assert same_bits(t.to_dense(), O.to_dense(val, idx, lay))
+    other = seeded(shape, dtype, seed=1)
+    want = O.gather_merged(O.merge(to_np(other), lay), idx, lay.n)
+    got = t._gather(other.to(DEV))
+    assert same_bits(getattr(got, "val", got), want)
