@@ -696,9 +696,13 @@ struct GemmF32Params {
 // 16 reduction positions x 4 groups per wavefront fall on 64 different banks.
 // XKM: the same for the activation-side operand, X[K, T] (Y = X^T * A: the weight gradient of a
 // linear layer from the upstream gradient and the activations as they lie).
-template <int WM, int WN, int WK, int MI, int NJ, bool FAST, bool AKM, bool XKM>
+// LOADS: what a step's loads may meet -- whole tiles and aligned rows only; the ends of the operands in any step; in the last
+// steps only (a loop of its own for the steps before).
+enum { F32_ALIGNED, F32_ANY, F32_ENDS };
+template <int WM, int WN, int WK, int MI, int NJ, int LOADS, bool AKM, bool XKM>
 __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
 {
+    constexpr bool FAST = LOADS == F32_ALIGNED;
     static_assert(WM * WN * WK == 4, "four wavefronts");
     constexpr int BM = WM * MI * 32, BN = WN * NJ * 32, BKT = 16 * WK, PITCH = BKT + 4;
     constexpr int KV = BKT / 4;                                      // float4 per tile row
@@ -799,15 +803,19 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
         ap[v] = first_ptr(P.a, P.lda, o0, P.O, (AE % 256 == 0 || tid + v * 256 < AE) ? tid + v * 256 : 0, AKM);
     // one load / LDS store of a tile: first the activations, then the weight
     constexpr int NG = XV + AV, CSX = XKM ? 4 : 1, CSA = AKM ? 4 : 1, NS = CSX * XV + CSA * AV;
-    auto load_op = [&](Stage &G, int64_t k0, int o) {
+    // (whole_tag: the tile holds no end of the reduction, so nothing is guarded)
+    auto load_op = [&](Stage &G, int64_t k0, int o, auto whole_tag) {
+        constexpr bool WHOLE = decltype(whole_tag)::value;
         if (o < XV) {
             const int e = tid + o * 256;
             if constexpr (FAST) G.x[o] = *(const f32x4 *)(xp[o] + (XKM ? k0 * P.ldx : k0));
+            else if constexpr (WHOLE) G.x[o] = *(const f32x4_any *)(xp[o] + (XKM ? k0 * P.ldx : k0));
             else if (XE % 256 == 0 || e < XE)
                 G.x[o] = load_any(P.x, xp[o], P.ldx, tok0, P.T, e, k0, XKM);
         } else {
             const int v = o - XV, e = tid + v * 256;
             if constexpr (FAST) G.a[v] = *(const f32x4 *)(ap[v] + (AKM ? k0 * P.lda : k0));
+            else if constexpr (WHOLE) G.a[v] = *(const f32x4_any *)(ap[v] + (AKM ? k0 * P.lda : k0));
             else if (AE % 256 == 0 || e < AE)
                 G.a[v] = load_any(P.a, ap[v], P.lda, o0, P.O, e, k0, AKM);
         }
@@ -829,7 +837,7 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
     };
     auto load_tile = [&](Stage &G, int64_t k0) {
 #pragma unroll
-        for (int o = 0; o < NG; o++) load_op(G, k0, o);
+        for (int o = 0; o < NG; o++) load_op(G, k0, o, std::false_type{});
     };
     auto store_tile = [&](const Stage &G, int buf) {
 #pragma unroll
@@ -885,7 +893,7 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
     // ahead of their use), then the barrier, second half step the fragment reads of tile st+1.
     // The fences keep that order; without them the scheduler moves the barrier up to the first
     // MFMA and the next step's LDS stores up to the loads they wait for.
-    auto step = [&](int st, const Frags &cur, Frags &nxt, Stage &G, bool more, bool more3) {
+    auto step = [&](int st, const Frags &cur, Frags &nxt, Stage &G, bool more, bool more3, auto whole_tag) {
         pin();
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -895,7 +903,7 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
             for (int o = 0; o < NS + NG; o++)
                 if (o * NH / (NS + NG) == m) {
                     if (o < NS) { if (more) store_op(G, (st + 1) & 1, o); }   // last read before the barrier of step st-1
-                    else if (more3) load_op(G, (int64_t)(st + 3) * BKT, o - NS);
+                    else if (more3) load_op(G, (int64_t)(st + 3) * BKT, o - NS, whole_tag);
                 }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -911,13 +919,20 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
         }
     };
     int st = 0;
+    if constexpr (LOADS == F32_ENDS) {
+        const int whole = (XKM && P.T < 4) || (AKM && P.O < 4) ? 0 : (int)(P.K / BKT);
+        for (; st + 4 < whole; st += 2) {
+            step(st, F0, F1, G1, true, true, std::true_type{});
+            step(st + 1, F1, F0, G0, true, true, std::true_type{});
+        }
+    }
     for (; st + 4 < steps; st += 2) {
-        step(st, F0, F1, G1, true, true);
-        step(st + 1, F1, F0, G0, true, true);
+        step(st, F0, F1, G1, true, true, std::false_type{});
+        step(st + 1, F1, F0, G0, true, true, std::false_type{});
     }
     for (; st < steps; st += 2) {
-        step(st, F0, F1, G1, st + 1 < steps, st + 3 < steps);
-        if (st + 1 < steps) step(st + 1, F1, F0, G0, st + 2 < steps, st + 4 < steps);
+        step(st, F0, F1, G1, st + 1 < steps, st + 3 < steps, std::false_type{});
+        if (st + 1 < steps) step(st + 1, F1, F0, G0, st + 2 < steps, st + 4 < steps, std::false_type{});
     }
     pin();
 
@@ -972,17 +987,24 @@ static void launch_gemm_f32(const GemmF32Params &Q, int form, hipStream_t st)
     dim3 grid((unsigned)((Q.O + BN - 1) / BN), (unsigned)((Q.T + BM - 1) / BM));
     const bool fast = Q.vec && Q.K % BKT == 0 && (form < 1 || (Q.O % 4 == 0 && Q.O >= 4)) &&
                       (form < 2 || (Q.T % 4 == 0 && Q.T >= 4));
-#define NMG_F32_LAUNCH(FAST_, AKM_, XKM_) \
-    hipLaunchKernelGGL((gemm_nt_f32_kernel<WM, WN, WK, MI, NJ, FAST_, AKM_, XKM_>), grid, dim3(256), 0, st, Q)
+    // Guards are branches, and with a branch in the loop the compiler waits for every load in flight: us, guards in every step ->
+    // in the last, row-major weight: W B for 2816 x 2944, 259 columns 97 -> 69 (260 columns: 57), 999 columns 188 -> 159; 512 x 768,
+    // K 3071 37.5 -> 33.5, 36 x 221, K 1618 15.0 -> 12.2.  With both operands reduction-major 36 x 221, K 1618 22 -> 16.4, 1612 x 694,
+    // K 1482 77.6 -> 69.9, but on short reductions fetching the second loop's code costs more: 100 x 1444, K 773 14.5 -> 16.2, 225 x 89,
+    // K 307 7.9 -> 8.7.
+    const bool ends = Q.K >= 16 * BKT;
+#define NMG_F32_LAUNCH(LOADS_, AKM_, XKM_) \
+    hipLaunchKernelGGL((gemm_nt_f32_kernel<WM, WN, WK, MI, NJ, LOADS_, AKM_, XKM_>), grid, dim3(256), 0, st, Q)
     if (form == 0) {
-        if (fast) NMG_F32_LAUNCH(true, false, false);
-        else NMG_F32_LAUNCH(false, false, false);
+        if (fast) NMG_F32_LAUNCH(F32_ALIGNED, false, false);
+        else NMG_F32_LAUNCH(F32_ENDS, false, false);
     } else if (form == 1) {
-        if (fast) NMG_F32_LAUNCH(true, true, false);
-        else NMG_F32_LAUNCH(false, true, false);
+        if (fast) NMG_F32_LAUNCH(F32_ALIGNED, true, false);
+        else NMG_F32_LAUNCH(F32_ENDS, true, false);
     } else {
-        if (fast) NMG_F32_LAUNCH(true, true, true);
-        else NMG_F32_LAUNCH(false, true, true);
+        if (fast) NMG_F32_LAUNCH(F32_ALIGNED, true, true);
+        else if (ends) NMG_F32_LAUNCH(F32_ENDS, true, true);
+        else NMG_F32_LAUNCH(F32_ANY, true, true);
     }
 #undef NMG_F32_LAUNCH
 }

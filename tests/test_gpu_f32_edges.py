@@ -10,7 +10,9 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("form", ["nt", "nn", "tn"])
-@pytest.mark.parametrize("O,K,T", [(1, 1, 1), (3, 17, 2), (4, 16, 5), (5, 33, 4), (33, 15, 65), (98, 70, 131), (257, 129, 67), (771, 62, 1025), (2139, 333, 504), (3070, 96, 516)])
+@pytest.mark.parametrize("O,K,T", [(1, 1, 1), (3, 17, 2), (4, 16, 5), (5, 33, 4), (33, 15, 65), (98, 70, 131), (257, 129, 67), (771, 62, 1025), (2139, 333, 504), (3070, 96, 516),
+                                   # the loop without guards and the steps behind it: whole steps, one more and one less position; fewer than four rows
+                                   (70, 144, 99), (130, 319, 65), (98, 257, 131), (1024, 321, 257), (5, 256, 3), (3, 300, 200), (200, 300, 3)])
 @pytest.mark.parametrize("pad,off", [(0, 0), (1, 1), (3, 2)])
 def test_gemm_forms(form, O, K, T, pad, off):
     print(f"case {form} O={O} K={K} T={T} pad={pad} off={off}", flush=True)
