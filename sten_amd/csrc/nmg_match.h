@@ -141,7 +141,12 @@ constexpr int kMatchTables = 6;      // c ints each, and four counts (three of t
 constexpr int kMatchPad = 64;        // bytes behind the proposals: a batch of eight keys past the end of the last group
 
 // First rounds of a tile with `real_rows` < m real positions.  All columns' keys are sorted by pattern and key in
-// every round (compare-exchange network), since most of them are refused and sit in few, long groups.  A refused
+// every round, since most of them are refused and sit in few, long groups: places counted by all pairs, in larger tiles a
+// compare-exchange network.  Patterns that agree in the real positions are a class: a column sums and compares once for each
+// class (2 to 30 of them for up to 70 patterns).  One such tile is as long as the launch, four to five rounds of 6 to 50 us, half of it
+// the sort.  us, pattern by pattern -> by classes: 4:8:32 7742 x 933 fp32 608 -> 457, 512 x 4099 fp16 84 -> 65, 2:8:32 2001 x 2001 fp32 95 -> 75,
+// 3:8:8 997 x 1003 fp16 215 -> 140, 3:6:12 1152 x 1792 fp32 59 -> 59.  Sorts that lost: runs of 64 merged by binary search (gathers at
+// random places of LDS, 1.5 x), keys broadcast from a wavefront's lanes (1.2 x).  A refused
 // column skips the patterns of its class that those ahead of it are certain to fill: all of them that have no other
 // class with the same score to turn to, which bit 0 of a key says here.  Stops when at most `few` columns are pending;
 // leaves s_mem, s_occ, the waiting columns in s_np[1] and the pending ones in s_arr and s_np[0].
@@ -160,31 +165,102 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
     int *s_list = s_occ + c, *s_at = s_list + c, *s_last = s_at + c, *s_np = s_last + c;      // the classes, largest patterns first
     const int tt = threadIdx.x % NT, real_mask = (1 << real_rows) - 1;
     auto column = [](uint64_t key) { return (int)((key >> 1) & 0x7FFFu); };
+    int *s_class = s_np + 4;                                   // smallest pattern of every class
+    uint64_t *s_least = (uint64_t *)(s_class + ((c + 1) & ~1));    // least last key of a class's patterns, without the pattern
+    int classes = 0;
+    constexpr uint64_t EDGE = 0xFFFFFFFFFFFFull;      // score and column of a key
     auto propose = [&](int o, uint32_t at_score, int below) -> uint64_t {      // at that score only patterns up to `below`
         float a[8];
 #pragma unroll
         for (int r = 0; r < 8; r++) a[r] = match_abs(s_d[o * so + min(r, m - 1) * sr]);
-        uint32_t best = 0, bmask = 0;
-        int bp = 0;
-        bool tied = false;
-        for (int p = 0; p < c; p++) {
-            const uint32_t mk = __builtin_amdgcn_readfirstlane(s_mask[p]);
-            const uint64_t last = s_mem[p * g + g - 1];
+        auto score_of = [&](uint32_t mk) {
             float acc = 0;
 #pragma unroll
-            for (int r = 0; r < 7; r++) {
-                if (r >= real_rows) break;
-                acc += (mk >> r) & 1 ? a[r] : 0.f;      // (adding 0 changes nothing)
+            for (int r = 0; r < 7; r++)
+                acc += __uint_as_float(__float_as_uint(a[r]) & (uint32_t)__builtin_amdgcn_sbfe((int)mk, r, 1));      // (adding 0 changes nothing)
+            return __float_as_uint(acc);
+        };
+        if (c <= 8) {      // few patterns: one by one (1000 x 1001 2:4:16 fp16 26.0 us, by classes 27.4)
+            uint32_t best = 0, bmask = 0;
+            int bp = 0;
+            bool tied = false;
+            for (int p0 = 0; p0 < c; p0 += 4) {      // four patterns' reads in flight; beyond the last the last again
+                uint32_t mk4[4];
+                uint64_t last4[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int p = min(p0 + u, c - 1);
+                    mk4[u] = s_mask[p] & (uint32_t)real_mask;
+                    last4[u] = s_mem[p * g + g - 1];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int p = p0 + u;
+                    const uint32_t sb = score_of(mk4[u]);
+                    if (p < c && sb >= best && !(sb == at_score && p > below) && match_key(sb, o << 1, p) > last4[u]) {
+                        tied = sb == best && (tied || mk4[u] != bmask);
+                        best = sb;
+                        bp = p;
+                        bmask = mk4[u];
+                    }
+                }
             }
-            const uint32_t sb = __float_as_uint(acc);
-            if (sb >= best && !(sb == at_score && p > below) && match_key(sb, o << 1, p) > last) {
-                tied = sb == best && (tied || ((mk ^ bmask) & real_mask) != 0);
-                best = sb;
-                bp = p;
-                bmask = mk;
-            }
+            return best == 0 ? 0 : match_key(best, o << 1, bp) | (tied ? 1 : 0);
         }
-        return best == 0 ? 0 : match_key(best, o << 1, bp) | (tied ? 1 : 0);
+        auto edge_of = [&](uint32_t sb) { return ((uint64_t)sb << 16) | (uint32_t)(o << 1); };
+        // the largest pattern of class k that takes the column; -1: none
+        auto within = [&](int k, uint32_t sb) {
+            const int end = s_last[s_class[k]];
+            int at = k > 0 ? s_last[s_class[k - 1]] + 1 : 0;
+            if (sb == at_score && below >= 0 && s_last[below] == end) at = s_at[below];
+            for (; at <= end; at++) {
+                const int p = s_list[at];
+                if (!(sb == at_score && p > below) && edge_of(sb) > (s_mem[p * g + g - 1] & EDGE)) return p;
+            }
+            return -1;
+        };
+        for (uint32_t under = ~0u;;) {      // scores below it (a second time where the best score's patterns are above `below`)
+            uint32_t best = 0;
+            int from = -1;
+            bool several = false;
+            for (int k0 = 0; k0 < classes; k0 += 4) {      // four classes' reads in flight; beyond the last the last again
+                int p4[4];
+                uint32_t mk4[4];
+                uint64_t least4[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int k = min(k0 + u, classes - 1);
+                    p4[u] = s_class[k];
+                    least4[u] = s_least[k];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) mk4[u] = s_mask[p4[u]] & (uint32_t)real_mask;
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const uint32_t sb = score_of(mk4[u]);
+                    if (k0 + u < classes && sb < under && sb >= best && edge_of(sb) > least4[u]) {
+                        several = sb == best && from >= 0;
+                        best = sb;
+                        from = k0 + u;
+                    }
+                }
+            }
+            if (best == 0) return 0;
+            int bp = -1, found = 0;
+            if (!several) {
+                bp = within(from, best);
+                found = 1;
+            } else {
+                for (int k = 0; k < classes; k++) {
+                    if (score_of(s_mask[s_class[k]] & (uint32_t)real_mask) != best) continue;
+                    const int q = within(k, best);
+                    if (q >= 0) found++;
+                    bp = max(bp, q);
+                }
+            }
+            if (bp >= 0) return match_key(best, o << 1, bp) | (found > 1 ? 1 : 0);
+            under = best;
+        }
     };
     for (int p = tt; p < c; p += NT) {
         int before = 0, above = 0, size = 0;      // patterns of classes with a smaller mask, of the same one
@@ -198,6 +274,18 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
         s_at[p] = before + above;
         s_last[p] = before + size - 1;
     }
+    if (c > 8) {      // (else the patterns one by one)
+        match_sync<NT>();
+        for (int q = 0; q < c; q++) classes += s_at[q] == s_last[q] ? 1 : 0;
+        for (int p = tt; p < c; p += NT)
+            if (s_at[p] == s_last[p]) {
+                int k = 0;
+                for (int q = 0; q < c; q++) k += s_at[q] == s_last[q] && s_at[q] < s_at[p] ? 1 : 0;
+                s_class[k] = p;
+                s_least[k] = 0;
+            }
+    }
+    match_sync<NT>();
     for (int e = tt; e < real_cols; e += NT) s_arr[e] = propose(e, 0, 0);
     int span = 1;      // log2
     while ((1 << span) < real_cols) span++;
@@ -265,6 +353,12 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
         }
         match_sync<NT>();
         left = s_np[0];
+        for (int k = tt; k < classes; k += NT) {
+            const int end = s_last[s_class[k]], before = k > 0 ? s_last[s_class[k - 1]] : -1;
+            uint64_t least = ~0ull;
+            for (int at = before + 1; at <= end; at++) least = min(least, s_mem[s_list[at] * g + g - 1] & EDGE);
+            s_least[k] = least;
+        }
         match_sync<NT>();
         if (left <= few) break;
         for (int e = tt; e < real_cols; e += NT) {
@@ -283,7 +377,7 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
         }
     }
     // the lists, the pending columns in front of s_arr
-    constexpr int MOST = 10;      // keys that a thread holds while it re-orders s_arr
+    constexpr int MOST = 5;      // keys that a thread holds while it re-orders s_arr: five columns at most (match_launch)
     uint64_t mine[MOST];
     int waiting = 0;
     if (tt == 0) s_np[0] = 0;
@@ -995,6 +1089,7 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     off += cols * 8 + kMatchPad;
     Q.r_int = off;
     off = up(off + (kMatchTables * c + 4) * 4, 16);
+    if (Q.view.S % m != 0) off = up(off + ((c + 1) & ~1) * 4 + c * 8, 16);      // the classes of a partial block
     // the tiles of a wavefront run the same offsets of their regions: spread them over the banks
     if (NT < 64)
         while (off % 256 != (NT == 16 ? 64 : 128)) off += 16;

@@ -102,3 +102,21 @@ def test_columns_that_want_the_same_patterns(n, m, g, dtype):
             t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
             assert np.array_equal(to_np(t.idx), idx)
             assert same_bits(t.val, val)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n,m,g", [(2, 8, 32), (3, 6, 12), (4, 8, 4), (3, 8, 8), (5, 8, 2), (2, 6, 1), (3, 7, 1), (6, 8, 1), (1, 8, 32), (2, 4, 16)])
+def test_partial_blocks_whose_classes_tie(n, m, g, dtype):
+    # every number of real positions; equal magnitudes make a column's best score one of several classes', zeros leave classes
+    # without a score, and one chunk is short: the order inside a class and the second choice at the same score decide
+    cols = math.comb(m, n) * g
+    gen = torch.Generator().manual_seed(n * 100 + m * 10 + g)
+    for rest in range(1, m):
+        for kind in range(3):
+            w = torch.randint(0, (2, 3, 9)[kind], (cols + cols // 3 + 1, m + rest), generator=gen).float() * 0.5
+            w = (w * torch.where(torch.rand(w.shape, generator=gen) < 0.5, -1.0, 1.0)).to(dtype)
+            print(f"case {n}:{m}:{g} {dtype} rest={rest} kind={kind}", flush=True)
+            val, idx, _ = oracle_sparsify(w, n, m, 1, g, 0)
+            t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=1, group_size=g, group_dim=0)
+            assert np.array_equal(to_np(t.idx), idx)
+            assert same_bits(t.val, val)
