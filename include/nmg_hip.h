@@ -169,7 +169,7 @@ int nmg_spmm_smfmac_ct(const void *d_fp_val, const void *d_fp_idx, int64_t M, in
  * is caller-owned device memory, 16-byte aligned, written and read inside the call only.
  * slices <= 1 is the unsplit entry point with its default tile.  K % 64 == 0, T > 16.
  * nmg_spmm_densefrag_splitk (declared with the densefrag entry points) is the same for the
- * dense-matrix-core route.
+ * dense-matrix-core route, its slices from nmg_densefrag_plan.
  * No counterpart in the reference (sten_impls.py:44-140 calls one generated loop nest). */
 int nmg_splitk_plan(int64_t M, int64_t K, int64_t T, int *slices, int64_t *workspace_bytes);
 int nmg_spmm_smfmac_splitk(const void *d_fp_val, const void *d_fp_idx, int64_t M, int64_t K,
@@ -252,7 +252,7 @@ int nmg_densefrag(const void *d_pk_val, const void *d_pk_pat, int64_t G, int64_t
                   void *d_df, int n, int m, int dtype, void *stream);
 
 /* Y[T, O] = X[T, K] * A^T (+ bias), A given as densefrag.  variant 0 = 256 outputs x 128 tokens
- * per workgroup, 1 = 256 x 256, -1 = whichever needs fewer rounds of tiles on 256 CUs.  X must be
+ * per workgroup, 1 = 256 x 256, -1 = the fastest of these and 128 x 128 for the extents.  X must be
  * 16-byte aligned with ldx a multiple of 8 and smaller than 2 GiB.
  * Replaces: the forward of sten_impls.py:143-174 for patterns outside 2-of-4, and supplies the
  * grad_input product the reference leaves to the dense fallback (sten.py:1586-1601). */
@@ -269,7 +269,9 @@ int nmg_spmm_densefrag_tt(const void *d_df, int64_t O, int64_t K, const void *d_
 /* The same result from activations X [T, K]: C [O, T] = A * X^T. */
 int nmg_spmm_densefrag_ct(const void *d_df, int64_t O, int64_t K, const void *d_x, int64_t ldx, void *d_c, int64_t ldc,
                           const void *d_bias, int64_t T, int dtype, void *stream);
-/* nmg_spmm_densefrag with the reduction cut into slices (see nmg_splitk_plan). */
+/* nmg_spmm_densefrag with the reduction cut into slices.  nmg_densefrag_plan gives the number of slices for a product of O
+ * outputs, reduction K and T tokens (1: nmg_spmm_densefrag as it is) and the bytes of its workspace. */
+int nmg_densefrag_plan(int64_t O, int64_t K, int64_t T, int *slices, int64_t *workspace_bytes);
 int nmg_spmm_densefrag_splitk(const void *d_df, int64_t O, int64_t K, const void *d_x, int64_t ldx,
                               void *d_y, int64_t ldy, const void *d_bias, int64_t T, int dtype, int slices,
                               void *d_workspace, int64_t workspace_bytes, void *stream);

@@ -24,6 +24,8 @@
 #include "nmg_common.h"
 #include "nmg_tile.h"
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace nmg {
@@ -169,8 +171,10 @@ struct DfParams {
     int64_t part_ld;
 };
 
-constexpr int DD_D = 2;    // K steps in flight (a dense K step takes twice the MFMA time of a sparse one)
-constexpr int DD_NS = 4;   // activation stages in LDS (>= DD_D + 1)
+// K steps in flight and activation stages in LDS (>= steps + 1), by the blocks of 16 outputs of a wavefront: a step of four blocks takes
+// twice the MFMA time of one of two, and that of a sparse step
+constexpr int dd_steps(int ab) { return ab == 4 ? 2 : 4; }
+constexpr int dd_stages(int ab) { return ab == 4 ? 4 : 8; }
 
 // V_MFMA_F32_16X16X32: of the two dense forms of the instruction the one that draws less power
 // per flop (from registers, random operands: 1.76-1.97 against 1.61-1.71 PFLOP/s for 32 x 32 x 16),
@@ -207,12 +211,12 @@ template <> struct DfMma16<__hip_bfloat16> {
 // lane's 16 bytes are those of its output row at the lane's reduction positions, a load touches 64 bytes of 16 rows
 // (the two loads of a K step the two halves of a 128-byte line).  Both operands of Y = X A^T as they lie.
 // CT = true stores the result transposed, C [O, T].
-template <typename T, int TB, int NH, bool XT = false, bool CT = XT, bool ROWA = false>
+template <typename T, int TB, int NH, bool XT = false, bool CT = XT, bool ROWA = false, int AB = 4>
 __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
 {
     using Mm = DfMma16<T>;
-    constexpr int AB = 4;                                 // blocks of 16 outputs per wavefront
-    constexpr int TF = 256, TT = TB * 16;                 // workgroup tile: outputs x tokens
+    constexpr int DD_D = dd_steps(AB), DD_NS = dd_stages(AB);
+    constexpr int TF = 64 * AB, TT = TB * 16;                 // workgroup tile: outputs x tokens
     constexpr int STAGE = TT * 128;                       // activation bytes per K step
     constexpr int XL = TT / 32;                           // DMA loads per wavefront per K step
     constexpr int OPS = XL + 2 * AB;                      // memory operations per wavefront per K step
@@ -248,11 +252,11 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     const int kp_lo = slice * kp_per;
     const int KP = min(KPT, kp_lo + kp_per) - kp_lo;
     const int first = P.turn ? (int)(blockIdx.x & 7) * KP / 8 : 0;
-    const int ob0 = (int)(f0 / 32) + wave * 2;
+    const int ob0 = (int)(f0 / 32) + wave * (AB / 2);
 
-    const unsigned char *av_base[2];
+    const unsigned char *av_base[AB / 2];
 #pragma unroll
-    for (int o = 0; o < 2; o++)
+    for (int o = 0; o < AB / 2; o++)
         av_base[o] = (const unsigned char *)P.df +
                      (ROWA ? (int64_t)kp_lo * 128 : (((int64_t)(ob0 + o) * KPT + kp_lo) * 4) * 1024);
     const int r16 = lane & 15, kq = lane >> 4;
@@ -261,7 +265,7 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     if constexpr (ROWA) {
 #pragma unroll
         for (int ab = 0; ab < AB; ab++) {
-            int64_t row = f0 + wave * 64 + ab * 16 + r16;
+            int64_t row = f0 + wave * (16 * AB) + ab * 16 + r16;
             if (row >= P.O) row = P.O - 1;            // clamped rows are computed, never stored
             row_a[ab] = (uint32_t)(row * P.lda * 2 + kq * 16);
         }
@@ -413,12 +417,19 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     //      the barrier that ended that step.  The two fragment sets alternate by phase; NP is
     //      even, so the set read after the barrier (for phase 0 of the next step) is set 0.
     static_assert(DD_NS > DD_D, "a stage must not be refilled while the step that reads it is in flight");
+    static_assert(AB == 2 || AB == 4, "the waits list the registers of two or four blocks");
     auto landed = [&](WSet &w) {
-        asm volatile("s_waitcnt vmcnt(%8) lgkmcnt(0)"
-                     : "+v"(w.a[0][0]), "+v"(w.a[0][1]), "+v"(w.a[1][0]), "+v"(w.a[1][1]),
-                       "+v"(w.a[2][0]), "+v"(w.a[2][1]), "+v"(w.a[3][0]), "+v"(w.a[3][1])
-                     : "n"((DD_D - 1) * OPS)
-                     : "memory");
+        if constexpr (AB == 4)
+            asm volatile("s_waitcnt vmcnt(%8) lgkmcnt(0)"
+                         : "+v"(w.a[0][0]), "+v"(w.a[0][1]), "+v"(w.a[1][0]), "+v"(w.a[1][1]),
+                           "+v"(w.a[AB - 2][0]), "+v"(w.a[AB - 2][1]), "+v"(w.a[AB - 1][0]), "+v"(w.a[AB - 1][1])
+                         : "n"((DD_D - 1) * OPS)
+                         : "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(%4) lgkmcnt(0)"
+                         : "+v"(w.a[0][0]), "+v"(w.a[0][1]), "+v"(w.a[1][0]), "+v"(w.a[1][1])
+                         : "n"((DD_D - 1) * OPS)
+                         : "memory");
     };
 
     // prologue: steps 0 .. DD_D-1 in flight, then wait for step 0
@@ -501,42 +512,50 @@ walked:
     pin_acc();
     // The loads of the steps beyond the last are still in flight and nothing reads what they bring:
     // every register of the ring passes through the final wait.
-    static_assert(DD_D == 2, "the final wait lists three weight sets");
-    asm volatile("s_waitcnt vmcnt(0)"
-                 : "+v"(ws[0].a[0][0]), "+v"(ws[0].a[0][1]), "+v"(ws[0].a[1][0]), "+v"(ws[0].a[1][1]),
-                   "+v"(ws[0].a[2][0]), "+v"(ws[0].a[2][1]), "+v"(ws[0].a[3][0]), "+v"(ws[0].a[3][1]),
-                   "+v"(ws[1].a[0][0]), "+v"(ws[1].a[0][1]), "+v"(ws[1].a[1][0]), "+v"(ws[1].a[1][1]),
-                   "+v"(ws[1].a[2][0]), "+v"(ws[1].a[2][1]), "+v"(ws[1].a[3][0]), "+v"(ws[1].a[3][1]),
-                   "+v"(ws[2].a[0][0]), "+v"(ws[2].a[0][1]), "+v"(ws[2].a[1][0]), "+v"(ws[2].a[1][1]),
-                   "+v"(ws[2].a[2][0]), "+v"(ws[2].a[2][1]), "+v"(ws[2].a[3][0]), "+v"(ws[2].a[3][1])
-                 :
-                 : "memory");
+    if constexpr (AB == 4) {
+        static_assert(AB != 4 || DD_D == 2, "the final wait lists three weight sets");
+        asm volatile("s_waitcnt vmcnt(0)"
+                     : "+v"(ws[0].a[0][0]), "+v"(ws[0].a[0][1]), "+v"(ws[0].a[1][0]), "+v"(ws[0].a[1][1]),
+                       "+v"(ws[0].a[AB - 2][0]), "+v"(ws[0].a[AB - 2][1]), "+v"(ws[0].a[AB - 1][0]), "+v"(ws[0].a[AB - 1][1]),
+                       "+v"(ws[1].a[0][0]), "+v"(ws[1].a[0][1]), "+v"(ws[1].a[1][0]), "+v"(ws[1].a[1][1]),
+                       "+v"(ws[1].a[AB - 2][0]), "+v"(ws[1].a[AB - 2][1]), "+v"(ws[1].a[AB - 1][0]), "+v"(ws[1].a[AB - 1][1]),
+                       "+v"(ws[2].a[0][0]), "+v"(ws[2].a[0][1]), "+v"(ws[2].a[1][0]), "+v"(ws[2].a[1][1]),
+                       "+v"(ws[2].a[AB - 2][0]), "+v"(ws[2].a[AB - 2][1]), "+v"(ws[2].a[AB - 1][0]), "+v"(ws[2].a[AB - 1][1])
+                     :
+                     : "memory");
+    } else {
+#pragma unroll
+        for (int st = 0; st <= DD_D; st++) {
+            WSet &w = ws[st];
+            asm volatile("s_waitcnt vmcnt(0)" : "+v"(w.a[0][0]), "+v"(w.a[0][1]), "+v"(w.a[1][0]), "+v"(w.a[1][1]) : : "memory");
+        }
+    }
     asm volatile("s_barrier" ::: "memory");
     if (P.ksplit > 1) {
         store_partial_tile16<AB, TB>(acc, P.part + (int64_t)slice * P.T * P.part_ld, P.part_ld, lane,
-                                     f0 + wave * 64, t0, P.T);
+                                     f0 + wave * (16 * AB), t0, P.T);
         return;
     }
     const TileOut out{P.y, P.bias, P.O, P.T, P.ldy};
     if constexpr (CT)
-        store_tile16_t<T, AB, TB>(acc, smem + wave * (AB * 16 * (TT * 2 + 16)), lane, f0 + wave * 64, t0, out);
+        store_tile16_t<T, AB, TB>(acc, smem + wave * (AB * 16 * (TT * 2 + 16)), lane, f0 + wave * (16 * AB), t0, out);
     else
-        store_tile16<T, AB, TB>(acc, smem + wave * (TT * (AB * 32 + 16)), lane, f0 + wave * 64, t0, out);
+        store_tile16<T, AB, TB>(acc, smem + wave * (TT * (AB * 32 + 16)), lane, f0 + wave * (16 * AB), t0, out);
 }
 
-template <typename T, int TB, int NH, bool XT = false, bool CT = XT, bool ROWA = false> static int launch_dense16(DfParams &P, hipStream_t s)
+template <typename T, int TB, int NH, bool XT = false, bool CT = XT, bool ROWA = false, int AB = 4> static int launch_dense16(DfParams &P, hipStream_t s)
 {
     constexpr int TT = TB * 16;
-    P.tiles_m = (int)((P.O + 255) / 256);
+    P.tiles_m = (int)((P.O + 64 * AB - 1) / (64 * AB));
     P.tiles_n = (int)((P.T + TT - 1) / TT);
     const int slices = P.ksplit > 1 ? P.ksplit : 1;
     dim3 grid((unsigned)(P.tiles_m * P.tiles_n * slices));
     P.turn = stagger_xcds(grid.x, P.KP / slices, P.KP * (P.O + P.T) * 128) ? 1 : 0;
-    constexpr size_t ring = (size_t)DD_NS * TT * 128;
-    constexpr size_t stg = CT ? (size_t)4 * 64 * (TT * 2 + 16) : (size_t)4 * TT * (4 * 32 + 16);
+    constexpr size_t ring = (size_t)dd_stages(AB) * TT * 128;
+    constexpr size_t stg = CT ? (size_t)4 * 16 * AB * (TT * 2 + 16) : (size_t)4 * TT * (AB * 32 + 16);
     constexpr size_t lds = ring > stg ? ring : stg;
     static_assert(lds <= 160 * 1024, "LDS");
-    auto k = dense16_direct_kernel<T, TB, NH, XT, CT, ROWA>;
+    auto k = dense16_direct_kernel<T, TB, NH, XT, CT, ROWA, AB>;
     NMG_HIP_TRY(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k, grid, dim3(256), lds, s, P);
     NMG_HIP_TRY(hipGetLastError());
@@ -555,16 +574,54 @@ static bool dense16_square(int64_t O, int64_t T)
     return t256 >= 256 && fill256 * 1.055 >= fill128;
 }
 
+// The tiles of the direct kernel: 256 outputs x 128 tokens, 256 x 256 and, narrow, 128 x 128.
+enum { DENSE_WIDE, DENSE_SQUARE, DENSE_NARROW };
+
+static inline int64_t dense16_tiles(int tile, int64_t O, int64_t T)
+{
+    return (tile == DENSE_NARROW ? (O + 127) / 128 : (O + 255) / 256) * (tile == DENSE_SQUARE ? (T + 255) / 256 : (T + 127) / 128);
+}
+
+// Time in us of a product whose reduction of `steps` K steps is cut into `slices`, one workgroup per CU: whole rounds of 256
+// workgroups and a last one that is the faster the fewer it has, a step and a fixed part per round; with slices the second kernel and
+// the partial sums, written and read once; and the weight comes from memory in any case.  The constants are those of 17 weights
+// of 512^2 to 16384 x 2048 and 1024 x 16384 with 17 to 6000 tokens in 1 to 16 slices (fp16 4:8, weights new in every pass), 9 % off in
+// the mean; what it chooses is 1 % behind the best of those measured.
+static double dense16_cost(int tile, int slices, int64_t O, int64_t steps, int64_t T)
+{
+    static const struct { double step, fixed, crowd; } of[] = {{0.54, 4.3, 0.44}, {0.89, 11.0, 0.49}, {0.30, 3.8, 0.63}};
+    const auto c = of[tile];
+    const int64_t groups = dense16_tiles(tile, O, T) * slices, rest = groups % 256;
+    const double walk = (double)((steps + slices - 1) / slices) * c.step;
+    double t = (double)(groups / 256) * (walk * (1 + c.crowd) + c.fixed);
+    if (rest) t += walk * (1 + c.crowd * (double)rest / 256) + c.fixed;
+    if (slices > 1) t += 2.6 + (double)slices * (double)T * (double)O * 8 * 0.21e-6;
+    const double mem = (double)O * (double)steps * 128 * 0.15e-6 + c.fixed;
+    return std::sqrt(std::sqrt(t * t * t * t + mem * mem * mem * mem));
+}
+
+// The tile of a product.  Where 128 x 128 needs more than one round it is behind (4096 x 4096 x 2048 tokens: 256 wide tiles 52.8 us, 512
+// narrow 65.7).  Below, it leaves fewer CUs idle: x 777 in two slices of wide tiles and their sum 36.7, 224 narrow tiles 30.0;
+// 1024 x 1024 x 777 16.6 -> 9.7; 768 x 3072 x 4096 31.5 -> 22.1.  256 x 256 moves the fewest bytes per flop and is for what wide
+// tiles do not take in one round: 4096 x 11008 x 2500, 320 wide tiles 265, 160 square 195; but 752 against 384 412 and 428.
+static int dense16_tile(int slices, int64_t O, int64_t steps, int64_t T)
+{
+    const double wide = dense16_cost(DENSE_WIDE, slices, O, steps, T);
+    if (dense16_tiles(DENSE_NARROW, O, T) * slices <= 256) return dense16_cost(DENSE_NARROW, slices, O, steps, T) < wide ? DENSE_NARROW : DENSE_WIDE;
+    // (4 % between the two is within the error of the model)
+    if (slices == 1 && dense16_tiles(DENSE_WIDE, O, T) > 256 && dense16_cost(DENSE_SQUARE, 1, O, steps, T) * 1.04 < wide) return DENSE_SQUARE;
+    return DENSE_WIDE;
+}
+
 template <typename T, bool CT = false> static int launch_dense(DfParams &P, int variant, hipStream_t s)
 {
-    // Variant 0: 256 outputs x 128 tokens per workgroup, 1: 256 x 256.  The larger tile moves fewer
-    // bytes per flop through the vector caches and is 5-6 % faster per flop in steady state; one
-    // workgroup per CU either way, so what decides is how full the last round of tiles is.
+    // Variant 0: 256 outputs x 128 tokens per workgroup, 1: 256 x 256, -1: the faster one of all tiles.
     // (A sixteen-phase form of the 256 x 256 tile on the 32 x 32 x 16 instruction once gave wrong
     // values now and then; the forms here pass the static check of their hand-tracked loads and
     // the repeated full-chip test.)
-    if (variant < 0) variant = P.ksplit <= 1 && dense16_square(P.O, P.T) ? 1 : 0;
-    if (variant == 1) return launch_dense16<T, 16, 4, false, CT>(P, s);
+    const int tile = variant < 0 ? dense16_tile(P.ksplit > 1 ? P.ksplit : 1, P.O, P.KP, P.T) : variant;
+    if (tile == DENSE_NARROW) return launch_dense16<T, 8, 2, false, CT, false, 2>(P, s);
+    if (tile == DENSE_SQUARE) return launch_dense16<T, 16, 4, false, CT>(P, s);
     return launch_dense16<T, 8, 2, false, CT>(P, s);
 }
 
@@ -759,6 +816,30 @@ extern "C" int nmg_spmm_densefrag_ct(const void *d_df, int64_t O, int64_t K, con
     return dtype == NMG_F16 ? launch_dense<__half, true>(P, -1, s) : launch_dense<__hip_bfloat16, true>(P, -1, s);
 }
 
+extern "C" int nmg_densefrag_plan(int64_t O, int64_t K, int64_t T, int *slices, int64_t *workspace_bytes)
+{
+    NMG_REQUIRE(O >= 0 && K >= 0 && T >= 0, NMG_ERR_ARG, "negative extent");
+    NMG_REQUIRE(slices && workspace_bytes, NMG_ERR_ARG, "null output pointer");
+    const int64_t steps = K / 64;
+    int best = 1;
+    if (O > 0 && T > 0 && steps > 0) {
+        double least = dense16_cost(dense16_tile(1, O, steps, T), 1, O, steps, T);
+        // at most a workgroup per CU and eight slices (sixteen for a handful of tiles), at least four steps each
+        const int64_t wide = dense16_tiles(DENSE_WIDE, O, T);
+        for (int64_t s = 2; s <= std::min<int64_t>(wide <= 8 ? 16 : 8, steps / 4) && wide * s <= 256; s++) {
+            if (splitk_fit(steps, s) != s) continue;
+            const double t = dense16_cost(dense16_tile((int)s, O, steps, T), (int)s, O, steps, T);
+            if (t < least) {
+                least = t;
+                best = (int)s;
+            }
+        }
+    }
+    *slices = best;
+    *workspace_bytes = best > 1 ? (int64_t)best * T * ((O + 255) / 256) * 256 * 4 : 0;
+    return NMG_OK;
+}
+
 extern "C" int nmg_spmm_densefrag_splitk(const void *d_df, int64_t O, int64_t K, const void *d_x, int64_t ldx,
                                          void *d_y, int64_t ldy, const void *d_bias, int64_t T, int dtype,
                                          int slices, void *d_workspace, int64_t workspace_bytes, void *stream)
@@ -794,5 +875,5 @@ extern "C" int nmg_spmm_densefrag_splitk(const void *d_df, int64_t O, int64_t K,
     P.part = (float *)d_workspace;
     P.part_ld = tiles_m * 256;
     hipStream_t s = (hipStream_t)stream;
-    return dtype == NMG_F16 ? launch_dense16<__half, 8, 2>(P, s) : launch_dense16<__hip_bfloat16, 8, 2>(P, s);
+    return dtype == NMG_F16 ? launch_dense<__half>(P, -1, s) : launch_dense<__hip_bfloat16>(P, -1, s);
 }

@@ -616,10 +616,7 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
         const int64_t ldx = dense16 ? (T > 1 ? x.stride(0) : K) : pitch_of(xq), K = Kp;
         int slices = 1;
         int64_t bytes = 0;
-        if (opt.dense_variant == -1)
-            // (the plan leaves 16 tokens and fewer to the streaming kernel of the sparse-core operand;
-            // here they are cut like 17)
-            check(nmg_splitk_plan(O, K, std::max<int64_t>(T, 17), &slices, &bytes));
+        if (opt.dense_variant == -1) check(nmg_densefrag_plan(O, K, T, &slices, &bytes));
         if (opt.slices >= 0) slices = (int)opt.slices;
         if (slices > 1) {
             // few tiles for the chip: the reduction is cut into slices, summed by a second kernel
@@ -727,8 +724,9 @@ bool tt_split_pays(const Options &opt, int64_t O, int64_t K, int64_t N, bool spa
         return false;
     int slices = 1;
     int64_t bytes = 0;
-    check(nmg_splitk_plan(O, K, N, &slices, &bytes));
-    const double saved = (double)up(K, 64) * (1.0 - 1.0 / slices) * (sparse ? 0.45 : 0.6);
+    check(sparse ? nmg_splitk_plan(O, K, N, &slices, &bytes) : nmg_densefrag_plan(O, round_up(K, 64), N, &slices, &bytes));
+    const bool narrow = !sparse && up(O, 128) * up(N, 128) <= 256;
+    const double saved = (double)up(K, 64) * (1.0 - 1.0 / slices) * (sparse ? 0.45 : narrow ? 0.4 : 0.6);
     return slices > 1 && saved > 11.0 + (double)slices * (double)(N * O) * 8 / 4e6;
 }
 
