@@ -95,7 +95,7 @@ __global__ __launch_bounds__(512, 2) void spmm_dense_pipe_kernel(DenseParams P)
 
     int id = blockIdx.x;
     const int ntiles = P.tiles_m * P.tiles_n;
-    if ((ntiles & 7) == 0) id = (id & 7) * (ntiles >> 3) + (id >> 3);
+    id = xcd_run(id, ntiles);
     constexpr int GH = 4;
     const int band = id / (GH * P.tiles_n);
     const int band_h = min(P.tiles_m - band * GH, GH);

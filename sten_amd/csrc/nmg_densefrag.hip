@@ -239,7 +239,7 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     // slices of the reduction: the slices of a tile are workgroups ntiles apart
     const int slice = P.ksplit > 1 ? id / ntiles : 0;
     id -= slice * ntiles;
-    if ((ntiles & 7) == 0) id = (id & 7) * (ntiles >> 3) + (id >> 3);
+    id = xcd_run(id, ntiles);
     constexpr int GH = 4;
     const int band = id / (GH * P.tiles_n);
     const int band_h = min(P.tiles_m - band * GH, GH);

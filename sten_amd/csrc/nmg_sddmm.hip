@@ -215,7 +215,7 @@ __global__ __launch_bounds__(256, 1) void sddmm16_kernel(SddmmParams P)
     // a compact block of tiles whose operands stay in that XCD's L2.
     int id = blockIdx.x;
     const int ntiles = P.tiles_p * P.tiles_l;
-    if ((ntiles & 7) == 0) id = (id & 7) * (ntiles >> 3) + (id >> 3);
+    id = xcd_run(id, ntiles);
     constexpr int GH = 4;
     const int band = id / (GH * P.tiles_l);
     const int band_h = min(P.tiles_p - band * GH, GH);

@@ -95,7 +95,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void spmm_smfmac_kernel(SmfPara
     // contiguous run of tiles (token tile fastest) and let it reuse its weight rows from its L2.
     int id = blockIdx.x;
     const int ntiles = P.tiles_m * P.tiles_n;
-    if ((ntiles & 7) == 0) id = (id & 7) * (ntiles >> 3) + (id >> 3);
+    id = xcd_run(id, ntiles);
     const int tile_m = id / P.tiles_n, tile_n = id - tile_m * P.tiles_n;
     const int64_t f0 = (int64_t)tile_m * BMf, t0 = (int64_t)tile_n * BNt;
 
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
     // slices of the reduction: the slices of a tile are workgroups ntiles apart
     const int slice = P.ksplit > 1 ? id / ntiles : 0;
     id -= slice * ntiles;
-    if ((ntiles & 7) == 0) id = (id & 7) * (ntiles >> 3) + (id >> 3);
+    id = xcd_run(id, ntiles);
     const int GH = P.band;
     const int band = id / (GH * P.tiles_n);
     const int band_h = min(P.tiles_m - band * GH, GH);

@@ -81,3 +81,24 @@ def test_dense_products_of_every_tile(dtype, R, C, T, slices):
         # its transposed result
         c = sten.spmm_tt(w, x.to(DEV).t().contiguous())
         assert within(c, prod.T, 0.0, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tiles", [(1, 1), (1, 7), (3, 3), (1, 9), (5, 3), (1, 23), (3, 11)])
+def test_every_tile_once(tiles):
+    # counts of tiles of 256 x 128 with every remainder by the 8 runs that the workgroups are dealt to
+    R, C, T = tiles[0] * 256 - 8, 128, tiles[1] * 128 - 4
+    for n, m, g, opt in ((2, 4, 16, {"variant": 6}), (2, 4, 16, {"variant": 0}), (4, 8, 4, {"dense_variant": 0})):
+        print(f"case {tiles} {n}:{m} {opt}", flush=True)
+        W, x = whole((R, C), torch.float16, R), whole((T, C), torch.float16, T)
+        w = sten.GroupedNMTensor.from_dense(W.to(DEV), n, m, sparse_dim=1, group_size=g, group_dim=0)
+        w.spmm_opt.update(opt)
+        prod = to_np(x).astype(np.float64) @ to_np(w.to_dense()).astype(np.float64).T
+        y = sten.spmm(w, x.to(DEV), reduce_dim=1, kernel="smfmac" if m == 4 else "densefrag")
+        assert within(y, prod, 0.0, torch.float16)
+    # the gradient in the weight's own pattern
+    w = sten.get_sparsifier_implementation(sten.GroupedNMSparsifier, torch.Tensor, sten.GroupedNMTensor)(
+        sten.GroupedNMSparsifier(2, 4, 16, sparse_dim=1, group_dim=0), whole((R, T), torch.float16, 1).to(DEV).requires_grad_(True))
+    B, go = whole((T, C), torch.float16, 2).to(DEV), whole((R, C), torch.float16, 3)
+    torch.mm(w, B).backward(go.to(DEV))
+    assert within(w.grad.wrapped_tensor.to_dense(), to_np(go).astype(np.float64) @ to_np(B).astype(np.float64).T, 0.0, torch.float16)
