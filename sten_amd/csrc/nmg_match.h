@@ -180,7 +180,7 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
                 acc += __uint_as_float(__float_as_uint(a[r]) & (uint32_t)__builtin_amdgcn_sbfe((int)mk, r, 1));      // (adding 0 changes nothing)
             return __float_as_uint(acc);
         };
-        if (c <= 8) {      // few patterns: one by one (1000 x 1001 2:4:16 fp16 26.0 us, by classes 27.4)
+        if (classes == 0) {
             uint32_t best = 0, bmask = 0;
             int bp = 0;
             bool tied = false;
@@ -274,11 +274,15 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
         s_at[p] = before + above;
         s_last[p] = before + size - 1;
     }
-    if (c > 8) {      // (else the patterns one by one)
+    // Few patterns, or few that agree: one by one, which reads half as much per sum (us, one by one against by classes: 1000 x 1001
+    // 2:4:16 fp16 26.0, 27.4; 1536 x 2157 2:5:8 bf16, 4 classes of 10, 51, 54; x 2176 3:6:12, 14 of 20, 62, 70; x 2163, 8 of 20, 69, 72,
+    // fp32 69, 66; x 2162, 4 of 20, 62, 60).
+    if (c > 15) {
         match_sync<NT>();
         for (int q = 0; q < c; q++) classes += s_at[q] == s_last[q] ? 1 : 0;
+        if (3 * classes > 2 * c) classes = 0;
         for (int p = tt; p < c; p += NT)
-            if (s_at[p] == s_last[p]) {
+            if (classes > 0 && s_at[p] == s_last[p]) {
                 int k = 0;
                 for (int q = 0; q < c; q++) k += s_at[q] == s_last[q] && s_at[q] < s_at[p] ? 1 : 0;
                 s_class[k] = p;
