@@ -167,11 +167,14 @@ int nmg_spmm_smfmac_ct(const void *d_fp_val, const void *d_fp_idx, int64_t M, in
  * order (+ bias) and rounds once.  nmg_splitk_plan gives the number of slices for a product of M
  * outputs, reduction K and T tokens (1 = do not split) and the workspace in bytes; the workspace
  * is caller-owned device memory, 16-byte aligned, written and read inside the call only.
+ * nmg_smfmac_plan gives the number that is fastest with the tiles that the kernels choose for it (1024 x 1024 x 1024 tokens: 16.8 us
+ * in two slices, 9.7 whole); nmg_splitk_plan brings the workgroups of 256 x 128 towards one per CU.
  * slices <= 1 is the unsplit entry point with its default tile.  K % 64 == 0, T > 16.
  * nmg_spmm_densefrag_splitk (declared with the densefrag entry points) is the same for the
  * dense-matrix-core route, its slices from nmg_densefrag_plan.
  * No counterpart in the reference (sten_impls.py:44-140 calls one generated loop nest). */
 int nmg_splitk_plan(int64_t M, int64_t K, int64_t T, int *slices, int64_t *workspace_bytes);
+int nmg_smfmac_plan(int64_t M, int64_t K, int64_t T, int *slices, int64_t *workspace_bytes);
 int nmg_spmm_smfmac_splitk(const void *d_fp_val, const void *d_fp_idx, int64_t M, int64_t K,
                            const void *d_x, int64_t ldx, void *d_y, int64_t ldy, const void *d_bias,
                            int64_t T, int dtype, int slices, void *d_workspace, int64_t workspace_bytes,

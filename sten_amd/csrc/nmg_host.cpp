@@ -511,7 +511,7 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
         const void *fv = w.ops.fp_val.data_ptr(), *fi = w.ops.fp_idx.data_ptr();
         int slices = 1;
         int64_t bytes = 0;
-        if (T > 16) check(nmg_splitk_plan(O, Kp, T, &slices, &bytes));
+        if (T > 16) check(nmg_smfmac_plan(O, Kp, T, &slices, &bytes));
         if (slices > 1) {
             Tensor ws = workspace(split_ws(slices, T, O), x);
             check(nmg_spmm_smfmac_splitk(fv, fi, O, Kp, xq.data_ptr(), pitch_of(xq), yp, O, bp, T, dt, slices, ws.data_ptr(), ws.numel() * 4, stream));
@@ -541,7 +541,7 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
             // few tiles for the chip: the reduction is cut into slices, summed by a second kernel
             int slices = 1;
             int64_t bytes = 0;
-            check(nmg_splitk_plan(O, K, T, &slices, &bytes));
+            check(nmg_smfmac_plan(O, K, T, &slices, &bytes));
             if (opt.slices >= 0) slices = (int)opt.slices;
             if (slices > 1) {
                 Tensor ws = workspace(split_ws(slices, T, O), x);
@@ -714,7 +714,7 @@ bool transposed_pays(int64_t O, int64_t K, int64_t N, bool as_it_lies)
 
 // Whether op(W) B with few columns is better cut along the reduction (as spmm does it, its result transposed
 // back) than run whole on the CUs that its tiles occupy.  A reduction step of 64 takes about 0.45 us on the sparse and
-// 0.6 us on the dense cores; the cut saves the steps of all slices but one and costs about 11 us of launches beside
+// 0.6 us on the dense cores, 0.4 on tiles of 128 x 128; the cut saves the steps of all slices but one and costs about 11 us of launches beside
 // the partial sums, written and read once.  us, whole -> cut: sparse cores 4096 x 11008 x 32 columns 81 -> 27, x 512
 // 102 -> 58, 4096 x 4096 x 128 31 -> 25 (8 slices), x 512 32 -> 41 (4 slices); dense cores 1024 x 16384 x 128 141 -> 31,
 // 4096 x 4096 x 512 46 -> 41, x 1024 50 -> 57.
@@ -724,9 +724,9 @@ bool tt_split_pays(const Options &opt, int64_t O, int64_t K, int64_t N, bool spa
         return false;
     int slices = 1;
     int64_t bytes = 0;
-    check(sparse ? nmg_splitk_plan(O, K, N, &slices, &bytes) : nmg_densefrag_plan(O, round_up(K, 64), N, &slices, &bytes));
-    const bool narrow = !sparse && up(O, 128) * up(N, 128) <= 256;
-    const double saved = (double)up(K, 64) * (1.0 - 1.0 / slices) * (sparse ? 0.45 : narrow ? 0.4 : 0.6);
+    check(sparse ? nmg_smfmac_plan(O, K, N, &slices, &bytes) : nmg_densefrag_plan(O, round_up(K, 64), N, &slices, &bytes));
+    const bool narrow = up(O, 128) * up(N, 128) <= 256;      // (tiles of 128 x 128)
+    const double saved = (double)up(K, 64) * (1.0 - 1.0 / slices) * (narrow ? 0.4 : sparse ? 0.45 : 0.6);
     return slices > 1 && saved > 11.0 + (double)slices * (double)(N * O) * 8 / 4e6;
 }
 

@@ -288,8 +288,9 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void spmm_smfmac_kernel(SmfPara
 // MFMAs of a phase run while the activation fragments of the next one are read from LDS into a
 // second register set.  Short phases pay: with four MFMAs per phase the 256 x 128 tile is 3-12 %
 // faster than with eight (fewer fragments wait in registers, the LDS reads are spread thinner).
-constexpr int DR_D = 3;                 // K steps in flight
-constexpr int DR_NS = 4;                // activation stages in LDS (>= DR_D + 1)
+// K steps in flight and activation stages in LDS (>= steps + 1), by the blocks of 32 features of a wavefront
+constexpr int dr_steps(int fb) { return fb == 2 ? 3 : 6; }
+constexpr int dr_stages(int fb) { return fb == 2 ? 4 : 8; }
 
 //
 // XT = true is the product with both dense operands transposed, C[M, T] = W * B for B [K, T]
@@ -305,6 +306,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
     using S = Smf<T>;
     static_assert(WM * WN == 4, "four wavefronts");
     static_assert(TB % NH == 0, "token blocks split evenly into phases");
+    constexpr int DR_D = dr_steps(FB), DR_NS = dr_stages(FB);
     constexpr int TF = WM * FB * 32, TT = WN * TB * 32;   // workgroup tile: features x tokens
     constexpr int STAGE = TT * 128;                       // activation bytes per K step
     constexpr int XL = TT / 32;                           // DMA loads per wavefront per K step
@@ -528,12 +530,16 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
     // kp+DR_D-DR_NS < kp, completed (lgkmcnt(0), same wait) before the barrier of their step.
     static_assert(DR_NS > DR_D, "a stage must not be refilled while the step that reads it is in flight");
     static_assert(NP % 2 == 0, "fragment sets alternate by phase across K steps");
-    static_assert(FB == 2, "the wait lists the registers of two fragment rows");
+    static_assert(FB == 1 || FB == 2, "the waits list the registers of one or two fragment rows");
     auto landed = [&](WSet &w) {
-        asm volatile("s_waitcnt vmcnt(%6) lgkmcnt(0)"
-                     : "+a"(w.a[0][0]), "+a"(w.a[0][1]), "+v"(w.ix[0]), "+a"(w.a[1][0]), "+a"(w.a[1][1]), "+v"(w.ix[1])
-                     : "n"((DR_D - 1) * OPS)
-                     : "memory");
+        if constexpr (FB == 1)
+            asm volatile("s_waitcnt vmcnt(%3) lgkmcnt(0)" : "+a"(w.a[0][0]), "+a"(w.a[0][1]), "+v"(w.ix[0]) : "n"((DR_D - 1) * OPS) : "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(%6) lgkmcnt(0)"
+                         : "+a"(w.a[0][0]), "+a"(w.a[0][1]), "+v"(w.ix[0]), "+a"(w.a[FB - 1][0]), "+a"(w.a[FB - 1][1]),
+                           "+v"(w.ix[FB - 1])
+                         : "n"((DR_D - 1) * OPS)
+                         : "memory");
     };
 
     // prologue: steps 0 .. DR_D-1 in flight, then wait for step 0
@@ -640,14 +646,20 @@ walked:
     // The loads of the steps beyond the last are still in flight and nothing reads what they bring:
     // every register of the ring passes through the final wait, so that none of them is given to
     // the epilogue while a load may still land in it.
-    static_assert(DR_D == 3 && FB == 2, "the final wait lists four weight sets of two fragment rows");
-    asm volatile("s_waitcnt vmcnt(0)"
-                 : "+a"(ws[0].a[0][0]), "+a"(ws[0].a[0][1]), "+a"(ws[0].a[1][0]), "+a"(ws[0].a[1][1]), "+v"(ws[0].ix[0]), "+v"(ws[0].ix[1]),
-                   "+a"(ws[1].a[0][0]), "+a"(ws[1].a[0][1]), "+a"(ws[1].a[1][0]), "+a"(ws[1].a[1][1]), "+v"(ws[1].ix[0]), "+v"(ws[1].ix[1]),
-                   "+a"(ws[2].a[0][0]), "+a"(ws[2].a[0][1]), "+a"(ws[2].a[1][0]), "+a"(ws[2].a[1][1]), "+v"(ws[2].ix[0]), "+v"(ws[2].ix[1]),
-                   "+a"(ws[3].a[0][0]), "+a"(ws[3].a[0][1]), "+a"(ws[3].a[1][0]), "+a"(ws[3].a[1][1]), "+v"(ws[3].ix[0]), "+v"(ws[3].ix[1])
-                 :
-                 : "memory");
+    if constexpr (FB == 2) {
+        static_assert(FB != 2 || DR_D == 3, "the final wait lists four weight sets");
+        asm volatile("s_waitcnt vmcnt(0)"
+                     : "+a"(ws[0].a[0][0]), "+a"(ws[0].a[0][1]), "+a"(ws[0].a[FB - 1][0]), "+a"(ws[0].a[FB - 1][1]), "+v"(ws[0].ix[0]), "+v"(ws[0].ix[FB - 1]),
+                       "+a"(ws[1].a[0][0]), "+a"(ws[1].a[0][1]), "+a"(ws[1].a[FB - 1][0]), "+a"(ws[1].a[FB - 1][1]), "+v"(ws[1].ix[0]), "+v"(ws[1].ix[FB - 1]),
+                       "+a"(ws[2].a[0][0]), "+a"(ws[2].a[0][1]), "+a"(ws[2].a[FB - 1][0]), "+a"(ws[2].a[FB - 1][1]), "+v"(ws[2].ix[0]), "+v"(ws[2].ix[FB - 1]),
+                       "+a"(ws[3].a[0][0]), "+a"(ws[3].a[0][1]), "+a"(ws[3].a[FB - 1][0]), "+a"(ws[3].a[FB - 1][1]), "+v"(ws[3].ix[0]), "+v"(ws[3].ix[FB - 1])
+                     :
+                     : "memory");
+    } else {
+#pragma unroll
+        for (int st = 0; st <= DR_D; st++)
+            asm volatile("s_waitcnt vmcnt(0)" : "+a"(ws[st].a[0][0]), "+a"(ws[st].a[0][1]), "+v"(ws[st].ix[0]) : : "memory");
+    }
     asm volatile("s_barrier" ::: "memory");
     if (P.ksplit > 1) {
         store_partial_tile<FB, TB>(acc, P.part + (int64_t)slice * P.T * P.part_ld, P.part_ld, lane,
@@ -667,7 +679,7 @@ template <typename T, int FB, int TB, int WM, int WN, int NH, bool XT = false, b
 static int launch_smfmac_direct(SmfParams &P, hipStream_t s)
 {
     constexpr int TF = WM * FB * 32, TT = WN * TB * 32;
-    static_assert(TF == 256, "the operand is padded to 256 lines");
+    static_assert(256 % TF == 0, "the operand is padded to 256 lines");
     P.tiles_m = (int)((P.M + TF - 1) / TF);
     P.tiles_n = (int)((P.T + TT - 1) / TT);
     // An XCD works on 32 consecutive tiles of the walk at a time, a block of `band` line tiles x
@@ -677,7 +689,7 @@ static int launch_smfmac_direct(SmfParams &P, hipStream_t s)
     const int slices = P.ksplit > 1 ? P.ksplit : 1;
     dim3 grid((unsigned)(P.tiles_m * P.tiles_n * slices));
     P.turn = !P.in_order && stagger_xcds(grid.x, P.KP / slices, P.KP * (int64_t)(P.MB * 32 * 72 + P.T * 128)) ? 1 : 0;
-    constexpr size_t ring = (size_t)DR_NS * TT * 128;
+    constexpr size_t ring = (size_t)dr_stages(FB) * TT * 128;
     constexpr size_t stg = CT ? (size_t)4 * FB * 32 * (TB * 64 + 16) : (size_t)4 * TB * 32 * (FB * 64 + 16);
     constexpr size_t lds = ring > stg ? ring : stg;
     static_assert(lds <= 160 * 1024, "LDS");
@@ -1172,7 +1184,32 @@ static int launch_smfmac_cfg(SmfParams &P, hipStream_t s)
     return NMG_OK;
 }
 
-// The tile of the direct kernel: 6 = 256 x 128, 8 = 256 x 256.
+// Time in us of a product on tiles of 256 x 128 or, narrow, 128 x 128, its reduction of `steps` K steps cut into `slices`, one
+// workgroup per CU: whole rounds of 256 workgroups and a last one that is the faster the fewer it has, a step and a fixed part per
+// round; with slices the second kernel and the partial sums, written and read once.  A narrow step is bound by its LDS reads, which are
+// those of a wide one, and it fetches twice the bytes per flop, which tells where the operands are large.  The constants are
+// those of 8 weights of 512^2 to 16384 x 2048 and 4096 x 11008 with 17 to 6000 tokens in 1 to 16 slices (fp16 2:4, weights new in
+// every pass), 9 % off in the mean; what it chooses is 1 % behind the best of those measured.
+static double smfmac_cost(bool narrow, int slices, int64_t M, int64_t steps, int64_t T)
+{
+    const int64_t groups = (narrow ? (M + 127) / 128 : (M + 255) / 256) * ((T + 127) / 128) * slices, rest = groups % 256;
+    const double walk = (double)((steps + slices - 1) / slices) * (narrow ? 0.245 : 0.28), fixed = narrow ? 5.06 : 5.2, crowd = narrow ? 0.4 : 0.79;
+    double t = (double)(groups / 256) * (walk * (1 + crowd) + fixed);
+    if (rest) t += walk * (1 + crowd * (double)rest / 256) + fixed;
+    if (slices > 1) t += 2.45 + (double)slices * (double)T * (double)M * 8 * 0.21e-6;
+    if (narrow) t += 0.4 * std::max(0.0, (double)(M * 72 + T * 128) * (double)steps * 1e-6 - 46);
+    return t;
+}
+
+// Whether tiles of 128 x 128 are the faster ones.  Where they need more than one round they are behind (4096 x 4096 x 2000 tokens: 256
+// wide tiles 37.1 us, 512 narrow 50.4).  Below, they leave fewer CUs idle: 1024 x 1024 x 1024 10.6 -> 9.7, 4096 x 4096 x 777 26.6 -> 24.1,
+// 768 x 3072 x 2000 21.2 -> 18.4; with slices 2048 x 8192 x 300 24.0 -> 21.9; but 4096 x 11008 x 777 in two slices 57.0, narrow 61.4.
+static bool smfmac_narrow(int slices, int64_t M, int64_t steps, int64_t T)
+{
+    return (M + 127) / 128 * ((T + 127) / 128) * slices <= 256 && smfmac_cost(true, slices, M, steps, T) < smfmac_cost(false, slices, M, steps, T);
+}
+
+// The tile of the direct kernel: 6 = 256 x 128, 7 = 128 x 128, 8 = 256 x 256.
 static int smfmac_tile(const SmfParams &P)
 {
     // Large-batch default.  The 256 x 256 tile moves a quarter fewer bytes per flop through the
@@ -1182,7 +1219,8 @@ static int smfmac_tile(const SmfParams &P)
     // one (both are one workgroup per CU: 260 and 448 registers per lane).
     const int64_t tm = (P.M + 255) / 256, t256 = tm * ((P.T + 255) / 256), t128 = tm * ((P.T + 127) / 128);
     const double cost128 = (double)((t128 + 255) / 256), cost256 = (double)((t256 + 255) / 256) * 2.0 / 1.025;
-    return (P.ksplit <= 1 && cost256 < cost128) ? 8 : 6;
+    if (P.ksplit <= 1 && cost256 < cost128) return 8;
+    return smfmac_narrow(1, P.M, P.KP, P.T) ? 7 : 6;
 }
 
 template <typename T> static int launch_smfmac(SmfParams &P, int variant, hipStream_t s)
@@ -1210,10 +1248,12 @@ template <typename T> static int launch_smfmac(SmfParams &P, int variant, hipStr
         if ((P.M + 31) / 32 >= 256) return launch_smfmac_skinny<T, 4, 4>(P, s);
         return launch_smfmac_skinny<T, 16, 1>(P, s);
     case 6:                                                     // 256 x 128, weights straight to registers
+    case 7:                                                     // 128 x 128
     case 8:                                                     // 256 x 256
         if (P.K % 64 != 0 || P.T * P.ldx * 2 >= (int64_t)1 << 31)
             return launch_smfmac_cfg<T, 2, 2, 4, 2, 1>(P, s);
         if (variant == 8) return launch_smfmac_direct<T, 2, 8, 4, 1, 4>(P, s);
+        if (variant == 7) return launch_smfmac_direct<T, 1, 4, 4, 1, 1>(P, s);
         return launch_smfmac_direct<T, 2, 4, 4, 1, 2>(P, s);
     }
     return NMG_ERR_ARG;
@@ -1273,6 +1313,27 @@ extern "C" int nmg_splitk_plan(int64_t M, int64_t K, int64_t T, int *slices,
     return NMG_OK;
 }
 
+extern "C" int nmg_smfmac_plan(int64_t M, int64_t K, int64_t T, int *slices, int64_t *workspace_bytes)
+{
+    NMG_REQUIRE(M >= 0 && K >= 0 && T >= 0, NMG_ERR_ARG, "negative extent");
+    NMG_REQUIRE(slices && workspace_bytes, NMG_ERR_ARG, "null output pointer");
+    const int64_t steps = K / 64, wide = (M + 255) / 256 * ((T + 127) / 128);
+    int best = 1;
+    if (T > 16 && K % 64 == 0 && steps > 0 && wide > 0) {
+        auto cost = [&](int s) { return smfmac_cost(smfmac_narrow(s, M, steps, T), s, M, steps, T); };
+        double least = cost(1);
+        // at most a workgroup per CU and eight slices (sixteen for a handful of tiles), at least four steps each
+        for (int64_t s = 2; s <= std::min<int64_t>(wide <= 8 ? 16 : 8, steps / 4) && wide * s <= 256; s++) {
+            if (splitk_fit(steps, s) != s || cost((int)s) >= least) continue;
+            least = cost((int)s);
+            best = (int)s;
+        }
+    }
+    *slices = best;
+    *workspace_bytes = best > 1 ? (int64_t)best * T * ((M + 255) / 256) * 256 * 4 : 0;
+    return NMG_OK;
+}
+
 extern "C" int nmg_spmm_smfmac_splitk(const void *d_fp_val, const void *d_fp_idx, int64_t M, int64_t K,
                                       const void *d_x, int64_t ldx, void *d_y, int64_t ldy,
                                       const void *d_bias, int64_t T, int dtype, int slices,
@@ -1314,8 +1375,12 @@ extern "C" int nmg_spmm_smfmac_splitk(const void *d_fp_val, const void *d_fp_idx
     P.part = (float *)d_workspace;
     P.part_ld = tiles_m * 256;
     hipStream_t s = (hipStream_t)stream;
-    return dtype == NMG_F16 ? launch_smfmac_direct<__half, 2, 4, 4, 1, 2>(P, s)
-                            : launch_smfmac_direct<__hip_bfloat16, 2, 4, 4, 1, 2>(P, s);
+    const bool narrow = smfmac_narrow(slices, M, KP, T);
+    auto launch = [&](auto tag) -> int {
+        using T16 = decltype(tag);
+        return narrow ? launch_smfmac_direct<T16, 1, 4, 4, 1, 1>(P, s) : launch_smfmac_direct<T16, 2, 4, 4, 1, 2>(P, s);
+    };
+    return dtype == NMG_F16 ? launch(__half{}) : launch(__hip_bfloat16{});
 }
 
 // ---- both dense operands transposed: C[M, T] = W * B (+ bias per row), B [K, T] ------------------
@@ -1380,7 +1445,9 @@ extern "C" int nmg_spmm_smfmac_ct(const void *d_fp_val, const void *d_fp_idx, in
     hipStream_t s = (hipStream_t)stream;
     auto launch = [&](auto tag) -> int {
         using T16 = decltype(tag);
-        if (smfmac_tile(P) == 8) return launch_smfmac_direct<T16, 2, 8, 4, 1, 4, false, true>(P, s);
+        const int tile = smfmac_tile(P);
+        if (tile == 8) return launch_smfmac_direct<T16, 2, 8, 4, 1, 4, false, true>(P, s);
+        if (tile == 7) return launch_smfmac_direct<T16, 1, 4, 4, 1, 1, false, true>(P, s);
         return launch_smfmac_direct<T16, 2, 4, 4, 1, 2, false, true>(P, s);
     };
     return dtype == NMG_F16 ? launch(__half{}) : launch(__hip_bfloat16{});

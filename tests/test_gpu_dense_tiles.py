@@ -1,4 +1,4 @@
-"""The direct kernel of the dense matrix cores on the tiles it takes by itself: 256 x 128, 128 x 128, slices of either."""
+"""The direct kernels on the tiles that they take by themselves: 256 x 128, 128 x 128, slices of either, 256 x 256."""
 import ctypes
 
 import numpy as np
@@ -12,25 +12,28 @@ from sten_amd import native
 DEV = "cuda:0"
 
 
-def plan(O, K, T):
+def plan(O, K, T, entry="nmg_densefrag_plan"):
     slices, ws = ctypes.c_int(0), ctypes.c_int64(0)
-    assert native.load().nmg_densefrag_plan(O, K, T, ctypes.byref(slices), ctypes.byref(ws)) == 0
+    assert getattr(native.load(), entry)(O, K, T, ctypes.byref(slices), ctypes.byref(ws)) == 0
     return slices.value, ws.value
 
 
-def test_plan_leaves_no_slice_empty():
+@pytest.mark.parametrize("entry", ["nmg_densefrag_plan", "nmg_smfmac_plan"])
+def test_plan_leaves_no_slice_empty(entry):
     for O in (1, 100, 128, 129, 256, 1000, 4096, 16384, 50000):
         for K in (0, 64, 192, 256, 512, 576, 4096, 11008):
             for T in (0, 1, 17, 128, 129, 777, 4096):
-                s, ws = plan(O, K, T)
+                s, ws = plan(O, K, T, entry)
                 steps = K // 64
                 assert s == 1 or (2 <= s <= 16 and (s - 1) * -(-steps // s) < steps and steps // s >= 4)
                 assert ws == (0 if s == 1 else s * T * -(-O // 256) * 256 * 4)
-    assert plan(16384, 4096, 4096)[0] == 1 and plan(1024, 16384, 128)[0] > 1
+                if entry == "nmg_smfmac_plan" and T <= 16:
+                    assert s == 1
+    assert plan(16384, 4096, 4096, entry)[0] == 1 and plan(1024, 16384, 128, entry)[0] > 1 and plan(1024, 1000, 128, entry)[0] == 1
     lib = native.load()
     s, ws = ctypes.c_int(0), ctypes.c_int64(0)
-    assert lib.nmg_densefrag_plan(-1, 64, 64, ctypes.byref(s), ctypes.byref(ws)) == 1
-    assert lib.nmg_densefrag_plan(64, 64, 64, None, ctypes.byref(ws)) == 1
+    assert getattr(lib, entry)(-1, 64, 64, ctypes.byref(s), ctypes.byref(ws)) == 1
+    assert getattr(lib, entry)(64, 64, 64, None, ctypes.byref(ws)) == 1
 
 
 def whole(shape, dtype, seed):
@@ -48,12 +51,15 @@ def within(y, prod, bias, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("pattern", [(4, 8, 4), (2, 4, 16)])
 @pytest.mark.parametrize("R,C,T,slices", [
     (128, 64, 17, -1),        # one step, fewer than are in flight
     (127, 128, 128, -1),
     (129, 192, 129, -1),      # a last tile of one output and one token
     (255, 256, 300, -1),      # four steps, as many as are in flight
     (33, 320, 130, -1),
+    (256, 384, 100, -1),      # six and seven: as in flight on the sparse cores, and one more
+    (256, 448, 100, -1),
     (384, 512, 31, -1),       # as many steps as stages
     (1000, 576, 777, -1),     # one more; outputs that are no multiple of 16
     (1640, 1920, 386, -1),
@@ -66,15 +72,16 @@ def within(y, prod, bias, dtype):
     (640, 1088, 300, 4),      # of 5, 5, 5 and 2: the last shorter than the steps in flight
     (1100, 4096, 129, -1),    # what the plan takes
 ])
-def test_dense_products_of_every_tile(dtype, R, C, T, slices):
-    print(f"case {dtype} {R}x{C} T={T} slices={slices} plan={plan(R, C, T)}", flush=True)
+def test_products_of_every_tile(dtype, pattern, R, C, T, slices):
+    n, m, g = pattern
+    print(f"case {dtype} {n}:{m} {R}x{C} T={T} slices={slices} plans={plan(R, C, T)} {plan(R, C, T, 'nmg_smfmac_plan')}", flush=True)
     W, x = whole((R, C), dtype, R + C + T), whole((T, C), dtype, 1)
-    w = sten.GroupedNMTensor.from_dense(W.to(DEV), 4, 8, sparse_dim=1, group_size=4, group_dim=0)
+    w = sten.GroupedNMTensor.from_dense(W.to(DEV), n, m, sparse_dim=1, group_size=g, group_dim=0)
     if slices >= 0:
         w.spmm_opt["slices"] = slices
     D = to_np(w.to_dense()).astype(np.float64)
     bias = whole((R,), dtype, 2)
-    y = sten.spmm(w, x.to(DEV), bias.to(DEV), reduce_dim=1, kernel="densefrag")
+    y = sten.spmm(w, x.to(DEV), bias.to(DEV), reduce_dim=1, kernel="densefrag" if m == 8 else "smfmac")
     prod = to_np(x).astype(np.float64) @ D.T
     assert within(y, prod, to_np(bias).astype(np.float64), dtype)
     if slices < 0:
