@@ -236,10 +236,19 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     // a compact block of tiles whose weights and activations stay in that XCD's L2.
     int id = blockIdx.x;
     const int ntiles = P.tiles_m * P.tiles_n;
-    // slices of the reduction: the slices of a tile are workgroups ntiles apart
-    const int slice = P.ksplit > 1 ? id / ntiles : 0;
-    id -= slice * ntiles;
-    id = xcd_run(id, ntiles);
+    // Slices of the reduction: an XCD's run goes over slices and tiles, so that few XCDs fetch the same operands (us, against runs of tiles
+    // within every slice: 2:4 4096 x 11008 x 200 tokens 30.1 -> 25.1, 1024 x 16384 x 777 37 -> 28.7; 4:8 x 300 29.0 -> 20.3); but in short
+    // slices an XCD's workgroups wait for the same lines (2:4 2048 x 8192 x 128, 16 steps a slice, 14.7 -> 16.8).
+    const int kp_per = P.ksplit > 1 ? (P.KP + P.ksplit - 1) / P.ksplit : P.KP;
+    int slice = 0;
+    if (kp_per >= 20) {
+        id = xcd_run(id, gridDim.x);
+        if (P.ksplit > 1) slice = id / ntiles;
+        id -= slice * ntiles;
+    } else {
+        if (P.ksplit > 1) slice = id / ntiles;
+        id = xcd_run(id - slice * ntiles, ntiles);
+    }
     constexpr int GH = 4;
     const int band = id / (GH * P.tiles_n);
     const int band_h = min(P.tiles_m - band * GH, GH);
@@ -248,7 +257,6 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     const int64_t f0 = (int64_t)tile_m * TF, t0 = (int64_t)tile_n * TT;
     // K steps kp_lo .. kp_lo + KP - 1 of the operand's KPT (the host leaves no slice empty)
     const int KPT = P.KP;
-    const int kp_per = P.ksplit > 1 ? (KPT + P.ksplit - 1) / P.ksplit : KPT;
     const int kp_lo = slice * kp_per;
     const int KP = min(KPT, kp_lo + kp_per) - kp_lo;
     const int first = P.turn ? (int)(blockIdx.x & 7) * KP / 8 : 0;
