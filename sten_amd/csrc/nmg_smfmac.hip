@@ -1214,6 +1214,8 @@ static double smfmac_cost(bool narrow, int slices, int64_t M, int64_t steps, int
 // 768 x 3072 x 2000 21.2 -> 18.4; with slices 2048 x 8192 x 300 24.0 -> 21.9; but 4096 x 11008 x 777 in two slices 57.0, narrow 61.4.
 static bool smfmac_narrow(int slices, int64_t M, int64_t steps, int64_t T)
 {
+    // (a quarter of the tokens and less, in slices: its steps save nothing, 4096 x 4096 x 32 in 8 slices 11.6, narrow 12.0)
+    if (slices > 1 && T <= 32) return false;
     return (M + 127) / 128 * ((T + 127) / 128) * slices <= 256 && smfmac_cost(true, slices, M, steps, T) < smfmac_cost(false, slices, M, steps, T);
 }
 
