@@ -24,18 +24,14 @@
 // pipeline above, the single-precision one -- gemm_nt_f32_kernel, V_MFMA_F32_32X32X2_F32 -- with
 // its own three-stage loop; single-precision products with more than 16 tokens run on it).
 #include "nmg_common.h"
+#include "nmg_tile.h"
 
 #include <type_traits>
 
 namespace nmg {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void *lds_ptr_t;
-typedef const __attribute__((address_space(1))) void *glb_ptr_t;
 
 template <typename T> struct Dmma;
 template <> struct Dmma<__half> {
@@ -46,13 +42,6 @@ template <> struct Dmma<__hip_bfloat16> {
     using F = bf16x8;
     __device__ static f32x16 run(F a, F b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 };
-
-__device__ __forceinline__ uint16_t dn_bits16(float x, __half *) { return __half_as_ushort(__float2half(x)); }
-__device__ __forceinline__ uint16_t dn_bits16(float x, __hip_bfloat16 *)
-{
-    __hip_bfloat16 b = __float2bfloat16(x);
-    return *reinterpret_cast<uint16_t *>(&b);
-}
 
 struct DenseParams {
     const void *pk_val;
@@ -340,12 +329,7 @@ __global__ __launch_bounds__(512, 2) void spmm_dense_pipe_kernel(DenseParams P)
     // ================================== matrix wavefronts ==================================
     const int wm = wave >> 1, wn = wave & 1;
     f32x16 acc[FA][FB];
-#pragma unroll
-    for (int i = 0; i < FA; i++)
-#pragma unroll
-        for (int j = 0; j < FB; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+    start_sums<T>(acc, P.bias, lane, o0 + wm * 128, P.O);
 
     const int j = lane & 31, h = lane >> 5;
     struct Frags {
@@ -426,60 +410,9 @@ __global__ __launch_bounds__(512, 2) void spmm_dense_pipe_kernel(DenseParams P)
         __builtin_amdgcn_sched_barrier(0);
     }
 
-    // ---- epilogue: D[row = output][col = token] -> LDS [token][output] -> 16-byte stores ----
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    unsigned char *stg = smem + wave * (64 * DN_OUT_ROW);
-#pragma unroll
-    for (int tb = 0; tb < FB; tb++)
-#pragma unroll
-        for (int fb = 0; fb < FA; fb++)
-#pragma unroll
-            for (int rq = 0; rq < 4; rq++) {
-                uint16_t hh[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) hh[i] = dn_bits16(acc[fb][tb][rq * 4 + i], (T *)nullptr);
-                uint2 pk;
-                pk.x = (uint32_t)hh[0] | ((uint32_t)hh[1] << 16);
-                pk.y = (uint32_t)hh[2] | ((uint32_t)hh[3] << 16);
-                *(uint2 *)(stg + (tb * 32 + j) * DN_OUT_ROW + (fb * 32 + rq * 8 + h * 4) * 2) = pk;
-            }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    uint16_t *Y = (uint16_t *)P.y;
-    const T *bias = (const T *)P.bias;
-    const bool vec_ok = (P.ldy & 7) == 0 && ((uintptr_t)P.y & 15) == 0;
-    const int fc = lane & 15;
-    const int64_t f = o0 + wm * 128 + fc * 8;
-    float bv[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) bv[i] = (bias && f + i < P.O) ? to_f32(bias[f + i]) : 0.f;
-#pragma unroll 4
-    for (int it = 0; it < 16; it++) {
-        const int tl = it * 4 + (lane >> 4);
-        const int64_t tok = t0 + wn * 64 + tl;
-        u32x4 v = *(const u32x4 *)(stg + tl * DN_OUT_ROW + fc * 16);
-        if (tok >= P.T || f >= P.O) continue;
-        if (bias) {
-            uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint16_t lo = (uint16_t)(w[i] & 0xFFFF), hi = (uint16_t)(w[i] >> 16);
-                T tlo = *reinterpret_cast<T *>(&lo), thi = *reinterpret_cast<T *>(&hi);
-                lo = dn_bits16(to_f32(tlo) + bv[2 * i], (T *)nullptr);
-                hi = dn_bits16(to_f32(thi) + bv[2 * i + 1], (T *)nullptr);
-                w[i] = (uint32_t)lo | ((uint32_t)hi << 16);
-            }
-            v.x = w[0]; v.y = w[1]; v.z = w[2]; v.w = w[3];
-        }
-        uint16_t *dst = Y + tok * P.ldy + f;
-        if (vec_ok && f + 7 < P.O) {
-            *(u32x4 *)dst = v;
-        } else {
-            uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                if (f + i < P.O) dst[i] = (uint16_t)(w[i >> 1] >> ((i & 1) * 16));
-        }
-    }
+    static_assert(DN_OUT_ROW == FA * 64 + 16, "row of the staging area");
+    const TileOut out{P.y, P.O, P.T, P.ldy};
+    smf_store_tile<T, FA, FB>(acc, smem + wave * (64 * DN_OUT_ROW), lane, o0 + wm * 128, t0 + wn * 64, out);
 }
 
 template <typename T, int N, int M> static int launch_dense_nm(DenseParams &P, int reduce_sparse, hipStream_t s)

@@ -345,10 +345,7 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     };
 
     f32x4 acc[AB][TB];
-#pragma unroll
-    for (int i = 0; i < AB; i++)
-#pragma unroll
-        for (int t = 0; t < TB; t++) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    start_sums<T>(acc, P.ksplit > 1 ? nullptr : P.bias, lane, f0 + wave * (16 * AB), P.O);   // (slices: the sum adds it)
     auto pin_acc = [&]() {
 #pragma unroll
         for (int i = 0; i < AB; i++)
@@ -538,13 +535,14 @@ walked:
             asm volatile("s_waitcnt vmcnt(0)" : "+v"(w.a[0][0]), "+v"(w.a[0][1]), "+v"(w.a[1][0]), "+v"(w.a[1][1]) : : "memory");
         }
     }
-    asm volatile("s_barrier" ::: "memory");
+    // (no-ops: the compiler does not see that `from_acc` reads what a product may just have written)
+    asm volatile("s_barrier\n\ts_nop 15" ::: "memory");
     if (P.ksplit > 1) {
         store_partial_tile16<AB, TB>(acc, P.part + (int64_t)slice * P.T * P.part_ld, P.part_ld, lane,
                                      f0 + wave * (16 * AB), t0, P.T);
         return;
     }
-    const TileOut out{P.y, P.bias, P.O, P.T, P.ldy};
+    const TileOut out{P.y, P.O, P.T, P.ldy};
     if constexpr (CT)
         store_tile16_t<T, AB, TB>(acc, smem + wave * (AB * 16 * (TT * 2 + 16)), lane, f0 + wave * (16 * AB), t0, out);
     else

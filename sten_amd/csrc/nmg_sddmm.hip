@@ -47,15 +47,6 @@ template <> __device__ __forceinline__ uint16_t sd_bits16<__hip_bfloat16>(float 
     return __builtin_bit_cast(uint16_t, b);
 }
 
-// An accumulator, read where it is used: without this the compiler copies all 256 accumulation
-// registers to architectural ones at the end of the product loop, and spills to make room.
-__device__ __forceinline__ float sd_from_acc(float a)
-{
-    float v;
-    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
-    return v;
-}
-
 // ------------------------------------------------------------------------------- slot map
 // slot[b][q] (b = block of the sparse dim, q = line of the padded group dim, Gpad = chunks * c*g):
 // the slot s with idx[(q / cg) * nb + b][s] == q % cg.  Every line has exactly one slot per block
@@ -509,7 +500,7 @@ __global__ __launch_bounds__(256, 1) void sddmm16_kernel(SddmmParams P)
             for (int x = 0; x < 8; x++) {
                 uint16_t hh[4];
 #pragma unroll
-                for (int r = 0; r < 4; r++) hh[r] = sd_bits16<T>(sd_from_acc(acc[x][y][r]));
+                for (int r = 0; r < 4; r++) hh[r] = sd_bits16<T>(from_acc(acc[x][y][r]));
                 uint2 pk;
                 pk.x = (uint32_t)hh[0] | ((uint32_t)hh[1] << 16);
                 pk.y = (uint32_t)hh[2] | ((uint32_t)hh[3] << 16);
@@ -522,41 +513,40 @@ __global__ __launch_bounds__(256, 1) void sddmm16_kernel(SddmmParams P)
         // ---- dense product: stage [line][position] in the output type, then whole rows: a
         // wavefront stores two lines per instruction, 16 bytes per lane
         asm volatile("s_barrier" ::: "memory");   // every wavefront is done with the ring
-#pragma unroll
-        for (int y = 0; y < 8; y++)
+        auto stage = [&](auto biased_tag) {
+            constexpr bool BIASED = decltype(biased_tag)::value;
 #pragma unroll
             for (int x = 0; x < 8; x++) {
-                uint16_t hh[4];
+                const int pos = wm * 128 + x * 16 + kq * 4;
+                float bv[4];
 #pragma unroll
-                for (int r = 0; r < 4; r++) hh[r] = sd_bits16<T>(sd_from_acc(acc[x][y][r]));
-                uint2 pk;
-                pk.x = (uint32_t)hh[0] | ((uint32_t)hh[1] << 16);
-                pk.y = (uint32_t)hh[2] | ((uint32_t)hh[3] << 16);
-                const int line = wn * 128 + y * 16 + j16, pos = wm * 128 + x * 16 + kq * 4;
-                *(uint2 *)(smem + line * SD_PITCH + pos * 2) = pk;
+                for (int r = 0; r < 4; r++) bv[r] = BIASED ? bias_of<T>(P.bias, p0 + pos + r, P.S) : 0.f;
+#pragma unroll
+                for (int y = 0; y < 8; y++) {
+                    uint16_t hh[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float sum = from_acc(acc[x][y][r]);
+                        hh[r] = sd_bits16<T>(BIASED ? sum + bv[r] : sum);
+                    }
+                    uint2 pk;
+                    pk.x = (uint32_t)hh[0] | ((uint32_t)hh[1] << 16);
+                    pk.y = (uint32_t)hh[2] | ((uint32_t)hh[3] << 16);
+                    *(uint2 *)(smem + (wn * 128 + y * 16 + j16) * SD_PITCH + pos * 2) = pk;
+                }
             }
+        };
+        if (P.bias) stage(std::true_type{});
+        else stage(std::false_type{});
         __syncthreads();
         const int64_t pos = p0 + (lane & 31) * 8;
-        float bv[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) bv[e] = (P.bias && pos + e < P.S) ? to_f32(((const T *)P.bias)[pos + e]) : 0.f;
         for (int it = wave; it < 128; it += 4) {
             const int row = 2 * it + (lane >> 5);
             const int64_t line = l0 + row;
             const unsigned char *src = smem + row * SD_PITCH + (lane & 31) * 16;
-            uint2 lo = *(const uint2 *)src, hi = *(const uint2 *)(src + 8);   // (rows are 8-byte aligned)
-            if (line >= P.G || pos >= P.S) continue;                          // S % 8 == 0: a piece is whole or absent
-            uint32_t w[4] = {lo.x, lo.y, hi.x, hi.y};
-            if (P.bias) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    uint16_t a = (uint16_t)w[e], b = (uint16_t)(w[e] >> 16);
-                    a = sd_bits16<T>(to_f32(__builtin_bit_cast(T, a)) + bv[2 * e]);
-                    b = sd_bits16<T>(to_f32(__builtin_bit_cast(T, b)) + bv[2 * e + 1]);
-                    w[e] = (uint32_t)a | ((uint32_t)b << 16);
-                }
-            }
-            *(u32x4 *)((uint16_t *)P.val + line * P.ldv + pos) = u32x4{w[0], w[1], w[2], w[3]};
+            const uint2 lo = *(const uint2 *)src, hi = *(const uint2 *)(src + 8);   // (rows are 8-byte aligned)
+            if (line >= P.G || pos >= P.S) continue;                                // S % 8 == 0: a piece is whole or absent
+            *(u32x4 *)((uint16_t *)P.val + line * P.ldv + pos) = u32x4{lo.x, lo.y, hi.x, hi.y};
         }
     } else if constexpr (MODE > 8) {
         // ---- epilogue in registers, m == 8.  The lanes q even / odd round and pack their halves of
@@ -594,8 +584,8 @@ __global__ __launch_bounds__(256, 1) void sddmm16_kernel(SddmmParams P)
                     for (int qd = 0; qd < 2; qd++)
 #pragma unroll
                         for (int w = 0; w < 2; w++) {
-                            const uint16_t lo16 = sd_bits16<T>(sd_from_acc(acc[2 * xp + qd][y][2 * w]));
-                            const uint16_t hi16 = sd_bits16<T>(sd_from_acc(acc[2 * xp + qd][y][2 * w + 1]));
+                            const uint16_t lo16 = sd_bits16<T>(from_acc(acc[2 * xp + qd][y][2 * w]));
+                            const uint16_t hi16 = sd_bits16<T>(from_acc(acc[2 * xp + qd][y][2 * w + 1]));
                             d[qd * 2 + w] = (uint32_t)lo16 | ((uint32_t)hi16 << 16);
                         }
                     uint32_t blkw[4];   // positions 0,1 | 2,3 | 4,5 | 6,7 of the lane's block
@@ -664,7 +654,7 @@ __global__ __launch_bounds__(256, 1) void sddmm16_kernel(SddmmParams P)
                         const int x = xq * 4 + e;
                         uint16_t hh[4];
 #pragma unroll
-                        for (int r = 0; r < 4; r++) hh[r] = sd_bits16<T>(sd_from_acc(acc[x][y][r]));
+                        for (int r = 0; r < 4; r++) hh[r] = sd_bits16<T>(from_acc(acc[x][y][r]));
                         uint32_t lo = (uint32_t)hh[0] | ((uint32_t)hh[1] << 16);
                         uint32_t hi = (uint32_t)hh[2] | ((uint32_t)hh[3] << 16);
                         if (!INTERIOR && !line_ok) lo = hi = 0;

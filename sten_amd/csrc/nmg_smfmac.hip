@@ -435,12 +435,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
     };
 
     f32x16 acc[FB][TB];
-#pragma unroll
-    for (int i = 0; i < FB; i++)
-#pragma unroll
-        for (int j = 0; j < TB; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+    start_sums<T>(acc, P.ksplit > 1 ? nullptr : P.bias, lane, f0 + wm * FB * 32, P.M);   // (slices: the sum adds it)
 
     // 256 accumulators fill the architectural registers exactly; left alone the allocator
     // puts them all there and spills everything else.  Pin half of them to the accumulation
@@ -674,7 +669,7 @@ walked:
                                    f0 + wm * FB * 32, t0 + wn * TB * 32, P.T);
         return;
     }
-    const TileOut out{P.y, P.bias, P.M, P.T, P.ldy};
+    const TileOut out{P.y, P.M, P.T, P.ldy};
     if constexpr (CT)
         smf_store_tile_t<T, FB, TB>(acc, smem + wave * (FB * 32 * (TB * 64 + 16)), lane, f0 + wm * FB * 32,
                                     t0 + wn * TB * 32, out);

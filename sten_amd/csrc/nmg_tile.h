@@ -31,12 +31,59 @@ inline bool stagger_xcds(unsigned workgroups, int steps, int64_t operand_bytes)
     return workgroups <= 256 && steps >= 64 && operand_bytes <= (int64_t)192 << 20;
 }
 
-// Where an output tile goes: Y[T, M] row-major with leading dimension ldy, optional bias[M].
+// Where an output tile goes: Y[T, M] row-major with leading dimension ldy.
 struct TileOut {
     void *y;
-    const void *bias;
     int64_t M, T, ldy;
 };
+
+// A sum starts with its feature's bias (bias[M]; zero without one): single precision, rounded once.  Added behind the
+// rounding of the sum, as the epilogues once did, a product is rounded twice (4096^2 4:8 bf16: 2.35e-3 off in 2-norm
+// instead of 1.66e-3); added to the sums in the epilogue, in a body with a bias beside one without, the 256 x 256 tiles spill.
+// The loads have no branch each, which would make each a round trip to memory; what a feature beyond the last one gets is
+// never stored.
+template <typename T> __device__ __forceinline__ float bias_of(const void *bias, int64_t f, int64_t M)
+{
+    return to_f32(((const T *)bias)[f < M ? f : M - 1]);
+}
+
+// a lane of the 32 x 32 form holds features 8*(r/4) + 4*(l/32) + r%4 of a block
+template <typename T, int FB, int TB>
+__device__ __forceinline__ void start_sums(f32x16 (&acc)[FB][TB], const void *bias, int lane, int64_t fw, int64_t M)
+{
+    float b[FB][16] = {};
+    if (bias) {
+#pragma unroll
+        for (int fb = 0; fb < FB; fb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) b[fb][r] = bias_of<T>(bias, fw + fb * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), M);
+    }
+#pragma unroll
+    for (int fb = 0; fb < FB; fb++)
+#pragma unroll
+        for (int tb = 0; tb < TB; tb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[fb][tb][r] = b[fb][r];
+}
+
+// ... and one of the 16 x 16 form features 4*(l/16) + 0..3
+template <typename T, int AB, int TB>
+__device__ __forceinline__ void start_sums(f32x4 (&acc)[AB][TB], const void *bias, int lane, int64_t fw, int64_t M)
+{
+    float b[AB][4] = {};
+    if (bias) {
+#pragma unroll
+        for (int ab = 0; ab < AB; ab++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) b[ab][i] = bias_of<T>(bias, fw + ab * 16 + 4 * (lane >> 4) + i, M);
+    }
+#pragma unroll
+    for (int ab = 0; ab < AB; ab++)
+#pragma unroll
+        for (int tb = 0; tb < TB; tb++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[ab][tb][i] = b[ab][i];
+}
 
 // Epilogue of the pipelined kernels.  D[row = feature][col = token]; a lane holds token
 // l%32 and features 8*(r/4) + 4*(l/32) + r%4.  The wavefront's TB*32 tokens x FB*32 features are
@@ -44,8 +91,8 @@ struct TileOut {
 // lane and FB*64 B contiguous per token row.  fw / tw = first feature / token of the wavefront.
 // The caller guarantees that no load into LDS is pending.
 // Second half of the staged epilogues: NROWS token rows of FB*64 B (+16 B pad) lie in `stg`; every
-// lane moves 16 B per pass, FB*64 B contiguous per token row, adding the bias on the way.
-template <typename T, int FB, int NROWS>
+// lane moves 16 B per pass, FB*64 B contiguous per token row.
+template <int FB, int NROWS>
 __device__ __forceinline__ void store_staged_rows(const unsigned char *stg, int lane, int64_t fw, int64_t tw,
                                                   const TileOut &P)
 {
@@ -53,31 +100,15 @@ __device__ __forceinline__ void store_staged_rows(const unsigned char *stg, int 
     constexpr int CPR = FB * 4;             // 16-byte chunks per row
     constexpr int RPP = 64 / CPR;           // token rows per pass of the wavefront
     uint16_t *Y = (uint16_t *)P.y;
-    const T *bias = (const T *)P.bias;
     const bool vec_ok = (P.ldy & 7) == 0 && ((uintptr_t)P.y & 15) == 0;
     const int fc = lane % CPR;                      // 8-feature chunk of the row
     const int64_t f = fw + fc * 8;
-    float bv[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) bv[i] = (bias && f + i < P.M) ? to_f32(bias[f + i]) : 0.f;
 #pragma unroll 4
     for (int it = 0; it < NROWS / RPP; it++) {
         const int tl = it * RPP + lane / CPR;
         const int64_t tok = tw + tl;
-        u32x4 v = *(const u32x4 *)(stg + tl * ROW + fc * 16);
+        const u32x4 v = *(const u32x4 *)(stg + tl * ROW + fc * 16);
         if (tok >= P.T || f >= P.M) continue;
-        if (bias) {
-            uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint16_t lo = (uint16_t)(w[i] & 0xFFFF), hi = (uint16_t)(w[i] >> 16);
-                T tlo = *reinterpret_cast<T *>(&lo), thi = *reinterpret_cast<T *>(&hi);
-                lo = f32_to_bits16(to_f32(tlo) + bv[2 * i], (T *)nullptr);
-                hi = f32_to_bits16(to_f32(thi) + bv[2 * i + 1], (T *)nullptr);
-                w[i] = (uint32_t)lo | ((uint32_t)hi << 16);
-            }
-            v.x = w[0]; v.y = w[1]; v.z = w[2]; v.w = w[3];
-        }
         uint16_t *dst = Y + tok * P.ldy + f;
         if (vec_ok && f + 7 < P.M) {
             *(u32x4 *)dst = v;
@@ -112,7 +143,16 @@ __device__ __forceinline__ void smf_store_tile(const f32x16 (&acc)[FB][TB], unsi
                 *(uint2 *)(stg + (tb * 32 + j) * ROW + (fb * 32 + rq * 8 + h * 4) * 2) = pk;
             }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    store_staged_rows<T, FB, TB * 32>(stg, lane, fw, tw, P);
+    store_staged_rows<FB, TB * 32>(stg, lane, fw, tw, P);
+}
+
+// A sum out of its accumulation register, one read where it is used: left to the compiler all of them (256 a lane in
+// the 256 x 256 tile) are copied to the other registers at the head of the epilogue, for which some are spilled.
+__device__ __forceinline__ float from_acc(float a)
+{
+    float v;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
+    return v;
 }
 
 // The 16 x 16 form of the instruction: a lane holds token l%16 and outputs 4*(l/16) + 0..3 of every
@@ -126,29 +166,28 @@ __device__ __forceinline__ void store_tile16(const f32x4 (&acc)[AB][TB], unsigne
     const int j = lane & 15, q = lane >> 4;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int tb = 0; tb < TB; tb++)
+    for (int tb = 0; tb < TB; tb++) {
 #pragma unroll
         for (int ab = 0; ab < AB; ab++) {
             uint16_t hh[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) hh[i] = f32_to_bits16(acc[ab][tb][i], (T *)nullptr);
+            for (int i = 0; i < 4; i++) hh[i] = f32_to_bits16(from_acc(acc[ab][tb][i]), (T *)nullptr);
             uint2 pk;
             pk.x = (uint32_t)hh[0] | ((uint32_t)hh[1] << 16);
             pk.y = (uint32_t)hh[2] | ((uint32_t)hh[3] << 16);
             *(uint2 *)(stg + (tb * 16 + j) * ROW + (ab * 16 + q * 4) * 2) = pk;
         }
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    store_staged_rows<T, AB / 2, TB * 16>(stg, lane, fw, tw, P);
+    store_staged_rows<AB / 2, TB * 16>(stg, lane, fw, tw, P);
 }
 
 // The same epilogue for a transposed output, Y[M, T] row-major (tokens contiguous): the
 // wavefront's FB*32 features x TB*32 tokens are staged as [feature][token], so that a lane stores
-// 16 bytes = 8 tokens of one feature row and TB*64 bytes per row are contiguous.  The bias of a
-// feature is added to its whole row.
+// 16 bytes = 8 tokens of one feature row and TB*64 bytes per row are contiguous.
 // Second half of the transposed epilogues: NROWS output rows of TB*64 B (+16 B pad) lie in `stg`
-// as [output][token]; a lane moves 16 bytes = 8 tokens of one output row per pass.  The bias of an
-// output is added to its whole row.
-template <typename T, int TB, int NROWS>
+// as [output][token]; a lane moves 16 bytes = 8 tokens of one output row per pass.
+template <int TB, int NROWS>
 __device__ __forceinline__ void store_staged_rows_t(const unsigned char *stg, int lane, int64_t fw, int64_t tw,
                                                     const TileOut &P)
 {
@@ -156,7 +195,6 @@ __device__ __forceinline__ void store_staged_rows_t(const unsigned char *stg, in
     constexpr int CPR = TB * 4;             // 16-byte chunks per row
     constexpr int RPP = 64 / CPR;           // feature rows per pass of the wavefront
     uint16_t *Y = (uint16_t *)P.y;
-    const T *bias = (const T *)P.bias;
     const bool vec_ok = (P.ldy & 7) == 0 && ((uintptr_t)P.y & 15) == 0;
     const int tc = lane % CPR;                      // 8-token chunk of the row
     const int64_t tok = tw + tc * 8;
@@ -164,21 +202,8 @@ __device__ __forceinline__ void store_staged_rows_t(const unsigned char *stg, in
     for (int it = 0; it < NROWS / RPP; it++) {
         const int fl = it * RPP + lane / CPR;
         const int64_t f = fw + fl;
-        u32x4 v = *(const u32x4 *)(stg + fl * ROW + tc * 16);
+        const u32x4 v = *(const u32x4 *)(stg + fl * ROW + tc * 16);
         if (f >= P.M || tok >= P.T) continue;
-        if (bias) {
-            const float bv = to_f32(bias[f]);
-            uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint16_t lo = (uint16_t)(w[i] & 0xFFFF), hi = (uint16_t)(w[i] >> 16);
-                T tlo = *reinterpret_cast<T *>(&lo), thi = *reinterpret_cast<T *>(&hi);
-                lo = f32_to_bits16(to_f32(tlo) + bv, (T *)nullptr);
-                hi = f32_to_bits16(to_f32(thi) + bv, (T *)nullptr);
-                w[i] = (uint32_t)lo | ((uint32_t)hi << 16);
-            }
-            v.x = w[0]; v.y = w[1]; v.z = w[2]; v.w = w[3];
-        }
         uint16_t *dst = Y + f * P.ldy + tok;
         if (vec_ok && tok + 7 < P.T) {
             *(u32x4 *)dst = v;
@@ -208,7 +233,7 @@ __device__ __forceinline__ void smf_store_tile_t(const f32x16 (&acc)[FB][TB], un
                 *(uint16_t *)(stg + f * ROW + (tb * 32 + j) * 2) = f32_to_bits16(acc[fb][tb][r], (T *)nullptr);
             }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    store_staged_rows_t<T, TB, FB * 32>(stg, lane, fw, tw, P);
+    store_staged_rows_t<TB, FB * 32>(stg, lane, fw, tw, P);
 }
 
 // The 16 x 16 form, transposed output: AB blocks of 16 outputs x TB16 blocks of 16 tokens (an even
@@ -222,15 +247,16 @@ __device__ __forceinline__ void store_tile16_t(const f32x4 (&acc)[AB][TB16], uns
     const int j = lane & 15, q = lane >> 4;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int tb = 0; tb < TB16; tb++)
+    for (int tb = 0; tb < TB16; tb++) {
 #pragma unroll
         for (int ab = 0; ab < AB; ab++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
                 *(uint16_t *)(stg + (ab * 16 + q * 4 + r) * ROW + (tb * 16 + j) * 2) =
-                    f32_to_bits16(acc[ab][tb][r], (T *)nullptr);
+                    f32_to_bits16(from_acc(acc[ab][tb][r]), (T *)nullptr);
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    store_staged_rows_t<T, TB16 / 2, AB * 16>(stg, lane, fw, tw, P);
+    store_staged_rows_t<TB16 / 2, AB * 16>(stg, lane, fw, tw, P);
 }
 
 // ---- reductions cut into slices (products with fewer tiles than the GPU has CUs) ----

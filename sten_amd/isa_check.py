@@ -12,8 +12,9 @@ error.  This tool re-reads the device assembly the compiler produced and proves,
     instruction wrote it (the compiler keeps that distance for its own instructions only), and
   * no loop that streams operands holds scratch traffic, which would break the per-step count
     of operations the waits rely on, and no scratch load is issued while hand-issued loads are
-    outstanding: the compiler's wait for it drains them all (other spills are reported, not
-    refused),
+    outstanding: the compiler's wait for it drains them all (other spills are told apart in the
+    report and fail the check too: an epilogue that spilled blocks of accumulators was compiled so
+    that one word of a block was never put back),
 
 by simulating the in-order vector-memory counter along every kernel (loop bodies are walked again
 with the state their back edge carries, so what a loop hands to its next iteration is checked too).
@@ -148,7 +149,7 @@ notes = []
 
 
 def check_kernel(name, body):
-    """List of problems of one kernel (empty = clean); remarks that are no problems go to `notes`."""
+    """List of problems of one kernel (empty = clean); spills outside the streaming loops go to `notes`."""
     prog = parse(body)
     labels = {p[1]: i for i, p in enumerate(prog) if p[0] == "label"}
     problems = scalar_hazards(name, prog)
@@ -246,8 +247,8 @@ def check_kernel(name, body):
     walk(0, len(prog), [], False, 2)
     # Spills: a spilled register with a load in flight is caught above (the scratch operation reads
     # it).  Scratch traffic inside a loop that streams operands would also disturb the counted
-    # waits' budget of operations per step, so there it is an error; before and after the loops
-    # (a value parked across the product) it is only reported.
+    # waits' budget of operations per step, so there it is a problem of the kernel; before and after
+    # the loops (a value parked across the product) it goes to the notes.
     loops = []
     for i, (kind, payload, _) in enumerate(prog):
         if kind != "inst":
@@ -306,9 +307,9 @@ def main(argv=None):
     for p in problems:
         print(p)
     for q in sorted(set(n.split(" @")[0] for n in notes)):
-        print(f"note: {q}: spills outside the streaming loops")
-    print(f"isa_check: {total} kernels, {len(problems)} problems")
-    return 1 if problems else 0
+        print(f"{q}: spills outside the streaming loops")
+    print(f"isa_check: {total} kernels, {len(problems)} problems, {len(notes)} spills outside the loops")
+    return 1 if problems or notes else 0
 
 
 if __name__ == "__main__":
