@@ -163,7 +163,7 @@ struct DfParams {
     int64_t lda;         // ROWA: row pitch of the weight, in elements
     int KP;              // K steps of 64
     int tiles_m, tiles_n;
-    int turn;            // XCD x starts its walk of the reduction x / 8 of the way in
+    int turn;            // band b of the tiles starts its walk of the reduction b / bands of the way in
     // reduction cut into slices (0 / 1: whole): slice s of a tile stores its sums in single
     // precision at part[s][token][output], part_ld outputs per token
     int ksplit;
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     const int KPT = P.KP;
     const int kp_lo = slice * kp_per;
     const int KP = min(KPT, kp_lo + kp_per) - kp_lo;
-    const int first = P.turn ? (int)(blockIdx.x & 7) * KP / 8 : 0;
+    const int first = P.turn ? band * KP / ((P.tiles_m + GH - 1) / GH) : 0;
     const int ob0 = (int)(f0 / 32) + wave * (AB / 2);
 
     const unsigned char *av_base[AB / 2];
@@ -556,7 +556,7 @@ template <typename T, int TB, int NH, bool XT = false, bool CT = XT, bool ROWA =
     P.tiles_n = (int)((P.T + TT - 1) / TT);
     const int slices = P.ksplit > 1 ? P.ksplit : 1;
     dim3 grid((unsigned)(P.tiles_m * P.tiles_n * slices));
-    P.turn = stagger_xcds(grid.x, P.KP / slices, P.KP * (P.O + P.T) * 128) ? 1 : 0;
+    P.turn = stagger_bands(grid.x, P.KP / slices, P.KP * (P.O + P.T) * 128) ? 1 : 0;
     constexpr size_t ring = (size_t)dd_stages(AB) * TT * 128;
     constexpr size_t stg = CT ? (size_t)4 * 16 * AB * (TT * 2 + 16) : (size_t)4 * TT * (AB * 32 + 16);
     constexpr size_t lds = ring > stg ? ring : stg;

@@ -62,7 +62,7 @@ struct SmfParams {
     int MB, KP;          // feature blocks of 32, k pairs of 64
     int tiles_m, tiles_n;
     int band;            // direct kernel: line tiles per band of the tile walk (4 or 8)
-    int turn;            // direct kernel: XCD x starts its walk of the reduction x / 8 of the way in
+    int turn;            // direct kernel: band b of the tiles starts its walk of the reduction b / bands of the way in
     bool in_order;       // a tile asked for by number: sums in the order of the reduction, alike for every tile
     // direct kernel with the reduction cut into slices (0 / 1: whole): slice s of a tile writes
     // its sums in single precision to part[s][token][feature], part_ld features per token
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
     const int KPT = P.KP;
     const int kp_lo = slice * kp_per;
     const int KP = min(KPT, kp_lo + kp_per) - kp_lo;
-    const int first = P.turn ? (int)(blockIdx.x & 7) * KP / 8 : 0;
+    const int first = P.turn ? band * KP / ((P.tiles_m + GH - 1) / GH) : 0;
     const int wm = wave / WN, wn = wave % WN;
     const int mb0 = (int)(f0 / 32) + wm * FB;
 
@@ -691,7 +691,7 @@ static int launch_smfmac_direct(SmfParams &P, hipStream_t s)
     P.band = (int64_t)TT * 2 * 8 > (int64_t)TF * 9 ? 8 : 4;   // bytes per reduction position: TT * 2 against TF * 9 / 8
     const int slices = P.ksplit > 1 ? P.ksplit : 1;
     dim3 grid((unsigned)(P.tiles_m * P.tiles_n * slices));
-    P.turn = !P.in_order && stagger_xcds(grid.x, P.KP / slices, P.KP * (int64_t)(P.MB * 32 * 72 + P.T * 128)) ? 1 : 0;
+    P.turn = !P.in_order && stagger_bands(grid.x, P.KP / slices, P.KP * (int64_t)(P.MB * 32 * 72 + P.T * 128)) ? 1 : 0;
     constexpr size_t ring = (size_t)dr_stages(FB) * TT * 128;
     constexpr size_t stg = CT ? (size_t)4 * FB * 32 * (TB * 64 + 16) : (size_t)4 * TB * 32 * (FB * 64 + 16);
     constexpr size_t lds = ring > stg ? ring : stg;

@@ -20,13 +20,18 @@ __device__ __forceinline__ uint16_t f32_to_bits16(float x, __hip_bfloat16 *)
 
 // Grids of at most one workgroup per CU: all workgroups walk the reduction in step, so that the XCDs that share a weight
 // or an activation (2 and 4 of the 8 where the tiles are 16 x 16) ask memory for the same line at the same moment and all
-// wait for it.  Started x / 8 of the reduction apart, XCD by XCD, the first one to come by brings a line into the
-// memory-side cache and the others find it there.  Operands new in every pass, us: 4096 x 11008 2:4 fp16 x 2048 tokens
-// 114.5 -> 106, x 777 67 -> 60.5; its transpose on the dense cores x 512 58.5 -> 54; torch.mm 4096^2 x 2048 with both
-// gradients 183 -> 177.  Shorter walks put the XCDs a few steps apart only (21 steps of 64: 39.4 -> 42, 32 steps: 56.8 -> 59);
+// wait for it.  So every band of output tiles starts b / bands of the reduction further on: of the XCDs that share
+// activations the first one to come by brings a line into the memory-side cache and the others find it there.  The start depends
+// on the outputs alone, so that an activation row is summed in the same order wherever it stands among the tokens.  Operands
+// new in every pass, us, in step -> apart: 4096 x 11008 2:4 fp16 x 2048 tokens 115.4 -> 111.7, x 777 67.5 -> 59.8; its transpose
+// on the dense cores x 512 57.5 -> 55.6; 8192 x 4096 x 777 43.8 -> 37.7.  A start for every XCD, an eighth apart, sums equal rows
+// differently and is not faster over the range (111.8, 62.4, 55.4, 38.8; the first of them and torch.mm 4096^2 x 2048, timed alone in longer
+// runs, 3 and 1.6 % faster: 104.7 against 107.7, 175.8 against 178.6).  Starts of single output tiles 1 to 20 steps apart
+// in a band: 111.7 to 129, an XCD's workgroups no longer share lines in its L2; bands of two tiles 112.5, 59.3, 55.1, 37.4.
+// Shorter walks put the bands a few steps apart only (21 steps of 64: 39.4 -> 42, 32 steps: 56.8 -> 59);
 // operands beyond that cache of 256 MB are gone before the others come by (268 MB, dense cores, 16384 x 4096 transposed x
 // 4096: 0.5 to 0.8 % of a training step lost); and with more than one round of workgroups the XCDs drift apart by themselves.
-inline bool stagger_xcds(unsigned workgroups, int steps, int64_t operand_bytes)
+inline bool stagger_bands(unsigned workgroups, int steps, int64_t operand_bytes)
 {
     return workgroups <= 256 && steps >= 64 && operand_bytes <= (int64_t)192 << 20;
 }

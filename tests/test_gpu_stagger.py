@@ -51,3 +51,30 @@ def test_matrix_product_and_its_gradients(sd):
         assert rel_l2(to_np(y), to_np(D @ B.detach().double())) <= 1e-3
         assert rel_l2(to_np(B.grad), to_np(D.t() @ go.double())) <= 1e-3
         assert rel_l2(to_np(w.grad.wrapped_tensor.to_dense()), to_np(go.double() @ B.detach().double().t())) <= 1e-3
+
+
+def bits(t):
+    return t.contiguous().view(torch.int16)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("R,C,T,n,m,g,rd,opt", [
+    (4096, 4224, 2000, 2, 4, 16, 1, {}),                   # 256 x 128 on the sparse cores, several bands of tiles
+    (4096, 4224, 777, 2, 4, 16, 1, {}),
+    (512, 4224, 2100, 2, 4, 16, 1, {"slices": 1}),         # one band
+    (1100, 8448, 300, 2, 4, 16, 1, {"slices": 2}),
+    (2048, 4224, 2000, 4, 8, 4, 1, {}),                    # dense cores
+    (1100, 4224, 500, 4, 8, 4, 1, {"slices": 1}),
+    (4224, 2048, 600, 2, 4, 16, 0, {"slices": 1}),
+    (8448, 1100, 300, 2, 4, 16, 0, {"slices": 2}),
+])
+def test_a_row_of_activations_gives_the_same_bits_in_every_tile(R, C, T, n, m, g, rd, opt, dtype):
+    print(f"case {dtype} {R}x{C} T={T} {n}:{m}:{g} reduce_dim={rd} {opt}", flush=True)
+    w = sten.GroupedNMTensor.from_dense(seeded((R, C), dtype, seed=1).to(DEV), n, m, sparse_dim=1, group_size=g, group_dim=0)
+    w.spmm_opt.update(opt)
+    x = seeded((1, C if rd == 1 else R), dtype, seed=2).to(DEV).expand(T, -1).contiguous()
+    y = bits(sten.spmm(w, x, reduce_dim=rd))
+    assert bool((y == y[:1]).all())
+    if rd == 1:
+        c = bits(sten.spmm_tt(w, x.t().contiguous()))
+        assert bool((c == c[:, :1]).all())
