@@ -164,6 +164,7 @@ struct DfParams {
     int KP;              // K steps of 64
     int tiles_m, tiles_n;
     int turn;            // band b of the tiles starts its walk of the reduction b / bands of the way in
+    bool in_order;       // a tile asked for by number: sums in the order of the reduction, alike for every tile
     // reduction cut into slices (0 / 1: whole): slice s of a tile stores its sums in single
     // precision at part[s][token][output], part_ld outputs per token
     int ksplit;
@@ -556,7 +557,7 @@ template <typename T, int TB, int NH, bool XT = false, bool CT = XT, bool ROWA =
     P.tiles_n = (int)((P.T + TT - 1) / TT);
     const int slices = P.ksplit > 1 ? P.ksplit : 1;
     dim3 grid((unsigned)(P.tiles_m * P.tiles_n * slices));
-    P.turn = stagger_bands(grid.x, P.KP / slices, P.KP * (P.O + P.T) * 128) ? 1 : 0;
+    P.turn = !P.in_order && stagger_bands(grid.x, P.KP / slices, P.KP * (P.O + P.T) * 128) ? 1 : 0;
     constexpr size_t ring = (size_t)dd_stages(AB) * TT * 128;
     constexpr size_t stg = CT ? (size_t)4 * 16 * AB * (TT * 2 + 16) : (size_t)4 * TT * (AB * 32 + 16);
     constexpr size_t lds = ring > stg ? ring : stg;
@@ -625,6 +626,7 @@ template <typename T, bool CT = false> static int launch_dense(DfParams &P, int 
     // (A sixteen-phase form of the 256 x 256 tile on the 32 x 32 x 16 instruction once gave wrong
     // values now and then; the forms here pass the static check of their hand-tracked loads and
     // the repeated full-chip test.)
+    P.in_order = variant >= 0;
     const int tile = variant < 0 ? dense16_tile(P.ksplit > 1 ? P.ksplit : 1, P.O, P.KP, P.T) : variant;
     if (tile == DENSE_NARROW) return launch_dense16<T, 8, 2, false, CT, false, 2>(P, s);
     if (tile == DENSE_SQUARE) return launch_dense16<T, 16, 4, false, CT>(P, s);

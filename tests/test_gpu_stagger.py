@@ -78,3 +78,13 @@ def test_a_row_of_activations_gives_the_same_bits_in_every_tile(R, C, T, n, m, g
     if rd == 1:
         c = bits(sten.spmm_tt(w, x.t().contiguous()))
         assert bool((c == c[:, :1]).all())
+
+
+@pytest.mark.parametrize("n,m,g,name,variants", [(2, 4, 16, "variant", (6, 8)), (4, 8, 4, "dense_variant", (0, 1))])
+def test_tiles_asked_for_by_number_keep_the_order_of_the_reduction(n, m, g, name, variants):
+    w = sten.GroupedNMTensor.from_dense(seeded((1100, 4224), torch.float16, seed=1).to(DEV), n, m, sparse_dim=1, group_size=g, group_dim=0)
+    x, got = seeded((600, 4224), torch.float16, seed=2).to(DEV), []
+    for v in variants:
+        w.spmm_opt[name] = v
+        got.append(bits(sten.spmm(w, x, reduce_dim=1)))
+    assert torch.equal(*got)
