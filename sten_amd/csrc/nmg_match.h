@@ -15,11 +15,11 @@
 // (2:8:32), 299 of 2240 (4:8:32).
 //
 // Later rounds insert proposals into the lists lane by lane (the code says how).  4096 x 4096 2:4:16 fp16: 99 -> 58 us,
-// 8192 x 8192 2:8:32: 727 -> 201 us, 4096 x 4096 4:8:32: 390 -> 140 us.  What bounds it is the issue of vector instructions (1200 for a
+// 8192 x 8192 2:8:32: 727 -> 201 us, 4096 x 4096 4:8:32: 390 -> 123 us.  What bounds it is the issue of vector instructions (1200 for a
 // wavefront of two tiles 2:4:16, 0.74 of the time; 0.66 at 2:8:32) and, in the later rounds, chains of LDS round trips: of the 201 us,
 // tile data and results take 52, the first proposals 15, the first round 44, the later rounds 90.  A list in 16 lanes of one or two
 // keys, merged two proposals at a time, and eight lanes (2:4: two) on a column's patterns took these from 122 (whole kernel 233; 2:4:16
-// 59.3 -> 57.8, 1:8:32 43.5 -> 39.5, 4:8:32 170 -> 136, fp32 238 -> 200).  Other group sizes, 4096 x 4096
+// 59.3 -> 57.8, 1:8:32 43.5 -> 39.5, 4:8:32 170 -> 123, fp32 240 -> 191).  Other group sizes, 4096 x 4096
 // fp16 with the blocks along the contiguous / the slow dim, the batched walk -> this: 2:4:4 168 -> 116 / 231 -> 113 us, 2:4:8 115 -> 75 /
 // 146 -> 76, 2:4:32 118 -> 105 / 135 -> 116, 2:4:64 130 -> 118 / 146 -> 129, 1:4:8 99 -> 69 / 151 -> 70, 1:2:8 192 -> 147 /
 // 302 -> 145, 2:8:8 293 -> 130 / 326 -> 134, 4:8:16 870 -> 366 / 810 -> 388.  Slower than the walk is 1:4:17 (107 -> 110), and where the
@@ -830,9 +830,11 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                             bp = p;
                         }
                     };
-                    // (many patterns and more columns than one pass of the lanes takes: a column per lane, as a lone tile waits
-                    // less for it.  4:8:32 fp16, lanes of a column -> this: 1024 x 1024 22.2 -> 20.8 us, 4096 x 4096 141 -> 136, fp32 189 -> 200.)
-                    if (SG != 0 && (SC <= 32 || pend * EL <= A)) {
+                    // (Many patterns and more than twice as many columns as lanes: a column per lane is as much work without the exchange
+                    // between lanes.  With fewer its last pass leaves most lanes idle: a lone tile of 2240 real columns, 4:8:32, has 300
+                    // of them.  us, a column per lane from A / EL columns on -> from 2 A on: 2240 x 1024 fp16 61 -> 53, 4096 x 4096 fp16 133 -> 123,
+                    // fp32 209 -> 191; 1024 x 1024, with few pending columns, 20.5 either way.)
+                    if (SG != 0 && (SC <= 32 || pend <= 2 * A)) {
                         const int sub = tt % EL;
                         for (int e = tt / EL; e < pend; e += A / EL) {
                             const int o = (int)pending[e];
