@@ -275,12 +275,13 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
         s_last[p] = before + size - 1;
     }
     // Few patterns, or few that agree: one by one, which reads half as much per sum (us, one by one against by classes: 1000 x 1001
-    // 2:4:16 fp16 26.0, 27.4; 1536 x 2157 2:5:8 bf16, 4 classes of 10, 51, 54; x 2176 3:6:12, 14 of 20, 62, 70; x 2163, 8 of 20, 69, 72,
-    // fp32 69, 66; x 2162, 4 of 20, 62, 60).
+    // 2:4:16 fp16 26.0, 27.4; 1536 x 2157 2:5:8 bf16, 4 classes of 10, 51, 54; x 2176 3:6:12, 14 of 20, 58, 66, 4 of 20, 60, 58; 2:8:32,
+    // 16 of 28, 143, 135, 22 of 28, 143, 150).  Where half of a block and more is kept, so that most columns turn to few classes, also
+    // below 13 patterns fewer: 3:6:12, 8 of 20, bf16 65, 70, fp16 64, 66; 6:8:16, 16 of 28, 105, 112.
     if (c > 15) {
         match_sync<NT>();
         for (int q = 0; q < c; q++) classes += s_at[q] == s_last[q] ? 1 : 0;
-        if (3 * classes > 2 * c) classes = 0;
+        if (3 * classes > 2 * c || (2 * __popc(s_mask[0]) >= m && c - classes < 13)) classes = 0;
         for (int p = tt; p < c; p += NT)
             if (classes > 0 && s_at[p] == s_last[p]) {
                 int k = 0;
