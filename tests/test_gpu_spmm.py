@@ -283,7 +283,7 @@ def test_spmm_sparse_matrix_cores(variant, dtype, M, K, T, n, m, g):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,K,T,n,m,g,slices", [
-    (512, 1152, 40, 2, 4, 16, None),     # planned: 2 tiles, 18 K steps -> 2 slices
+    (512, 1152, 40, 2, 4, 16, None),     # planned: 18 K steps in 4 slices of 5, 5, 5 and 3
     (512, 1152, 129, 2, 4, 16, 3),       # two token tiles, uneven slices (6 + 6 + 6)
     (1000, 2048, 200, 2, 4, 8, 7),       # ragged lines and tokens, slices of 5, 5, ..., 2
     (300, 704, 17, 1, 4, 4, 11),         # one K step per slice
@@ -298,7 +298,7 @@ def test_split_reduction_matches_dense(dtype, M, K, T, n, m, g, slices):
         w.spmm_opt["slices"] = slices
     else:
         planned, ws = ctypes.c_int(0), ctypes.c_int64(0)
-        assert native.load().nmg_splitk_plan(M, K, T, ctypes.byref(planned), ctypes.byref(ws)) == 0
+        assert native.load().nmg_smfmac_plan(M, K, T, ctypes.byref(planned), ctypes.byref(ws)) == 0
         assert planned.value > 1 and ws.value == planned.value * T * ((M + 255) // 256) * 256 * 4
     x = seeded((T, K), dtype, seed=1)
     b = seeded((M,), dtype, seed=2)
@@ -306,6 +306,9 @@ def test_split_reduction_matches_dense(dtype, M, K, T, n, m, g, slices):
         y = sten.spmm(w, x.to(DEV), bias, reduce_dim=1)
         ref = to_np(x).astype(np.float64) @ Wd.T + (0 if bias is None else to_np(b).astype(np.float64))
         assert rel_l2(to_np(y), ref) <= TOL[dtype]
+    if slices is None:                            # the plan is what the product takes
+        w.spmm_opt["slices"] = planned.value
+        assert torch.equal(sten.spmm(w, x.to(DEV), b.to(DEV), reduce_dim=1), y)
     w.spmm_opt["slices"] = 1                      # the same product on whole reductions
     y1 = sten.spmm(w, x.to(DEV), b.to(DEV), reduce_dim=1)
     assert rel_l2(to_np(y), to_np(y1)) <= 2 * TOL[dtype]
@@ -328,12 +331,15 @@ def test_split_reduction_dense_route(dtype, M, K, T, n, m, g, rd, slices):
         w.spmm_opt["slices"] = slices
     else:
         planned, ws = ctypes.c_int(0), ctypes.c_int64(0)
-        assert native.load().nmg_splitk_plan(Oo, R, T, ctypes.byref(planned), ctypes.byref(ws)) == 0
-        assert planned.value > 1
+        assert native.load().nmg_densefrag_plan(Oo, R, T, ctypes.byref(planned), ctypes.byref(ws)) == 0
+        assert planned.value > 1 and ws.value == planned.value * T * ((Oo + 255) // 256) * 256 * 4
     x = seeded((T, R), dtype, seed=1)
     y = sten.spmm(w, x.to(DEV), reduce_dim=rd, kernel="densefrag")
     ref = to_np(x).astype(np.float64) @ (Wd.T if rd == 1 else Wd)
     assert rel_l2(to_np(y), ref) <= TOL[dtype]
+    if slices is None:
+        w.spmm_opt["slices"] = planned.value
+        assert torch.equal(sten.spmm(w, x.to(DEV), reduce_dim=rd, kernel="densefrag"), y)
     w.spmm_opt["slices"] = 1
     y1 = sten.spmm(w, x.to(DEV), reduce_dim=rd, kernel="densefrag")
     assert rel_l2(to_np(y), to_np(y1)) <= 2 * TOL[dtype]
