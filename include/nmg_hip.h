@@ -105,7 +105,8 @@ int nmg_rowpack_expand(const void *d_pk_val, const void *d_pk_pat, int64_t G, in
 /* Y[T, G] = X[T, S] * W2^T      (reduce_sparse = 1)   W2 = the [G, S] weight view
  * Y[T, S] = X[T, G] * W2        (reduce_sparse = 0)
  * X, Y row-major with leading dimensions ldx, ldy (elements).  X/Y/pk_val share `dtype`
- * (F32, F16 or BF16); accumulation is fp32.  `bias` (length = output features, same dtype) may be
+ * (F32, F16 or BF16); accumulation is fp32, the bias
+ * included, and a 16-bit result is rounded once (so in every product below).  `bias` (length = output features, same dtype) may be
  * NULL.  `kernel` is one of NMG_KERNEL_*.
  * Replaces: `__program_<name>(state, A_idx, A_val, B, C, groups)` produced by
  * dace_gnm_mult.py:572-1007 and called from sten_impls.py:111-138, plus the bias add of

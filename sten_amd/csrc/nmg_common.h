@@ -90,7 +90,8 @@ __device__ __forceinline__ float to_f32(__hip_bfloat16 x) { return __bfloat162fl
 // (of tiles / 8, the first tiles % 8 of them one more), which the caller's walk makes a compact block whose operands stay in that
 // XCD's L2.  Against leaving counts that are no multiple of 8 in the order of the ids, neighbours on different XCDs, us: 2:4
 // 11008 x 4096 x 6000 tokens (2021 tiles) 422 -> 312, 2176 x 4096 x 9000 163 -> 113, 1640 x 1920 x 3500 23.5 -> 18.9; 4:8
-// 11008 x 4096 x 6000 484 -> 412; few tiles in slices 0.86 to 1.05 of the time.
+// 11008 x 4096 x 6000 484 -> 412; of 242 products of 33 to 1024 tokens the fastest 0.71, the slowest 1.03 of the time (2:4 2304 x 4096
+// x 384, four slices of 16 steps, 17.5 -> 18.0).
 __device__ __forceinline__ int xcd_run(int id, int tiles)
 {
     const int xcd = id & 7;

@@ -237,9 +237,9 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
     // a compact block of tiles whose weights and activations stay in that XCD's L2.
     int id = blockIdx.x;
     const int ntiles = P.tiles_m * P.tiles_n;
-    // Slices of the reduction: an XCD's run goes over slices and tiles, so that few XCDs fetch the same operands (us, against runs of tiles
-    // within every slice: 2:4 4096 x 11008 x 200 tokens 30.1 -> 25.1, 1024 x 16384 x 777 37 -> 28.7; 4:8 x 300 29.0 -> 20.3); but in short
-    // slices an XCD's workgroups wait for the same lines (2:4 2048 x 8192 x 128, 16 steps a slice, 14.7 -> 16.8).
+    // Slices of the reduction: an XCD's run goes over slices and tiles, so that few XCDs fetch the same operands (us, weights from memory,
+    // against runs of tiles within every slice: 2:4 4096 x 11008 x 200 tokens 34.3 -> 33.2, 1024 x 16384 x 777 38.7 -> 35.4; 4:8 x 300 30.4 -> 27.8);
+    // but in short slices an XCD's workgroups wait for the same lines (2:4 2048 x 8192 x 128, 16 steps a slice, 17.3 -> 19.3).
     const int kp_per = P.ksplit > 1 ? (P.KP + P.ksplit - 1) / P.ksplit : P.KP;
     int slice = 0;
     if (kp_per >= 20) {
@@ -591,9 +591,13 @@ static inline int64_t dense16_tiles(int tile, int64_t O, int64_t T)
 
 // Time in us of a product whose reduction of `steps` K steps is cut into `slices`, one workgroup per CU: whole rounds of 256
 // workgroups and a last one that is the faster the fewer it has, a step and a fixed part per round; with slices the second kernel and
-// the partial sums, written and read once; and the weight comes from memory in any case.  The constants are those of 17 weights
-// of 512^2 to 16384 x 2048 and 1024 x 16384 with 17 to 6000 tokens in 1 to 16 slices (fp16 4:8, weights new in every pass), 9 % off in
-// the mean; what it chooses is 1 % behind the best of those measured.
+// the partial sums, written and read once; and the weight comes from memory in any case (fitted without
+// the term of smfmac_cost for the narrow tile's fetches).  The constants are those of 17 weights
+// of 512^2 to 16384 x 2048 and 1024 x 16384 with 17 to 6000 tokens in 1 to 16 slices (fp16 4:8, weights new in every pass), fitted before the
+// slices' workgroups were dealt out by XCD.  Against the best of every tile and slice as the kernels are now, 16 weights x 33 to 4096 tokens:
+// 1.6 % behind in the mean, 3 % and more in 47 of 224 (8192 x 1024 x 4096 72.0, 57.7; 512 x 16384 x 450 25.3, 21.9), and 2.1 % for 8 weights
+// that no fit has seen (profiles/tile_slice_sweep.txt).  Row operands keep a rule of their own (dense16_square): the product of
+// rows has the square tile only, against another kernel.
 static double dense16_cost(int tile, int slices, int64_t O, int64_t steps, int64_t T)
 {
     static const struct { double step, fixed, crowd; } of[] = {{0.54, 4.3, 0.44}, {0.89, 11.0, 0.49}, {0.30, 3.8, 0.63}};

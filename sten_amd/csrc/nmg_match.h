@@ -873,7 +873,8 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                         }
                     }
                     match_sync<A>();
-                    // a pattern's proposals into its list, AT at a time
+                    // a pattern's proposals into its list, AT at a time (compiled patterns: two, their buckets hold an even number; any
+                    // other n:m:g may have an odd one and takes one at a time, two were not tried for it)
                     auto merge = [&](int p) {
                         constexpr int AT = SG != 0 ? 2 : 1;
                         static_assert(SG == 0 || (SG / 2 < 8 ? SG / 2 : 8) % AT == 0, "whole batches");

@@ -323,9 +323,9 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
 
     int id = blockIdx.x;
     const int ntiles = P.tiles_m * P.tiles_n;
-    // Slices of the reduction: an XCD's run goes over slices and tiles, so that few XCDs fetch the same operands (us, against runs of tiles
-    // within every slice: 2:4 4096 x 11008 x 200 tokens 30.1 -> 25.1, 1024 x 16384 x 777 37 -> 28.7; 4:8 x 300 29.0 -> 20.3); but in short
-    // slices an XCD's workgroups wait for the same lines (2:4 2048 x 8192 x 128, 16 steps a slice, 14.7 -> 16.8).
+    // Slices of the reduction: an XCD's run goes over slices and tiles, so that few XCDs fetch the same operands (us, weights from memory,
+    // against runs of tiles within every slice: 2:4 4096 x 11008 x 200 tokens 34.3 -> 33.2, 1024 x 16384 x 777 38.7 -> 35.4; 4:8 x 300 30.4 -> 27.8);
+    // but in short slices an XCD's workgroups wait for the same lines (2:4 2048 x 8192 x 128, 16 steps a slice, 17.3 -> 19.3).
     const int kp_per = P.ksplit > 1 ? (P.KP + P.ksplit - 1) / P.ksplit : P.KP;
     int slice = 0;
     if (kp_per >= 20) {
@@ -1190,9 +1190,14 @@ static int launch_smfmac_cfg(SmfParams &P, hipStream_t s)
 // Time in us of a product on tiles of 256 x 128 or, narrow, 128 x 128, its reduction of `steps` K steps cut into `slices`, one
 // workgroup per CU: whole rounds of 256 workgroups and a last one that is the faster the fewer it has, a step and a fixed part per
 // round; with slices the second kernel and the partial sums, written and read once.  A narrow step is bound by its LDS reads, which are
-// those of a wide one, and it fetches twice the bytes per flop, which tells where the operands are large.  The constants are
+// those of a wide one, and it fetches twice the bytes per flop, which tells where the operands are large: the last term, in the
+// narrow tile's bytes as fitted.  The weight's time from memory has no term of its own here, as it has in dense16_cost: the sparse operand is
+// half of the dense one, and a term for it came out as zero.  The constants are
 // those of 8 weights of 512^2 to 16384 x 2048 and 4096 x 11008 with 17 to 6000 tokens in 1 to 16 slices (fp16 2:4, weights new in
-// every pass), 9 % off in the mean; what it chooses is 1 % behind the best of those measured.
+// every pass; other patterns and bf16 take the same bytes and instructions), fitted before the slices' workgroups were dealt out by XCD.
+// Against the best of every tile and slice as the kernels are now, 16 weights x 33 to 4096 tokens: 1.3 % behind in the mean, 3 % and more
+// in 26 of 224 (768 x 3072 x 3000 23.3, 18.6; 4096 x 11008 x 128 28.9, 24.5), and 1.6 % for 8 weights that no fit has seen
+// (profiles/tile_slice_sweep.txt).
 static double smfmac_cost(bool narrow, int slices, int64_t M, int64_t steps, int64_t T)
 {
     const int64_t groups = (narrow ? (M + 127) / 128 : (M + 255) / 256) * ((T + 127) / 128) * slices, rest = groups % 256;
