@@ -212,9 +212,9 @@ int nmg_spmm_smfmac_splitk_noalloc(const void *d_fp_val, const void *d_fp_idx, i
  * patterns the sparse matrix cores cannot take, where it runs at the dense library's speed.
  * dtype F16 / BF16: K % 64 == 0, rows 16-byte aligned, operands < 2 GiB.
  * dtype F32: any K > 0 and any row pitch, on V_MFMA_F32_32X32X2_F32 or, products of many tiles, on the
- * bf16 matrix cores with every number in three parts (no larger an error against 64 bits; results
- * that are not finite or as a whole below 2^-64 are computed on the fp32 instruction); nmg_gemm_nn and
- * nmg_gemm_tn too.  It is what single-precision products run on, after nmg_to_dense.
+ * bf16 matrix cores with every number in three parts (no larger an error against 64 bits, for numbers of
+ * any size; what operands beyond 2^104 or sums beyond 2^80 are part of is computed on the fp32 instruction);
+ * nmg_gemm_nn and nmg_gemm_tn too.  It is what single-precision products run on, after nmg_to_dense.
  * No counterpart in the reference (its nmg path has no backward, sten.py:1690-1693). */
 int nmg_gemm_nt(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy,
                 const void *d_bias, int64_t O, int64_t K, int64_t T, int dtype, void *stream);

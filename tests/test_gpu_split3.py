@@ -77,3 +77,36 @@ def test_zeros(form):
     (x if form != "tn" else x.t())[1000:] = 0.0
     y = product(form, a, x)
     assert float(y[1000:].abs().max()) == 0.0 and float(y[:1000].abs().min(1).values.max()) > 0.0
+
+
+@pytest.mark.parametrize("form", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("e", [-100, -108, -114, -120, -126, -140])
+def test_small_rows_among_ordinary_ones(form, e):
+    # a few rows of small numbers on either side, in tiles whose other sums are of ordinary size: every row for itself
+    print(f"case {form} 2^{e}", flush=True)
+    O, K, T = 2048, 1024, 2048
+    a, x = operands(form, O, K, T)
+    rows_a, rows_x = (a if form == "nt" else a.t()), (x if form != "tn" else x.t())
+    small = torch.tensor([3, 200, 2047], device=DEV)
+    rows_a[small] = (rows_a[small].double() * 2.0 ** e).float()
+    rows_x[small] = (rows_x[small].double() * 2.0 ** e).float()
+    y, want = product(form, a, x).double(), exact(form, a, x)
+    # K / 2 roundings at the most as above, and half a unit of the smallest fp32 number (2^-149) for every sum
+    unit = 2.0 ** -150
+    for got, w in ((y, want), (y.t(), want.t())):
+        others = torch.ones(got.shape[1], dtype=torch.bool, device=DEV)
+        others[small] = False
+        got, w = got[:, others], w[:, others]      # (small times small: below every fp32 number)
+        off = ((got - w).norm(dim=1) - unit * w.shape[1] ** 0.5).clamp_min(0) / w.norm(dim=1)
+        assert float(off.max()) <= 1e-6
+    assert float(y[small][:, small].abs().max()) <= 2.0 ** (2 * e + 10)
+
+
+@pytest.mark.parametrize("form", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("ea,ex", [(80, -118), (-118, 80), (90, -120), (100, -126), (104, -126)])
+def test_small_numbers_times_large_ones(form, ea, ex):
+    print(f"case {form} 2^{ea} 2^{ex}", flush=True)
+    a, x = operands(form, 2048, 1024, 2048)
+    a, x = (a.double() * 2.0 ** ea).float(), (x.double() * 2.0 ** ex).float()
+    y, want = product(form, a, x), exact(form, a, x)
+    assert float((y.double() - want).norm() / want.norm()) <= 1e-6      # as above
