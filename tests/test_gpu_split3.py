@@ -110,3 +110,24 @@ def test_small_numbers_times_large_ones(form, ea, ex):
     a, x = (a.double() * 2.0 ** ea).float(), (x.double() * 2.0 ** ex).float()
     y, want = product(form, a, x), exact(form, a, x)
     assert float((y.double() - want).norm() / want.norm()) <= 1e-6      # as above
+
+
+@pytest.mark.parametrize("form", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 2.0 ** 110, -3.0 * 2.0 ** 122])
+def test_numbers_that_have_no_parts_in_single_rows(form, value):
+    # one such number in one row of a block of 64, at every place of a row in its 32: whichever sums of a lane they reach
+    print(f"case {form} {value}", flush=True)
+    O, K, T = 2048, 1024, 2048
+    for weights in (True, False):
+        a, x = operands(form, O, K, T)
+        rows = torch.arange(32, device=DEV) * 65
+        ((a if form == "nt" else a.t()) if weights else (x if form != "tn" else x.t()))[rows, 9] = value
+        y, want = product(form, a, x), exact(form, a, x)
+        assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(torch.isinf(y), torch.isinf(want.float()))
+        y, want = (y.t(), want.t()) if weights else (y, want)
+        for got, w in zip((y[rows], y), (want[rows], want)):
+            ok = torch.isfinite(w) & torch.isfinite(w.float())
+            if got is y:
+                ok[rows] = False
+            if bool(ok.any()):      # K / 2 roundings, as above
+                assert float((got[ok].double() - w[ok]).norm() / w[ok].norm()) <= 1e-6
