@@ -131,3 +131,26 @@ def test_numbers_that_have_no_parts_in_single_rows(form, value):
                 ok[rows] = False
             if bool(ok.any()):      # K / 2 roundings, as above
                 assert float((got[ok].double() - w[ok]).norm() / w[ok].norm()) <= 1e-6
+
+
+@pytest.mark.parametrize("form", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 2.0 ** 110])
+def test_equal_rows_have_equal_sums(form, value):
+    # equal rows of either operand, some in tiles that hold a number without parts, some in tiles of ordinary numbers only
+    print(f"case {form} {value}", flush=True)
+    O, K, T = 2048, 1024, 2048
+    a, x = operands(form, O, K, T)
+    rows_a, rows_x = (a if form == "nt" else a.t()), (x if form != "tn" else x.t())
+    same = torch.tensor([1, 100, 130, 700, 1500, 2046], device=DEV)
+    rows_a[same], rows_x[same] = rows_a[1].clone(), rows_x[1].clone()
+    plain = product(form, a, x)
+    rows_x[5, 7] = value
+    rows_a[1490, 9] = value
+    y = product(form, a, x)
+    others = torch.ones(2048, dtype=torch.bool, device=DEV)
+    others[1490] = False
+    assert torch.equal(y[same][:, others], y[1, others].expand(len(same), -1))
+    others[1490], others[5] = True, False
+    assert torch.equal(y[others][:, same], y[others][:, 1:2].expand(-1, len(same)))
+    others[1490] = False
+    assert torch.equal(y[others][:, others], plain[others][:, others])      # (rows 5 and 1490 of either operand left out)
