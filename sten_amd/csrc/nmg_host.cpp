@@ -467,7 +467,7 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
     if (x.dim() != 2 || x.size(1) != K) fail("activations must be [tokens, ", K, "], got ", shape_text(x));
     c10::DeviceGuard device(x.device());
     at::AutoDispatchBelowADInplaceOrView raw;
-    if (x.stride(1) != 1) x = x.contiguous();
+    if (x.stride(1) != 1 || !rows_lie(x)) x = x.contiguous();      // (the kernels take no rows that share memory)
     const int64_t T = x.size(0);
     const int64_t ldx = T > 1 ? x.stride(0) : K;      // the stride of a dim of extent 1 means nothing
     Tensor y = new_empty({T, O}, x);
