@@ -167,7 +167,6 @@ struct DfParams {
     int64_t lda;         // ROWA: row pitch of the weight, in elements
     int KP;              // K steps of 64
     int tiles_m, tiles_n;
-    int tail;            // reduction positions of the last K step where they are fewer than 64 (multiple of 8), else 0
     int turn;            // band b of the tiles starts its walk of the reduction b / bands of the way in
     bool in_order;       // a tile asked for by number: sums in the order of the reduction, alike for every tile
     // reduction cut into slices (0 / 1: whole): slice s of a tile stores its sums in single
@@ -175,6 +174,7 @@ struct DfParams {
     int ksplit;
     float *part;
     int64_t part_ld;
+    int tail;            // reduction positions of the last K step where they are fewer than 64 (multiple of 8), else 0
 };
 
 // K steps in flight and activation stages in LDS (>= steps + 1), by the blocks of 16 outputs of a wavefront: a step of four blocks takes

@@ -62,7 +62,6 @@ struct SmfParams {
     int MB, KP;          // feature blocks of 32, k pairs of 64
     int tiles_m, tiles_n;
     int band;            // direct kernel: line tiles per band of the tile walk (4 or 8)
-    int tail;            // direct kernel: reduction positions of the last K step where they are fewer than 64 (multiple of 8), else 0
     int turn;            // direct kernel: band b of the tiles starts its walk of the reduction b / bands of the way in
     bool in_order;       // a tile asked for by number: sums in the order of the reduction, alike for every tile
     // direct kernel with the reduction cut into slices (0 / 1: whole): slice s of a tile writes
@@ -70,6 +69,7 @@ struct SmfParams {
     int ksplit;
     float *part;
     int64_t part_ld;
+    int tail;            // direct kernel: reduction positions of the last K step where they are fewer than 64 (multiple of 8), else 0
 };
 
 constexpr int SMF_ROW = 144;  // bytes per token row in LDS: 64 k * 2 B + 16 B pad (conflict-free b128 reads)
