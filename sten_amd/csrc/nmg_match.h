@@ -86,6 +86,7 @@ struct MatchParams {
     int unit;                                  // bytes of one load of the tile data (16, 8, 4, or one element)
     int out4;                                  // four slots per thread on the way out
     int lanes_log2;                            // lanes that hold a pattern's list in the later rounds; 0: no such rounds
+    int listed;                                // a partial block's refused columns have a list of their own in LDS
     uint32_t masks[32];                        // position mask of every pattern, four per word
     uint64_t magic_cols, magic_g;
 };
@@ -270,10 +271,10 @@ template <int NT, int KPT> __device__ __forceinline__ void match_sort(uint64_t *
 
 template <typename T, int NT, int KPT, int SN, int SM, int SG>
 __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, int r_int, int c, int m, int g, int so, int sr,
-                                           int real_cols, int real_rows, int few)
+                                           int real_cols, int real_rows, int few, int listed)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    for (int *x : {&region_at, &r_mem, &r_arr, &r_int, &c, &m, &g, &so, &sr, &real_cols, &real_rows, &few})
+    for (int *x : {&region_at, &r_mem, &r_arr, &r_int, &c, &m, &g, &so, &sr, &real_cols, &real_rows, &few, &listed})
         *x = __builtin_amdgcn_readfirstlane(*x);      // (arguments come in vector registers)
     const uint32_t *s_mask = (const uint32_t *)smem + c;
     const T *s_d = (const T *)(smem + region_at);
@@ -287,7 +288,7 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
     auto column = [](uint64_t key) { return (int)((key >> 1) & 0x7FFFu); };
     int *s_class = s_np + 4;                                   // smallest pattern of every class
     uint64_t *s_least = (uint64_t *)(s_class + ((c + 1) & ~1));    // least last key of a class's patterns, without the pattern
-    uint16_t *s_ref = (uint16_t *)(s_least + c);      // KPT > 1: where in s_arr the refused ones are
+    uint16_t *s_ref = (uint16_t *)(s_least + c);      // where in s_arr the refused ones are, if `listed`
     int classes = 0;
     constexpr uint64_t EDGE = 0xFFFFFFFFFFFFull;      // score and column of a key
     auto propose = [&](int o, uint32_t at_score, int below) -> uint64_t {      // at that score only patterns up to `below`
@@ -468,7 +469,7 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
             if (r == g - 1) s_mem[p * g + g - 1] = key;
             if (r >= g) {
                 const int nr = atomicAdd(s_np, 1);
-                if (KPT > 1) s_ref[nr] = (uint16_t)e;
+                if (KPT > 1 && listed) s_ref[nr] = (uint16_t)e;
                 if (key & 1) atomicMin(&s_occ[p], e);
             }
         }
@@ -482,8 +483,8 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
         }
         match_sync<NT>();
         if (left <= few) break;
-        for (int i = tt; i < (KPT > 1 ? left : real_cols); i += NT) {
-            const int e = KPT > 1 ? (int)s_ref[i] : i;
+        for (int i = tt; i < (KPT > 1 && listed ? left : real_cols); i += NT) {
+            const int e = KPT > 1 && listed ? (int)s_ref[i] : i;
             const uint64_t key = s_arr[e];
             if (key == 0) continue;
             const int p = match_pattern(key), r = e - s_start[p];
@@ -707,7 +708,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
             // (what is left for the lists: a refused column tries there the patterns of a class one by one.  Up to a quarter
             // of the columns, 3:6:12 1003 x 2001 fp32 45.3 -> 45.0 us, 512 x 1792 46.8 -> 39.5; but 2:8:32 1005 x 5000 74 -> 92)
             match_partial<T, THREADS, KPT, SN, SM, SG>(head_bytes + tm * Q.region_bytes, Q.r_mem, Q.r_arr, Q.r_int, c, m, g, RC ? 1 : m,
-                                                       RC ? ldc : 1, there, (int)(Q.view.S - mb * m), there / (c <= 20 ? 4 : 8));
+                                                       RC ? ldc : 1, there, (int)(Q.view.S - mb * m), there / (c <= 20 ? 4 : 8), Q.listed);
         }
     auto group_of = [&](int s) { return SG ? s / SG : (int)(((uint64_t)s * Q.magic_g) >> 32); };
     auto at = [&](int o, int r) { return RC ? r * ldc + o : o * m + r; };
@@ -1227,13 +1228,19 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     off += cols * 8 + kMatchPad;
     Q.r_int = off;
     off = up(off + (kMatchTables * c + 4) * 4, 16);
-    if (Q.view.S % m != 0) off = up(off + ((c + 1) & ~1) * 4 + c * 8 + (match_keys(NT, CPT) > 1 ? cols * 2 : 0), 16);      // the classes of a partial block, its refused columns
+    constexpr int LDS = 160 * 1024;
+    const int head = up(c * 8, 16);
+    if (Q.view.S % m != 0) {      // the classes of a partial block, and a list of its refused columns where the tile leaves room for it
+        off = up(off + ((c + 1) & ~1) * 4 + c * 8, 16);
+        Q.listed = match_keys(NT, CPT) > 1 && head + TILES * up(off + cols * 2, 16) <= LDS;
+        if (Q.listed) off = up(off + cols * 2, 16);
+    }
     // the tiles of a wavefront run the same offsets of their regions: spread them over the banks
     if (NT < 64)
         while (off % 256 != (NT == 16 ? 64 : 128)) off += 16;
     Q.region_bytes = off;
-    const size_t lds = (size_t)up(c * 8, 16) + (size_t)TILES * off;
-    if (lds > 160 * 1024) return NMG_OK;
+    const size_t lds = (size_t)head + (size_t)TILES * off;
+    if (lds > LDS) return NMG_OK;
     // Two wavefronts per tile where every CU gets eight tiles and their data fits beside each other, else four: us with two /
     // four, 4096 x 4096 fp16 2:4:64 118 / 157 and 2:8:16 130 / 135, the latter in fp32 (22 KB a tile) 162 / 137;
     // 777 x 1001 fp16 2:4:64 (750 tiles) 52 / 39, 2:8:16 85 / 56.

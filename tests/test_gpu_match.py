@@ -142,3 +142,19 @@ def test_partial_blocks_of_any_number_of_columns(n, m, g, columns, dtype):
         t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=1, group_size=g, group_dim=0)
         assert np.array_equal(to_np(t.idx), idx)
         assert same_bits(t.val, val)
+
+
+@pytest.mark.parametrize("n,m,g", [(4, 8, 45), (4, 8, 46), (4, 8, 47), (3, 8, 58), (3, 8, 59)])
+@pytest.mark.parametrize("along", [0, 1])
+def test_largest_tiles_with_a_partial_block(n, m, g, along):
+    # single precision: but for 4:8:45 the tile leaves no room in LDS for a list of a partial block's refused columns, and no other
+    # compressor takes a tile of this size
+    cols = math.comb(m, n) * g
+    gen = torch.Generator().manual_seed(g)
+    w = torch.randn(cols, 2 * m + 5, generator=gen) * 0.02
+    w = w if along == 1 else w.t().contiguous()
+    print(f"case {n}:{m}:{g} along={along}", flush=True)
+    val, idx, _ = oracle_sparsify(w, n, m, along, g, 1 - along)
+    t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
+    assert np.array_equal(to_np(t.idx), idx)
+    assert same_bits(t.val, val)
