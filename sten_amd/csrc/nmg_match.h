@@ -283,12 +283,13 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
     int *s_list = s_occ + c, *s_at = s_list + c, *s_last = s_at + c, *s_np = s_last + c;      // the classes, largest patterns first
     if (SG != 0) g = SG;
     if (SM != 0) m = SM;
+    const bool lists = KPT > 1 && (SG != 0 || listed);      // (tiles of the compiled group sizes have room for the list)
     if (SM != 0 && SN != 0) c = match_binom(SM ? SM : 1, SN);
     const int tt = threadIdx.x % NT, real_mask = (1 << real_rows) - 1;
     auto column = [](uint64_t key) { return (int)((key >> 1) & 0x7FFFu); };
     int *s_class = s_np + 4;                                   // smallest pattern of every class
     uint64_t *s_least = (uint64_t *)(s_class + ((c + 1) & ~1));    // least last key of a class's patterns, without the pattern
-    uint16_t *s_ref = (uint16_t *)(s_least + c);      // where in s_arr the refused ones are, if `listed`
+    uint16_t *s_ref = (uint16_t *)(s_least + c);      // where in s_arr the refused ones are, if there is room (`lists`)
     int classes = 0;
     constexpr uint64_t EDGE = 0xFFFFFFFFFFFFull;      // score and column of a key
     auto propose = [&](int o, uint32_t at_score, int below) -> uint64_t {      // at that score only patterns up to `below`
@@ -469,7 +470,7 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
             if (r == g - 1) s_mem[p * g + g - 1] = key;
             if (r >= g) {
                 const int nr = atomicAdd(s_np, 1);
-                if (KPT > 1 && listed) s_ref[nr] = (uint16_t)e;
+                if (lists) s_ref[nr] = (uint16_t)e;
                 if (key & 1) atomicMin(&s_occ[p], e);
             }
         }
@@ -483,8 +484,8 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
         }
         match_sync<NT>();
         if (left <= few) break;
-        for (int i = tt; i < (KPT > 1 && listed ? left : real_cols); i += NT) {
-            const int e = KPT > 1 && listed ? (int)s_ref[i] : i;
+        for (int i = tt; i < (lists ? left : real_cols); i += NT) {
+            const int e = lists ? (int)s_ref[i] : i;
             const uint64_t key = s_arr[e];
             if (key == 0) continue;
             const int p = match_pattern(key), r = e - s_start[p];
