@@ -788,11 +788,15 @@ static double dense16_best(int64_t O, int64_t steps, int64_t T, int *slices)
 // by both models.  us, direct kernel in slices and their sum -> this, weights from memory: 512 x 1024, 16 tokens 7.1 -> 3.6, 640 x 1408, 1
 // 7.2 -> 3.2, 2048^2, 8 7.9 -> 4.2, 32 8.6 -> 4.8, 4096^2, 16 14.6 -> 10.1, 10624 x 1664, 8 14.5 -> 9.0, 8192^2, 16 30.2 -> 25.2;
 // long reductions of few outputs stay: 888 x 8128, 16 11.0, 15.3.
+static bool few_takes(int64_t O, int64_t K, int64_t T) { return T <= 64 && O > 0 && K > 0 && T > 0 && O <= ((int64_t)1 << 24); }
+static bool few_ahead(int64_t O, int64_t K, int64_t T, double direct_us)
+{
+    return few_cost(few_tile(O, K, T), O, K, T) * (T > 16 ? 1.15 : 1.0) < direct_us;
+}
 static bool few_pays(int64_t O, int64_t K, int64_t T)
 {
-    if (T > 64 || O <= 0 || K <= 0 || T <= 0 || O > ((int64_t)1 << 24)) return false;
     int slices;
-    return few_cost(few_tile(O, K, T), O, K, T) * (T > 16 ? 1.15 : 1.0) < dense16_best(O, (K + 63) / 64, T, &slices);
+    return few_takes(O, K, T) && few_ahead(O, K, T, dense16_best(O, (K + 63) / 64, T, &slices));
 }
 
 template <typename T, bool CT = false> static int launch_dense(DfParams &P, int variant, hipStream_t s)
@@ -1034,7 +1038,10 @@ extern "C" int nmg_densefrag_plan(int64_t O, int64_t K, int64_t T, int *slices, 
     NMG_REQUIRE(O >= 0 && K >= 0 && T >= 0, NMG_ERR_ARG, "negative extent");
     NMG_REQUIRE(slices && workspace_bytes, NMG_ERR_ARG, "null output pointer");
     int best = 1;
-    if (O > 0 && T > 0 && K / 64 > 0 && !few_pays(O, K, T)) dense16_best(O, K / 64, T, &best);
+    if (O > 0 && T > 0 && K / 64 > 0) {
+        const double us = dense16_best(O, K / 64, T, &best);
+        if (few_takes(O, K, T) && few_ahead(O, K, T, us)) best = 1;
+    }
     *slices = best;
     *workspace_bytes = best > 1 ? (int64_t)best * T * ((O + 255) / 256) * 256 * 4 : 0;
     return NMG_OK;

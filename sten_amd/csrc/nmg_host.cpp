@@ -744,7 +744,9 @@ bool transposed_pays(int64_t O, int64_t K, int64_t N, bool as_it_lies)
 // 0.6 us on the dense cores, 0.4 on tiles of 128 x 128; the cut saves the steps of all slices but one and costs about 11 us of launches beside
 // the partial sums, written and read once.  us, whole -> cut: sparse cores 4096 x 11008 x 32 columns 81 -> 27, x 512
 // 102 -> 58, 4096 x 4096 x 128 31 -> 25 (8 slices), x 512 32 -> 41 (4 slices); dense cores 1024 x 16384 x 128 141 -> 31,
-// 4096 x 4096 x 512 46 -> 41, x 1024 50 -> 57.
+// 4096 x 4096 x 512 46 -> 41, x 1024 50 -> 57.  The kernel for few tokens walks no steps one after the other and has no partial sums: 32
+// columns 2048 x 2048 18.8 -> 12.4, 1024 x 4096 28.0 -> 14.4, 4096 x 4096 33.7 -> 20.4, 8192 x 2048 23.1 -> 18.6; 64 columns 1000 x 3000
+// 23.2 -> 15.5, 512 x 4096 28.0 -> 15.2.
 bool tt_split_pays(const Options &opt, int64_t O, int64_t K, int64_t N, bool sparse)
 {
     if (opt.kernel != "auto" || opt.variant != -1 || opt.dense_variant != -1 || opt.slices >= 0 || !opt.expand || N * round_up(K, 64) * 2 >= k2G)
@@ -753,8 +755,9 @@ bool tt_split_pays(const Options &opt, int64_t O, int64_t K, int64_t N, bool spa
     int64_t bytes = 0;
     check(sparse ? nmg_smfmac_plan(O, K, N, &slices, &bytes) : nmg_densefrag_plan(O, round_up(K, 64), N, &slices, &bytes));
     const bool narrow = up(O, 128) * up(N, 128) <= 256;      // (tiles of 128 x 128)
-    const double saved = (double)up(K, 64) * (1.0 - 1.0 / slices) * (narrow ? 0.4 : sparse ? 0.45 : 0.6);
-    return slices > 1 && saved > 11.0 + (double)slices * (double)(N * O) * 8 / 4e6;
+    const double walk = (double)up(K, 64) * (narrow ? 0.4 : sparse ? 0.45 : 0.6);
+    if (!sparse && slices == 1 && nmg_densefrag_few(O, round_up(K, 64), N)) return walk > 11.0;
+    return slices > 1 && walk * (1.0 - 1.0 / slices) > 11.0 + (double)slices * (double)(N * O) * 8 / 4e6;
 }
 
 Tensor tt_split(State &w, const Tensor &b, int rd)

@@ -45,3 +45,20 @@ def test_what_it_does_not_take():
     for K, T, ldx in ((12, 1, 64), (64, 65, 64), (64, 1, 60), (0, 1, 64)):
         with pytest.raises(native.NmgError):
             native.check(lib.nmg_spmm_densefrag_few(*args(K, T, ldx)))
+
+
+@pytest.mark.parametrize("O,K,N", [(1024, 4096, 17), (1024, 4096, 32), (1000, 3000, 64), (2048, 2048, 40), (4096, 4096, 32), (520, 4096, 64)])
+@pytest.mark.parametrize("rd", [0, 1])
+def test_few_columns_take_it(O, K, N, rd):
+    # op(W) @ B with few columns: the kernel for few tokens on the transposed operands, so the same sums bit for bit.  (A walk over
+    # the whole reduction adds in another order: of 32 columns x 1024 outputs some dozens then round to the other side.)
+    print(f"case {O}x{K} N={N} rd={rd}", flush=True)
+    assert native.load().nmg_densefrag_few(O, -(-K // 64) * 64, N) == 1
+    gen = torch.Generator(DEV).manual_seed(O + K + N)
+    shape = (O, K) if rd == 1 else (K, O)
+    w = sten.GroupedNMTensor.from_dense(torch.randn(*shape, device=DEV, generator=gen).half(), 4, 8, sparse_dim=1, group_size=2, group_dim=0)
+    b = torch.randn(K, N, device=DEV, generator=gen).half()
+    c = sten.spmm_tt_dense(w, b, reduce_dim=rd)
+    assert torch.equal(c, sten.spmm(w, b.t().contiguous(), reduce_dim=rd).t())
+    dense = w.to_dense().double()
+    assert rel_l2(to_np(c), to_np((dense if rd == 1 else dense.t()) @ b.double())) <= TOL[torch.float16]
