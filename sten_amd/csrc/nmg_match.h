@@ -283,7 +283,7 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
     int *s_list = s_occ + c, *s_at = s_list + c, *s_last = s_at + c, *s_np = s_last + c;      // the classes, largest patterns first
     if (SG != 0) g = SG;
     if (SM != 0) m = SM;
-    const bool lists = KPT > 1 && (SG != 0 || listed);      // (tiles of the compiled group sizes have room for the list)
+    const bool lists = KPT > 1 && (SG != 0 || listed);      // (at the compiled group sizes the list costs nothing)
     if (SM != 0 && SN != 0) c = match_binom(SM ? SM : 1, SN);
     const int tt = threadIdx.x % NT, real_mask = (1 << real_rows) - 1;
     auto column = [](uint64_t key) { return (int)((key >> 1) & 0x7FFFu); };
@@ -1229,12 +1229,16 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     off += cols * 8 + kMatchPad;
     Q.r_int = off;
     off = up(off + (kMatchTables * c + 4) * 4, 16);
-    constexpr int LDS = 160 * 1024;
+    constexpr int LDS = 160 * 1024, MOST = match_waves(NT, SM != 0, RC) * 4 / (THREADS / 64);      // workgroups that fit a CU's wavefronts
     const int head = up(c * 8, 16);
-    if (Q.view.S % m != 0) {      // the classes of a partial block, and a list of its refused columns where the tile leaves room for it
+    if (Q.view.S % m != 0) {
+        // the classes of a partial block, and a list of its refused columns where that costs no workgroup of a CU (us, two workgroups without the
+        // list against one with it: 3:6:100 fp32 2001 x 1999 102, 168)
         off = up(off + ((c + 1) & ~1) * 4 + c * 8, 16);
-        Q.listed = match_keys(NT, CPT) > 1 && head + TILES * up(off + cols * 2, 16) <= LDS;
-        if (Q.listed) off = up(off + cols * 2, 16);
+        const int with = up(off + cols * 2, 16);
+        auto per_cu = [&](int region) { return std::min(MOST, LDS / (head + TILES * region)); };
+        Q.listed = match_keys(NT, CPT) > 1 && (SG != 0 || per_cu(with) == per_cu(off));
+        if (Q.listed) off = with;
     }
     // the tiles of a wavefront run the same offsets of their regions: spread them over the banks
     if (NT < 64)
