@@ -700,7 +700,11 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
         real_rows = (int)min(Q.view.S - mb * m, (int64_t)m);
     }
     // the partial blocks among the workgroup's tiles, all threads on one after the other
-    if (Q.view.S % m != 0)
+    // (kept out of the way of launches that have none: us, eight copies of the call and any branch -> this, 4096^2 fp16, 2:4:16 59.2 -> 59.0, as
+    // without a list of refused columns, 3:6:12, blocks along the slow dim, 76.0 -> 75.4)
+    const bool partial = __builtin_amdgcn_readfirstlane(Q.view.S % m != 0 ? 1 : 0) != 0;
+    if (__builtin_expect(partial, 0))
+#pragma unroll 1
         for (int tm = 0; tm < TILES && tile0 + tm < Q.outer; tm++) {
             int64_t b, kc, mb;
             locate(tm, b, kc, mb);
@@ -1267,21 +1271,14 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     return NMG_OK;
 }
 
+// The patterns of this repository's benchmark and tests at their group sizes, in a source of their own (nmg_match_fixed.hip).
+template <typename T> int match_fixed(MatchParams &Q, bool rc, hipStream_t stream, bool *done);
+
 template <typename T, bool RC> static int match_dispatch(MatchParams &Q, hipStream_t stream, bool *done)
 {
-    const int n = Q.n, m = Q.m, g = Q.g;
-    auto is = [&](int a, int b, int d) { return n == a && m == b && g == d; };
-    // The patterns of this repository's benchmark and tests at their group sizes: pattern, list and tile extents folded in
-    // (4096 x 4096 fp16, any pattern -> compiled: 2:4:16 107 -> 64 us, 2:8:32 128 -> 71).
-    if (is(2, 4, 16)) return match_launch<T, 32, 3, 2, 4, 16, RC>(Q, stream, done);
-    if (is(1, 8, 32)) return match_launch<T, 64, 4, 1, 8, 32, RC>(Q, stream, done);
-    if (is(3, 6, 12)) return match_launch<T, 64, 4, 3, 6, 12, RC>(Q, stream, done);
-    if (is(2, 8, 32)) return match_launch<T, 256, 4, 2, 8, 32, RC>(Q, stream, done);
-    if (is(4, 8, 32)) {
-        // (fp32 tiles with the data in LDS leave one workgroup per CU)
-        const int rc = match_launch<T, 512, 5, 4, 8, 32, RC>(Q, stream, done);
-        if (rc != NMG_OK || *done) return rc;
-    }
+    const int n = Q.n, m = Q.m;
+    const int fixed = match_fixed<T>(Q, RC, stream, done);
+    if (fixed != NMG_OK || *done) return fixed;
     // Small tiles, a quarter of a wavefront each: what counts is the instructions of a proposal.  The kernels compiled for
     // a pattern, any g, need the fewest (4096 x 4096 fp16, any pattern -> compiled: 2:4:8 112 -> 75 us, 1:4:8 107 -> 69, 1:2:16
     // 131 -> 94, 1:5:4 164 -> 122).

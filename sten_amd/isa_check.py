@@ -271,11 +271,11 @@ def check_kernel(name, body):
 
 def assembly_of(source):
     """Device assembly of one HIP source, compiled with the flags of the library."""
-    from .build import FLAGS
+    from .build import FLAGS, OPTIONS
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     with tempfile.TemporaryDirectory() as tmp:
         out = os.path.join(tmp, "k.s")
-        cmd = [hipcc] + FLAGS + ["--cuda-device-only", "-S", os.path.join(CSRC, source), "-o", out]
+        cmd = [hipcc] + FLAGS + OPTIONS.get(source, []) + ["--cuda-device-only", "-S", os.path.join(CSRC, source), "-o", out]
         subprocess.run(cmd, check=True, stdout=subprocess.PIPE, stderr=subprocess.PIPE)
         return open(out).read()
 
