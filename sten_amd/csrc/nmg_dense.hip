@@ -1058,9 +1058,10 @@ static int gemm_f32_host(const void *d_a, int64_t lda, const void *d_x, int64_t 
         const double cost = (double)((tiles + 255) / 256) * S.bm * S.bn / eff;
         if (c == 0 || cost < best_cost) { best = c; best_cost = cost; rounds = (tiles + 255) / 256; }
     }
-    // its time in us (guards cost a fifth), and 4 % to make the other kernel worth while
+    // its time in us (guards cost a fifth; 64 x 64 and 32 x 32 take less than their share of the rule above), and 4 % to make the other
+    // kernel worth while
     const bool even = Q.vec && K % 32 == 0 && (form < 1 || O % 4 == 0) && (form < 2 || T % 4 == 0);
-    const double us = best_cost * 3.63e-6 * (double)K * (even ? 1.0 : 1.2) + 3.5 + 1.25 * (double)rounds;
+    const double us = best_cost * 3.63e-6 * (double)K * (even ? 1.0 : 1.2) * (best >= 4 ? 0.91 : 1.0) + 3.5 + 1.25 * (double)rounds;
     if (split3_gemm(d_a, lda, d_x, ldx, d_y, ldy, d_bias, O, K, T, form, 0.96 * us, st)) {
         NMG_HIP_TRY(hipGetLastError());
         return NMG_OK;
