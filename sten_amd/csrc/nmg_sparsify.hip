@@ -1022,30 +1022,34 @@ static int launch_scatter_tiled(bool gather, ScatterParams &P, hipStream_t s, bo
     auto lds_of = [&](int tiles, bool pd) {
         return (size_t)(gc ? tiles * P.m : P.cols) * pitch_of(tiles, pd) * sizeof(T);
     };
-    // Tiles of many columns.  Group dim contiguous: a row of the region is long however few tiles there are, so as many as keep
-    // several workgroups on a CU.  Else the rows are runs of the tiles' positions: 4 tiles, or 2 where 4 take nearly all of the LDS.
+    // Tiles of many columns.  Small tensors, about what the caches of a few CUs hold, have too few workgroups of them: a slot per thread is ahead
+    // (4:8:32 fp32 1001^2, along the blocks, gather / dense 8.4 / 10.3 against 13.5 / 12.5 us; 2048 x 1536 25 / 42 against 15 / 14).
+    const double mi = (double)P.view.G * (double)P.view.S * (double)(P.outer / (P.view.num_blocks * P.view.num_chunks)) / (1 << 20);
+    if (per_tile > (gc && gather ? 16 : 32) * 1024 && mi <= (gather ? 2.5 : gc ? 0.5 : 1.5)) return NMG_OK;
+    // Group dim contiguous: a row of the region is long however few tiles there are, so as many as keep several workgroups on a CU.  Else the
+    // rows are runs of the tiles' positions: 4 tiles, or 2 where 4 take nearly all of the LDS (dense: with a row's padding more than it).
     // us, gather / dense, before -> this: 4:8:32 fp32 3712 x 3584 group dim contiguous (a slot per thread) 69 / 102 -> 25 / 31, else
     // 97 / 156 -> 35 / 31; 12160 x 1408 bf16 38 / 20 (4 tiles) -> 18 / 17, 37 / 28 -> 34 / 24; 2:8:32 8192^2 fp16 55 / 51 (4 / 8 tiles)
-    // -> 52 / 44, 2048 x 1536 fp32 8.0 / 8.4 -> 6.7 / 6.8.  Few workgroups are not faster than a slot per
-    // thread (4:8:32 1024^2, gather by 128 of them: fp16 6.5 -> 7.2, fp32 7.5 -> 8.2; dense by 64 8.9 -> 10.6).
+    // -> 52 / 44, 2048 x 1536 fp32 8.0 / 8.4 -> 6.7 / 6.8.  13 patterns x 9 sizes, two types, both dims: 0.86 of the time with 8 or 4 tiles or a slot
+    // per thread, at the most 1.12 of it (2:8:32 fp32 4096 x 1024 dense 9.5 -> 10.6).
     if (gc && per_tile * 8 > 48 * 1024) nt = (int)std::min<int64_t>(nt, std::max<int64_t>(1, 32 * 1024 / per_tile));
     if (!gc && lds_of(nt, pad) > 150 * 1024) nt = (int)std::min<int64_t>(4, P.view.num_blocks);
     // (rows that do not lie on 16 bytes are read and written element by element, and longer runs are then ahead: 4:8:32 fp16 12971 x 2722
     // gather 116, with 2 tiles 124; dense 117, 127)
     const bool odd_rows = !gc && P.view.stride_g * (int64_t)sizeof(T) % 16 != 0, four = odd_rows && lds_of(nt, false) <= 150 * 1024 && nt >= 4;
-    if (!gc && !four && lds_of(nt, pad) > 128 * 1024) nt = 2;
+    if (!gc && !four && lds_of(nt, pad) > (gather ? 128 : 150) * 1024) nt = 2;
     if (lds_of(nt, pad) > 150 * 1024) pad = false;    // rows without the vector of padding
     if (lds_of(nt, pad) > 150 * 1024) return NMG_OK;
-    if (per_tile > 32 * 1024 && !four && (gather || !gc) && chunks * ((P.view.num_blocks + nt - 1) / nt) < (gather ? 256 : 128)) return NMG_OK;
     TiledParams Q{};
     Q.sp = P;
     Q.nt = nt;
     Q.pitch = pitch_of(nt, pad);
     Q.groups_per_chunk = (int)((P.view.num_blocks + nt - 1) / nt);
-    // Runs that are no whole lines of 128 bytes share their lines with the next workgroup's: one XCD for both.  us, gather / dense, dealt
-    // round-robin -> this: 4:8:32 12160 x 1408 bf16 (runs of 32 bytes) 34 / 24 -> 23 / 22, 3712 x 3584 fp32 (64) 35 / 31 -> 32 / 31, 3:6:12
-    // 9216 x 4608 fp16 (96) 52 / 64 -> 45 / 61; whole lines lose: 2:4:16 16384 x 4096 58 / 54 -> 64 / 57.
-    Q.runs = !gc && !odd_rows && nt * P.m * (int)sizeof(T) % 128 != 0 ? 1 : 0;
+    // Runs that are no whole lines of 128 bytes share their lines with the next workgroup's: one XCD for both.  us, gather, dealt
+    // round-robin -> this: 4:8:32 12160 x 1408 bf16 (runs of 32 bytes) 34 -> 23, 3712 x 3584 fp32 (64) 35 -> 32, 3:6:12 9216 x 4608 fp16 (96) 52 -> 45;
+    // whole lines lose: 2:4:16 16384 x 4096 58 -> 64.  Dense only the short runs, 4:8:32 4096^2 fp16 22.4 -> 20.5; else it loses, 3:6:50 fp32 1024 x
+    // 4096 17.0 -> 20.0, 2:4:64 fp16 2048 x 1536 7.0 -> 7.5.
+    Q.runs = !gc && !odd_rows && nt * P.m * (int)sizeof(T) % 128 != 0 && (gather || (nt == 2 && sizeof(T) == 2)) ? 1 : 0;
     Q.magic_cols = (((uint64_t)1 << 32) + P.cols - 1) / P.cols;
     Q.magic_g = (((uint64_t)1 << 32) + P.g - 1) / P.g;
     const size_t lds = lds_of(nt, pad);
