@@ -222,7 +222,7 @@ int nmg_gemm_nt(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void
 /* The same single-precision product with the weight-side operand reduction-major:
  * Y[T, O] = X[T, K] * A[K, O] (+ bias[o]).  It is how torch.mm(W_nmg, B) and its gradient with
  * respect to B run in fp32 without transposing copies: X is the expanded weight (or its transpose,
- * both from nmg_rowpack_expand), A is B as it lies in memory, Y is the result as torch.mm lays it
+ * both from nmg_to_dense), A is B as it lies in memory, Y is the result as torch.mm lays it
  * out (the reference's transpose_b / transpose_c, dace_gnm_mult.py:572-627).  dtype F32 only; any
  * extents and pitches, 128-bit loads where rows are 16-byte aligned and O % 4 == 0. */
 int nmg_gemm_nn(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy,

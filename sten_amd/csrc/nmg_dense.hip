@@ -946,9 +946,9 @@ static void launch_gemm_f32(const GemmF32Params &Q, int form, hipStream_t st)
 // Few tiles for the chip: 16 outputs x 16 tokens a workgroup on V_MFMA_F32_16X16X4_F32, both operands as rows, the reduction dealt out
 // to its 16 wavefronts in chunks of 32 positions, from memory into registers (nothing is used twice in a workgroup), sums added
 // through LDS.  The kernel above is bound there by the walk of four wavefronts through the reduction on few CUs; this one by
-// two or three rounds of loads, and from 4096 outputs on by the stream of the weight (3.3 TB/s).  us, tile of 32 x 32 -> this, operands
-// of 256 MB in turn: 256 x 1664, 9 tokens 10.3 -> 7.5, 384 x 1792, 27 11.9 -> 9.0, 768 x 768, 64 7.6 -> 5.6, 4024 x 1808, 2 14.4 -> 8.8,
-// 4096 x 4096, 16 22.2 -> 19.4, 1001 x 777, 27 8.9 -> 5.2.  With one operand reduction-major (16 lanes on a line of 64 bytes, an element
+// two or three rounds of loads, and from 4096 outputs on by the stream of the weight (2.9 TB/s).  us, tile of 32 x 32 -> this, operands
+// of 256 MB in turn: 256 x 1664, 9 tokens 10.9 -> 8.1, 384 x 1792, 27 12.5 -> 9.5, 768 x 768, 64 8.1 -> 5.9, 4024 x 1808, 2 15.9 -> 10.1,
+// 4096 x 4096, 16 26.9 -> 23.4, 1001 x 777, 27 10.4 -> 5.9.  With one operand reduction-major (16 lanes on a line of 64 bytes, an element
 // a lane) it gains half of that or nothing, 4024 x 1808, 2 18.8 either way, and is not there.
 // Lane (j, g) holds row j of both operands, positions 4 g .. 4 g + 3 and 16 + 4 g .. of a chunk; MFMA e takes element e of both.
 __global__ __launch_bounds__(1024) void gemm_f32_few_kernel(GemmF32Params P)

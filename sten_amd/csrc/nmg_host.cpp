@@ -143,9 +143,12 @@ constexpr int64_t kOstreamAutoTokens = 2;   // ... and up to where it is ahead o
 constexpr int64_t kGstreamMaxTokens = 16;   // nmg_spmm_gstream: tokens up to which the stream of the weight bounds the product
 // Activations whose rows are no whole number of 128-byte lines, a copy in whole K steps of 64 against the rows as they lie: a tile's
 // piece of a row then reaches into two lines, and every line tile reads it again, from memory where no cache holds the activations; from some
-// size on that costs more than the copy and its launch.  us, copy / as they lie, operands in the caches and (from memory): 2:4 1768 x 2216 x 298
-// tokens 19.1 / 16.0 (21.7 / 20.6), 11256 x 672 x 240 11.4 / 9.1 (18.1 / 16.2), 512 x 1000 x 32 13.1 / 9.5 (15.0 / 11.6); beyond the line 4000 x 2056 x 500 18.8 / 16.9 (26.9 / 29.0), 2048 x 2056 x 1024
-// (27.1 / 28.4), 4096 x 4088 x 500 (40.6 / 47.1), 8000 x 2504 x 200 (30.0 / 33.8), 8200 x 8104 x 260 45.8 / 52.9; 2352 x 9488 x 570 would gain (51.5 / 46.0).
+// size on that costs more than the copy and its launch.  Time with the copy over time as they lie, 29 weights of 520 x 200 to 8200 x 8104
+// with 32 to 2000 tokens, 2:4 / 4:8, weights and activations from memory: up to 7.2 Mi weights 1.07 to 1.45 / 1.05 to 1.43 at 100 to 500 tokens,
+// up to 64 tokens 1.22 to 1.41 / 1.0 (the kernel for few tokens, either way) to 1.31.  Beyond the line 7.8 to 13.7 Mi weights would still gain
+// (1.02 to 1.21 / 1.0 to 1.20), as would more tokens (1.0 to 1.45; 1768 x 4088 x 1000 alone loses, 0.98); 16 Mi and more lose as often as not
+// (0.84 to 1.12 / 0.90 to 1.15, most with many outputs and a short reduction: 12000 x 2056 0.84 to 0.94), but up to 64 tokens
+// still gain 1.04 to 1.27 / 1.0 to 1.25.  With everything in the caches 1.0 to 1.7 up to 14 Mi, 0.86 to 1.23 beyond.
 constexpr int64_t kRaggedMost = 15 << 19;
 constexpr int64_t kF32GemmMaxTokens = 65535 * 32;   // one launch of the fp32 GEMM: token tiles of 32 in grid.y
 
@@ -467,8 +470,8 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
     if (x.dim() != 2 || x.size(1) != K) fail("activations must be [tokens, ", K, "], got ", shape_text(x));
     c10::DeviceGuard device(x.device());
     at::AutoDispatchBelowADInplaceOrView raw;
-    if (x.stride(1) != 1 || !rows_lie(x)) x = x.contiguous();      // (the kernels take no rows that share memory)
     const int64_t T = x.size(0);
+    if (x.stride(1) != 1 || (T > 1 && x.stride(0) < K)) x = x.contiguous();      // (the kernels take no rows that share memory)
     const int64_t ldx = T > 1 ? x.stride(0) : K;      // the stride of a dim of extent 1 means nothing
     Tensor y = new_empty({T, O}, x);
     if (bias.defined()) bias = bias.to(x.scalar_type()).contiguous();

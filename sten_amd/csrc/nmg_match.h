@@ -141,20 +141,6 @@ __device__ __forceinline__ int match_column(uint64_t key) { return (int)(key & 0
 constexpr int kMatchTables = 6;      // c ints each, and four counts (three of them for partial blocks only)
 constexpr int kMatchPad = 64;        // bytes behind the proposals: a batch of eight keys past the end of the last group
 
-// First rounds of a tile with `real_rows` < m real positions.  All columns' keys are sorted by pattern and key in
-// every round, since most of them are refused and sit in few, long groups.  Patterns that agree in the real positions are a class: where
-// there are few, a column sums and compares once for each class.  One such tile is as long as the launch: three to seven rounds, each a
-// sort, a pass over the keys and the new proposals.  The sort is a compare-exchange network on keys in registers (10 stages of 55 for
-// 896 keys in LDS) and for the patterns of the compiled kernels a column's sums are folded in, as those of the other tiles (18
-// instructions a pattern against 36).  us, network in LDS or places counted by all pairs and sums from masks -> now: 3:6:12 512 x 1792 fp32
-// 52 -> 40, 1280 x 2176 bf16 56 -> 37, 2:8:32 3054 x 3960 bf16 148 -> 61 (3056 x 3960, without partial blocks, 50), 2001 x 2001 fp32 80 -> 50,
-// 4:8:32 512 x 4099 fp16 100 -> 59, 1005 x 3000 bf16 581 -> 273, 2:4:16 1001 x 1000 fp16 26 -> 22; any pattern, 3:8:8 997 x 1003 fp16
-// 162 -> 137.  Of the 2:8:32 one 14 us came from the refused columns proposing one per lane instead of where they lie.  Sorts that lost:
-// runs of 64 merged by binary search (gathers at random places of LDS, 1.5 x), keys broadcast from a wavefront's lanes (1.2 x).  A refused
-// column skips the patterns of its class that those ahead of it are certain to fill: all of them that have no other
-// class with the same score to turn to, which bit 0 of a key says here.  Stops when at most `few` columns are pending;
-// leaves s_mem, s_occ, the waiting columns in s_np[1] and the pending ones in s_arr and s_np[0].
-// A function of its own: its registers are not those of the other tiles.
 // Value of lane (this one ^ X), X = 2^k or 2^k - 1.
 template <int X> __device__ __forceinline__ uint32_t match_lane_xor(uint32_t v)
 {
@@ -269,6 +255,20 @@ template <int NT, int KPT> __device__ __forceinline__ void match_sort(uint64_t *
     __syncthreads();
 }
 
+// First rounds of a tile with `real_rows` < m real positions.  All columns' keys are sorted by pattern and key in
+// every round, since most of them are refused and sit in few, long groups.  Patterns that agree in the real positions are a class: where
+// there are few, a column sums and compares once for each class.  One such tile is as long as the launch: three to seven rounds, each a
+// sort, a pass over the keys and the new proposals.  The sort is a compare-exchange network on keys in registers (10 stages of 55 for
+// 896 keys in LDS) and for the patterns of the compiled kernels a column's sums are folded in, as those of the other tiles (18
+// instructions a pattern against 36).  us, network in LDS or places counted by all pairs and sums from masks -> now: 3:6:12 512 x 1792 fp32
+// 53 -> 40, 1280 x 2176 bf16 57 -> 37, 2:8:32 3054 x 3960 bf16 143 -> 60 (3056 x 3960, without partial blocks, 50), 2001 x 2001 fp32 80 -> 51,
+// 4:8:32 512 x 4099 fp16 100 -> 60, 1005 x 3000 bf16 536 -> 279, 7742 x 933 fp32 437 -> 253, 2:4:16 1001 x 1000 fp16 24 -> 21; any pattern,
+// 3:8:8 997 x 1003 fp16 163 -> 122.  Of the 2:8:32 one 14 us came from the refused columns proposing one per lane instead of where they lie.  Sorts that lost:
+// runs of 64 merged by binary search (gathers at random places of LDS, 1.5 x), keys broadcast from a wavefront's lanes (1.2 x).  A refused
+// column skips the patterns of its class that those ahead of it are certain to fill: all of them that have no other
+// class with the same score to turn to, which bit 0 of a key says here.  Stops when at most `few` columns are pending;
+// leaves s_mem, s_occ, the waiting columns in s_np[1] and the pending ones in s_arr and s_np[0].
+// A function of its own: its registers are not those of the other tiles.
 template <typename T, int NT, int KPT, int SN, int SM, int SG>
 __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, int r_int, int c, int m, int g, int so, int sr,
                                            int real_cols, int real_rows, int few, int listed)
