@@ -10,29 +10,29 @@
 // patterns' lists are kept sorted and are the result.
 //
 // The walk batched by "until the next pattern fills", which this replaced, took up to one round per pattern
-// over all free columns (6 / 28 / 70 rounds for 2:4, 2:8, 4:8).  Random weights need 4 / 7 / 8 rounds here,
-// and all but the first concern a few columns: 13 of 96 are sent away in total (2:4:16), 113 of 896
-// (2:8:32), 299 of 2240 (4:8:32).
-//
-// Later rounds insert proposals into the lists lane by lane (the code says how).  4096 x 4096 2:4:16 fp16: 99 -> 58 us,
-// 8192 x 8192 2:8:32: 727 -> 201 us, 4096 x 4096 4:8:32: 390 -> 123 us.  What bounds it is the issue of vector instructions (1200 for a
-// wavefront of two tiles 2:4:16, 0.74 of the time; 0.66 at 2:8:32) and, in the later rounds, chains of LDS round trips: of the 201 us,
-// tile data and results take 52, the first proposals 15, the first round 44, the later rounds 90.  A list in 16 lanes of one or two
-// keys, merged two proposals at a time, and eight lanes (2:4: two) on a column's patterns took these from 122 (whole kernel 233; 2:4:16
-// 59.3 -> 57.8, 1:8:32 43.5 -> 39.5, 4:8:32 170 -> 123, fp32 240 -> 191).  Other group sizes, 4096 x 4096
-// fp16 with the blocks along the contiguous / the slow dim, the batched walk -> this: 2:4:4 168 -> 116 / 231 -> 113 us, 2:4:8 115 -> 75 /
-// 146 -> 76, 2:4:32 118 -> 105 / 135 -> 116, 2:4:64 130 -> 118 / 146 -> 129, 1:4:8 99 -> 69 / 151 -> 70, 1:2:8 192 -> 147 /
-// 302 -> 145, 2:8:8 293 -> 130 / 326 -> 134, 4:8:16 870 -> 366 / 810 -> 388.  Slower than the walk is 1:4:17 (107 -> 110), and where the
-// sparse extent is odd and slow, 1:4:32 (4095 x 4093: 118 -> 126) and 1:2:64 (172 -> 182).
+// over all free columns (6 / 28 / 70 rounds for 2:4, 2:8, 4:8).  Random weights need 3.5 / 6 / 8 rounds here,
+// and all but the first concern a few columns: 12 of 96 are proposed again in total (2:4:16), 106 of 896
+// (2:8:32), 276 of 2240 (4:8:32).
 //
 // A round over all columns:
 //   1. every pending column computes its proposal (one thread per column; threshold of a pattern = key of its
 //      last slot, 0 while it has room);
-//   2. counting sort of the proposals by pattern;
-//   3. every proposal finds its rank: proposals of its pattern that are larger (all pairs) plus kept keys
-//      that are larger (binary search); every kept key of a pattern with proposals moves down by the
-//      proposals above it;
+//   2. counting sort of all columns' proposals, kept and new, by pattern and by bins of the score below the tile's largest;
+//   3. every proposal finds its rank: those in larger bins of its pattern plus those of its own bin that are larger (all pairs);
 //   4. what ranks below the pattern's capacity is written to its slot, the rest is pending.
+// A quarter of the columns and fewer (any n:m:g: half) insert into the lists lane by lane (the code says how).
+//
+// us, 4096 x 4096 fp16 with the blocks along the contiguous / the slow dim (8192 x 8192 for 2:8:32), batched walk -> ranks among all
+// proposals of a pattern -> this: 2:4:16 99 -> 58 / 57 -> 50 / 50, 1:8:32 37 -> 31, 3:6:12 75 / 73 -> 61 / 59, 2:8:32 727 -> 182 / 190 -> 138 / 147,
+// 4:8:32 390 -> 128 / 124 -> 73 / 73; any n:m:g: 2:4:4 168 / 231 -> 110 / 109 -> 87, 2:4:8 115 / 146 -> 71 -> 57, 2:4:32 118 / 135 -> 104 / 114 ->
+// 93 / 103, 2:4:64 130 / 146 -> 113 / 124 -> 107, 1:2:8 192 / 302 -> 143 / 138 -> 132, 2:8:8 293 / 326 -> 130 / 134 -> 102, 4:8:16 870 / 810 ->
+// 280 / 293 -> 220 / 228, 2:4:100 144 / 160 -> 130.  What each part gave, 2:8:32: bins 43 -> 20 us of the first round, score and pattern compared as one
+// double 17 -> 7 (a select behind a select on the same condition takes 17 to 40 clocks, a 64-bit maximum 4), the sorted keys in the place of the lists (six
+// workgroups a CU instead of five) 168 -> 150, the reads of a column's patterns in flight together 150 -> 145.  4:8:32: 125 -> 102, and 73 where the
+// later rounds are inlined: in a function their addresses are not known to lie in LDS.  Of the 147 us of 2:8:32 now, tile data and results
+// take 39 to 45, first proposals 10, the first round 25, the later ones 68: chains of LDS round trips and the issue of vector instructions,
+// 1500 a wavefront.
+//
 // Columns that have no pattern with room and a positive score wait.  In the walk they come last, together
 // with the zero columns beyond the end of the group dim, in descending column order, and each takes the
 // largest pattern with room: that is written in closed form.
@@ -139,7 +139,7 @@ __device__ __forceinline__ int match_pattern(uint64_t key) { return 255 - (int)(
 __device__ __forceinline__ int match_column(uint64_t key) { return (int)(key & 0xFFFFu); }
 
 constexpr int kMatchTables = 6;      // c ints each, and four counts (three of them for partial blocks only)
-constexpr int kMatchPad = 64;        // bytes behind the proposals: a batch of eight keys past the end of the last group
+constexpr int kMatchPad = 32;        // bytes behind the proposals: a batch of four keys past the end of the last bin
 
 // Value of lane (this one ^ X), X = 2^k or 2^k - 1.
 template <int X> __device__ __forceinline__ uint32_t match_lane_xor(uint32_t v)
@@ -154,6 +154,51 @@ template <int X> __device__ __forceinline__ uint32_t match_lane_xor(uint32_t v)
     else if constexpr (X == 15) return dpp(v, std::integral_constant<int, 0x140>{});
     else if constexpr (X < 32) return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (X << 10) | 0x1F);
     else return (uint32_t)__shfl_xor((int)v, X);
+}
+
+// Larger one of two edges (score in the high word, pattern in the low one; a positive double, never a NaN: scores are at most 0x7FFFFFFF and
+// a double's NaNs begin at 0x7FF00000, above every float).  One instruction, where fmax canonicalises its operands first.  The compiler does not
+// know it for a vector instruction: `s_nop 1` before a move between lanes reads its result.
+__device__ __forceinline__ uint64_t match_larger(uint64_t a, uint64_t b)
+{
+    uint64_t r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ uint64_t match_smaller(uint64_t a, uint64_t b)
+{
+    uint64_t r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Largest of LANES consecutive lanes, in all of them.
+template <int LANES> __device__ __forceinline__ uint32_t match_top(uint32_t v)
+{
+    v = max(v, match_lane_xor<1>(v));
+    v = max(v, match_lane_xor<2>(v));
+    v = max(v, match_lane_xor<7>(v));
+    v = max(v, match_lane_xor<15>(v));
+    if constexpr (LANES >= 32) v = max(v, match_lane_xor<16>(v));
+    if constexpr (LANES >= 64) v = max(v, match_lane_xor<32>(v));
+    return v;
+}
+
+// Bins of a pattern in the first round, by score: 8 (four to an octave below the tile's largest score, the last one open) where a lane then
+// has at most four of the tile's bins to sum up, else 4 (two to an octave).
+constexpr int match_bins_log2(int nt, int c) { return 8 * c <= 4 * (nt < 64 ? nt : 64) ? 3 : 2; }
+constexpr int match_bin_bytes(int bins) { return (4 + bins + 4) * 4; }      // a multiple of 16: bins come in fours
+
+// Bytes of a tile's s_arr: a round's bins; then the later rounds' two lists of pending columns and the patterns' buckets (a batch is read past the
+// last); then the waiting columns, flags and runs of the closed form; a partial block's proposals.  One after the other in the same place: 2:8:32 takes
+// 25.8 KB a tile of fp16 instead of 29.5, six workgroups of a CU instead of five.
+constexpr int match_few(int sg) { return sg != 0 ? 4 : 2; }
+static inline int match_scratch(int cols, int c, int g, int bins_log2, bool lists, bool partial, int few)
+{
+    int bytes = std::max(match_bin_bytes(c << bins_log2), 4 * cols + cols / 4 + 16);
+    if (lists) bytes = std::max(bytes, ((few + 1) / 2 + c * std::min(g / 2, 8) + 2) * 8);
+    if (partial) bytes = std::max(bytes, cols * 8);
+    return (bytes + 15) & ~15;
 }
 
 // Sorts s_arr[0 .. count), count <= NT * KPT, larger keys first, all NT threads at it: thread t has the keys t * KPT .. + KPT - 1 in registers, steps
@@ -532,7 +577,7 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
 // (2:4:12 with 4 / 6: 136 / 125), which spill more where the columns are contiguous (1:8:8 with 5 / 6: 77 / 87).
 constexpr int match_waves(int nt, bool compiled, bool rc)
 {
-    return nt > 256 ? 4 : compiled ? (nt == 256 ? 5 : nt == 64 ? 6 : 7) : nt > 64 ? 4 : rc ? 5 : 6;
+    return nt > 256 ? 4 : compiled ? (nt == 256 ? 6 : nt == 64 ? 6 : 7) : nt > 64 ? 4 : rc ? 5 : 6;
 }
 
 // Columns of a tile per thread of its workgroup, up to a power of two.
@@ -567,12 +612,15 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
     const int head_bytes = (c * 8 + 15) & ~15;
     unsigned char *region = smem + head_bytes + (size_t)tile * Q.region_bytes;
     T *s_d = (T *)region;
-    uint64_t *s_mem = (uint64_t *)(region + Q.r_mem);     // kept keys, every pattern's in descending order; 0: free slot
-    uint64_t *s_arr = (uint64_t *)(region + Q.r_arr);     // pending columns, then the proposals grouped by pattern
+    uint64_t *s_mem = (uint64_t *)(region + Q.r_mem);     // kept keys, every pattern's in descending order; 0: free slot.  Sorted keys before
+    uint64_t *s_arr = (uint64_t *)(region + Q.r_arr);     // a partial block's proposals; else see match_scratch
     int *s_dem = (int *)(region + Q.r_int);               // proposals of the round per pattern
     int *s_start = s_dem + c;                             // first of them in s_arr
     int *s_occ = s_start + c;                             // slots taken
     int *s_np = s_occ + 4 * c;                            // pending columns, waiting columns, pending columns of the later rounds
+    // A round's bins, larger patterns' behind smaller ones', of a pattern larger scores first; two counts in front of them
+    int *s_bin = (int *)s_arr + 4;
+    const int nbl2 = match_bins_log2(NT, c), nbins = c << nbl2;
 
     // ---- where the tiles lie ----
     // Workgroups go to the 8 XCDs in turn, each with an L2 of its own, and neighbours along the sparse dim share
@@ -687,10 +735,6 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
         }
         s_pos[p] = pos;
     }
-    for (int s = tt; s < cols; s += NT) s_mem[s] = 0;
-    for (int p = tt; p < kMatchTables * c + 4; p += NT) s_dem[p] = 0;
-    __syncthreads();
-
     const bool live = tile0 + tile < Q.outer;
     int real_cols = cols, real_rows = m;
     if (live) {
@@ -699,6 +743,14 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
         real_cols = (int)min(Q.view.G - kc * cols, (int64_t)cols);
         real_rows = (int)min(Q.view.S - mb * m, (int64_t)m);
     }
+    if (real_rows == m && real_cols > 0) {
+        for (int b = tt; b < match_bin_bytes(nbins) / 16; b += NT) ((int4 *)s_arr)[b] = int4{0, 0, 0, 0};
+    } else {
+        for (int s = tt; s < cols; s += NT) s_mem[s] = 0;
+    }
+    for (int p = tt; p < kMatchTables * c + 4; p += NT) s_dem[p] = 0;
+    __syncthreads();
+
     // the partial blocks among the workgroup's tiles, all threads on one after the other
     // (kept out of the way of launches that have none: us, eight copies of the call and any branch -> this, 4096^2 fp16, 2:4:16 59.2 -> 59.0, as
     // without a list of refused columns, 3:6:12, blocks along the slow dim, 76.0 -> 75.4)
@@ -720,7 +772,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 
     // Proposal of column o: its best pattern among those with room or a last key below the column's (the
     // larger pattern on equal scores); 0 where no such pattern has a positive score.  THR = false: all have room.
-    auto propose = [&](int o, auto thr_tag) -> uint64_t {
+    auto propose = [&](int o, auto thr_tag) __attribute__((always_inline)) -> uint64_t {      // (a call takes addresses that say no more that they lie in LDS)
         constexpr bool THR = decltype(thr_tag)::value;
         float a[8];
         if (!RC && sizeof(T) == 2 && SM == 8) {
@@ -739,19 +791,17 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 #pragma unroll
             for (int r = 0; r < 8; r++) a[r] = r < m ? match_abs(s_d[at(o, r)]) : 0.f;
         }
-        uint32_t best = 0;
-        int bp = 0, later = 0;
+        uint64_t best = 0;      // score and pattern
+        int later = 0;
+        uint32_t zero;      // not to be known for one: the patterns' numbers would take a register each for all columns
+        asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
         auto consider = [&](float acc, int p) {
-            const uint32_t sb = __float_as_uint(acc);
-            bool ok = sb >= best;
+            uint32_t sb = __float_as_uint(acc);
             if (THR) {
                 const uint64_t last = s_mem[p * g + g - 1 + later];
-                ok = ok && match_key(sb, o, p) > last;
+                if (!(match_key(sb, o, p) > last)) sb = 0;
             }
-            if (ok) {
-                best = sb;
-                bp = p;
-            }
+            best = match_larger(best, ((uint64_t)sb << 32) | (zero + (uint32_t)p));
         };
         if constexpr (SM != 0) {
             constexpr MatchMasks<SN ? SN : 1, SM ? SM : 1> tab;
@@ -770,145 +820,164 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                 if (SC > 8 && p % 8 == 7) {
                     if (THR) asm volatile("" : "+v"(later), "+v"(best));
 #pragma unroll
-                    for (int r = 0; r < SM; r++) asm volatile("" : "+v"(a[r]), "+v"(best));
+                    for (int r = 0; r < SM; r++) asm volatile("" : "+v"(a[r]), "+v"(best), "+v"(zero));
                 }
             }
         } else {
-            uint32_t four = Q.masks[0];
-            for (int p = 0; p < c; p++) {
-                const uint32_t mk = four & 0xFFu;
-                four = (p & 3) == 3 ? Q.masks[((p + 1) >> 2) & 31] : four >> 8;
-                float acc = 0;
+            for (int p0 = 0; p0 < c; p0 += 4) {      // (beyond the last pattern no mask: no score)
+                const uint32_t four = Q.masks[p0 >> 2];
 #pragma unroll
-                for (int r = 0; r < 8; r++)
-                    acc += __uint_as_float(__float_as_uint(a[r]) & (0u - ((mk >> r) & 1u)));      // a[r] or 0, without a branch
-                consider(acc, p);
+                for (int u = 0; u < 4; u++) {
+                    float acc = 0;
+#pragma unroll
+                    for (int r = 0; r < 8; r++)
+                        acc += __uint_as_float(__float_as_uint(a[r]) & (0u - ((four >> (8 * u + r)) & 1u)));      // a[r] or 0, without a branch
+                    consider(acc, min(p0 + u, c - 1));
+                }
             }
         }
-        return best == 0 ? 0 : match_key(best, o, bp);
+        return (best >> 32) == 0 ? 0 : match_key((uint32_t)(best >> 32), o, (int)(best & 0xFFu));
     };
 
     if (live) {
-        int pend = real_cols;
         // a quarter of the tile and fewer go on in the registers below
         const bool lists = LISTS && (SG != 0 || Q.lanes_log2 != 0);
-        const int few = lists ? cols / 4 : 0;
+        const int few = lists ? cols / match_few(SG) : 0;
+        uint16_t *pending = (uint16_t *)s_arr;
         // every proposal that is not the last word of its column is refused once per (column, pattern) at most
         const int limit = cols * c + 2;
+        int pend = real_cols, round = 0;
+        uint64_t own[CPT] = {};      // this thread's columns' proposals, kept or new; 0: none
         if (real_rows < m) {
             pend = s_np[0];
             match_sync<NT>();
-        }
-        for (int round = real_rows < m ? 1 : 0; round < limit && pend > (round == 0 ? 0 : few); round++) {
-            const int ns = (pend + NT - 1) / NT;
-            // 1. proposals
-            if (round == 0) {
-                for (int e = tt; e < pend; e += NT) s_arr[e] = propose(e, std::false_type{});
-            } else {
-                for (int e = tt; e < pend; e += NT) s_arr[e] = propose((int)s_arr[e], std::true_type{});
+            if (pend > few) {      // (tiles without lists)
+                for (int s = tt; s < cols; s += NT) s_arr[s] = 0;
+                match_sync<NT>();
+                for (int s = tt; s < cols; s += NT)
+                    if (s_mem[s] != 0) s_arr[match_column(s_mem[s])] = s_mem[s];
+                match_sync<NT>();
+#pragma unroll
+                for (int i = 0; i < CPT; i++) own[i] = tt + NT * i < real_cols ? s_arr[tt + NT * i] : 0;
             }
-            // 2. counting sort by pattern
-            uint64_t key[CPT];
+            round = 1;
+        }
+        for (; round < limit && pend > (round == 0 ? 0 : few); round++) {
+            // 1. proposals
+            uint32_t top = 0;
+            if (round == 0) {
+#pragma unroll 1
+                for (int e = tt; e < real_cols; e += NT) {
+                    const uint64_t key = propose(e, std::false_type{});
+                    s_mem[e] = key;
+                    top = max(top, (uint32_t)(key >> 16));
+                }
+#pragma unroll
+                for (int i = 0; i < CPT; i++) own[i] = tt + NT * i < real_cols ? s_mem[tt + NT * i] : 0;      // this thread's own entries
+            } else {
+                match_sync<NT>();
+                for (int b = tt; b < match_bin_bytes(nbins) / 16; b += NT) ((int4 *)s_arr)[b] = int4{0, 0, 0, 0};
+                if (tt < 2) s_np[tt] = 0;
+                match_sync<NT>();
+#pragma unroll 1
+                for (int i = 0; i < CPT; i++) {
+                    const int o = tt + NT * i;
+                    uint64_t mine = own[0];
+#pragma unroll
+                    for (int u = 1; u < CPT; u++) mine = u == i ? own[u] : mine;
+                    if (o < real_cols) {
+                        if (mine != 0 && mine < s_mem[match_pattern(mine) * g + g - 1]) mine = 0;      // refused
+                        if (mine == 0) mine = propose(o, std::true_type{});
+                        top = max(top, (uint32_t)(mine >> 16));
+                    }
+#pragma unroll
+                    for (int u = 0; u < CPT; u++) own[u] = u == i ? mine : own[u];
+                }
+            }
+            top = match_top<(NT < 64 ? NT : 64)>(top);
+            if constexpr (NT > 64) {
+                if ((tt & 63) == 0) atomicMax((unsigned *)s_bin - 4, top);
+                __syncthreads();
+                top = ((unsigned *)s_bin)[-4];
+            }
+            // 2. counting sort by pattern and score
+            auto bin_of = [&](uint64_t key) {
+                return (match_pattern(key) << nbl2) + (int)min((top - (uint32_t)(key >> 16)) >> (24 - nbl2), (1u << nbl2) - 1);
+            };
             int pos[CPT];
 #pragma unroll
             for (int i = 0; i < CPT; i++) {
-                const int e = tt + NT * i;
-                key[i] = 0;
                 pos[i] = 0;
-                if (i < ns && e < pend) {
-                    key[i] = s_arr[e];      // this thread's own entries
-                    if (key[i] != 0) pos[i] = atomicAdd(&s_dem[match_pattern(key[i])], 1);
-                    else atomicAdd(s_np + 1, 1);      // waits
-                }
+                if (own[i] != 0) pos[i] = atomicAdd(&s_bin[bin_of(own[i])], 1);
+                else if (tt + NT * i < real_cols) atomicAdd(s_np + 1, 1);      // waits
             }
             match_sync<NT>();
-            if (tt < 64) {
+            if (tt < 64) {      // four or eight bins a lane
                 constexpr int LANES = NT < 64 ? NT : 64;
-                const int p0 = 2 * tt, p1 = p0 + 1;
-                const int d0 = p0 < c ? s_dem[p0] : 0, d1 = p1 < c ? s_dem[p1] : 0;
-                const int excl = match_prefix<LANES>(d0 + d1) - (d0 + d1);
-                if (p0 < c) s_start[p0] = excl;
-                if (p1 < c) s_start[p1] = excl + d0;
-                if (tt == LANES - 1) s_np[0] = excl + d0 + d1;      // proposals of this round
+                int4 *mine = (int4 *)s_bin + (nbl2 == 3 ? tt : 2 * tt), d0{}, d1{};
+                const int first = nbl2 == 3 ? 4 * tt : 8 * tt;
+                if (first < nbins) d0 = mine[0];
+                if (nbl2 == 2 && first + 4 < nbins) d1 = mine[1];
+                d0.y += d0.x;
+                d0.z += d0.y;
+                d0.w += d0.z;
+                int sum = d0.w;
+                if (nbl2 == 2) {
+                    d1.x += d0.w;
+                    d1.y += d1.x;
+                    d1.z += d1.y;
+                    sum = d1.w += d1.z;
+                }
+                const int excl = match_prefix<LANES>(sum) - sum;
+                if (first < nbins + 1) mine[0] = int4{excl, excl + d0.x, excl + d0.y, excl + d0.z};
+                if (nbl2 == 2 && first + 4 < nbins + 1) mine[1] = int4{excl + d0.w, excl + d1.x, excl + d1.y, excl + d1.z};
+                if (tt == LANES - 1) s_bin[-3] = s_bin[nbins] = excl + sum;      // proposals of this round
             }
             match_sync<NT>();
-            const int props = s_np[0];
+            const int props = s_bin[-3];
 #pragma unroll
             for (int i = 0; i < CPT; i++)
-                if (i < ns && key[i] != 0) s_arr[s_start[match_pattern(key[i])] + pos[i]] = key[i];
-            if (tt < 8) s_arr[props + tt] = 0;      // what the last batch of the last group reads
+                if (own[i] != 0) s_mem[s_bin[bin_of(own[i])] + pos[i]] = own[i];
+            if (tt < 4) s_mem[props + tt] = 0;      // what the last batch of the last bin reads
             match_sync<NT>();
             // 3. ranks.  Thread e takes the proposal that the sort put at e: the lanes of a wavefront then read the
-            //    same few groups.  A proposal that has seen as many larger keys as its pattern has slots stops.
-            const int nr = (props + NT - 1) / NT;
+            //    same few bins.  A proposal that has seen as many larger keys as its pattern has slots stops.
+            uint64_t key[CPT];
 #pragma unroll
             for (int i = 0; i < CPT; i++) {
                 const int e = tt + NT * i;
                 key[i] = 0;
-                if (i < nr && e < props) {
-                    const uint64_t mine = s_arr[e];
-                    const int p = match_pattern(mine), d = s_dem[p];
-                    int r = 0;
-                    if (round > 0) {
-                        const uint64_t *kept = s_mem + p * g;
-                        for (int step = 1 << (31 - __clz(g)); step > 0; step >>= 1)
-                            if (r + step <= g && kept[r + step - 1] > mine) r += step;
-                    }
-                    const uint64_t *grp_k = s_arr + s_start[p];
-                    // whole batches: behind the group lie smaller keys
-                    for (int j0 = 0; j0 < d && r < g; j0 += 8) {
-                        uint64_t k8[8];
+                if (e < props) {
+                    const uint64_t mine = s_mem[e];
+                    const int bin = bin_of(mine), s0 = s_bin[bin], s1 = s_bin[bin + 1];
+                    int r = s0 - s_bin[match_pattern(mine) << nbl2];      // the larger bins
+                    // whole batches: behind the bin lie smaller keys
+                    for (int j0 = s0; j0 < s1 && r < g; j0 += 4) {
+                        uint64_t k4[4];
 #pragma unroll
-                        for (int u = 0; u < 8; u++) k8[u] = grp_k[j0 + u];
+                        for (int u = 0; u < 4; u++) k4[u] = s_mem[j0 + u];
 #pragma unroll
-                        for (int u = 0; u < 8; u++) r += k8[u] > mine ? 1 : 0;
+                        for (int u = 0; u < 4; u++) r += k4[u] > mine ? 1 : 0;
                     }
                     key[i] = mine;
                     pos[i] = r;
                 }
             }
-            uint64_t mkey[CPT];      // kept keys that move, and by how much
-            int mshift[CPT];
-            if (round > 0) {
-#pragma unroll
-                for (int i = 0; i < CPT; i++) {
-                    const int s = tt + NT * i;
-                    mshift[i] = 0;
-                    if (s < cols) {
-                        const int p = group_of(s), d = s_dem[p];
-                        if (d > 0) {
-                            mkey[i] = s_mem[s];
-                            const uint64_t *grp_k = s_arr + s_start[p];
-                            if (mkey[i] != 0)
-                                for (int j = 0; j < d; j++) mshift[i] += grp_k[j] > mkey[i] ? 1 : 0;
-                        }
-                    }
-                }
-            }
-            if (tt == 0) s_np[0] = 0;
+            for (int p = tt; p < c; p += NT) s_occ[p] = min(g, s_bin[(p + 1) << nbl2] - s_bin[p << nbl2]);
             match_sync<NT>();
-            // 4. the new lists; what a pattern has no slot for is pending
-            if (round > 0) {
-#pragma unroll
-                for (int i = 0; i < CPT; i++)
-                    if (mshift[i] > 0) {
-                        const int p = match_pattern(mkey[i]);
-                        const int s = tt + NT * i + mshift[i];
-                        if (s - p * g < g) s_mem[s] = mkey[i];
-                        else s_arr[atomicAdd(s_np, 1)] = (uint64_t)match_column(mkey[i]);
-                    }
-            }
+            // 4. the new lists in the place of the sorted keys; what a pattern has no slot for is pending
 #pragma unroll
             for (int i = 0; i < CPT; i++)
-                if (i < nr && key[i] != 0) {
-                    const int p = match_pattern(key[i]);
-                    if (pos[i] < g) s_mem[p * g + pos[i]] = key[i];
-                    else s_arr[atomicAdd(s_np, 1)] = (uint64_t)match_column(key[i]);
+                if (key[i] != 0) {
+                    if (pos[i] < g) {
+                        s_mem[match_pattern(key[i]) * g + pos[i]] = key[i];
+                    } else {
+                        const int k = atomicAdd(s_np, 1);
+                        if (k < few) pending[k] = (uint16_t)match_column(key[i]);
+                    }
                 }
-            for (int p = tt; p < c; p += NT) {
-                s_occ[p] = min(g, s_occ[p] + s_dem[p]);
-                s_dem[p] = 0;
-            }
+            for (int p = tt; p < c; p += NT)
+                for (int s = s_occ[p]; s < g; s++) s_mem[p * g + s] = 0;
             match_sync<NT>();
             pend = s_np[0];
         }
@@ -917,13 +986,13 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
             // Later rounds: a few columns, whatever the pattern.  L lanes hold a pattern's list, KPL keys each in descending
             // order, and insert a proposal by one shift along the lanes.  A pattern takes at most `bucket` proposals in a round;
             // the rest stay pending.  In a tile of several wavefronts the first one ends the matching alone, without barriers.
-            constexpr int EIGHT = 8, KPL = SG > 16 ? 2 : 1;
-            const int ll = SG != 0 ? 4 : Q.lanes_log2, L = 1 << ll, bucket = min(g / 2, 8);
+            constexpr int EIGHT = 8, LL = SG > 16 && SC <= 8 ? 4 : 3, KPL = SG > 8 << (LL - 2) ? 4 : 2;
+            const int ll = SG != 0 ? LL : Q.lanes_log2, L = 1 << ll, bucket = min(g / 2, 8);
             static_assert(SG <= 32 && SG != 1, "a list fits its lanes; lists and buckets fit the proposals' place");
-            uint16_t *pending = (uint16_t *)s_arr, *next = pending + cols;
-            uint64_t *s_bkt = s_arr + (cols + 1) / 2;      // free places hold 0
-            {
-                constexpr int I = (CPT + 3) / 4;      // the columns left over come as entries of eight bytes
+            uint16_t *next = pending + few;
+            uint64_t *s_bkt = s_arr + (few + 1) / 2;      // free places hold 0
+            if (real_rows < m) {
+                constexpr int I = (CPT + 3) / 4;      // a partial block's columns come as entries of eight bytes
                 uint16_t o[I];
 #pragma unroll
                 for (int i = 0; i < I; i++) o[i] = tt + NT * i < pend ? (uint16_t)s_arr[tt + NT * i] : 0;
@@ -931,8 +1000,8 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 #pragma unroll
                 for (int i = 0; i < I; i++)
                     if (tt + NT * i < pend) pending[tt + NT * i] = o[i];
-                for (int i = tt; i < c * bucket; i += NT) s_bkt[i] = 0;
             }
+            for (int i = tt; i < c * bucket; i += NT) s_bkt[i] = 0;
             // a column's patterns go to EL lanes; the positions of a lane's patterns stay in registers
             constexpr int EL = SC >= 16 ? 8 : SC >= 8 ? 4 : 2, PER = SG != 0 ? (SC + EL - 1) / EL : 1;
             uint32_t mypos[PER];
@@ -940,13 +1009,13 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 #pragma unroll
                 for (int i = 0; i < PER; i++) mypos[i] = s_pos[min(tt % EL + EL * i, SC - 1)];
             }
-            int round = 0;
-            auto late = [&](auto active_tag, int until) {      // threads of the tile that take part
+            round = 0;
+            auto late = [&](auto active_tag, int until) __attribute__((always_inline)) {      // threads of the tile that take part
                 constexpr int A = decltype(active_tag)::value, W = A < 64 ? A : 64, WAVES = A / W;
                 const int rows_log2 = (W == 64 ? 6 : W == 32 ? 5 : 4) - ll, rows = 1 << rows_log2;
                 const int wave = tt / W, lane = tt % W, row = lane >> ll, r = lane & (L - 1);
-                for (const int limit = cols * c + 2; round < limit && pend > until; round++) {
-                    match_sync<A>();
+                match_sync<A>();
+                for (; round < limit && pend > until; round++) {
                     int *count = s_np + 2 + (round & 1);      // zero; the other one is cleared on the way
                     auto put = [&](int o, uint64_t key) {
                         if (key == 0) {
@@ -957,49 +1026,53 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                         if (place < bucket) s_bkt[p * bucket + place] = key;
                         else next[atomicAdd(count, 1)] = (uint16_t)o;
                     };
-                    auto best_of = [&](int o, int p, uint32_t ps, uint32_t &best, int &bp) {
+                    // score (0: refused) and pattern of a column's edge.  No branch: the reads of a lane's patterns go out together.
+                    auto edge = [&](int o, int p, uint32_t ps) {
                         float acc = match_abs(s_d[at(o, (int)(ps & 15u))]);
 #pragma unroll
                         for (int j = 1; j < n; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
-                        const uint32_t sb = __float_as_uint(acc);
-                        if (sb >= best && match_key(sb, o, p) > s_mem[p * g + g - 1]) {
-                            best = sb;
-                            bp = p;
-                        }
+                        uint32_t sb = __float_as_uint(acc);
+                        if (!(match_key(sb, o, p) > s_mem[p * g + g - 1])) sb = 0;
+                        return ((uint64_t)sb << 32) | (uint32_t)p;
                     };
-                    // (Many patterns and more than twice as many columns as lanes: a column per lane is as much work without the exchange
-                    // between lanes.  With fewer its last pass leaves most lanes idle: a lone tile of 2240 real columns, 4:8:32, has 300
-                    // of them.  us, a column per lane from A / EL columns on -> from 2 A on: 2240 x 1024 fp16 61 -> 53, 4096 x 4096 fp16 133 -> 123,
-                    // fp32 209 -> 191; 1024 x 1024, with few pending columns, 20.5 either way.)
-                    if (SG != 0 && (SC <= 32 || pend <= 2 * A)) {
+                    auto other = [&](uint64_t top, auto ctrl) {      // the larger one of two lanes
+                        asm("s_nop 1" : "+v"(top));
+                        return match_larger(top, match_swap<decltype(ctrl)::value>(top));
+                    };
+                    constexpr std::integral_constant<int, 0xB1> by_1{};      // lanes 1 apart, 2 apart, the two quads
+                    constexpr std::integral_constant<int, 0x4E> by_2{};
+                    constexpr std::integral_constant<int, 0x141> by_4{};
+                    // A column's patterns over EL lanes, or a column per lane, which is less work where there are enough columns for it: in
+                    // tiles of a wavefront from a quarter of the lanes on (us, 4096 x 4096 3:6:12 from 16 / 32 / never: 61.3 / 63.3 / 63.7), with
+                    // many patterns from twice as many as lanes on (4:8:32 from 32 / 1024: 85 / 73).
+                    if (SG != 0 && (A <= 64 ? pend <= A / 4 : SC <= 32 || pend <= 2 * A)) {
                         const int sub = tt % EL;
                         for (int e = tt / EL; e < pend; e += A / EL) {
                             const int o = (int)pending[e];
-                            uint32_t best = 0;
-                            int bp = 0;
+                            uint64_t top = 0;
 #pragma unroll
-                            for (int i = 0; i < PER; i++) best_of(o, min(sub + EL * i, SC - 1), mypos[i], best, bp);
-                            uint64_t top = ((uint64_t)best << 32) | (uint32_t)bp;
-                            top = max(top, match_swap<0xB1>(top));                    // lanes 1 apart, 2 apart, the two quads
-                            if (EL >= 4) top = max(top, match_swap<0x4E>(top));
-                            if (EL >= 8) top = max(top, match_swap<0x141>(top));
+                            for (int i = 0; i < PER; i++) {
+                                top = match_larger(top, edge(o, min(sub + EL * i, SC - 1), mypos[i]));
+                                if (PER > 4 && i % 3 == 2) asm volatile("" : "+v"(top)::"memory");      // (all reads at once do not fit the registers)
+                            }
+                            top = other(top, by_1);
+                            if (EL >= 4) top = other(top, by_2);
+                            if (EL >= 8) top = other(top, by_4);
                             if (sub == 0) put(o, (top >> 32) == 0 ? 0 : match_key((uint32_t)(top >> 32), o, (int)(top & 0xFFu)));
                         }
                     } else if (SG == 0 && c > 8 && pend * EIGHT <= A) {
                         const int e = tt / EIGHT, sub = tt % EIGHT;
                         if (e < pend) {
                             const int o = (int)pending[e];
-                            uint32_t best = 0;
-                            int bp = 0;
+                            uint64_t top = 0;
 #pragma unroll 3
                             for (int i = 0; i < (c + EIGHT - 1) / EIGHT; i++) {
                                 const int p = min(sub + EIGHT * i, c - 1);
-                                best_of(o, p, s_pos[p], best, bp);
+                                top = match_larger(top, edge(o, p, s_pos[p]));
                             }
-                            uint64_t top = ((uint64_t)best << 32) | (uint32_t)bp;
-                            top = max(top, match_swap<0xB1>(top));
-                            top = max(top, match_swap<0x4E>(top));
-                            top = max(top, match_swap<0x141>(top));
+                            top = other(top, by_1);
+                            top = other(top, by_2);
+                            top = other(top, by_4);
                             if (sub == 0) put(o, (top >> 32) == 0 ? 0 : match_key((uint32_t)(top >> 32), o, (int)(top & 0xFFu)));
                         }
                     } else {
@@ -1009,17 +1082,20 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                         }
                     }
                     match_sync<A>();
-                    // a pattern's proposals into its list, AT at a time (compiled patterns: two, their buckets hold an even number; any
-                    // other n:m:g may have an odd one and takes one at a time, two were not tried for it)
+                    // a pattern's proposals into its list, two at a time
                     auto merge = [&](int p) {
-                        constexpr int AT = SG != 0 ? 2 : 1;
-                        static_assert(SG == 0 || (SG / 2 < 8 ? SG / 2 : 8) % AT == 0, "whole batches");
+                        constexpr int AT = 2;
+                        constexpr bool EVEN = SG != 0 && (SG / 2 < 8 ? SG / 2 : 8) % AT == 0;      // whole batches, zeros behind the last
                         uint64_t *list = s_mem + p * g + r * KPL, *bkt = s_bkt + p * bucket;
                         uint64_t key[KPL], in[AT], ahead[AT];
+                        // what the list will have no place for is known beforehand: one request for its places
+                        const int asked = min(s_dem[p], bucket), had = s_occ[p], refused = had + asked - g;
+                        int to = 0;
+                        if (r == (g - 1) / KPL && refused > 0) to = atomicAdd(count, refused);
 #pragma unroll
                         for (int i = 0; i < KPL; i++) key[i] = r * KPL + i < g ? list[i] : 0;
 #pragma unroll
-                        for (int u = 0; u < AT; u++) in[u] = bkt[u];
+                        for (int u = 0; u < AT; u++) in[u] = EVEN || u < asked ? bkt[u] : 0;
                         for (int j = AT; in[0] != 0; j += AT) {
 #pragma unroll
                             for (int u = 0; u < AT; u++) ahead[u] = bkt[j + u];      // (the last batch reads past the bucket)
@@ -1027,56 +1103,47 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 #pragma unroll
                             for (int u = 0; u < AT; u++) {
                                 // key(i) = max(key(i), min(key(i - 1), in)): the keys are positive doubles and no NaN
-                                auto lo = [](uint64_t x, uint64_t y) {
-                                    return __builtin_bit_cast(uint64_t, __builtin_fmin(__builtin_bit_cast(double, x), __builtin_bit_cast(double, y)));
-                                };
-                                auto hi = [](uint64_t x, uint64_t y) {
-                                    return __builtin_bit_cast(uint64_t, __builtin_fmax(__builtin_bit_cast(double, x), __builtin_bit_cast(double, y)));
-                                };
+                                asm("s_nop 1" : "+v"(key[KPL - 1]));      // (a move between lanes reads a result two instructions later at the earliest)
                                 uint64_t before = match_swap<(SG != 0 ? 0x111 : 0x138)>(key[KPL - 1]);      // row_shr:1, wave_shr:1
                                 if (r == 0) before = in[u];
-                                out[u] = lo(key[(g - 1) % KPL], in[u]);
+                                out[u] = match_smaller(key[(g - 1) % KPL], in[u]);
 #pragma unroll
-                                for (int i = KPL - 1; i > 0; i--) key[i] = hi(key[i], lo(key[i - 1], in[u]));
-                                key[0] = hi(key[0], lo(before, in[u]));
+                                for (int i = KPL - 1; i > 0; i--) key[i] = match_larger(key[i], match_smaller(key[i - 1], in[u]));
+                                key[0] = match_larger(key[0], match_smaller(before, in[u]));
                             }
-                            if (r == (g - 1) / KPL) {      // what the list has no place for
-                                int has = 0;
+                            if (r == (g - 1) / KPL) {
 #pragma unroll
-                                for (int u = 0; u < AT; u++) has += out[u] != 0 ? 1 : 0;
-                                if (has != 0) {
-                                    int to = atomicAdd(count, has);
-#pragma unroll
-                                    for (int u = 0; u < AT; u++)
-                                        if (out[u] != 0) next[to++] = (uint16_t)match_column(out[u]);
-                                }
+                                for (int u = 0; u < AT; u++)
+                                    if (out[u] != 0) next[to++] = (uint16_t)match_column(out[u]);
                             }
 #pragma unroll
-                            for (int u = 0; u < AT; u++) in[u] = j < bucket ? ahead[u] : 0;
+                            for (int u = 0; u < AT; u++) in[u] = (EVEN ? j < bucket : j + u < asked) ? ahead[u] : 0;
                         }
 #pragma unroll
                         for (int i = 0; i < KPL; i++)
                             if (r * KPL + i < g) list[i] = key[i];
                         if (r < bucket) bkt[r] = 0;
-                        if (r == 0) s_dem[p] = 0;
-                    };
-                    // The patterns with proposals, `rows` at a time; wavefront w has those with p / rows = w (mod WAVES).
-                    for (int p0 = 0; p0 < c; p0 += W) {
-                        const int dl = p0 + lane < c && ((p0 + lane) >> rows_log2) % WAVES == wave ? s_dem[p0 + lane] : 0;
-                        uint64_t open = __ballot(dl > 0);
-                        if (W < 64) open = (open >> (threadIdx.x & 63 & ~(W - 1))) & ((1ull << (W & 63)) - 1);
-                        using Bits = typename std::conditional<W == 64, uint64_t, uint32_t>::type;
-                        Bits left = (Bits)open;
-                        while (left != 0) {
-                            int p = -1;
-#pragma unroll
-                            for (int i = 0; i < rows; i++) {
-                                const int q = W == 64 ? __ffsll((unsigned long long)left) : __ffs((unsigned)left);      // 0: none
-                                if (row == i) p = q - 1;
-                                left &= left - 1;
-                            }
-                            if (p >= 0) merge(p0 + p);
+                        if (r == 0) {
+                            s_dem[p] = 0;
+                            s_occ[p] = min(had + asked, g);
                         }
+                    };
+                    if constexpr (WAVES > 1) {
+                        // a pattern to every list of lanes, in as many turns as that takes
+                        for (int p = wave * rows + row; p < c; p += WAVES * rows)
+                            if (s_dem[p] != 0) merge(p);
+                    } else {
+                        // the patterns with proposals, numbered through
+                        int open = 0;
+                        for (int p0 = 0; p0 < c; p0 += W) {
+                            const bool has = p0 + lane < c && s_dem[p0 + lane] != 0;
+                            uint64_t b = __ballot(has);
+                            if (W < 64) b = (b >> (threadIdx.x & 63 & ~(W - 1))) & ((1ull << (W & 63)) - 1);
+                            if (has) s_start[open + __popcll(b & ((1ull << lane) - 1))] = p0 + lane;
+                            open += __popcll(b);
+                        }
+                        match_sync<W>();
+                        for (int k = row; k < open; k += rows) merge(s_start[k]);
                     }
                     if (tt == 0) s_np[2 + ((round & 1) ^ 1)] = 0;
                     match_sync<A>();
@@ -1095,13 +1162,6 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                 __syncthreads();
             } else {
                 late(std::integral_constant<int, NT>{}, 0);
-                match_sync<NT>();
-            }
-            if (real_cols - s_np[1] < cols) {      // slots taken per pattern, for the columns that come last
-                for (int p = tt; p < c; p += NT) s_occ[p] = 0;
-                match_sync<NT>();
-                for (int s = tt; s < cols; s += NT)
-                    if (s_mem[s] != 0) atomicAdd(&s_occ[group_of(s)], 1);
                 match_sync<NT>();
             }
         }
@@ -1228,9 +1288,14 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     auto up = [](int x, int a) { return (x + a - 1) / a * a; };
     int off = RC ? m * up(cols, V) * (int)sizeof(T) : up(cols * m * (int)sizeof(T), 16);
     Q.r_mem = off;
-    off += cols * 8;
+    off = up(off + cols * 8 + kMatchPad, 16);
+    // Lists of 2 to 64 keys that fit the lanes of a tile.  Below 32 columns a round over all of them is the shorter way
+    // (4096 x 4096 fp16, lists -> rounds: 2:4:4 204 -> 192 us, 1:2:8 238 -> 215; from there on 2:4:8 147 -> 140, 2:4:32
+    // 131 -> 117, 2:8:8 188 -> 140, 4:8:16 482 -> 365, rounds -> lists).
+    Q.lanes_log2 = Q.g < 2 || Q.g > 128 ? 0 : Q.g <= 16 ? 3 : Q.g <= 32 ? 4 : Q.g <= 64 ? 5 : 6;
+    if ((1 << Q.lanes_log2) > NT || cols < 24) Q.lanes_log2 = 0;
     Q.r_arr = off;
-    off += cols * 8 + kMatchPad;
+    off += match_scratch(cols, c, Q.g, match_bins_log2(NT, c), SG != 0 || Q.lanes_log2 != 0, Q.view.S % m != 0, cols / match_few(SG));
     Q.r_int = off;
     off = up(off + (kMatchTables * c + 4) * 4, 16);
     constexpr int LDS = 160 * 1024, MOST = match_waves(NT, SM != 0, RC) * 4 / (THREADS / 64);      // workgroups that fit a CU's wavefronts
@@ -1254,11 +1319,6 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     // four, 4096 x 4096 fp16 2:4:64 118 / 157 and 2:8:16 130 / 135, the latter in fp32 (22 KB a tile) 162 / 137;
     // 777 x 1001 fp16 2:4:64 (750 tiles) 52 / 39, 2:8:16 85 / 56.
     if (NT == 128 && (lds > 20 * 1024 || Q.outer < 8 * 256)) return NMG_OK;
-    // Lists of 2 to 64 keys that fit the lanes of a tile.  Below 32 columns a round over all of them is the shorter way
-    // (4096 x 4096 fp16, lists -> rounds: 2:4:4 204 -> 192 us, 1:2:8 238 -> 215; from there on 2:4:8 147 -> 140, 2:4:32
-    // 131 -> 117, 2:8:8 188 -> 140, 4:8:16 482 -> 365, rounds -> lists).
-    Q.lanes_log2 = Q.g < 2 || Q.g > 64 ? 0 : Q.g <= 16 ? 4 : Q.g <= 32 ? 5 : 6;
-    if ((1 << Q.lanes_log2) > NT || cols < 32) Q.lanes_log2 = 0;
     Q.out4 = cols % 4 == 0 && (uintptr_t)Q.val % 16 == 0 && (uintptr_t)Q.idx % 8 == 0;
     auto kern = match_kernel<T, NT, CPT, SN, SM, SG, RC>;
     if (lds > 64 * 1024)

@@ -158,3 +158,33 @@ def test_largest_tiles_with_a_partial_block(n, m, g, along):
     t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
     assert np.array_equal(to_np(t.idx), idx)
     assert same_bits(t.val, val)
+
+
+# The first round sorts by pattern and by bins of the score, four to an octave (two where a tile has many patterns): scores in one bin, at the bins'
+# bounds, many octaves below the largest, subnormal, infinite.  Lists of up to 128 keys, two or four to a lane; tiles of 23 and 24 columns.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,m,g", [(2, 4, 16), (1, 8, 32), (3, 6, 12), (2, 8, 32), (4, 8, 32), (2, 4, 4), (1, 4, 6), (1, 4, 5), (2, 4, 65),
+                                   (1, 4, 128), (1, 4, 129), (3, 8, 8), (4, 8, 6)])
+def test_scores_of_any_size(n, m, g, dtype):
+    cols = math.comb(m, n) * g
+    gen = torch.Generator().manual_seed(n * 100 + m * 10 + g)
+    for kind in ("equal", "powers", "tails", "subnormal", "infinite"):
+        w = torch.randn(cols + cols // 2, 2 * m, generator=gen)
+        if kind == "equal":
+            w = torch.full_like(w, 0.5)
+        elif kind == "powers":
+            w = 2.0 ** torch.randint(-9, 1, w.shape, generator=gen) * (1 + 0.25 * torch.randint(0, 4, w.shape, generator=gen))
+        elif kind == "tails":
+            w = w * torch.exp(2 * torch.randn(w.shape, generator=gen))
+        elif kind == "subnormal":
+            w = w * 8 * torch.finfo(dtype).smallest_normal / 64
+        else:
+            w[torch.rand(w.shape, generator=gen) < 0.05] = math.inf
+        w = w.to(dtype)
+        for along in (0, 1):
+            x = w if along == 1 else w.t().contiguous()
+            print(f"case {n}:{m}:{g} {dtype} {kind} along={along}", flush=True)
+            val, idx, _ = oracle_sparsify(x, n, m, along, g, 1 - along)
+            t = sten.GroupedNMTensor.from_dense(x.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
+            assert np.array_equal(to_np(t.idx), idx)
+            assert same_bits(t.val, val)
