@@ -240,6 +240,15 @@ int nmg_gemm_nn(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void
 int nmg_gemm_tn(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy,
                 const void *d_bias, int64_t O, int64_t K, int64_t T, int dtype, void *stream);
 
+/* The single-precision product (`form` 0: nmg_gemm_nt, 1: nmg_gemm_nn, 2: nmg_gemm_tn) on the bf16 matrix cores with the reduction cut into
+ * slices, which a second kernel adds up in order: products whose results are too few tiles for the chip (1021 x 1999
+ * results over 2047: 85 us whole, 66 in two slices).  nmg_gemm_f32_plan gives the number of slices (1: the entry points
+ * above) and the bytes of its workspace. */
+int nmg_gemm_f32_plan(int64_t lda, int64_t ldx, int64_t O, int64_t K, int64_t T, int form, int *slices, int64_t *workspace_bytes);
+int nmg_gemm_f32_splitk(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy, const void *d_bias,
+                        int64_t O, int64_t K, int64_t T, int form, int slices, void *d_workspace, int64_t workspace_bytes,
+                        void *stream);
+
 /* dst [dst_rows, dst_cols] = src [rows, cols] in a 16-bit type, zeros beyond the source; any pitches and
  * alignments.  Brings operands into the shape of the matrix-core products (row starts, K steps), or a padded
  * result back.  No counterpart in the reference. */

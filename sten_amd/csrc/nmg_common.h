@@ -49,6 +49,11 @@ int dense_rows16(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, voi
 // launched, where it does not take the extents or is not expected to beat `other_us`.
 bool split3_gemm(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy, const void *d_bias, int64_t O,
                  int64_t K, int64_t T, int form, double other_us, hipStream_t st);
+// The slices of the reduction with which it is fastest, and its time in us (1e30: extents that it does not take); the product in
+// slices, their sums at d_part [slices][T][O up to a multiple of 4].
+double split3_plan(int64_t lda, int64_t ldx, int64_t O, int64_t K, int64_t T, int form, int *slices);
+int split3_gemm_slices(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy, const void *d_bias, int64_t O,
+                       int64_t K, int64_t T, int form, int slices, float *d_part, hipStream_t st);
 // Y[G, S] = L[T, G]^T P[T, S] (+ bias[s]) in a 16-bit type on the matrix cores (nmg_sddmm.hip).
 int dense_tn16(const void *d_lines, int64_t ld_lines, const void *d_pos, int64_t ld_pos, int64_t T, int64_t G, int64_t S,
                void *d_y, int64_t ldy, const void *d_bias, int dtype, void *stream);

@@ -1017,6 +1017,29 @@ static const GemmF32Shape kGemmF32Shapes[] = {
     {128, 128, 1.00}, {128, 96, 0.97}, {128, 64, 0.92}, {64, 96, 0.88}, {64, 64, 0.80}, {32, 32, 0.55},
 };
 
+// One round of 16 x 16 tiles (a second one costs more than it gains: 768 x 768, 100 tokens 7.6 against 8.7).
+static bool gemm_f32_few(int64_t O, int64_t T, int form)
+{
+    return form == 0 && O <= 4096 && T <= 4096 && ((O + 15) / 16) * ((T + 15) / 16) <= 256;
+}
+
+// The tile of a product on the fp32 instruction and its time in us (guards cost a fifth; 64 x 64 and 32 x 32 take less than their share of
+// the rule above).
+static double gemm_f32_us(int64_t O, int64_t K, int64_t T, int form, bool even, int *shape)
+{
+    double best_cost = 0;
+    int64_t rounds = 0;
+    for (int c = 0; c < (int)(sizeof(kGemmF32Shapes) / sizeof(kGemmF32Shapes[0])); c++) {
+        const GemmF32Shape &S = kGemmF32Shapes[c];
+        const int64_t tiles = ((T + S.bm - 1) / S.bm) * ((O + S.bn - 1) / S.bn);
+        const double eff = form == 2 && S.bm == 64 && S.bn == 96 ? 0.68 : S.eff;
+        const double cost = (double)((tiles + 255) / 256) * S.bm * S.bn / eff;
+        if (c == 0 || cost < best_cost) { *shape = c; best_cost = cost; rounds = (tiles + 255) / 256; }
+    }
+    even = even && K % 32 == 0 && (form < 1 || O % 4 == 0) && (form < 2 || T % 4 == 0);
+    return best_cost * 3.63e-6 * (double)K * (even ? 1.0 : 1.2) * (*shape >= 4 ? 0.91 : 1.0) + 3.5 + 1.25 * (double)rounds;
+}
+
 }  // namespace nmg
 
 using namespace nmg;
@@ -1042,26 +1065,14 @@ static int gemm_f32_host(const void *d_a, int64_t lda, const void *d_x, int64_t 
     Q.vec = (lda % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)d_a % 16) == 0 && ((uintptr_t)d_x % 16) == 0) ? 1 : 0;
     hipStream_t st = (hipStream_t)stream;
     NMG_REQUIRE((T + 31) / 32 <= 65535, NMG_ERR_UNSUPPORTED, "too many tokens for one launch");
-    // one round of 16 x 16 tiles (a second one costs more than it gains: 768 x 768, 100 tokens 7.6 against 8.7)
-    if (form == 0 && O <= 4096 && T <= 4096 && ((O + 15) / 16) * ((T + 15) / 16) <= 256) {
+    if (gemm_f32_few(O, T, form)) {
         hipLaunchKernelGGL(gemm_f32_few_kernel, dim3((unsigned)((O + 15) / 16), (unsigned)((T + 15) / 16)), dim3(1024), 0, st, Q);
         NMG_HIP_TRY(hipGetLastError());
         return NMG_OK;
     }
     int best = 0;
-    double best_cost = 0;
-    int64_t rounds = 0;
-    for (int c = 0; c < (int)(sizeof(kGemmF32Shapes) / sizeof(kGemmF32Shapes[0])); c++) {
-        const GemmF32Shape &S = kGemmF32Shapes[c];
-        const int64_t tiles = ((T + S.bm - 1) / S.bm) * ((O + S.bn - 1) / S.bn);
-        const double eff = form == 2 && S.bm == 64 && S.bn == 96 ? 0.68 : S.eff;
-        const double cost = (double)((tiles + 255) / 256) * S.bm * S.bn / eff;
-        if (c == 0 || cost < best_cost) { best = c; best_cost = cost; rounds = (tiles + 255) / 256; }
-    }
-    // its time in us (guards cost a fifth; 64 x 64 and 32 x 32 take less than their share of the rule above), and 4 % to make the other
-    // kernel worth while
-    const bool even = Q.vec && K % 32 == 0 && (form < 1 || O % 4 == 0) && (form < 2 || T % 4 == 0);
-    const double us = best_cost * 3.63e-6 * (double)K * (even ? 1.0 : 1.2) * (best >= 4 ? 0.91 : 1.0) + 3.5 + 1.25 * (double)rounds;
+    const double us = gemm_f32_us(O, K, T, form, Q.vec, &best);
+    // (4 % to make the other kernel worth while)
     if (split3_gemm(d_a, lda, d_x, ldx, d_y, ldy, d_bias, O, K, T, form, 0.96 * us, st)) {
         NMG_HIP_TRY(hipGetLastError());
         return NMG_OK;
@@ -1076,6 +1087,47 @@ static int gemm_f32_host(const void *d_a, int64_t lda, const void *d_x, int64_t 
     }
     NMG_HIP_TRY(hipGetLastError());
     return NMG_OK;
+}
+
+extern "C" int nmg_gemm_f32_plan(int64_t lda, int64_t ldx, int64_t O, int64_t K, int64_t T, int form, int *slices, int64_t *workspace_bytes)
+{
+    NMG_REQUIRE(O >= 0 && K >= 0 && T >= 0 && form >= 0 && form <= 2, NMG_ERR_ARG, "negative extent, or no such form");
+    NMG_REQUIRE(slices && workspace_bytes, NMG_ERR_ARG, "null output pointer");
+    *slices = 1;
+    *workspace_bytes = 0;
+    if (O == 0 || K == 0 || T == 0 || gemm_f32_few(O, T, form)) return NMG_OK;
+    // Against the time on the fp32 instruction, which the model above puts too high or too low here, by form and tile (165 products of 2^27 to
+    // 2^33 multiplications with at most 140 tiles of 128 x 128, all forms, odd extents among them, in every number of slices: with this choice
+    // they take 0.935 of the time of whole ones, with the best 0.93, none more than 1 % longer than whole).  us, whole -> slices: 256 x 2176
+    // results over 2724, both operands reduction-major 100 -> 38, 1024 x 1024 over 4096 74.5 -> 59, 1021 x 1999 over 2047 85 -> 66, 768 x 2673
+    // over 3200 108 -> 83; below about 30 us the two launches cost more than they save (1024 x 176 over 1152: 9.8, 19.8).
+    int shape, best;
+    const double us = split3_plan(lda, ldx, O, K, T, form, &best);
+    const bool even = lda % 4 == 0 && ldx % 4 == 0;
+    const double fixed = 4.75, model = gemm_f32_us(O, K, T, form, even, &shape) - fixed;
+    const bool guards = !(even && K % 32 == 0 && O % 4 == 0 && T % 4 == 0);
+    const double whole = fixed + model * (form == 0 ? (shape == 5 ? 0.7 : 1.0) : form == 1 ? (shape == 5 ? 0.85 : shape == 4 ? 1.2 : 1.0) : guards ? 1.4 : 1.0);
+    if (best > 1 && us < 0.95 * whole) {
+        *slices = best;
+        *workspace_bytes = best * T * ((O + 3) / 4 * 4) * 4;
+    }
+    return NMG_OK;
+}
+
+extern "C" int nmg_gemm_f32_splitk(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy, const void *d_bias,
+                                   int64_t O, int64_t K, int64_t T, int form, int slices, void *d_workspace, int64_t workspace_bytes,
+                                   void *stream)
+{
+    NMG_REQUIRE(O >= 0 && K >= 0 && T >= 0 && form >= 0 && form <= 2, NMG_ERR_ARG, "negative extent, or no such form");
+    NMG_REQUIRE(lda >= (form == 0 ? K : O) && ldx >= (form == 2 ? T : K) && ldy >= O, NMG_ERR_ARG, "leading dimension smaller than row length");
+    if (slices <= 1) return gemm_f32_host(d_a, lda, d_x, ldx, d_y, ldy, d_bias, O, K, T, form, stream);
+    if (O == 0 || T == 0) return NMG_OK;
+    NMG_REQUIRE(slices <= 256, NMG_ERR_ARG, "%d slices", slices);
+    const int64_t need = slices * T * ((O + 3) / 4 * 4) * 4;
+    NMG_REQUIRE(d_workspace && workspace_bytes >= need && ((uintptr_t)d_workspace % 16) == 0, NMG_ERR_ARG,
+                "workspace of %lld bytes (16-byte aligned) needed, %lld given", (long long)need, (long long)workspace_bytes);
+    NMG_REQUIRE(d_a && d_x && d_y, NMG_ERR_ARG, "null device pointer");
+    return split3_gemm_slices(d_a, lda, d_x, ldx, d_y, ldy, d_bias, O, K, T, form, slices, (float *)d_workspace, (hipStream_t)stream);
 }
 
 extern "C" int nmg_gemm_nn(const void *d_a, int64_t lda, const void *d_x, int64_t ldx, void *d_y, int64_t ldy,

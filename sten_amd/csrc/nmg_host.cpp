@@ -441,6 +441,19 @@ Tensor workspace(int64_t floats, const Tensor &like) { return new_empty({std::ma
 
 int64_t split_ws(int slices, int64_t T, int64_t O) { return slices * T * up(O, 256) * 256; }
 
+// A product in single precision, operands as they lie (form 0: nmg_gemm_nt, 1: nmg_gemm_nn, 2: nmg_gemm_tn), its reduction in slices where
+// its results are too few tiles for the chip.
+void product_f32(int form, const Tensor &a, int64_t lda, const Tensor &x, int64_t ldx, Tensor &y, const void *bias, int64_t O, int64_t K, int64_t T)
+{
+    int slices = 1;
+    int64_t bytes = 0;
+    check(nmg_gemm_f32_plan(lda, ldx, O, K, T, form, &slices, &bytes));
+    Tensor ws;
+    if (slices > 1) ws = workspace(bytes / 4, y);
+    check(nmg_gemm_f32_splitk(a.data_ptr(), lda, x.data_ptr(), ldx, y.data_ptr(), O, bias, O, K, T, form, slices,
+                              slices > 1 ? ws.data_ptr() : nullptr, bytes, stream_of(y)));
+}
+
 // The code of the kernel that takes what no other route does; KeyError for a name that there is no kernel of.
 int kernel_code(const std::string &name)
 {
@@ -676,8 +689,7 @@ Tensor spmm(State &w, Tensor x, Tensor bias, int rd, const char *kernel)
         // One dense copy [R, C] serves both directions: row-major operand of the product that
         // reduces along dim 1, reduction-major operand of the one that reduces along dim 0.
         Tensor a = dense_operand(w, 1, opt.cache_dense, 1);
-        auto entry = rd == 1 ? nmg_gemm_nt : nmg_gemm_nn;
-        check(entry(a.data_ptr(), a.stride(0), xp, ldx, yp, O, bp, O, K, T, dt, stream));
+        product_f32(rd == 1 ? 0 : 1, a, a.stride(0), x, ldx, y, bp, O, K, T);
         return y;
     }
     const int64_t Kp = round_up(K, 64);
@@ -712,10 +724,8 @@ Tensor mm_f32(State &w, Tensor b, int rd, const Options &opt)
     const int64_t N = b.size(1);
     // the one dense copy [R, C]: row-major row operand of W @ B, reduction-major row operand of W^T @ B
     Tensor wd = dense_operand(w, 1, opt.cache_dense, 1);
-    auto entry = rd == 1 ? nmg_gemm_nn : nmg_gemm_tn;
     Tensor c = new_empty({O, N}, b);
-    check(entry(b.data_ptr(), K > 1 ? b.stride(0) : N, wd.data_ptr(), wd.stride(0), c.data_ptr(), N, nullptr, N, K, O,
-                dtype_code(b.scalar_type()), stream_of(b)));
+    product_f32(rd == 1 ? 1 : 2, b, K > 1 ? b.stride(0) : N, wd, wd.stride(0), c, nullptr, N, K, O);
     return c;
 }
 
@@ -936,8 +946,7 @@ Tensor dense_product(bool tn, Tensor x, Tensor a)
             a = a.to(at::kFloat).contiguous();
         }
         Tensor y = new_empty({T, O}, x);
-        auto entry = tn ? nmg_gemm_tn : nmg_gemm_nt;
-        check(entry(a.data_ptr(), a.stride(0), x.data_ptr(), x.stride(0), y.data_ptr(), O, nullptr, O, K, T, NMG_F32, stream));
+        product_f32(tn ? 2 : 0, a, a.stride(0), x, x.stride(0), y, nullptr, O, K, T);
         return half ? y.to(dt) : y;
     }
     if (tn) {

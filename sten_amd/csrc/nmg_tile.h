@@ -3,6 +3,8 @@
 #pragma once
 #include "nmg_common.h"
 
+#include <type_traits>
+
 namespace nmg {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -350,17 +352,22 @@ template <typename T, int U> __global__ __launch_bounds__(256) void splitk_sum_k
         }
     }
     const float o[4] = {sum.x, sum.y, sum.z, sum.w};
-    uint16_t *dst = (uint16_t *)P.y + tok * P.ldy + f;
+    T *dst = (T *)P.y + tok * P.ldy + f;
     const T *bias = (const T *)P.bias;
-    uint16_t h[4];
+    using Bits = std::conditional_t<std::is_same<T, float>::value, float, uint16_t>;
+    Bits h[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) h[i] = f32_to_bits16(o[i] + (bias && f + i < P.M ? to_f32(bias[f + i]) : 0.f), (T *)nullptr);
+    for (int i = 0; i < 4; i++) {
+        const float total = o[i] + (bias && f + i < P.M ? to_f32(bias[f + i]) : 0.f);
+        if constexpr (std::is_same<T, float>::value) h[i] = total;
+        else h[i] = f32_to_bits16(total, (T *)nullptr);
+    }
     if (f + 4 <= P.M) {
-        __builtin_memcpy(dst, h, 8);
+        __builtin_memcpy(dst, h, sizeof(h));
     } else {
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            if (f + i < P.M) dst[i] = h[i];
+            if (f + i < P.M) ((Bits *)dst)[i] = h[i];
     }
 }
 

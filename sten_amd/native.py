@@ -102,6 +102,8 @@ SIGNATURES = {
     "nmg_lanepack8": (_I, [_P, _P, _I64, _I64, _I, _P, _P, _I, _P]),
     "nmg_spmm_sstream": (_I, [_P, _P, _I64, _I64, _P, _I64, _P, _I64, _P, _I64, _I, _I, _I, _P]),
     "nmg_gemm_nt": (_I, [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I, _P]),
+    "nmg_gemm_f32_plan": (_I, [_I64, _I64, _I64, _I64, _I64, _I, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int64)]),
+    "nmg_gemm_f32_splitk": (_I, [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I, _I, _P, _I64, _P]),
     "nmg_gemm_nn": (_I, [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I, _P]),
     "nmg_gemm_tn": (_I, [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I, _P]),
 }
