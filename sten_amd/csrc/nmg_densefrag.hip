@@ -335,9 +335,15 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
             const unsigned char *xb = x_base + (int64_t)at * XSTEP;
 #pragma unroll
             for (int q = 0; q < XL; q++)
-                if (q == i)
-                    __builtin_amdgcn_global_load_lds((glb_ptr_t)(xb + x_off[q]),
-                                                     (lds_ptr_t)(base + (wave * XL + q) * 1024), 16, 0, 0);
+                if (q == i) {
+                    // (XT: left visible, the compiler makes the transposing reads of every step wait for all loads in flight)
+                    if constexpr (XT)
+                        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                                     :: "v"(x_off[q]), "s"(xb), "s"((uint32_t)(uintptr_t)(lds_ptr_t)(base + (wave * XL + q) * 1024)) : "memory");
+                    else
+                        __builtin_amdgcn_global_load_lds((glb_ptr_t)(xb + x_off[q]),
+                                                         (lds_ptr_t)(base + (wave * XL + q) * 1024), 16, 0, 0);
+                }
         } else {
             // Written as instructions so that their completion is tracked by the explicit vmcnt
             // waits below and by nothing else.
@@ -472,11 +478,16 @@ __global__ __launch_bounds__(256, 1) void dense16_direct_kernel(DfParams P)
 #pragma unroll
     for (int t = 0; t < BT; t++) read_one(fr[0], smem, 0, t);
 
-    for (int kp0 = 0; kp0 < KP; kp0 += DD_D + 1) {
+    // The transposed form on narrow tiles has whole turns of the ring in a loop of their own: with the exits inside, the compiler lays its
+    // steps out in an order that the check of the loads in flight does not follow.
+    int kp0 = 0;
+#pragma unroll
+    for (int part = XT && AB == 2 ? 0 : 1; part < 2; part++)
+    for (; part != 0 ? kp0 < KP : kp0 + DD_D < KP; kp0 += DD_D + 1) {
 #pragma unroll
         for (int u = 0; u <= DD_D; u++) {
             const int kp = kp0 + u;
-            if (kp >= KP) goto walked;      // (past the loop: a break would be tested again there)
+            if (part != 0 && kp >= KP) goto walked;      // (past the loop: a break would be tested again there)
             const unsigned char *base = smem + (kp & (DD_NS - 1)) * STAGE;
             const unsigned char *next = smem + ((kp + 1) & (DD_NS - 1)) * STAGE;
             // A phase: its MFMAs, and behind one MFMA each the fragment reads of the next phase and
@@ -812,6 +823,17 @@ template <typename T, bool CT = false> static int launch_dense(DfParams &P, int 
     return launch_dense16<T, 8, 2, false, CT>(P, s);
 }
 
+// C = A B from B as it lies, on the tile of the plain product.  us, with every step waiting for the loads that it had just issued (256 x 128
+// tiles only) -> now: 4096 x 4096 x 2048 columns 80.5 -> 62, 1024^3 20 -> 11, 512 x 4096 x 4096 78 -> 39, 768 x 768 x 512 16.3 -> 9.1,
+// 8192 x 4096 x 4096 (256 x 256 tiles) 340 -> 216.
+template <typename T> static int launch_dense_tt(DfParams &P, hipStream_t s)
+{
+    const int tile = dense16_tile(1, P.O, P.KP, P.T);
+    if (tile == DENSE_NARROW) return launch_dense16<T, 8, 2, true, true, false, 2>(P, s);
+    if (tile == DENSE_SQUARE) return launch_dense16<T, 16, 4, true>(P, s);
+    return launch_dense16<T, 8, 2, true>(P, s);
+}
+
 // Y[T, O] = X[T, K] A[O, K]^T (+ bias), both operands rows in memory, on 256 x 256 tiles.  The caller has checked
 // extents, pitches and alignment (nmg_gemm_nt).  Bound by the vector memory path: a weight load touches 16 rows.  us,
 // 256 x 128 kernel of nmg_gemm_nt -> this one: 4096 x 4096, K = 2048 (the weight gradient of torch.mm) 77 -> 68;
@@ -1000,10 +1022,7 @@ extern "C" int nmg_spmm_densefrag_tt(const void *d_df, int64_t O, int64_t K, con
     P.ldy = ldc;
     P.KP = (int)(K / 64);
     hipStream_t s = (hipStream_t)stream;
-    // 256 x 128 tiles only: the fragments of this form are LDS transpose reads, 8 bytes per lane, and
-    // the 256 x 256 tile, which doubles them per wavefront, measured slower (16384x4096 x 4096
-    // columns: 724 against 582 us; the plain product on a transposed copy: 360 + 60 for the copy).
-    return dtype == NMG_F16 ? launch_dense16<__half, 8, 2, true>(P, s) : launch_dense16<__hip_bfloat16, 8, 2, true>(P, s);
+    return dtype == NMG_F16 ? launch_dense_tt<__half>(P, s) : launch_dense_tt<__hip_bfloat16>(P, s);
 }
 
 // C[O, T] = A X^T for X [T, K]: the product above with a transposed result.

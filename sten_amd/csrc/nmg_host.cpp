@@ -739,17 +739,17 @@ void check_mm(const State &w, const Tensor &b, int64_t K)
 
 Tensor spmm_tt_dense(State &w, Tensor b, int rd);
 
-// C = op(W) B from a transposed copy of B rather than from B as it lies: the copy (4 us, K N / 0.55 * 10^6 us beyond
-// a few MB) and the kernel on it, whose activation fragments are 16-byte LDS reads, against a kernel whose fragments
-// are transposing reads at half that rate.  us, as it lies -> copy and kernel, sparse / dense cores: 4096 x 4096 x 2048
-// columns 85 -> 52 / 83 -> 66; 512 x 4096 x 4096 75 -> 50 / 70 -> 62; 1024^3 20 -> 15 / 20 -> 18; 768 x 768 x 512
-// 14.3 -> 13.3 / 16.3 -> 15.8; 4096 x 512 x 4096 29 -> 24 / 31 -> 28; 512 x 512 x 64 9.2 -> 11.4 / 10.9 -> 12.8.  What is
-// saved grows with the reduction steps that a CU walks, rounds of 256 tiles times the reduction.  Operands that need
-// a padded copy anyway take the transposed one.
+// C = op(W) B from a transposed copy of B rather than from B as it lies.  The copy takes about 3.5 + K N / 0.8 * 10^6 us; without it
+// the fragments of B are transposing LDS reads, at half the rate of plain ones, which costs nothing on tiles of 256 outputs and 0.1 us a
+// step of 64 on tiles of 128 x 128.  us, copy and kernel -> as it lies, sparse / dense cores: 4096 x 4096 x 2048 columns 55 -> 44 /
+// 70 -> 62; 1024^3 13 -> 10 / 15 -> 11; 512 x 4096 x 4096 39 -> 33 / 47 -> 39; 512 x 512 x 64 10 -> 6.7 / 10 -> 7.1; 768 x 768 x 512
+// 11.6 -> 8.4 / 12.4 -> 9.1; but 744 x 11520 x 272 60, 62 / 65, 72 and 3032 x 13888 x 400 74, 88 / 92, 101.  (57 random
+// products of up to 2^36 multiplications: 0.86 / 0.87 of the time.)  Operands that need a padded copy anyway take the transposed one.
 bool transposed_pays(int64_t O, int64_t K, int64_t N, bool as_it_lies)
 {
-    const int64_t rounds = up(up(O, 256) * up(N, 128), 256);
-    return N * round_up(K, 64) * 2 < k2G && (!as_it_lies || rounds * K >= 768);
+    if (N * round_up(K, 64) * 2 >= k2G) return false;
+    const bool narrow = up(O, 128) * up(N, 128) <= 256;
+    return !as_it_lies || (narrow && (double)up(K, 64) * 0.1 > 3.5 + (double)K * (double)N / 0.8e6);
 }
 
 // Whether op(W) B with few columns is better cut along the reduction (as spmm does it, its result transposed

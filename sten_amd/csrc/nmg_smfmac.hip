@@ -412,9 +412,15 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
             const unsigned char *xb = x_base + (int64_t)at * XSTEP;
 #pragma unroll
             for (int q = 0; q < XL; q++)
-                if (q == i)
-                    __builtin_amdgcn_global_load_lds((glb_ptr_t)(xb + x_off[q]),
-                                                     (lds_ptr_t)(base + (wave * XL + q) * 1024), 16, 0, 0);
+                if (q == i) {
+                    // (XT: left visible, the compiler makes the transposing reads of every step wait for all loads in flight)
+                    if constexpr (XT)
+                        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                                     :: "v"(x_off[q]), "s"(xb), "s"((uint32_t)(uintptr_t)(lds_ptr_t)(base + (wave * XL + q) * 1024)) : "memory");
+                    else
+                        __builtin_amdgcn_global_load_lds((glb_ptr_t)(xb + x_off[q]),
+                                                         (lds_ptr_t)(base + (wave * XL + q) * 1024), 16, 0, 0);
+                }
         } else {
             // Written as instructions so that their completion is tracked by the explicit vmcnt
             // waits below and by nothing else (left to itself the compiler waits for vmcnt(0) at
@@ -714,7 +720,7 @@ static int launch_smfmac_direct(SmfParams &P, hipStream_t s)
     constexpr size_t stg = CT ? (size_t)4 * FB * 32 * (TB * 64 + 16) : (size_t)4 * TB * 32 * (FB * 64 + 16);
     constexpr size_t lds = ring > stg ? ring : stg;
     static_assert(lds <= 160 * 1024, "LDS");
-    static_assert(!XT || (TT == 128 && WN == 1), "the transposed tile is 64 rows of 128 tokens");
+    static_assert(!XT || WN == 1, "a wavefront reads the transposed tile over all of its tokens");
     auto k = spmm_smfmac_direct_kernel<T, FB, TB, WM, WN, NH, XT, CT>;
     if constexpr (!CT)
         if (P.tail != 0) k = spmm_smfmac_direct_kernel<T, FB, TB, WM, WN, NH, XT, CT, true>;
@@ -1489,8 +1495,16 @@ extern "C" int nmg_spmm_smfmac_tt(const void *d_fp_val, const void *d_fp_idx, in
     P.MB = (int)((M + 255) / 256 * 8);
     P.KP = (int)(K / 64);
     hipStream_t s = (hipStream_t)stream;
-    return dtype == NMG_F16 ? launch_smfmac_direct<__half, 2, 4, 4, 1, 2, true>(P, s)
-                            : launch_smfmac_direct<__hip_bfloat16, 2, 4, 4, 1, 2, true>(P, s);
+    // us, with every step waiting for the loads that it had just issued, twice (256 x 128 tiles only) -> now: 4096 x 4096 x 2048 columns
+    // 81 -> 44, 1024^3 19 -> 10, 512 x 4096 x 4096 84 -> 33, 768 x 768 x 512 14.6 -> 8.4, 8192 x 4096 x 4096 364 -> 158 (wide tiles)
+    auto launch = [&](auto tag) -> int {
+        using T16 = decltype(tag);
+        const int tile = smfmac_tile(P);
+        if (tile == 8) return launch_smfmac_direct<T16, 2, 8, 4, 1, 4, true>(P, s);
+        if (tile == 7) return launch_smfmac_direct<T16, 1, 4, 4, 1, 1, true>(P, s);
+        return launch_smfmac_direct<T16, 2, 4, 4, 1, 2, true>(P, s);
+    };
+    return dtype == NMG_F16 ? launch(__half{}) : launch(__hip_bfloat16{});
 }
 
 // ---- C[M, T] = W * X^T (+ bias per row) for X [T, K]: the untransposed product with a transposed result ----
