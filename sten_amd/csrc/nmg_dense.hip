@@ -855,10 +855,15 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
     int st = 0;
     if constexpr (LOADS == F32_ENDS) {
         const int whole = (XKM && P.T < 4) || (AKM && P.O < 4) ? 0 : (int)(P.K / BKT);
+        // The guarded loads of the first tiles stand behind branches, and the compiler cannot count them: without this wait for them (vmcnt(0),
+        // nothing else) the loop waits for every load in flight once a turn.  us, without -> with: both operands reduction-major 1280 x 512,
+        // K 3690 130 -> 93, 1664 x 512, K 1381 46 -> 38, 640 x 2432, K 423 28.7 -> 26.4, one 376 x 511, K 3296 30.4 -> 26.4; none, no difference.
+        if (AKM && st + 4 < whole) __builtin_amdgcn_s_waitcnt(0x0f70);
         for (; st + 4 < whole; st += 2) {
             step(st, F0, F1, G1, true, true, std::true_type{});
             step(st + 1, F1, F0, G0, true, true, std::true_type{});
         }
+        if constexpr (XKM) asm volatile("" : "+s"(st));      // (the compiler made one loop of this and the next, with 64 x 64 tiles)
     }
     for (; st + 4 < steps; st += 2) {
         step(st, F0, F1, G1, true, true, std::false_type{});
@@ -923,10 +928,9 @@ static void launch_gemm_f32(const GemmF32Params &Q, int form, hipStream_t st)
                       (form < 2 || (Q.T % 4 == 0 && Q.T >= 4));
     // Guards are branches, and with a branch in the loop the compiler waits for every load in flight: us, guards in every step ->
     // in the last, row-major weight: W B for 2816 x 2944, 259 columns 97 -> 69 (260 columns: 57), 999 columns 188 -> 159; 512 x 768,
-    // K 3071 37.5 -> 33.5, 36 x 221, K 1618 15.0 -> 12.2.  With both operands reduction-major 36 x 221, K 1618 22 -> 16.4, 1612 x 694,
-    // K 1482 77.6 -> 69.9, but on short reductions fetching the second loop's code costs more: 100 x 1444, K 773 14.5 -> 16.2, 225 x 89,
-    // K 307 7.9 -> 8.7.
-    const bool ends = Q.K >= 16 * BKT;
+    // K 3071 37.5 -> 33.5, 36 x 221, K 1618 15.0 -> 12.2.  With both operands reduction-major 512 x 2432, K 237 18.7 -> 16.8, 2839 x 422,
+    // K 252 19.7 -> 17.7, 100 x 1444, K 773 14.3 -> 14.1; on fewer steps fetching the second loop's code costs more.
+    const bool ends = Q.K >= 8 * BKT;
 #define NMG_F32_LAUNCH(LOADS_, AKM_, XKM_) \
     hipLaunchKernelGGL((gemm_nt_f32_kernel<WM, WN, WK, MI, NJ, LOADS_, AKM_, XKM_>), grid, dim3(256), 0, st, Q)
     if (form == 0) {
@@ -1096,17 +1100,20 @@ extern "C" int nmg_gemm_f32_plan(int64_t lda, int64_t ldx, int64_t O, int64_t K,
     *slices = 1;
     *workspace_bytes = 0;
     if (O == 0 || K == 0 || T == 0 || gemm_f32_few(O, T, form)) return NMG_OK;
-    // Against the time on the fp32 instruction, which the model above puts too high or too low here, by form and tile (165 products of 2^27 to
+    // Against the time on the fp32 instruction, which the model above puts too high or too low here, by form and tile (276 products of 2^27 to
     // 2^33 multiplications with at most 140 tiles of 128 x 128, all forms, odd extents among them, in every number of slices: with this choice
-    // they take 0.935 of the time of whole ones, with the best 0.93, none more than 1 % longer than whole).  us, whole -> slices: 256 x 2176
-    // results over 2724, both operands reduction-major 100 -> 38, 1024 x 1024 over 4096 74.5 -> 59, 1021 x 1999 over 2047 85 -> 66, 768 x 2673
-    // over 3200 108 -> 83; below about 30 us the two launches cost more than they save (1024 x 176 over 1152: 9.8, 19.8).
+    // they take 0.933 of the time of whole ones, with the best 0.926, one of them more than 1 % longer than whole, 25.9 -> 26.6).  us, whole ->
+    // slices: 960 x 584 results over 4076, both operands reduction-major 98 -> 50, 1024 x 1024 over 4096 74.5 -> 59, 1021 x 1999 over 2047
+    // 85 -> 66, 768 x 2673 over 3200 108 -> 83; below about 30 us the two launches cost more than they save (1024 x 176 over 1152: 9.8, 19.8).
     int shape, best;
     const double us = split3_plan(lda, ldx, O, K, T, form, &best);
     const bool even = lda % 4 == 0 && ldx % 4 == 0;
     const double fixed = 4.75, model = gemm_f32_us(O, K, T, form, even, &shape) - fixed;
-    const bool guards = !(even && K % 32 == 0 && O % 4 == 0 && T % 4 == 0);
-    const double whole = fixed + model * (form == 0 ? (shape == 5 ? 0.7 : 1.0) : form == 1 ? (shape == 5 ? 0.85 : shape == 4 ? 1.2 : 1.0) : guards ? 1.4 : 1.0);
+    const bool guards = !(even && K % 32 == 0 && O % 4 == 0 && (form < 2 || T % 4 == 0));
+    const double share = form == 0 ? (shape == 5 ? 0.7 : 1.0)
+                         : form == 1 ? (shape == 5 ? 0.85 : shape == 4 ? (guards ? 0.95 : 1.2) : 1.0)
+                                     : (guards ? 1.15 : 1.0);
+    const double whole = fixed + model * share;
     if (best > 1 && us < 0.95 * whole) {
         *slices = best;
         *workspace_bytes = best * T * ((O + 3) / 4 * 4) * 4;

@@ -1,4 +1,4 @@
-"""Single-precision products with the reduction in slices (nmg_gemm_f32_splitk) against fp64."""
+"""Single-precision products, whole and with the reduction in slices (nmg_gemm_f32_splitk), against fp64."""
 import ctypes
 
 import pytest
@@ -51,6 +51,20 @@ def test_slices_against_fp64(form, O, K, T, slices, pad):
     ref = x.double() @ a.double().t() + (0 if bias is None else bias.double())
     y = _product(form, A, X, O, K, T, slices, bias, pad)
     assert ((y.double() - ref).norm() / ref.norm()).item() <= BOUND
+
+
+# Whole products with ends inside steps and groups of four: one step fewer than the loop for whole steps takes, as many, and several
+# turns of it, on tiles of 32 x 32 (steps of 64), 64 x 64 (16) and larger ones.  On the fp32 instruction sums are rounded once per 2 positions.
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [0, 1, 2])
+@pytest.mark.parametrize("O,K,T", [(36, 511, 221), (37, 513, 222), (36, 1618, 221), (1001, 127, 640), (1000, 131, 641), (1000, 383, 639),
+                                   (383, 263, 1281), (2664, 279, 263), (1283, 515, 510)])
+def test_whole_products_with_ends_against_fp64(form, O, K, T):
+    print(f"case f32 ends form={form} O={O} K={K} T={T}", flush=True)
+    A, X, a, x = _operands(form, O, K, T, 0)
+    ref = x.double() @ a.double().t()
+    y = _product(form, A, X, O, K, T, 1)
+    assert ((y.double() - ref).norm() / ref.norm()).item() <= 2.0 ** -24 * (K / 2) ** 0.5
 
 
 @pytest.mark.gpu
