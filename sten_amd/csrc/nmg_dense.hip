@@ -1099,7 +1099,8 @@ extern "C" int nmg_gemm_f32_plan(int64_t lda, int64_t ldx, int64_t O, int64_t K,
     NMG_REQUIRE(slices && workspace_bytes, NMG_ERR_ARG, "null output pointer");
     *slices = 1;
     *workspace_bytes = 0;
-    if (O == 0 || K == 0 || T == 0 || gemm_f32_few(O, T, form)) return NMG_OK;
+    // (below 2^28 multiplications slices gained nothing, and the models take a tenth of a microsecond that a small call would see)
+    if ((double)O * (double)K * (double)T < 268435456.0 || gemm_f32_few(O, T, form)) return NMG_OK;
     // Against the time on the fp32 instruction, which the model above puts too high or too low here, by form and tile (276 products of 2^27 to
     // 2^33 multiplications with at most 140 tiles of 128 x 128, all forms, odd extents among them, in every number of slices: with this choice
     // they take 0.933 of the time of whole ones, with the best 0.926, one of them more than 1 % longer than whole, 25.9 -> 26.6).  us, whole ->
