@@ -20,12 +20,13 @@
 //   2. counting sort of all columns' proposals, kept and new, by pattern and by bins of the score below the tile's largest;
 //   3. every proposal finds its rank: those in larger bins of its pattern plus those of its own bin that are larger (all pairs);
 //   4. what ranks below the pattern's capacity is written to its slot, the rest is pending.
-// A quarter of the columns and fewer (any n:m:g: half) insert into the lists lane by lane (the code says how).
+// A quarter of the columns and fewer (any n:m:g: half) insert into the lists lane by lane (the code says how).  Lists of more than 256 keys stay
+// with rounds over all columns (1:4:300 295 us, 250 when these took pending columns only).
 //
 // us, 4096 x 4096 fp16 with the blocks along the contiguous / the slow dim (8192 x 8192 for 2:8:32), batched walk -> ranks among all
 // proposals of a pattern -> this: 2:4:16 99 -> 58 / 57 -> 50 / 50, 1:8:32 37 -> 31, 3:6:12 75 / 73 -> 61 / 59, 2:8:32 727 -> 182 / 190 -> 138 / 147,
 // 4:8:32 390 -> 128 / 124 -> 73 / 73; any n:m:g: 2:4:4 168 / 231 -> 110 / 109 -> 87, 2:4:8 115 / 146 -> 71 -> 57, 2:4:32 118 / 135 -> 104 / 114 ->
-// 93 / 103, 2:4:64 130 / 146 -> 113 / 124 -> 107, 1:2:8 192 / 302 -> 143 / 138 -> 132, 2:8:8 293 / 326 -> 130 / 134 -> 102, 4:8:16 870 / 810 ->
+// 93 / 103, 2:4:64 130 / 146 -> 113 / 124 -> 107, 1:2:8 192 / 302 -> 143 / 138 -> 132, 2:8:8 293 / 326 -> 130 / 134 -> 102, 1:8:8 86 / 117 -> 79 -> 63, 4:8:16 870 / 810 ->
 // 280 / 293 -> 220 / 228, 2:4:100 144 / 160 -> 130.  What each part gave, 2:8:32: bins 43 -> 20 us of the first round, score and pattern compared as one
 // double 17 -> 7 (a select behind a select on the same condition takes 17 to 40 clocks, a 64-bit maximum 4), the sorted keys in the place of the lists (six
 // workgroups a CU instead of five) 168 -> 150, the reads of a column's patterns in flight together 150 -> 145.  4:8:32: 125 -> 102, and 73 where the
@@ -193,10 +194,15 @@ constexpr int match_bin_bytes(int bins) { return (4 + bins + 4) * 4; }      // a
 // last); then the waiting columns, flags and runs of the closed form; a partial block's proposals.  One after the other in the same place: 2:8:32 takes
 // 25.8 KB a tile of fp16 instead of 29.5, six workgroups of a CU instead of five.
 constexpr int match_few(int sg) { return sg != 0 ? 4 : 2; }
+constexpr int match_bucket(int g) { return g < 4 ? 1 : g / 2 < 8 ? g / 2 : 8; }      // proposals that a pattern takes in a later round
+// Keys of a list that a lane holds where g is not compiled in: 64 lanes hold lists of 128, with four keys a lane 256.  Tiles of two wavefronts
+// have a kernel for each (told apart by the columns a thread has room for): us, 4096 x 4096 fp16, two keys a lane -> four: 2:4:64 108 -> 113, 2:8:16 101 -> 105;
+// rounds -> lists of four keys a lane: 1:2:150 257 -> 205, 1:3:140 204 -> 141.
+constexpr int match_list_keys(int nt, int cpt) { return nt >= 256 || (nt == 128 && cpt > 4) ? 4 : 2; }
 static inline int match_scratch(int cols, int c, int g, int bins_log2, bool lists, bool partial, int few)
 {
     int bytes = std::max(match_bin_bytes(c << bins_log2), 4 * cols + cols / 4 + 16);
-    if (lists) bytes = std::max(bytes, ((few + 1) / 2 + c * std::min(g / 2, 8) + 2) * 8);
+    if (lists) bytes = std::max(bytes, ((few + 1) / 2 + c * match_bucket(g) + 2) * 8);
     if (partial) bytes = std::max(bytes, cols * 8);
     return (bytes + 15) & ~15;
 }
@@ -600,7 +606,6 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
     constexpr int THREADS = NT <= 64 ? 256 : NT;
     constexpr int TILES = THREADS / NT;
     constexpr int KPT = match_keys(NT, CPT);
-    constexpr bool LISTS = NT > 16 || SM != 0;
     const int n = SN ? SN : Q.n, m = SM ? SM : Q.m, g = SG ? SG : Q.g, c = SC ? SC : Q.c;
     const int cols = SC && SG ? SC * SG : Q.cols;
     constexpr int V = 16 / (int)sizeof(T);
@@ -841,7 +846,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 
     if (live) {
         // a quarter of the tile and fewer go on in the registers below
-        const bool lists = LISTS && (SG != 0 || Q.lanes_log2 != 0);
+        const bool lists = SG != 0 || Q.lanes_log2 != 0;
         const int few = lists ? cols / match_few(SG) : 0;
         uint16_t *pending = (uint16_t *)s_arr;
         // every proposal that is not the last word of its column is refused once per (column, pattern) at most
@@ -982,12 +987,12 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
             pend = s_np[0];
         }
 
-        if constexpr (LISTS) if (lists) {
+        if (lists) {
             // Later rounds: a few columns, whatever the pattern.  L lanes hold a pattern's list, KPL keys each in descending
             // order, and insert a proposal by one shift along the lanes.  A pattern takes at most `bucket` proposals in a round;
             // the rest stay pending.  In a tile of several wavefronts the first one ends the matching alone, without barriers.
-            constexpr int EIGHT = 8, LL = SG > 16 && SC <= 8 ? 4 : 3, KPL = SG > 8 << (LL - 2) ? 4 : 2;
-            const int ll = SG != 0 ? LL : Q.lanes_log2, L = 1 << ll, bucket = min(g / 2, 8);
+            constexpr int EIGHT = 8, LL = SG > 16 && SC <= 8 ? 4 : 3, KPL = SG == 0 ? match_list_keys(NT, CPT) : SG > 8 << (LL - 2) ? 4 : 2;
+            const int ll = SG != 0 ? LL : Q.lanes_log2, L = 1 << ll, bucket = match_bucket(g);
             static_assert(SG <= 32 && SG != 1, "a list fits its lanes; lists and buckets fit the proposals' place");
             uint16_t *next = pending + few;
             uint64_t *s_bkt = s_arr + (few + 1) / 2;      // free places hold 0
@@ -1103,10 +1108,13 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 #pragma unroll
                             for (int u = 0; u < AT; u++) {
                                 // key(i) = max(key(i), min(key(i - 1), in)): the keys are positive doubles and no NaN
+                                uint64_t tail = key[0];      // the list's last key, in its last lane
+#pragma unroll
+                                for (int i = 1; i < KPL; i++) tail = (g - 1) % KPL == i ? key[i] : tail;
                                 asm("s_nop 1" : "+v"(key[KPL - 1]));      // (a move between lanes reads a result two instructions later at the earliest)
                                 uint64_t before = match_swap<(SG != 0 ? 0x111 : 0x138)>(key[KPL - 1]);      // row_shr:1, wave_shr:1
                                 if (r == 0) before = in[u];
-                                out[u] = match_smaller(key[(g - 1) % KPL], in[u]);
+                                out[u] = match_smaller(tail, in[u]);
 #pragma unroll
                                 for (int i = KPL - 1; i > 0; i--) key[i] = match_larger(key[i], match_smaller(key[i - 1], in[u]));
                                 key[0] = match_larger(key[0], match_smaller(before, in[u]));
@@ -1289,11 +1297,11 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     int off = RC ? m * up(cols, V) * (int)sizeof(T) : up(cols * m * (int)sizeof(T), 16);
     Q.r_mem = off;
     off = up(off + cols * 8 + kMatchPad, 16);
-    // Lists of 2 to 64 keys that fit the lanes of a tile.  Below 32 columns a round over all of them is the shorter way
-    // (4096 x 4096 fp16, lists -> rounds: 2:4:4 204 -> 192 us, 1:2:8 238 -> 215; from there on 2:4:8 147 -> 140, 2:4:32
-    // 131 -> 117, 2:8:8 188 -> 140, 4:8:16 482 -> 365, rounds -> lists).
-    Q.lanes_log2 = Q.g < 2 || Q.g > 128 ? 0 : Q.g <= 16 ? 3 : Q.g <= 32 ? 4 : Q.g <= 64 ? 5 : 6;
-    if ((1 << Q.lanes_log2) > NT || cols < 24) Q.lanes_log2 = 0;
+    // Lists that fit the lanes of a tile; longer ones, and tiles of 16 columns with more than four patterns, go through rounds over all columns
+    // to the end.  us, 4096 x 4096 fp16, rounds -> lists: 1:8:8 101 -> 62, 2:5:2 (20 columns) 275 -> 224, 1:4:4 (16) 104 -> 93, 2:8:1 314 -> 223,
+    // 4:8:1 824 -> 434, 2:4:160 211 -> 123, 1:8:256 165 -> 82; but 1:8:2 (16) 115 -> 126.
+    Q.lanes_log2 = Q.g > 64 * match_list_keys(NT, CPT) ? 0 : Q.g <= 16 ? 3 : Q.g <= 32 ? 4 : Q.g <= 64 ? 5 : 6;
+    if ((1 << Q.lanes_log2) > NT || (cols < 18 && c > 4)) Q.lanes_log2 = 0;
     Q.r_arr = off;
     off += match_scratch(cols, c, Q.g, match_bins_log2(NT, c), SG != 0 || Q.lanes_log2 != 0, Q.view.S % m != 0, cols / match_few(SG));
     Q.r_int = off;
@@ -1352,11 +1360,12 @@ template <typename T, bool RC> static int match_dispatch(MatchParams &Q, hipStre
         if (m == 5 && n == 1) return match_launch<T, 16, 4, 1, 5, 0, RC>(Q, stream, done);
         if (m == 5 && n == 4) return match_launch<T, 16, 4, 4, 5, 0, RC>(Q, stream, done);
     }
-    if (Q.cols <= 64 && Q.c <= 32) return match_launch<T, 16, 4, 0, 0, 0, RC>(Q, stream, done);
-    if (Q.cols <= 128 && Q.c <= 20) return match_launch<T, 32, 4, 0, 0, 0, RC>(Q, stream, done);
+    // (a tile of many patterns: half a wavefront, 3:6:3 236 -> 184, 2:7:3 241 -> 171, 2:8:2 218 -> 166)
+    if (Q.cols <= 64 && Q.c <= (Q.cols > 48 ? 15 : 32)) return match_launch<T, 16, 4, 0, 0, 0, RC>(Q, stream, done);
+    if (Q.cols <= 128 && Q.c <= (Q.cols > 64 ? 20 : 60)) return match_launch<T, 32, 4, 0, 0, 0, RC>(Q, stream, done);
     if (Q.cols <= 256) return match_launch<T, 64, 4, 0, 0, 0, RC>(Q, stream, done);
     if (Q.cols <= 512) {
-        const int rc = match_launch<T, 128, 4, 0, 0, 0, RC>(Q, stream, done);
+        const int rc = Q.g > 128 ? match_launch<T, 128, 5, 0, 0, 0, RC>(Q, stream, done) : match_launch<T, 128, 4, 0, 0, 0, RC>(Q, stream, done);
         if (rc != NMG_OK || *done) return rc;
     }
     if (Q.cols <= 1024) return match_launch<T, 256, 4, 0, 0, 0, RC>(Q, stream, done);

@@ -188,3 +188,34 @@ def test_scores_of_any_size(n, m, g, dtype):
             t = sten.GroupedNMTensor.from_dense(x.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
             assert np.array_equal(to_np(t.idx), idx)
             assert same_bits(t.val, val)
+
+
+# Which later rounds a tile takes: lists of one key, of up to 128 and 256 (two and four to a lane), rounds over all columns beyond; tiles of 16, 18
+# and 20 columns; tiles of 48 and more columns on a quarter and on half of a wavefront.  Whole blocks and a partial one.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n,m,g", [(1, 8, 2), (1, 2, 9), (2, 5, 2), (1, 4, 4), (1, 8, 4), (1, 6, 8), (1, 8, 8), (2, 6, 4), (3, 6, 3), (2, 8, 2), (2, 8, 1), (3, 6, 1),
+                                   (4, 8, 1), (1, 2, 128), (1, 2, 129), (2, 4, 160), (1, 8, 256), (1, 2, 257), (1, 4, 257)])
+@pytest.mark.parametrize("rest", [0, 1])
+def test_later_rounds_of_any_tile(n, m, g, dtype, rest):
+    cols = math.comb(m, n) * g
+    gen = torch.Generator().manual_seed(n * 100 + m * 10 + g + rest)
+    for along in (0, 1):
+        w = torch.randn(2 * cols + cols // 2, 4 * m + rest, generator=gen).to(dtype)
+        x = w if along == 1 else w.t().contiguous()
+        print(f"case {n}:{m}:{g} {dtype} rest={rest} along={along}", flush=True)
+        val, idx, _ = oracle_sparsify(x, n, m, along, g, 1 - along)
+        t = sten.GroupedNMTensor.from_dense(x.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
+        assert np.array_equal(to_np(t.idx), idx)
+        assert same_bits(t.val, val)
+
+
+# Lists of more than 128 keys in tiles of two wavefronts, which take tensors of at least 2048 tiles.
+@pytest.mark.parametrize("n,m,g", [(1, 2, 128), (1, 2, 129), (1, 2, 256), (1, 3, 160)])
+def test_long_lists_in_tiles_of_two_wavefronts(n, m, g):
+    cols = math.comb(m, n) * g
+    w = torch.randn(8 * cols, 256 * m, generator=torch.Generator().manual_seed(g)).to(torch.float16)
+    print(f"case {n}:{m}:{g}", flush=True)
+    val, idx, _ = oracle_sparsify(w, n, m, 1, g, 0)
+    t = sten.GroupedNMTensor.from_dense(w.to(DEV), n, m, sparse_dim=1, group_size=g, group_dim=0)
+    assert np.array_equal(to_np(t.idx), idx)
+    assert same_bits(t.val, val)
