@@ -157,8 +157,13 @@ template <int X> __device__ __forceinline__ uint32_t match_lane_xor(uint32_t v)
     else return (uint32_t)__shfl_xor((int)v, X);
 }
 
-// Larger one of two edges (score in the high word, pattern in the low one; a positive double, never a NaN: scores are at most 0x7FFFFFFF and
-// a double's NaNs begin at 0x7FF00000, above every float).  One instruction, where fmax canonicalises its operands first.  The compiler does not
+// An edge's score (31 bits) and pattern as a positive double that is no NaN for any score.  (With the score as the high word those from 0x7FF00000
+// on, which a weight that is no number may give, would be NaNs, and the maximum below drops them.)
+__device__ __forceinline__ uint64_t match_edge(uint32_t score, uint32_t p) { return ((uint64_t)(score >> 1) << 32) | ((score << 31) | p); }
+__device__ __forceinline__ uint32_t match_edge_score(uint64_t edge) { return (uint32_t)(edge >> 31); }
+__device__ __forceinline__ int match_edge_pattern(uint64_t edge) { return (int)(edge & 0xFFu); }
+
+// Larger one of two edges or keys.  One instruction, where fmax canonicalises its operands first.  The compiler does not
 // know it for a vector instruction: `s_nop 1` before a move between lanes reads its result.
 __device__ __forceinline__ uint64_t match_larger(uint64_t a, uint64_t b)
 {
@@ -796,17 +801,43 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 #pragma unroll
             for (int r = 0; r < 8; r++) a[r] = r < m ? match_abs(s_d[at(o, r)]) : 0.f;
         }
-        uint64_t best = 0;      // score and pattern
+        // Many patterns: the score itself is the high word, and a column with a weight that could make it a NaN compares whole numbers (us, shifted
+        // edges -> this, 4096 x 4096 fp16: 4:8:32 77.5 -> 75.0, 2:8:32 48.8 -> 48.0; with the NaNs out of order 74.2, 47.3).  With few of them the
+        // test for it costs more than the shifts (1:8:16 57.5 -> 59.0, 7:8:12 66.5 -> 68.1).
+        constexpr bool RAW = SC > 8;
+        if constexpr (RAW) {
+            uint32_t largest = __float_as_uint(a[0]);
+#pragma unroll
+            for (int r = 1; r < SM; r++) largest = max(largest, __float_as_uint(a[r]));
+            if (__builtin_expect(largest >= 0x7FF00000u, 0)) {
+                uint32_t best = 0;
+                int bp = 0;
+#pragma unroll 1
+                for (int p = 0; p < SC; p++) {
+                    const uint32_t ps = s_pos[p];
+                    float acc = match_abs(s_d[at(o, (int)(ps & 15u))]);
+#pragma unroll 1
+                    for (int j = 1; j < SN; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
+                    const uint32_t sb = __float_as_uint(acc);
+                    if (sb >= best && (!THR || match_key(sb, o, p) > s_mem[p * g + g - 1])) {
+                        best = sb;
+                        bp = p;
+                    }
+                }
+                return best == 0 ? 0 : match_key(best, o, bp);
+            }
+        }
+        uint64_t best = 0;
         int later = 0;
-        uint32_t zero;      // not to be known for one: the patterns' numbers would take a register each for all columns
-        asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+        uint32_t zero = 0;      // not to be known for one: the patterns' numbers would take a register each for all columns
+        if constexpr (RAW) asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
         auto consider = [&](float acc, int p) {
             uint32_t sb = __float_as_uint(acc);
             if (THR) {
                 const uint64_t last = s_mem[p * g + g - 1 + later];
                 if (!(match_key(sb, o, p) > last)) sb = 0;
             }
-            best = match_larger(best, ((uint64_t)sb << 32) | (zero + (uint32_t)p));
+            best = match_larger(best, RAW ? ((uint64_t)sb << 32) | (zero + (uint32_t)p) : match_edge(sb, (uint32_t)p));
         };
         if constexpr (SM != 0) {
             constexpr MatchMasks<SN ? SN : 1, SM ? SM : 1> tab;
@@ -841,7 +872,8 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                 }
             }
         }
-        return (best >> 32) == 0 ? 0 : match_key((uint32_t)(best >> 32), o, (int)(best & 0xFFu));
+        const uint32_t score = RAW ? (uint32_t)(best >> 32) : match_edge_score(best);
+        return score == 0 ? 0 : match_key(score, o, match_edge_pattern(best));
     };
 
     if (live) {
@@ -1038,7 +1070,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                         for (int j = 1; j < n; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
                         uint32_t sb = __float_as_uint(acc);
                         if (!(match_key(sb, o, p) > s_mem[p * g + g - 1])) sb = 0;
-                        return ((uint64_t)sb << 32) | (uint32_t)p;
+                        return match_edge(sb, (uint32_t)p);
                     };
                     auto other = [&](uint64_t top, auto ctrl) {      // the larger one of two lanes
                         asm("s_nop 1" : "+v"(top));
@@ -1063,7 +1095,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                             top = other(top, by_1);
                             if (EL >= 4) top = other(top, by_2);
                             if (EL >= 8) top = other(top, by_4);
-                            if (sub == 0) put(o, (top >> 32) == 0 ? 0 : match_key((uint32_t)(top >> 32), o, (int)(top & 0xFFu)));
+                            if (sub == 0) put(o, match_edge_score(top) == 0 ? 0 : match_key(match_edge_score(top), o, match_edge_pattern(top)));
                         }
                     } else if (SG == 0 && c > 8 && pend * EIGHT <= A) {
                         const int e = tt / EIGHT, sub = tt % EIGHT;
@@ -1078,7 +1110,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                             top = other(top, by_1);
                             top = other(top, by_2);
                             top = other(top, by_4);
-                            if (sub == 0) put(o, (top >> 32) == 0 ? 0 : match_key((uint32_t)(top >> 32), o, (int)(top & 0xFFu)));
+                            if (sub == 0) put(o, match_edge_score(top) == 0 ? 0 : match_key(match_edge_score(top), o, match_edge_pattern(top)));
                         }
                     } else {
                         for (int e = tt; e < pend; e += A) {

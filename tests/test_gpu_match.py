@@ -190,6 +190,32 @@ def test_scores_of_any_size(n, m, g, dtype):
             assert same_bits(t.val, val)
 
 
+# A sum over a weight that is no number is larger than every other one, whatever number its bits stand for (those of 0x7FFF in 16 bits and 0x7FFFFFFF
+# lie where the high word of a double is no number either): equal ones take the places of infinities, in whole blocks and partial ones.
+@pytest.mark.parametrize("dtype,bits", [(torch.float16, 0x7E00), (torch.float16, 0x7FFF), (torch.float16, 0xFFFF), (torch.bfloat16, 0x7FC0), (torch.bfloat16, 0x7FFF),
+                                        (torch.float32, 0x7FC00000), (torch.float32, 0x7FF00001), (torch.float32, 0x7FFFFFFF)])
+@pytest.mark.parametrize("n,m,g", [(2, 4, 16), (1, 8, 32), (3, 6, 12), (2, 8, 32), (4, 8, 32), (2, 4, 4), (1, 4, 129), (3, 8, 8), (4, 8, 6)])
+@pytest.mark.parametrize("rest", [0, 1])
+def test_weights_that_are_no_numbers(n, m, g, dtype, bits, rest):
+    cols = math.comb(m, n) * g
+    gen = torch.Generator().manual_seed(n * 100 + m * 10 + g)
+    w = torch.randn(cols + cols // 2, 4 * m + rest, generator=gen).to(dtype)
+    odd = torch.rand(w.shape, generator=gen) < 0.03
+    whole = {2: torch.int16, 4: torch.int32}[w.element_size()]
+    value = bits - (1 << 8 * w.element_size()) if bits >> (8 * w.element_size() - 1) else bits
+    as_none, as_inf = w.view(whole).masked_fill(odd, value).view(dtype), w.masked_fill(odd, math.inf)
+    for along in (0, 1):
+        x, y = (t if along == 1 else t.t().contiguous() for t in (as_none, as_inf))
+        print(f"case {n}:{m}:{g} {dtype} {bits:x} rest={rest} along={along}", flush=True)
+        val, idx, _ = oracle_sparsify(y, n, m, along, g, 1 - along)
+        t = sten.GroupedNMTensor.from_dense(x.to(DEV), n, m, sparse_dim=along, group_size=g, group_dim=1 - along)
+        assert np.array_equal(to_np(t.idx), idx)
+        none = np.isinf(val.astype(np.float32))
+        assert np.array_equal(torch.isnan(t.val).cpu().numpy(), none)
+        assert bool((t.val.cpu().view(whole)[torch.from_numpy(none)] == value).all())
+        assert same_bits(t.val.masked_fill(torch.isnan(t.val), math.inf), val)
+
+
 # Which later rounds a tile takes: lists of one key, of up to 128 and 256 (two and four to a lane), rounds over all columns beyond; tiles of 16, 18
 # and 20 columns; tiles of 48 and more columns on a quarter and on half of a wavefront.  Whole blocks and a partial one.
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
