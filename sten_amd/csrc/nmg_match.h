@@ -20,8 +20,7 @@
 //   2. counting sort of all columns' proposals, kept and new, by pattern and by bins of the score below the tile's largest;
 //   3. every proposal finds its rank: those in larger bins of its pattern plus those of its own bin that are larger (all pairs);
 //   4. what ranks below the pattern's capacity is written to its slot, the rest is pending.
-// A quarter of the columns and fewer (any n:m:g: half) insert into the lists lane by lane (the code says how).  Lists of more than 256 keys stay
-// with rounds over all columns (1:4:300 295 us, 250 when these took pending columns only).
+// A quarter of the columns and fewer (any n:m:g: half) insert into the lists lane by lane, into long ones key by key (the code says how).
 //
 // us, 4096 x 4096 fp16 with the blocks along the contiguous / the slow dim (8192 x 8192 for 2:8:32), batched walk -> ranks among all
 // proposals of a pattern -> this: 2:4:16 99 -> 58 / 57 -> 50 / 50, 1:8:32 37 -> 31, 3:6:12 75 / 73 -> 61 / 59, 2:8:32 727 -> 182 / 190 -> 138 / 147,
@@ -199,15 +198,26 @@ constexpr int match_bin_bytes(int bins) { return (4 + bins + 4) * 4; }      // a
 // last); then the waiting columns, flags and runs of the closed form; a partial block's proposals.  One after the other in the same place: 2:8:32 takes
 // 25.8 KB a tile of fp16 instead of 29.5, six workgroups of a CU instead of five.
 constexpr int match_few(int sg) { return sg != 0 ? 4 : 2; }
-constexpr int match_bucket(int g) { return g < 4 ? 1 : g / 2 < 8 ? g / 2 : 8; }      // proposals that a pattern takes in a later round
 // Keys of a list that a lane holds where g is not compiled in: 64 lanes hold lists of 128, with four keys a lane 256.  Tiles of two wavefronts
 // have a kernel for each (told apart by the columns a thread has room for): us, 4096 x 4096 fp16, two keys a lane -> four: 2:4:64 108 -> 113, 2:8:16 101 -> 105;
 // rounds -> lists of four keys a lane: 1:2:150 257 -> 205, 1:3:140 204 -> 141.
 constexpr int match_list_keys(int nt, int cpt) { return nt >= 256 || (nt == 128 && cpt > 4) ? 4 : 2; }
-static inline int match_scratch(int cols, int c, int g, int bins_log2, bool lists, bool partial, int few)
+// Longer lists stay in LDS, a wavefront moves their keys (us, 4096 x 4096 fp16, rounds over all columns ->
+// this: 1:4:300 297 -> 168, 2:4:400 298 -> 142, 1:8:257 160 -> 80, 1:2:1000 1205 -> 640).  It takes many proposals at a time for what a shift along the lanes does with eight, which a partial block gains from with lists
+// of more than 64 keys: its columns want the same few patterns (2000 x 3000 bf16, blocks along the slow dim, 3:6:100 202 -> 125, 3:6:128 293 -> 152).
+// Whole blocks of up to 256 keys are faster in the lanes (7:8:160 106, 116; 2:6:100 125, 139).
+constexpr bool match_long(int nt, int cpt, int g, bool partial) { return nt >= 128 && g > (partial ? 64 : 64 * match_list_keys(nt, cpt)); }
+// Proposals that a pattern takes in a later round: what has room where the closed form, a first round's bins (short lists) or a partial block's
+// proposals lie anyway.  With one for lists of up to three keys 1:6:3 was slower than by rounds, 178 against 157; 150 with three, 2:8:2 167 -> 159.
+constexpr int match_bucket(bool longs, int g, bool partial)
+{
+    if (longs) return partial ? (g * 11 / 16 < 64 ? g * 11 / 16 : 64) : (g / 4 < 64 ? g / 4 : 64);
+    return g < 3 ? 2 : g == 3 ? 3 : g / 2 < 8 ? g / 2 : 8;
+}
+static inline int match_scratch(bool longs, int cols, int c, int g, int bins_log2, bool lists, bool partial, int few)
 {
     int bytes = std::max(match_bin_bytes(c << bins_log2), 4 * cols + cols / 4 + 16);
-    if (lists) bytes = std::max(bytes, ((few + 1) / 2 + c * match_bucket(g) + 2) * 8);
+    if (lists) bytes = std::max(bytes, ((few + 1) / 2 + c * match_bucket(longs, g, partial) + 2) * 8);
     if (partial) bytes = std::max(bytes, cols * 8);
     return (bytes + 15) & ~15;
 }
@@ -585,10 +595,11 @@ __device__ __noinline__ void match_partial(int region_at, int r_mem, int r_arr, 
 
 // Wavefronts per SIMD that the registers are cut for.  The kernels compiled for a pattern gain from the most, whatever
 // they spill (4096 x 4096 fp16 2:4:4 with 5 / 7: 134 / 116 us); so do those of up to a wavefront per tile that take any pattern
-// (2:4:12 with 4 / 6: 136 / 125), which spill more where the columns are contiguous (1:8:8 with 5 / 6: 77 / 87).
+// (2:4:12 with 4 / 6: 136 / 125), which spill more where the columns are contiguous (1:8:8 with 5 / 6: 77 / 87), and tiles of two and four wavefronts
+// where they are not (six workgroups of a CU instead of five, 2000 x 3000 bf16 1:7:48 48 -> 42, 1024 x 1536 fp32 1:3:128 31 -> 27).
 constexpr int match_waves(int nt, bool compiled, bool rc)
 {
-    return nt > 256 ? 4 : compiled ? (nt == 256 ? 6 : nt == 64 ? 6 : 7) : nt > 64 ? 4 : rc ? 5 : 6;
+    return nt > 256 ? 4 : compiled ? (nt == 256 ? 6 : nt == 64 ? 6 : 7) : nt > 64 ? (rc ? 4 : 6) : rc ? 5 : 6;
 }
 
 // Columns of a tile per thread of its workgroup, up to a power of two.
@@ -1013,8 +1024,16 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                         if (k < few) pending[k] = (uint16_t)match_column(key[i]);
                     }
                 }
-            for (int p = tt; p < c; p += NT)
-                for (int s = s_occ[p]; s < g; s++) s_mem[p * g + s] = 0;
+            if (SG == 0 && NT >= 32 && g > 16) {      // (slot by slot in one thread a pattern 1:2:1000 took 740 us, 640 now)
+#pragma unroll 1
+                for (int s = tt; s < cols; s += NT) {
+                    const int p = group_of(s);
+                    if (s - p * g >= s_occ[p]) s_mem[s] = 0;
+                }
+            } else {
+                for (int p = tt; p < c; p += NT)
+                    for (int s = s_occ[p]; s < g; s++) s_mem[p * g + s] = 0;
+            }
             match_sync<NT>();
             pend = s_np[0];
         }
@@ -1024,7 +1043,8 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
             // order, and insert a proposal by one shift along the lanes.  A pattern takes at most `bucket` proposals in a round;
             // the rest stay pending.  In a tile of several wavefronts the first one ends the matching alone, without barriers.
             constexpr int EIGHT = 8, LL = SG > 16 && SC <= 8 ? 4 : 3, KPL = SG == 0 ? match_list_keys(NT, CPT) : SG > 8 << (LL - 2) ? 4 : 2;
-            const int ll = SG != 0 ? LL : Q.lanes_log2, L = 1 << ll, bucket = match_bucket(g);
+            const bool longs = SG == 0 && match_long(NT, CPT, g, real_rows < m);
+            const int ll = SG != 0 ? LL : Q.lanes_log2, L = 1 << ll, bucket = match_bucket(longs, g, real_rows < m);
             static_assert(SG <= 32 && SG != 1, "a list fits its lanes; lists and buckets fit the proposals' place");
             uint16_t *next = pending + few;
             uint64_t *s_bkt = s_arr + (few + 1) / 2;      // free places hold 0
@@ -1168,7 +1188,49 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                             s_occ[p] = min(had + asked, g);
                         }
                     };
-                    if constexpr (WAVES > 1) {
+                    // the same for a list that the lanes have no room for, by a wavefront: places by search, then everything moves there
+                    auto merge_long = [&](int p) {
+                        uint64_t *list = s_mem + p * g, *bkt = s_bkt + p * bucket;
+                        const int asked = __builtin_amdgcn_readfirstlane(min(s_dem[p], bucket)), had = __builtin_amdgcn_readfirstlane(s_occ[p]);
+                        const int refused = had + asked - g;
+                        int to = 0;
+                        if (lane == 0 && refused > 0) to = atomicAdd(count, refused);
+                        to = __builtin_amdgcn_readfirstlane(to) - g;
+                        const uint64_t mine = lane < asked ? bkt[lane] : 0;
+                        int above = 0;      // kept keys in front of the proposal
+                        for (int step = 1 << (31 - __clz(had | 1)); step > 0; step >>= 1)
+                            if (above + step <= had && list[above + step - 1] > mine) above += step;
+                        int at = above;
+                        for (int j = 0; j < asked; j++) {
+                            const uint64_t k = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(mine >> 32), j) << 32) |
+                                               (uint32_t)__builtin_amdgcn_readlane((int)mine, j);
+                            at += k > mine ? 1 : 0;
+                        }
+                        const int first = (int)~match_top<64>(~(uint32_t)above);
+                        for (int s0 = (had - 1) & ~63; s0 >= 0 && s0 + 63 >= first; s0 -= 64) {      // the last keys first
+                            const int s = s0 + lane;
+                            const uint64_t k = s < had ? list[s] : 0;
+                            int d = s;
+                            for (int j = 0; j < asked; j++) d += __builtin_amdgcn_readlane(above, j) <= s ? 1 : 0;
+                            if (s < had) {
+                                if (d < g) list[d] = k;
+                                else next[to + d] = (uint16_t)match_column(k);
+                            }
+                        }
+                        if (lane < asked) {
+                            if (at < g) list[at] = mine;
+                            else next[to + at] = (uint16_t)match_column(mine);
+                        }
+                        if (lane == 0) {
+                            s_dem[p] = 0;
+                            s_occ[p] = min(had + asked, g);
+                        }
+                    };
+                    if (longs) {
+                        if constexpr (W == 64)
+                            for (int p = wave; p < c; p += WAVES)
+                                if (__builtin_amdgcn_readfirstlane(s_dem[p]) != 0) merge_long(p);
+                    } else if constexpr (WAVES > 1) {
                         // a pattern to every list of lanes, in as many turns as that takes
                         for (int p = wave * rows + row; p < c; p += WAVES * rows)
                             if (s_dem[p] != 0) merge(p);
@@ -1329,16 +1391,18 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     int off = RC ? m * up(cols, V) * (int)sizeof(T) : up(cols * m * (int)sizeof(T), 16);
     Q.r_mem = off;
     off = up(off + cols * 8 + kMatchPad, 16);
-    // Lists that fit the lanes of a tile; longer ones, and tiles of 16 columns with more than four patterns, go through rounds over all columns
-    // to the end.  us, 4096 x 4096 fp16, rounds -> lists: 1:8:8 101 -> 62, 2:5:2 (20 columns) 275 -> 224, 1:4:4 (16) 104 -> 93, 2:8:1 314 -> 223,
-    // 4:8:1 824 -> 434, 2:4:160 211 -> 123, 1:8:256 165 -> 82; but 1:8:2 (16) 115 -> 126.
-    Q.lanes_log2 = Q.g > 64 * match_list_keys(NT, CPT) ? 0 : Q.g <= 16 ? 3 : Q.g <= 32 ? 4 : Q.g <= 64 ? 5 : 6;
+    // Tiles of 16 columns with more than four patterns go through rounds over all columns to the end, those of a wavefront and less also with lists
+    // that do not fit their lanes.  us, 4096 x 4096 fp16, rounds -> lists: 1:8:8 101 -> 62, 2:5:2 (20 columns) 275 -> 224, 1:4:4 (16) 104 -> 93, 2:8:1 314 -> 223,
+    // 4:8:1 824 -> 434, 2:4:160 211 -> 123, 1:8:256 165 -> 82; but 1:8:2 (16) 115 -> 126.  (1:8:2 109 and 113 along the two dims, 125 and 130 with pending columns only.)
+    Q.lanes_log2 = match_long(NT, CPT, Q.g, false) ? 6 : Q.g > 64 * match_list_keys(NT, CPT) ? 0 : Q.g <= 16 ? 3 : Q.g <= 32 ? 4 : Q.g <= 64 ? 5 : 6;
     if ((1 << Q.lanes_log2) > NT || (cols < 18 && c > 4)) Q.lanes_log2 = 0;
     Q.r_arr = off;
-    off += match_scratch(cols, c, Q.g, match_bins_log2(NT, c), SG != 0 || Q.lanes_log2 != 0, Q.view.S % m != 0, cols / match_few(SG));
+    off += match_scratch(match_long(NT, CPT, Q.g, Q.view.S % m != 0), cols, c, Q.g, match_bins_log2(NT, c), SG != 0 || Q.lanes_log2 != 0, Q.view.S % m != 0, cols / match_few(SG));
     Q.r_int = off;
     off = up(off + (kMatchTables * c + 4) * 4, 16);
-    constexpr int LDS = 160 * 1024, MOST = match_waves(NT, SM != 0, RC) * 4 / (THREADS / 64);      // workgroups that fit a CU's wavefronts
+    // workgroups that fit a CU's wavefronts (for tiles of several wavefronts four a SIMD, though six may fit: a partial block without
+    // the list costs more than the other two give, 2000 x 3000 bf16 2:7:20 94 -> 109)
+    constexpr int LDS = 160 * 1024, MOST = (NT > 64 && SM == 0 ? 4 : match_waves(NT, SM != 0, RC)) * 4 / (THREADS / 64);
     const int head = up(c * 8, 16);
     if (Q.view.S % m != 0) {
         // the classes of a partial block, and a list of its refused columns where that costs no workgroup of a CU (us, two workgroups without the

@@ -86,7 +86,8 @@ def test_two_wavefronts_per_tile(n, m, g, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
-@pytest.mark.parametrize("n,m,g", [(2, 4, 16), (1, 8, 32), (2, 8, 32), (3, 6, 12), (4, 8, 32), (2, 4, 8), (2, 4, 32), (2, 8, 8), (3, 8, 8)])
+@pytest.mark.parametrize("n,m,g", [(2, 4, 16), (1, 8, 32), (2, 8, 32), (3, 6, 12), (4, 8, 32), (2, 4, 8), (2, 4, 32), (2, 8, 8), (3, 8, 8),
+                                   (2, 4, 129), (1, 4, 257), (2, 4, 320)])
 def test_columns_that_want_the_same_patterns(n, m, g, dtype):
     # magnitudes that fall along the block: most columns propose to one pattern, lists and buckets run over, and the
     # refusals come in long chains; mild, so that the later rounds see them, and steep
@@ -216,11 +217,12 @@ def test_weights_that_are_no_numbers(n, m, g, dtype, bits, rest):
         assert same_bits(t.val.masked_fill(torch.isnan(t.val), math.inf), val)
 
 
-# Which later rounds a tile takes: lists of one key, of up to 128 and 256 (two and four to a lane), rounds over all columns beyond; tiles of 16, 18
-# and 20 columns; tiles of 48 and more columns on a quarter and on half of a wavefront.  Whole blocks and a partial one.
+# Which later rounds a tile takes: lists of one key, of up to 128 and 256 (two and four to a lane), of more, which stay in LDS, as all of more than 64 keys
+# do in a partial block of more than 256 columns; tiles of 16, 18 and 20 columns; tiles of 48 and more columns on a quarter and on half of a wavefront.  Whole blocks and a partial one.
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("n,m,g", [(1, 8, 2), (1, 2, 9), (2, 5, 2), (1, 4, 4), (1, 8, 4), (1, 6, 8), (1, 8, 8), (2, 6, 4), (3, 6, 3), (2, 8, 2), (2, 8, 1), (3, 6, 1),
-                                   (4, 8, 1), (1, 2, 128), (1, 2, 129), (2, 4, 160), (1, 8, 256), (1, 2, 257), (1, 4, 257)])
+                                   (4, 8, 1), (1, 2, 128), (1, 2, 129), (2, 4, 160), (1, 8, 256), (1, 2, 257), (1, 4, 257),
+                                   (1, 2, 1), (2, 5, 3), (1, 6, 3), (1, 4, 64), (1, 4, 65), (2, 5, 65), (3, 6, 100), (1, 2, 320), (1, 3, 700), (2, 4, 400)])
 @pytest.mark.parametrize("rest", [0, 1])
 def test_later_rounds_of_any_tile(n, m, g, dtype, rest):
     cols = math.comb(m, n) * g
