@@ -334,10 +334,10 @@ __global__ __launch_bounds__(256, 1) void sddmm16_kernel(SddmmParams P)
             const int tok = NT ? nt_tok : (((wave & 1) * 8 + i) << 1) + tok_hi;
             const unsigned char *src = tok < st.rem ? st.b + g_off[i] : zero;
             asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                         :: "v"(src), "s"(st.dst + i * 1024) : "memory");
+                         :: "v"(src), "s"(st.dst + i * 1024) : "memory", "m0");
         } else {
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         :: "v"(g_off[i]), "s"(st.b), "s"(st.dst + i * 1024) : "memory");
+                         :: "v"(g_off[i]), "s"(st.b), "s"(st.dst + i * 1024) : "memory", "m0");
         }
     };
 

@@ -416,7 +416,7 @@ __global__ __launch_bounds__(256, 1) void spmm_smfmac_direct_kernel(SmfParams P)
                     // (XT: left visible, the compiler makes the transposing reads of every step wait for all loads in flight)
                     if constexpr (XT)
                         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                                     :: "v"(x_off[q]), "s"(xb), "s"((uint32_t)(uintptr_t)(lds_ptr_t)(base + (wave * XL + q) * 1024)) : "memory");
+                                     :: "v"(x_off[q]), "s"(xb), "s"((uint32_t)(uintptr_t)(lds_ptr_t)(base + (wave * XL + q) * 1024)) : "memory", "m0");
                     else
                         __builtin_amdgcn_global_load_lds((glb_ptr_t)(xb + x_off[q]),
                                                          (lds_ptr_t)(base + (wave * XL + q) * 1024), 16, 0, 0);

@@ -1,6 +1,10 @@
 """The static check of hand-tracked loads (sten_amd/isa_check.py) on small synthetic kernels:
 it must see a register touched while its load is in flight, honour counted waits, carry the state
 of a loop into its next iteration, and tell spills inside a streaming loop from spills outside."""
+import glob
+import os
+import re
+
 from sten_amd import isa_check as C
 
 
@@ -208,3 +212,14 @@ def test_spill_among_outstanding_hand_issued_loads_is_reported():
 \tv_add_u32_e32 v1, v10, v11
 """)
     assert clean == []
+
+
+def test_statements_that_write_m0_say_so():
+    # the compiler keeps values of its own in that register (addresses of loads into LDS), and may put them there once for several loads
+    found = 0
+    for path in glob.glob(os.path.join(os.path.dirname(C.__file__), "csrc", "*.h*")):
+        for statement in re.findall(r"asm volatile\((.*?)\);", open(path).read(), re.S):
+            if re.search(r"\bs_mov_b32 m0\b", statement):
+                found += 1
+                assert re.search(r':[^:]*"m0"[^:]*$', statement), f"{os.path.basename(path)}: {statement}"
+    assert found > 0
