@@ -19,12 +19,19 @@ error.  This tool re-reads the device assembly the compiler produced and proves,
 by simulating the in-order vector-memory counter along every kernel (loop bodies are walked again
 with the state their back edge carries, so what a loop hands to its next iteration is checked too).
 
+The compressor places single vector instructions as statements and moves their results between lanes:
+there it proves that
+
+  * no move between lanes reads a register less than two wait states after such an instruction wrote
+    it, and no lane read less than one (the compiler keeps that distance for its own only).
+
     python -m sten_amd.isa_check                  # all sources that contain hand-issued loads
     python -m sten_amd.isa_check file.s --kernels dense_direct   # an assembly file made elsewhere
 
 Exit status 0 = clean.  ``sten_amd.build`` runs it after compiling.
 """
 import argparse
+import concurrent.futures
 import os
 import re
 import subprocess
@@ -44,6 +51,9 @@ CHECKED = {
     "nmg_sstream.hip": ["sstream_kernel"],
     "nmg_ostream.hip": ["ostream_kernel"],
 }
+
+# sources whose kernels place vector instructions as statements, without hand-tracked loads
+LANES = {src: ["match_kernel"] for src in ("nmg_match_f16.hip", "nmg_match_bf16.hip", "nmg_match_f32.hip", "nmg_match_fixed.hip")}
 
 REG = re.compile(r"\b([va])(\d+)\b|\b([va])\[(\d+):(\d+)\]")
 SREG = re.compile(r"\bs(\d+)\b|\bs\[(\d+):(\d+)\]")
@@ -97,6 +107,35 @@ def scalar_hazards(name, prog):
             first = inst.split(None, 1)[1].split(",")[0]
             for r in sregs_of(first):
                 age[r] = 0
+    return problems
+
+
+def lane_hazards(name, prog):
+    """A vector register written by an instruction statement must rest two wait states before a move
+    between lanes (DPP) reads it, and one before a lane read does; in layout order."""
+    problems = []
+    age = {}      # vector register -> wait states since a statement wrote it
+    for i, (kind, inst, by_hand) in enumerate(prog):
+        if kind != "inst":
+            continue
+        op, _, rest = inst.partition(" ")
+        operands = rest.split(",")
+        rest_states = 2 if "_dpp" in op else 1 if op.startswith(("v_readlane", "v_readfirstlane")) else 0
+        if rest_states and len(operands) > 1:
+            young = sorted(r for r in regs_of(operands[1]) if age.get(r, 99) < rest_states)
+            if young:
+                problems.append(f"{name[:60]} @{i}: `{inst}` reads {young[:4]} less than {rest_states} wait states after a "
+                                "statement's vector instruction wrote them")
+        states = int(operands[0], 0) + 1 if op == "s_nop" else 1
+        for r in list(age):
+            age[r] += states
+            if age[r] > 2:
+                del age[r]
+        if op.startswith("v_"):
+            for r in regs_of(operands[0]):
+                age.pop(r, None)
+                if by_hand:
+                    age[r] = 0
     return problems
 
 
@@ -280,13 +319,17 @@ def assembly_of(source):
         return open(out).read()
 
 
-def check_text(asm_text, wanted):
+def check_lanes(name, body):
+    return lane_hazards(name, parse(body))
+
+
+def check_text(asm_text, wanted, check=check_kernel):
     problems, checked = [], 0
     for name, body in kernels_of(asm_text).items():
         if not any(w in name for w in wanted):
             continue
         checked += 1
-        problems += check_kernel(name, body)
+        problems += check(name, body)
     return checked, problems
 
 
@@ -300,8 +343,11 @@ def main(argv=None):
         n, p = check_text(open(args.asm).read(), args.kernels or [""])
         total, problems = n, p
     else:
-        for source, wanted in CHECKED.items():
-            n, p = check_text(assembly_of(source), args.kernels or wanted)
+        todo = [(source, wanted, check) for table, check in ((CHECKED, check_kernel), (LANES, check_lanes)) for source, wanted in table.items()]
+        with concurrent.futures.ThreadPoolExecutor(4) as pool:
+            texts = list(pool.map(assembly_of, [source for source, _, _ in todo]))
+        for (_, wanted, check), text in zip(todo, texts):
+            n, p = check_text(text, args.kernels or wanted, check)
             total += n
             problems += p
     for p in problems:

@@ -214,6 +214,24 @@ def test_spill_among_outstanding_hand_issued_loads_is_reported():
     assert clean == []
 
 
+def test_move_between_lanes_right_behind_a_statement():
+    def lanes(body):
+        return C.check_lanes("_Zk", body.strip("\n").split("\n"))
+
+    statement = """
+\t;;#ASMSTART
+\tv_max_f64 v[4:5], v[6:7], v[8:9]
+\t;;#ASMEND
+"""
+    move = "\tv_mov_b32_dpp v10, v5 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+    assert len(lanes(statement + move)) == 1
+    assert len(lanes(statement + "\ts_nop 0\n" + move)) == 1
+    assert lanes(statement + "\ts_nop 1\n" + move) == []
+    assert lanes(statement + "\tv_mov_b32_e32 v5, v1\n" + move) == []      # the compiler's own result: its own distance
+    assert len(lanes(statement + "\tv_readlane_b32 s2, v4, 3\n")) == 1
+    assert lanes(statement + "\ts_nop 0\n\tv_readlane_b32 s2, v4, 3\n") == []
+
+
 def test_statements_that_write_m0_say_so():
     # the compiler keeps values of its own in that register (addresses of loads into LDS), and may put them there once for several loads
     found = 0
