@@ -151,7 +151,8 @@ int nmg_spmm_smfmac(const void *d_fp_val, const void *d_fp_idx, int64_t M, int64
  * column), B [K, T] and C [M, T] row-major with leading dimensions ldb / ldc: what
  * torch.mm(W, B) asks for, without a transposing copy on either side (the tile of B is fetched as
  * it lies in memory and transposed by the LDS transpose reads of gfx950).  Large-batch kernel,
- * 256 lines x 128 columns per workgroup, any T; K % 64 == 0, ldb % 8 == 0, B 16-byte aligned.
+ * 128 lines x 128 columns per workgroup, 256 x 128 or 256 x 256 by the extents, any T; K % 64 == 0, ldb % 8 == 0,
+ * B 16-byte aligned.  Every row of B is read in whole pieces of 8 columns, the last one too.
  * Replaces: nmg_mult(..., transpose_b=True, transpose_c=True), dace_gnm_mult.py:572-627, whose
  * generated code makes the transposing copies of :813-915. */
 int nmg_spmm_smfmac_tt(const void *d_fp_val, const void *d_fp_idx, int64_t M, int64_t K, const void *d_b,
@@ -281,7 +282,7 @@ int nmg_spmm_densefrag(const void *d_df, int64_t O, int64_t K, const void *d_x, 
                        int64_t ldy, const void *d_bias, int64_t T, int dtype, int variant, void *stream);
 /* C[O, T] = A * B (+ bias[o] on row o) for B [K, T] and C as they lie in memory (row pitches ldb,
  * ldc), A given as densefrag: the dense-matrix-core product with both dense operands transposed.
- * K % 64 == 0, ldb % 8 == 0, B 16-byte aligned, ldb < 2^24.
+ * K % 64 == 0, ldb % 8 == 0, B 16-byte aligned, ldb < 2^24; tiles and reads of B as nmg_spmm_smfmac_tt.
  * No counterpart in the reference (its operators have no backward): this is the gradient with
  * respect to B of torch.mm(W, B), W^T * grad_out, taken without transposing copies; same
  * transpose_b / transpose_c meaning as dace_gnm_mult.py:572-627. */

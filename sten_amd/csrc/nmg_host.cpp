@@ -780,8 +780,11 @@ Tensor tt_split(State &w, const Tensor &b, int rd)
     return N % 8 == 0 ? transposed(y, N) : y.t().contiguous();
 }
 
+// The kernels read whole pieces of 8 columns, also in the last row: those of a view whose storage ends before must not be read as they lie.
 bool tt_as_it_lies(const Tensor &b)
 {
+    const int64_t end = b.storage_offset() + (b.size(0) - 1) * b.stride(0) + round_up(b.size(1), 8);
+    if (b.size(1) % 8 != 0 && end * b.element_size() > (int64_t)b.storage().nbytes()) return false;
     return b.stride(1) == 1 && b.stride(0) % 8 == 0 && b.stride(0) >= b.size(1) && aligned16(b) && b.stride(0) < (int64_t(1) << 24);
 }
 

@@ -48,6 +48,27 @@ def test_torch_mm_as_it_lies(R, C, N, dtype):
     check(sten.spmm_tt_dense(w, Gy, reduce_dim=0), Wd.t(), Gy, dtype, "dense cores, transposed weight")
 
 
+# A last row that ends with the storage, inside a piece of 8 columns, is not read as it lies.
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [17, 30, 133])
+def test_storage_that_ends_with_the_last_row(N):
+    w, B, _ = operands(256, 128, N, torch.float16)
+    pitch = B.stride(0)
+    short = torch.empty(127 * pitch + N, device=DEV, dtype=torch.float16).as_strided((128, N), (pitch, 1))
+    short.copy_(B)
+    print(f"case tt short storage N={N}", flush=True)
+    sten.spmm_tt(w, short), sten.spmm_tt_dense(w, short, reduce_dim=1)      # (packs the operands)
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        c, d = sten.spmm_tt(w, short), sten.spmm_tt_dense(w, short, reduce_dim=1)
+        torch.cuda.synchronize()
+    check(c, w.to_dense(), B, torch.float16, "sparse cores")
+    check(d, w.to_dense(), B, torch.float16, "dense cores")
+    names = [e.name for e in p.events() if "nmg::" in e.name]
+    if names:      # a copy and a product each
+        assert len(names) == 4, names
+
+
 # Which tiles those extents take: outputs and columns as (sparse, dense) kernels name them.
 @pytest.mark.gpu
 @pytest.mark.parametrize("R,N,C,sparse,dense", [
