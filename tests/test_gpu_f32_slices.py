@@ -3,7 +3,9 @@ import ctypes
 
 import pytest
 import torch
+from torch.profiler import ProfilerActivity, profile
 
+import sten_amd as sten
 from sten_amd import native
 
 DEV = "cuda:0"
@@ -102,3 +104,72 @@ def test_the_plan_leaves_no_slice_empty_and_sizes_its_workspace():
     assert 1 in seen and len(seen) > 3
     assert L.nmg_gemm_f32_plan(8, 8, -1, 8, 8, 0, ctypes.byref(slices), ctypes.byref(size)) != 0
     assert L.nmg_gemm_f32_plan(8, 8, 8, 8, 8, 3, ctypes.byref(slices), ctypes.byref(size)) != 0
+
+
+def _sums_of_slices(call):
+    """The call's result, and how many of its products came in slices (None where the profiler reports no kernels)."""
+    call()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        out = call()
+        torch.cuda.synchronize()
+    names = [e.name for e in p.events() if "nmg::" in e.name]
+    return out, sum("splitk_sum_kernel<float" in n for n in names) if names else None
+
+
+def _close(got, ref, name):
+    assert got.shape == ref.shape
+    assert ((got.double() - ref).norm() / ref.norm()).item() <= BOUND, name
+    # every element: BOUND of the root mean square is a standard deviation of those roundings, eight of them
+    assert (got.double() - ref).abs().max().item() <= 8 * BOUND * ref.pow(2).mean().sqrt().item(), name
+
+
+# The public calls whose products are in slices, one of the three in each case: forward with a bias, gradient of the input, of the weight, and the
+# same of torch.mm; operands with a pitch and an offset of their own, whole extents and odd ones.
+@pytest.mark.gpu
+@pytest.mark.parametrize("O,K,T", [(768, 3072, 1024), (3072, 768, 1024), (768, 1024, 3072), (767, 3071, 1021), (3071, 767, 1021), (767, 1021, 3071)])
+def test_public_calls_in_slices(O, K, T):
+    print(f"case f32 slices, public calls O={O} K={K} T={T}", flush=True)
+    g = torch.Generator(DEV).manual_seed(O)
+    lin = torch.nn.Linear(K, O, device=DEV)
+    with torch.no_grad():
+        lin.weight.copy_(torch.randn(O, K, device=DEV, generator=g))
+        lin.bias.copy_(torch.randn(O, device=DEV, generator=g))
+    sb = sten.SparsityBuilder()
+    sb.set_weight("weight", initial_sparsifier=sten.GroupedNMSparsifier(2, 4, 16, sparse_dim=1, group_dim=0), out_format=sten.GroupedNMTensor)
+    lin = sb.sparsify_model_inplace(lin)
+    W = lin.weight.wrapped_tensor.to_dense().double()
+
+    def strided(rows, cols):
+        wide = torch.randn(rows, cols + 6, device=DEV, generator=g)
+        return wide[:, 3:3 + cols]
+
+    x, gy = strided(T, K), strided(T, O)
+
+    def train():
+        lin.zero_grad(set_to_none=True)
+        leaf = x.detach().requires_grad_(True)
+        y = lin(leaf)
+        y.backward(gy)
+        return y.detach(), leaf.grad, lin.weight.grad.wrapped_tensor.to_dense()
+
+    (y, gx, gw), sums = _sums_of_slices(train)
+    assert sums in (None, 1), "the plan gives no slices: other extents"
+    _close(y, x.double() @ W.t() + lin.bias.detach().double(), "linear")
+    _close(gx, gy.double() @ W, "gradient of the input")
+    _close(gw, gy.double().t() @ x.double(), "gradient of the weight")
+
+    b, gc = strided(K, T), strided(O, T)
+
+    def mm():
+        lin.zero_grad(set_to_none=True)
+        leaf = b.detach().requires_grad_(True)
+        c = torch.mm(lin.weight, leaf)
+        c.backward(gc)
+        return c.detach(), leaf.grad, lin.weight.grad.wrapped_tensor.to_dense()
+
+    (c, gb, gw), sums = _sums_of_slices(mm)
+    assert sums in (None, 1), "the plan gives no slices: other extents"
+    _close(c, W @ b.double(), "mm")
+    _close(gb, W.t() @ gc.double(), "gradient of B")
+    _close(gw, gc.double() @ b.double().t(), "gradient of the weight of mm")
