@@ -631,8 +631,8 @@ struct GemmF32Params {
 // XKM: the same for the activation-side operand, X[K, T] (Y = X^T * A: the weight gradient of a
 // linear layer from the upstream gradient and the activations as they lie).
 // LOADS: what a step's loads may meet -- whole tiles and aligned rows only; the ends of the operands in any step; in the last
-// steps only (a loop of its own for the steps before).
-enum { F32_ALIGNED, F32_ANY, F32_ENDS };
+// steps only (a loop of its own for the steps before, whose loads the compiler counts or, DRAINED, waits for altogether).
+enum { F32_ALIGNED, F32_ANY, F32_ENDS, F32_ENDS_DRAINED };
 template <int WM, int WN, int WK, int MI, int NJ, int LOADS, bool AKM, bool XKM>
 __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
 {
@@ -853,12 +853,12 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
         }
     };
     int st = 0;
-    if constexpr (LOADS == F32_ENDS) {
+    if constexpr (LOADS >= F32_ENDS) {
         const int whole = (XKM && P.T < 4) || (AKM && P.O < 4) ? 0 : (int)(P.K / BKT);
         // The guarded loads of the first tiles stand behind branches, and the compiler cannot count them: without this wait for them (vmcnt(0),
         // nothing else) the loop waits for every load in flight once a turn.  us, without -> with: both operands reduction-major 1280 x 512,
-        // K 3690 130 -> 93, 1664 x 512, K 1381 46 -> 38, 640 x 2432, K 423 28.7 -> 26.4, one 376 x 511, K 3296 30.4 -> 26.4; none, no difference.
-        if (AKM && st + 4 < whole) __builtin_amdgcn_s_waitcnt(0x0f70);
+        // K 3690 130 -> 93, 1664 x 512, K 1381 46 -> 38, 640 x 2432, K 423 28.7 -> 26.4, one 376 x 511, K 3296 33.0 -> 27.5; none, no difference.
+        if (LOADS == F32_ENDS && AKM && st + 4 < whole) __builtin_amdgcn_s_waitcnt(0x0f70);
         for (; st + 4 < whole; st += 2) {
             step(st, F0, F1, G1, true, true, std::true_type{});
             step(st + 1, F1, F0, G0, true, true, std::true_type{});
@@ -931,6 +931,10 @@ static void launch_gemm_f32(const GemmF32Params &Q, int form, hipStream_t st)
     // K 3071 37.5 -> 33.5, 36 x 221, K 1618 15.0 -> 12.2.  With both operands reduction-major 512 x 2432, K 237 18.7 -> 16.8, 2839 x 422,
     // K 252 19.7 -> 17.7, 100 x 1444, K 773 14.3 -> 14.1; on fewer steps fetching the second loop's code costs more.
     const bool ends = Q.K >= 8 * BKT;
+    // One operand reduction-major: counted loads gain where a CU has one workgroup (32 x 32 tiles 0.975 of the time, 64 x 64 0.935, 128 x 64 0.965),
+    // but a second one covers the wait as well and counting has its price: 2085 x 209, K 2566 (462 tiles of 32 x 32) 44.3 -> 48.6, 897 x 405, K 2598
+    // 42.8 -> 45.8, and on tiles of 128 x 96 2783 x 3328, K 256 57.5 -> 67.0.
+    constexpr bool DRAINED = (BM == 128 && BN == 96) || BM == 32;
 #define NMG_F32_LAUNCH(LOADS_, AKM_, XKM_) \
     hipLaunchKernelGGL((gemm_nt_f32_kernel<WM, WN, WK, MI, NJ, LOADS_, AKM_, XKM_>), grid, dim3(256), 0, st, Q)
     if (form == 0) {
@@ -938,7 +942,8 @@ static void launch_gemm_f32(const GemmF32Params &Q, int form, hipStream_t st)
         else NMG_F32_LAUNCH(F32_ENDS, false, false);
     } else if (form == 1) {
         if (fast) NMG_F32_LAUNCH(F32_ALIGNED, true, false);
-        else NMG_F32_LAUNCH(F32_ENDS, true, false);
+        else if (DRAINED && (BM != 32 || (int64_t)grid.x * grid.y > 256)) NMG_F32_LAUNCH((DRAINED ? F32_ENDS_DRAINED : F32_ENDS), true, false);
+        else NMG_F32_LAUNCH((BM != 32 && DRAINED ? F32_ENDS_DRAINED : F32_ENDS), true, false);
     } else {
         if (fast) NMG_F32_LAUNCH(F32_ALIGNED, true, true);
         else if (ends) NMG_F32_LAUNCH(F32_ENDS, true, true);

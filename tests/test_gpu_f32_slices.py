@@ -56,11 +56,12 @@ def test_slices_against_fp64(form, O, K, T, slices, pad):
 
 
 # Whole products with ends inside steps and groups of four: one step fewer than the loop for whole steps takes, as many, and several
-# turns of it, on tiles of 32 x 32 (steps of 64), 64 x 64 (16) and larger ones.  On the fp32 instruction sums are rounded once per 2 positions.
+# turns of it, on tiles of 32 x 32 (steps of 64; up to one and more than one a CU), 64 x 64 (16) and larger ones, 128 x 96 among them.  On the fp32 instruction sums are rounded once per 2 positions.
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", [0, 1, 2])
 @pytest.mark.parametrize("O,K,T", [(36, 511, 221), (37, 513, 222), (36, 1618, 221), (1001, 127, 640), (1000, 131, 641), (1000, 383, 639),
-                                   (383, 263, 1281), (2664, 279, 263), (1283, 515, 510)])
+                                   (383, 263, 1281), (2664, 279, 263), (1283, 515, 510),
+                                   (2085, 515, 209), (1652, 145, 1576)])
 def test_whole_products_with_ends_against_fp64(form, O, K, T):
     print(f"case f32 ends form={form} O={O} K={K} T={T}", flush=True)
     A, X, a, x = _operands(form, O, K, T, 0)
