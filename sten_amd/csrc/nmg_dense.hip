@@ -1107,20 +1107,23 @@ extern "C" int nmg_gemm_f32_plan(int64_t lda, int64_t ldx, int64_t O, int64_t K,
     // (below 2^28 multiplications slices gained nothing, and the models take a tenth of a microsecond that a small call would see)
     if ((double)O * (double)K * (double)T < 268435456.0 || gemm_f32_few(O, T, form)) return NMG_OK;
     // Against the time on the fp32 instruction, which the model above puts too high or too low here, by form and tile (276 products of 2^27 to
-    // 2^33 multiplications with at most 140 tiles of 128 x 128, all forms, odd extents among them, in every number of slices: with this choice
-    // they take 0.933 of the time of whole ones, with the best 0.926, one of them more than 1 % longer than whole, 25.9 -> 26.6).  us, whole ->
-    // slices: 960 x 584 results over 4076, both operands reduction-major 98 -> 50, 1024 x 1024 over 4096 74.5 -> 59, 1021 x 1999 over 2047
+    // 2^33 multiplications with at most 140 tiles of 128 x 128, all forms, odd extents among them, in every number of slices; 8 to 12 %
+    // for what the models are off: 840 others of up to 2^32.5 that it cuts take 0.69 of the time of whole ones, six of
+    // them are more than 1 % longer, 24.0 -> 28.3 the most).  us, whole -> slices: 960 x 584 results over 4076, both operands reduction-major 98 -> 50, 1024 x 1024 over 4096 74.5 -> 59, 1021 x 1999 over 2047
     // 85 -> 66, 768 x 2673 over 3200 108 -> 83; below about 30 us the two launches cost more than they save (1024 x 176 over 1152: 9.8, 19.8).
     int shape, best;
     const double us = split3_plan(lda, ldx, O, K, T, form, &best);
-    const bool even = lda % 4 == 0 && ldx % 4 == 0;
-    const double fixed = 4.75, model = gemm_f32_us(O, K, T, form, even, &shape) - fixed;
-    const bool guards = !(even && K % 32 == 0 && O % 4 == 0 && (form < 2 || T % 4 == 0));
+    const bool even = lda % 4 == 0 && ldx % 4 == 0, rows = even && (form < 1 || O % 4 == 0) && (form < 2 || T % 4 == 0);
+    const double fixed = 4.75;
+    double model = gemm_f32_us(O, K, T, form, even, &shape) - fixed;
+    // (the model has guards for every K that is no multiple of 32; tiles that walk in steps of 16 have none for multiples of 16)
+    const bool short_steps = shape != 3 && shape != 5 && K % 16 == 0, guards = !(rows && (K % 32 == 0 || short_steps));
+    if (rows && K % 32 != 0 && short_steps) model /= 1.2;
     const double share = form == 0 ? (shape == 5 ? 0.7 : 1.0)
-                         : form == 1 ? (shape == 5 ? 0.85 : shape == 4 ? (guards ? 0.95 : 1.2) : 1.0)
+                         : form == 1 ? (shape == 5 ? 0.85 : shape == 4 ? (guards ? 0.95 : 1.05) : 1.0)
                                      : (guards ? 1.15 : 1.0);
     const double whole = fixed + model * share;
-    if (best > 1 && us < 0.95 * whole) {
+    if (best > 1 && us < (form == 2 && shape == 5 ? 0.88 : 0.92) * whole) {
         *slices = best;
         *workspace_bytes = best * T * ((O + 3) / 4 * 4) * 4;
     }
