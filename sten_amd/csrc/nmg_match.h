@@ -198,15 +198,15 @@ constexpr int match_bin_bytes(int bins) { return (4 + bins + 4) * 4; }      // a
 // last); then the waiting columns, flags and runs of the closed form; a partial block's proposals.  One after the other in the same place: 2:8:32 takes
 // 25.8 KB a tile of fp16 instead of 29.5, six workgroups of a CU instead of five.
 constexpr int match_few(int sg) { return sg != 0 ? 4 : 2; }
-// Keys of a list that a lane holds where g is not compiled in: 64 lanes hold lists of 128, with four keys a lane 256.  Tiles of two wavefronts
-// have a kernel for each (told apart by the columns a thread has room for): us, 4096 x 4096 fp16, two keys a lane -> four: 2:4:64 108 -> 113, 2:8:16 101 -> 105;
-// rounds -> lists of four keys a lane: 1:2:150 257 -> 205, 1:3:140 204 -> 141.
-constexpr int match_list_keys(int nt, int cpt) { return nt >= 256 || (nt == 128 && cpt > 4) ? 4 : 2; }
+// Keys of a list that a lane holds where g is not compiled in: 64 lanes hold lists of 128, with four keys a lane 256 (us, 4096 x 4096 fp16, tiles of two
+// wavefronts, two keys a lane -> four: 2:4:64 108 -> 113, 2:8:16 101 -> 105).
+constexpr int match_list_keys(int nt) { return nt >= 256 ? 4 : 2; }
 // Longer lists stay in LDS, a wavefront moves their keys (us, 4096 x 4096 fp16, rounds over all columns ->
-// this: 1:4:300 297 -> 168, 2:4:400 298 -> 142, 1:8:257 160 -> 80, 1:2:1000 1205 -> 640).  It takes many proposals at a time for what a shift along the lanes does with eight, which a partial block gains from with lists
-// of more than 64 keys: its columns want the same few patterns (2000 x 3000 bf16, blocks along the slow dim, 3:6:100 202 -> 125, 3:6:128 293 -> 152).
-// Whole blocks of up to 256 keys are faster in the lanes (7:8:160 106, 116; 2:6:100 125, 139).
-constexpr bool match_long(int nt, int cpt, int g, bool partial) { return nt >= 128 && g > (partial ? 64 : 64 * match_list_keys(nt, cpt)); }
+// this: 1:4:300 297 -> 168, 2:4:400 298 -> 142, 1:8:257 160 -> 80, 1:2:1000 1205 -> 640).  It takes many proposals at a time for what a shift along
+// the lanes does with eight, which a partial block gains from with lists of more than 64 keys: its columns want the same few patterns (2000 x 3000 bf16, blocks along the slow dim, 3:6:100 202 -> 125, 3:6:128 293 -> 152).
+// Whole blocks of up to 256 keys are faster in the lanes (7:8:160 106, 116; 2:6:100 125, 139), but two or three patterns take eight proposals each
+// in many rounds there (512 x 640 fp16 1:2:160 20.4 -> 17.4, 1:2:256 26.2 -> 20.6).
+constexpr bool match_long(int nt, int c, int g, bool partial) { return nt >= 128 && g > (partial || c <= 3 ? 64 : 64 * match_list_keys(nt)); }
 // Proposals that a pattern takes in a later round: what has room where the closed form, a first round's bins (short lists) or a partial block's
 // proposals lie anyway.  With one for lists of up to three keys 1:6:3 was slower than by rounds, 178 against 157; 150 with three, 2:8:2 167 -> 159.
 constexpr int match_bucket(bool longs, int g, bool partial)
@@ -1038,12 +1038,12 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
             pend = s_np[0];
         }
 
-        if (lists) {
+        if (lists && pend > 0) {
             // Later rounds: a few columns, whatever the pattern.  L lanes hold a pattern's list, KPL keys each in descending
             // order, and insert a proposal by one shift along the lanes.  A pattern takes at most `bucket` proposals in a round;
             // the rest stay pending.  In a tile of several wavefronts the first one ends the matching alone, without barriers.
-            constexpr int EIGHT = 8, LL = SG > 16 && SC <= 8 ? 4 : 3, KPL = SG == 0 ? match_list_keys(NT, CPT) : SG > 8 << (LL - 2) ? 4 : 2;
-            const bool longs = SG == 0 && match_long(NT, CPT, g, real_rows < m);
+            constexpr int EIGHT = 8, LL = SG > 16 && SC <= 8 ? 4 : 3, KPL = SG == 0 ? match_list_keys(NT) : SG > 8 << (LL - 2) ? 4 : 2;
+            const bool longs = SG == 0 && match_long(NT, c, g, real_rows < m);
             const int ll = SG != 0 ? LL : Q.lanes_log2, L = 1 << ll, bucket = match_bucket(longs, g, real_rows < m);
             static_assert(SG <= 32 && SG != 1, "a list fits its lanes; lists and buckets fit the proposals' place");
             uint16_t *next = pending + few;
@@ -1394,10 +1394,10 @@ static int match_launch(MatchParams &Q, hipStream_t stream, bool *done)
     // Tiles of 16 columns with more than four patterns go through rounds over all columns to the end, those of a wavefront and less also with lists
     // that do not fit their lanes.  us, 4096 x 4096 fp16, rounds -> lists: 1:8:8 101 -> 62, 2:5:2 (20 columns) 275 -> 224, 1:4:4 (16) 104 -> 93, 2:8:1 314 -> 223,
     // 4:8:1 824 -> 434, 2:4:160 211 -> 123, 1:8:256 165 -> 82; but 1:8:2 (16) 115 -> 126.  (1:8:2 109 and 113 along the two dims, 125 and 130 with pending columns only.)
-    Q.lanes_log2 = match_long(NT, CPT, Q.g, false) ? 6 : Q.g > 64 * match_list_keys(NT, CPT) ? 0 : Q.g <= 16 ? 3 : Q.g <= 32 ? 4 : Q.g <= 64 ? 5 : 6;
+    Q.lanes_log2 = match_long(NT, c, Q.g, false) ? 6 : Q.g > 64 * match_list_keys(NT) ? 0 : Q.g <= 16 ? 3 : Q.g <= 32 ? 4 : Q.g <= 64 ? 5 : 6;
     if ((1 << Q.lanes_log2) > NT || (cols < 18 && c > 4)) Q.lanes_log2 = 0;
     Q.r_arr = off;
-    off += match_scratch(match_long(NT, CPT, Q.g, Q.view.S % m != 0), cols, c, Q.g, match_bins_log2(NT, c), SG != 0 || Q.lanes_log2 != 0, Q.view.S % m != 0, cols / match_few(SG));
+    off += match_scratch(match_long(NT, c, Q.g, Q.view.S % m != 0), cols, c, Q.g, match_bins_log2(NT, c), SG != 0 || Q.lanes_log2 != 0, Q.view.S % m != 0, cols / match_few(SG));
     Q.r_int = off;
     off = up(off + (kMatchTables * c + 4) * 4, 16);
     // workgroups that fit a CU's wavefronts (for tiles of several wavefronts four a SIMD, though six may fit: a partial block without
@@ -1461,7 +1461,7 @@ template <typename T, bool RC> static int match_dispatch(MatchParams &Q, hipStre
     if (Q.cols <= 128 && Q.c <= (Q.cols > 64 ? 20 : 60)) return match_launch<T, 32, 4, 0, 0, 0, RC>(Q, stream, done);
     if (Q.cols <= 256) return match_launch<T, 64, 4, 0, 0, 0, RC>(Q, stream, done);
     if (Q.cols <= 512) {
-        const int rc = Q.g > 128 ? match_launch<T, 128, 5, 0, 0, 0, RC>(Q, stream, done) : match_launch<T, 128, 4, 0, 0, 0, RC>(Q, stream, done);
+        const int rc = match_launch<T, 128, 4, 0, 0, 0, RC>(Q, stream, done);
         if (rc != NMG_OK || *done) return rc;
     }
     if (Q.cols <= 1024) return match_launch<T, 256, 4, 0, 0, 0, RC>(Q, stream, done);
