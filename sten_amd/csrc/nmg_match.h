@@ -159,6 +159,13 @@ template <int X> __device__ __forceinline__ uint32_t match_lane_xor(uint32_t v)
 // An edge's score (31 bits) and pattern as a positive double that is no NaN for any score.  (With the score as the high word those from 0x7FF00000
 // on, which a weight that is no number may give, would be NaNs, and the maximum below drops them.)
 __device__ __forceinline__ uint64_t match_edge(uint32_t score, uint32_t p) { return ((uint64_t)(score >> 1) << 32) | ((score << 31) | p); }
+// Whether a pattern's positions are n from a multiple of n on.
+constexpr bool match_run(int mask, int n)
+{
+    for (int at = 0; at + n <= 8; at += n)
+        if (mask == ((1 << n) - 1) << at) return true;
+    return false;
+}
 __device__ __forceinline__ uint32_t match_edge_score(uint64_t edge) { return (uint32_t)(edge >> 31); }
 __device__ __forceinline__ int match_edge_pattern(uint64_t edge) { return (int)(edge & 0xFFu); }
 
@@ -619,6 +626,11 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int SC = SM ? match_binom(SM, SN) : 0;
+    // Where whole patterns make up a column, their sums, compared with themselves once a tile, find weights that are no numbers; columns of such a tile compare whole numbers, and
+    // edges have the score itself as their high word.  us, NaNs out of order -> all edges shifted (match_edge) -> this, 4096 x 4096 fp16: 3:6:12
+    // 61.0 -> 62.6 -> 61.1, 4:8:32 73.9 -> 77.5 -> 73.4, 2:8:32 47.2 -> 48.7 -> 47.3, 2:4:16 51.3 -> 52.0 -> 51.6.  (2:4 with a g that is not compiled in
+    // has no registers for the sums: 2:4:4 1024 x 1536 fp32 17.4 -> 17.8.)
+    constexpr bool RAW = SG != 0 && SN > 1 && SM % (SN ? SN : 1) == 0;
     constexpr int THREADS = NT <= 64 ? 256 : NT;
     constexpr int TILES = THREADS / NT;
     constexpr int KPT = match_keys(NT, CPT);
@@ -791,10 +803,32 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
     auto group_of = [&](int s) { return SG ? s / SG : (int)(((uint64_t)s * Q.magic_g) >> 32); };
     auto at = [&](int o, int r) { return RC ? r * ldc + o : o * m + r; };
 
+    bool odd = false;      // RAW: a column of the tile has a weight that is no number
+    float sums = 0;        // RAW: of this thread's columns
+    // Proposal of a column of such a tile: whole numbers are compared.
+    auto propose_odd = [&](int o, auto thr_tag) __attribute__((always_inline)) -> uint64_t {
+        uint32_t best = 0;
+        int bp = 0;
+#pragma unroll 1
+        for (int p = 0; p < SC; p++) {
+            const uint32_t ps = s_pos[p];
+            float acc = match_abs(s_d[at(o, (int)(ps & 15u))]);
+#pragma unroll 1
+            for (int j = 1; j < SN; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
+            const uint32_t sb = __float_as_uint(acc);
+            if (sb >= best && (!decltype(thr_tag)::value || match_key(sb, o, p) > s_mem[p * g + g - 1])) {
+                best = sb;
+                bp = p;
+            }
+        }
+        return best == 0 ? 0 : match_key(best, o, bp);
+    };
     // Proposal of column o: its best pattern among those with room or a last key below the column's (the
     // larger pattern on equal scores); 0 where no such pattern has a positive score.  THR = false: all have room.
     auto propose = [&](int o, auto thr_tag) __attribute__((always_inline)) -> uint64_t {      // (a call takes addresses that say no more that they lie in LDS)
         constexpr bool THR = decltype(thr_tag)::value;
+        if constexpr (RAW && THR)
+            if (odd) return propose_odd(o, thr_tag);
         float a[8];
         if (!RC && sizeof(T) == 2 && SM == 8) {
             const uint4 raw = *(const uint4 *)(s_d + o * 8);
@@ -812,36 +846,11 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 #pragma unroll
             for (int r = 0; r < 8; r++) a[r] = r < m ? match_abs(s_d[at(o, r)]) : 0.f;
         }
-        // Many patterns: the score itself is the high word, and a column with a weight that could make it a NaN compares whole numbers (us, shifted
-        // edges -> this, 4096 x 4096 fp16: 4:8:32 77.5 -> 75.0, 2:8:32 48.8 -> 48.0; with the NaNs out of order 74.2, 47.3).  With few of them the
-        // test for it costs more than the shifts (1:8:16 57.5 -> 59.0, 7:8:12 66.5 -> 68.1).
-        constexpr bool RAW = SC > 8;
-        if constexpr (RAW) {
-            uint32_t largest = __float_as_uint(a[0]);
-#pragma unroll
-            for (int r = 1; r < SM; r++) largest = max(largest, __float_as_uint(a[r]));
-            if (__builtin_expect(largest >= 0x7FF00000u, 0)) {
-                uint32_t best = 0;
-                int bp = 0;
-#pragma unroll 1
-                for (int p = 0; p < SC; p++) {
-                    const uint32_t ps = s_pos[p];
-                    float acc = match_abs(s_d[at(o, (int)(ps & 15u))]);
-#pragma unroll 1
-                    for (int j = 1; j < SN; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
-                    const uint32_t sb = __float_as_uint(acc);
-                    if (sb >= best && (!THR || match_key(sb, o, p) > s_mem[p * g + g - 1])) {
-                        best = sb;
-                        bp = p;
-                    }
-                }
-                return best == 0 ? 0 : match_key(best, o, bp);
-            }
-        }
         uint64_t best = 0;
         int later = 0;
         uint32_t zero = 0;      // not to be known for one: the patterns' numbers would take a register each for all columns
         if constexpr (RAW) asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+        float whole = 0;      // of the column
         auto consider = [&](float acc, int p) {
             uint32_t sb = __float_as_uint(acc);
             if (THR) {
@@ -852,6 +861,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
         };
         if constexpr (SM != 0) {
             constexpr MatchMasks<SN ? SN : 1, SM ? SM : 1> tab;
+            bool some = false;
 #pragma unroll
             for (int p = 0; p < SC; p++) {
                 float acc = 0;
@@ -863,6 +873,10 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                         any = true;
                     }
                 consider(acc, p);
+                if (RAW && match_run(tab.mask[p], SN)) {
+                    whole = some ? whole + acc : acc;
+                    some = true;
+                }
                 // all sums and thresholds in flight at once would not fit the registers
                 if (SC > 8 && p % 8 == 7) {
                     if (THR) asm volatile("" : "+v"(later), "+v"(best));
@@ -883,6 +897,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                 }
             }
         }
+        if (RAW && !THR) sums += whole;
         const uint32_t score = RAW ? (uint32_t)(best >> 32) : match_edge_score(best);
         return score == 0 ? 0 : match_key(score, o, match_edge_pattern(best));
     };
@@ -908,6 +923,19 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
 #pragma unroll
                 for (int i = 0; i < CPT; i++) own[i] = tt + NT * i < real_cols ? s_arr[tt + NT * i] : 0;
             }
+            if (RAW) {
+                uint32_t top = 0;
+                for (int s = tt; s < cols; s += NT) top = max(top, (uint32_t)(s_mem[s] >> 16));
+                top = match_top<(NT < 64 ? NT : 64)>(top);
+                if constexpr (NT > 64) {
+                    if (tt == 0) s_start[0] = 0;
+                    __syncthreads();
+                    if ((tt & 63) == 0) atomicMax((unsigned *)s_start, top);
+                    __syncthreads();
+                    top = ((unsigned *)s_start)[0];
+                }
+                odd = top > 0x7F800000u;
+            }
             round = 1;
         }
         for (; round < limit && pend > (round == 0 ? 0 : few); round++) {
@@ -919,6 +947,14 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                     const uint64_t key = propose(e, std::false_type{});
                     s_mem[e] = key;
                     top = max(top, (uint32_t)(key >> 16));
+                }
+                if (RAW && __builtin_expect(sums != sums, 0)) {
+#pragma unroll 1
+                    for (int e = tt; e < real_cols; e += NT) {
+                        const uint64_t key = propose_odd(e, std::false_type{});
+                        s_mem[e] = key;
+                        top = max(top, (uint32_t)(key >> 16));
+                    }
                 }
 #pragma unroll
                 for (int i = 0; i < CPT; i++) own[i] = tt + NT * i < real_cols ? s_mem[tt + NT * i] : 0;      // this thread's own entries
@@ -948,6 +984,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                 __syncthreads();
                 top = ((unsigned *)s_bin)[-4];
             }
+            if (RAW) odd = odd || top > 0x7F800000u;      // (every such column proposes with such a score, which the lists keep before all others)
             // 2. counting sort by pattern and score
             auto bin_of = [&](uint64_t key) {
                 return (match_pattern(key) << nbl2) + (int)min((top - (uint32_t)(key >> 16)) >> (24 - nbl2), (1u << nbl2) - 1);
@@ -1090,7 +1127,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                         for (int j = 1; j < n; j++) acc += match_abs(s_d[at(o, (int)((ps >> (4 * j)) & 15u))]);
                         uint32_t sb = __float_as_uint(acc);
                         if (!(match_key(sb, o, p) > s_mem[p * g + g - 1])) sb = 0;
-                        return match_edge(sb, (uint32_t)p);
+                        return RAW ? ((uint64_t)sb << 32) | (uint32_t)p : match_edge(sb, (uint32_t)p);
                     };
                     auto other = [&](uint64_t top, auto ctrl) {      // the larger one of two lanes
                         asm("s_nop 1" : "+v"(top));
@@ -1102,7 +1139,7 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                     // A column's patterns over EL lanes, or a column per lane, which is less work where there are enough columns for it: in
                     // tiles of a wavefront from a quarter of the lanes on (us, 4096 x 4096 3:6:12 from 16 / 32 / never: 61.3 / 63.3 / 63.7), with
                     // many patterns from twice as many as lanes on (4:8:32 from 32 / 1024: 85 / 73).
-                    if (SG != 0 && (A <= 64 ? pend <= A / 4 : SC <= 32 || pend <= 2 * A)) {
+                    if (SG != 0 && !odd && (A <= 64 ? pend <= A / 4 : SC <= 32 || pend <= 2 * A)) {
                         const int sub = tt % EL;
                         for (int e = tt / EL; e < pend; e += A / EL) {
                             const int o = (int)pending[e];
@@ -1115,7 +1152,8 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                             top = other(top, by_1);
                             if (EL >= 4) top = other(top, by_2);
                             if (EL >= 8) top = other(top, by_4);
-                            if (sub == 0) put(o, match_edge_score(top) == 0 ? 0 : match_key(match_edge_score(top), o, match_edge_pattern(top)));
+                            const uint32_t score = RAW ? (uint32_t)(top >> 32) : match_edge_score(top);
+                            if (sub == 0) put(o, score == 0 ? 0 : match_key(score, o, match_edge_pattern(top)));
                         }
                     } else if (SG == 0 && c > 8 && pend * EIGHT <= A) {
                         const int e = tt / EIGHT, sub = tt % EIGHT;
@@ -1130,7 +1168,8 @@ __global__ __launch_bounds__(NT <= 64 ? 256 : NT, match_waves(NT, SM != 0, RC)) 
                             top = other(top, by_1);
                             top = other(top, by_2);
                             top = other(top, by_4);
-                            if (sub == 0) put(o, match_edge_score(top) == 0 ? 0 : match_key(match_edge_score(top), o, match_edge_pattern(top)));
+                            const uint32_t score = RAW ? (uint32_t)(top >> 32) : match_edge_score(top);
+                            if (sub == 0) put(o, score == 0 ? 0 : match_key(score, o, match_edge_pattern(top)));
                         }
                     } else {
                         for (int e = tt; e < pend; e += A) {
