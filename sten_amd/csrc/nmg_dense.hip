@@ -857,7 +857,7 @@ __global__ __launch_bounds__(256) void gemm_nt_f32_kernel(GemmF32Params P)
         const int whole = (XKM && P.T < 4) || (AKM && P.O < 4) ? 0 : (int)(P.K / BKT);
         // The guarded loads of the first tiles stand behind branches, and the compiler cannot count them: without this wait for them (vmcnt(0),
         // nothing else) the loop waits for every load in flight once a turn.  us, without -> with: both operands reduction-major 1280 x 512,
-        // K 3690 130 -> 93, 1664 x 512, K 1381 46 -> 38, 640 x 2432, K 423 28.7 -> 26.4, one 376 x 511, K 3296 33.0 -> 27.5; none, no difference.
+        // K 3690 116 -> 92, 1664 x 512, K 1381 48 -> 39, 640 x 2432, K 423 29.4 -> 25.2, one 511 x 376, K 3296 32.7 -> 27.6; none, no difference.
         if (LOADS == F32_ENDS && AKM && st + 4 < whole) __builtin_amdgcn_s_waitcnt(0x0f70);
         for (; st + 4 < whole; st += 2) {
             step(st, F0, F1, G1, true, true, std::true_type{});

@@ -23,15 +23,15 @@
 // A quarter of the columns and fewer (any n:m:g: half) insert into the lists lane by lane, into long ones key by key (the code says how).
 //
 // us, 4096 x 4096 fp16 with the blocks along the contiguous / the slow dim (8192 x 8192 for 2:8:32), batched walk -> ranks among all
-// proposals of a pattern -> this: 2:4:16 99 -> 58 / 57 -> 50 / 50, 1:8:32 37 -> 31, 3:6:12 75 / 73 -> 61 / 59, 2:8:32 727 -> 182 / 190 -> 138 / 147,
-// 4:8:32 390 -> 128 / 124 -> 73 / 73; any n:m:g: 2:4:4 168 / 231 -> 110 / 109 -> 87, 2:4:8 115 / 146 -> 71 -> 57, 2:4:32 118 / 135 -> 104 / 114 ->
-// 93 / 103, 2:4:64 130 / 146 -> 113 / 124 -> 107, 1:2:8 192 / 302 -> 143 / 138 -> 132, 2:8:8 293 / 326 -> 130 / 134 -> 102, 1:8:8 86 / 117 -> 79 -> 63, 4:8:16 870 / 810 ->
-// 280 / 293 -> 220 / 228, 2:4:100 144 / 160 -> 130.  What each part gave, 2:8:32: bins 43 -> 20 us of the first round, score and pattern compared as one
-// double 17 -> 7 (a select behind a select on the same condition takes 17 to 40 clocks, a 64-bit maximum 4), the sorted keys in the place of the lists (six
-// workgroups a CU instead of five) 168 -> 150, the reads of a column's patterns in flight together 150 -> 145.  4:8:32: 125 -> 102, and 73 where the
-// later rounds are inlined: in a function their addresses are not known to lie in LDS.  Of the 147 us of 2:8:32 now, tile data and results
-// take 39 to 45, first proposals 10, the first round 25, the later ones 68: chains of LDS round trips and the issue of vector instructions,
-// 1500 a wavefront.
+// proposals of a pattern -> this: 2:4:16 99 -> 59 / 58 -> 51.5 / 51.5, 1:8:32 39 / 41 -> 32 / 34, 3:6:12 77 / 73 -> 63 / 61, 2:8:32 727 -> 195 / 197 -> 146 / 150,
+// 4:8:32 390 -> 120 / 114 -> 75 / 74; any n:m:g: 2:4:4 168 / 231 -> 111 / 110 -> 90, 2:4:8 115 / 146 -> 72 -> 59, 2:4:32 118 / 135 -> 104 / 114 ->
+// 94 / 104, 2:4:64 130 / 146 -> 115 / 123 -> 98 / 107, 1:2:8 192 / 302 -> 148 / 139 -> 137 / 130, 2:8:8 293 / 326 -> 131 / 133 -> 101 / 104, 1:8:8 86 / 117 -> 76 -> 60,
+// 4:8:16 870 / 810 -> 280 / 295 -> 233 / 239, 2:4:100 144 / 162 -> 121 / 135.  What each part gave, 2:8:32: bins 43 -> 20 us of the first round, score and pattern
+// compared as one double 17 -> 7 (a select behind a select on the same condition takes 17 to 40 clocks, a 64-bit maximum 4), the sorted keys in the place of the
+// lists (six workgroups a CU instead of five) 168 -> 150, the reads of a column's patterns in flight together 150 -> 145.  4:8:32: 125 -> 102, and 73 where the
+// later rounds are inlined: in a function their addresses are not known to lie in LDS.  Of the 151 us of 2:8:32 along the slow dim tile data and results
+// take 50, first proposals 14, the first round 20, the later ones 67, of the 54 of 2:4:16 (same box) 16, 5, 12 and 21: chains of LDS round trips and the issue
+// of vector instructions, 1500 and 1105 a wavefront.
 //
 // Columns that have no pattern with room and a positive score wait.  In the walk they come last, together
 // with the zero columns beyond the end of the group dim, in descending column order, and each takes the
